@@ -45,7 +45,8 @@ void launch_watpol(hipStream_t st, int nblk, int B, const DevSys* dsys, const in
   hipLaunchKernelGGL(k_watpol_force, g, t, 0, st, dsys);
   hipLaunchKernelGGL(k_watpol_finish, dim3(B), dim3(64), 0, st, dsys);
 }
-__global__ void k_reduce_energies(const DevSys*, int, int);
+__global__ void k_reduce_part(const DevSys*);
+__global__ void k_reduce_final(const DevSys*, int, int);
 __global__ void k_atom_terms(const DevSys*, uint32_t, const double*);
 
 static thread_local std::string g_err;
@@ -450,6 +451,7 @@ int instance_alloc(DevSys& S, DevAlloc& M, const qnb_params* p, int nslots) {
   AL(nq_lists, 2);
   S.nslots = nslots;
   AL(epart, (size_t)QNB_NE * nslots);
+  AL(ered_part, (size_t)QNB_NE * QNB_RED_BLOCKS);
   AL(ered, QNB_NE);
   AL(eatom, 2 * (size_t)nat);
   AL(sh_state, 3 * QNB_MAXSH);
@@ -693,7 +695,8 @@ static void launch_eval(qnb_handle* h, uint32_t mask) {
   const int with_pol = S.nwat > 0 && S.wpol && S.nshell > 0 && (mask & QNB_T_POL);
   if (with_qq) hipLaunchKernelGGL((k_qq<R, NS>), dim3(1), dim3(QQ_THREADS), 0, h->stream, h->dsys, mask);
   if (with_pol) launch_watpol(h->stream, (S.nwat + WP_THREADS - 1) / WP_THREADS, 1, h->dsys, (const int*)h->d_istep);
-  hipLaunchKernelGGL(k_reduce_energies, dim3(1), dim3(1024), 0, h->stream, h->dsys, with_qq, with_pol);
+  hipLaunchKernelGGL(k_reduce_part, dim3(QNB_RED_BLOCKS, 1), dim3(256), 0, h->stream, h->dsys);
+  hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(256), 0, h->stream, h->dsys, with_qq, with_pol);
 }
 
 template <typename R>

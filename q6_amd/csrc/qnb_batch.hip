@@ -29,7 +29,7 @@ __global__ void k_qforces(const DevSys*, uint32_t, int, double*, int);
 template <typename R, int NS>
 __global__ void k_qq(const DevSys*, uint32_t);
 void launch_watpol(hipStream_t st, int nblk, int B, const DevSys* dsys, const int* istep);
-__global__ void k_reduce_energies(const DevSys*, int, int);
+__global__ void k_reduce_part(const DevSys*);
 __global__ void k_atom_terms(const DevSys*, uint32_t, const double*);
 
 // per-instance MD record
@@ -475,9 +475,13 @@ __global__ void k_snap(const DevSys* __restrict__ systems, const MdDev* __restri
   for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) dst[k] = S.x[k];
 }
 
-__global__ void k_record(const DevSys* __restrict__ systems, const MdDev* __restrict__ mds) {
+// `energy`: the step's energy partials were reduced (k_reduce_part); their
+// second pass runs here, before the record that holds them
+__global__ __launch_bounds__(256) void k_record(const DevSys* __restrict__ systems, const MdDev* __restrict__ mds,
+                                                int energy, int with_qq, int with_pol) {
   const DevSys& S = systems[blockIdx.x];
   const MdDev& M = mds[blockIdx.x];
+  if (energy && want_energies(S)) reduce_final(S, with_qq, with_pol);
   const int step = *M.istep;
   if (threadIdx.x == 0 && M.xs_every > 0 && step % M.xs_every == 0 && M.ctr[2] < M.xs_max) M.ctr[2] += 1;
   if (M.ene_every <= 0 || step % M.ene_every != 0) return;
@@ -749,11 +753,12 @@ static void enqueue_step(qnb_batch* b, bool lists, bool energy) {
   if (b->anyqb) launch_qbonded(b->stream, B, b->dsys, b->dqb);
   // the reduction and the record do nothing on a step no instance samples
   // (energy is false only then); the record also counts stored snapshots
-  if (energy)
-    hipLaunchKernelGGL(k_reduce_energies, dim3(B), dim3(1024), 0, b->stream, b->dsys, (int)b->anyq, (int)b->anypol);
+  if (energy) hipLaunchKernelGGL(k_reduce_part, dim3(QNB_RED_BLOCKS, B), dim3(256), 0, b->stream, b->dsys);
   if (b->anysnap)
     hipLaunchKernelGGL(k_snap, dim3((3 * b->maxat + 255) / 256, B), dim3(256), 0, b->stream, b->dsys, b->dmd);
-  if (energy || b->anysnap) hipLaunchKernelGGL(k_record, dim3(B), dim3(64), 0, b->stream, b->dsys, b->dmd);
+  if (energy || b->anysnap)
+    hipLaunchKernelGGL(k_record, dim3(B), dim3(256), 0, b->stream, b->dsys, b->dmd, (int)energy, (int)b->anyq,
+                       (int)b->anypol);
   if (energy && b->exc_threads > 0)
     hipLaunchKernelGGL(k_exc_record, dim3((b->exc_threads + 63) / 64, B), dim3(64), 0, b->stream, b->dsys, b->dmd,
                        (const ExcDev*)b->dexc);

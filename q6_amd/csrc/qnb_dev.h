@@ -27,6 +27,8 @@ enum {
   E_Q0  // then per state s: qq_el, qq_vdw, qp_el, qp_vdw, qw_el, qw_vdw at E_Q0 + 6*s
 };
 #define QNB_NE (E_Q0 + 6 * QNB_MAXST)
+// blocks per system of the energy reduction's first pass (k_reduce_part)
+#define QNB_RED_BLOCKS 64
 
 struct DevSys {
   // sizes
@@ -155,6 +157,7 @@ struct DevSys {
   int* nq_lists;    // [2]: n_qw, n_qp
   double* epart;    // [nslots][QNB_NE]
   int nslots;
+  double* ered_part;  // [QNB_RED_BLOCKS][QNB_NE] partial sums of k_reduce_part
   double* ered;     // [QNB_NE]
   double* eatom;    // [natom][2]: per-atom LRF and radial-restraint energies
   // polarisation restraint state
@@ -416,6 +419,29 @@ __device__ __forceinline__ void store_energy_record(double* ep, const double (&p
     if (lane == slot[j]) v = vj;
   }
   if (lane < QNB_NE) *(__attribute__((address_space(1))) double*)(ep + lane) = v;
+}
+
+// Second pass of the energy reduction, one block of 256 threads: lane k of
+// wave c adds energy k of every fourth partial from c on, wave 0 adds the four
+// sums, the Q-Q record and the polarisation record, and writes ered.
+__device__ __forceinline__ void reduce_final(const DevSys& S, int with_qq, int with_pol) {
+  __shared__ double part[4][QNB_WAVE];
+  const int k = threadIdx.x % QNB_WAVE, c = threadIdx.x / QNB_WAVE;
+  double s = 0.0;
+  if (k < QNB_NE) {
+    const auto p = gp(S.ered_part);
+#pragma unroll
+    for (int g = 0; g < QNB_RED_BLOCKS / 4; g++) s += p[(size_t)(c + 4 * g) * QNB_NE + k];
+  }
+  part[c][k] = s;
+  __syncthreads();
+  if (c == 0 && k < QNB_NE) {
+    double t = ((part[0][k] + part[1][k]) + part[2][k]) + part[3][k];
+    if (with_qq && S.nqat > 0) t += S.epart[(size_t)S.ncgp * QNB_NE + k];
+    if (with_pol && S.nwat > 0 && S.wpol && S.nshell > 0) t += S.epart[(size_t)(S.ncgp + 1) * QNB_NE + k];
+    S.ered[k] = t;
+  }
+  __syncthreads();
 }
 
 // group contributions (calculate_exc): one pair of an energy array's list,

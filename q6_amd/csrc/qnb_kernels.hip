@@ -1959,48 +1959,52 @@ __global__ __launch_bounds__(64) void k_watpol_finish(const DevSys* __restrict__
 }
 
 // ---------------------------------------------------------------------------
-// Fixed-order reduction of the per-wave energy partials: wave c of the block
-// sums slots [c*n/16, (c+1)*n/16) with lane k on energy k (a wave reads one
-// 57-double slot per iteration), then thread k adds the 16 chunk sums in
-// order.  Runs on the sampled steps only.
-#define QNB_RED_CHUNKS 16
-__global__ __launch_bounds__(64 * QNB_RED_CHUNKS) void k_reduce_energies(const DevSys* __restrict__ systems,
-                                                                        int with_qq, int with_pol) {
-  const DevSys& S = systems[blockIdx.x];
+// Fixed-order reduction of the energy partials on the sampled steps, in two
+// passes: block g of QNB_RED_BLOCKS per system sums its share of the per-wave
+// records (a wave reads one 57-double record per iteration, lane k on energy
+// k) and of the per-atom LRF and radial energies into ered_part[g]; one block
+// per system then adds the QNB_RED_BLOCKS partials (reduce_final, qnb_dev.h;
+// the MD step does that inside k_record).  The records are written all over
+// the chip, so each read is a miss in this CU's caches and the pass is bound
+// by how many reads are in flight: one block of 1,024 threads per system,
+// whose thread 0 also added 1,024 atom sums in turn, took 68 us for 2,752
+// records and 11,056 atoms; with 64 blocks and the final pass a whole
+// evaluation of that system takes 62 us less (344 to 281 us).
+__global__ __launch_bounds__(256) void k_reduce_part(const DevSys* __restrict__ systems) {
+  const DevSys& S = systems[blockIdx.y];
   if (!want_energies(S)) return;
-  __shared__ double part[QNB_RED_CHUNKS][QNB_WAVE];
-  const int k = threadIdx.x % QNB_WAVE, c = threadIdx.x / QNB_WAVE;
-  const int n = S.ncgp, a0 = (int)((long)n * c / QNB_RED_CHUNKS), a1 = (int)((long)n * (c + 1) / QNB_RED_CHUNKS);
+  const int g = blockIdx.x, lane = threadIdx.x % QNB_WAVE, c = threadIdx.x / QNB_WAVE;
+  constexpr int NP = 4 * QNB_RED_BLOCKS;  // waves of a system
+  const int p = 4 * g + c;
+  const auto ep = gp(S.epart);
+  const int a0 = (int)((long)S.ncgp * p / NP), a1 = (int)((long)S.ncgp * (p + 1) / NP);
   double s = 0.0;
-  if (k < QNB_NE)
-    for (int a = a0; a < a1; a++) s += S.epart[(size_t)a * QNB_NE + k];
-  part[c][k] = s;
-  // per-atom LRF and radial-restraint energies: thread t sums a contiguous
-  // atom range, then the ranges are added in order
-  __shared__ double apart[64 * QNB_RED_CHUNKS][2];
-  {
-    const int t = threadIdx.x, nt = blockDim.x;
-    const int i0 = (int)((long)S.natom * t / nt), i1 = (int)((long)S.natom * (t + 1) / nt);
-    double l = 0.0, r = 0.0;
-    for (int i = i0; i < i1; i++) {
-      l += S.eatom[2 * i];
-      r += S.eatom[2 * i + 1];
-    }
-    apart[t][0] = l;
-    apart[t][1] = r;
+  if (lane < QNB_NE) {
+#pragma unroll 4
+    for (int a = a0; a < a1; a++) s += ep[(size_t)a * QNB_NE + lane];
   }
+  const auto ea = gp(S.eatom);
+  const int i0 = (int)((long)S.natom * p / NP), i1 = (int)((long)S.natom * (p + 1) / NP);
+  double l = 0.0, r = 0.0;
+  for (int i = i0 + lane; i < i1; i += QNB_WAVE) {
+    l += ea[2 * i];
+    r += ea[2 * i + 1];
+  }
+  l = wave_sum(l);
+  r = wave_sum(r);
+  if (lane == E_LRF) s += l;
+  if (lane == E_RAD) s += r;
+  __shared__ double part[4][QNB_WAVE];
+  part[c][lane] = s;
   __syncthreads();
-  if (c == 0 && k < QNB_NE) {
-    double t = 0.0;
-    for (int m = 0; m < QNB_RED_CHUNKS; m++) t += part[m][k];
-    if (k == E_LRF || k == E_RAD) {
-      const int col = k == E_LRF ? 0 : 1;
-      for (int m = 0; m < (int)blockDim.x; m++) t += apart[m][col];
-    }
-    if (with_qq && S.nqat > 0) t += S.epart[(size_t)S.ncgp * QNB_NE + k];
-    if (with_pol && S.nwat > 0 && S.wpol && S.nshell > 0) t += S.epart[(size_t)(S.ncgp + 1) * QNB_NE + k];
-    S.ered[k] = t;
-  }
+  if (c == 0 && lane < QNB_NE)
+    stg(S.ered_part + (size_t)g * QNB_NE + lane, ((part[0][lane] + part[1][lane]) + part[2][lane]) + part[3][lane]);
+}
+
+// the second pass alone (single-system evaluations)
+__global__ __launch_bounds__(256) void k_reduce_final(const DevSys* __restrict__ systems, int with_qq, int with_pol) {
+  const DevSys& S = systems[blockIdx.x];
+  if (want_energies(S)) reduce_final(S, with_qq, with_pol);
 }
 
 // explicit instantiations used by the host code
