@@ -32,18 +32,16 @@ __global__ void k_qq(const DevSys*, uint32_t);
 __global__ void k_pack_xq(const DevSys*);
 __global__ void k_pw_first(const DevSys*);
 __global__ void k_watpol_theta(const DevSys*, const int*);
-__global__ void k_watpol_rank(const DevSys*);
 __global__ void k_watpol_force(const DevSys*);
 __global__ void k_watpol_finish(const DevSys*);
 
-// SCAAS polarisation restraint: theta and shells, ranks, forces (blocks of
-// WP_THREADS waters, grid.y the instance), then the per-system sums
-void launch_watpol(hipStream_t st, int nblk, int B, const DevSys* dsys, const int* istep) {
-  const dim3 g(nblk, B), t(WP_THREADS);
-  hipLaunchKernelGGL(k_watpol_theta, g, t, 0, st, dsys, istep);
-  hipLaunchKernelGGL(k_watpol_rank, dim3(QNB_MAXSH, B), dim3(WP_RANK_THREADS), 0, st, dsys);
-  hipLaunchKernelGGL(k_watpol_force, g, t, 0, st, dsys);
-  hipLaunchKernelGGL(k_watpol_finish, dim3(B), dim3(64), 0, st, dsys);
+// SCAAS polarisation restraint: angles and shells, then ranks and forces
+// (grid.y the instance); `finish`: the per-system sums too, where no later
+// kernel of the caller runs them
+void launch_watpol(hipStream_t st, int nwat, int B, const DevSys* dsys, const int* istep, bool finish) {
+  hipLaunchKernelGGL(k_watpol_theta, dim3((nwat + WP_THREADS - 1) / WP_THREADS, B), dim3(WP_THREADS), 0, st, dsys, istep);
+  hipLaunchKernelGGL(k_watpol_force, dim3(nwat / WP_WATERS + QNB_MAXSH, B), dim3(256), 0, st, dsys);
+  if (finish) hipLaunchKernelGGL(k_watpol_finish, dim3(B), dim3(64), 0, st, dsys);
 }
 __global__ void k_reduce_part(const DevSys*);
 __global__ void k_reduce_final(const DevSys*, int, int);
@@ -457,11 +455,10 @@ int instance_alloc(DevSys& S, DevAlloc& M, const qnb_params* p, int nslots) {
   AL(sh_state, 3 * QNB_MAXSH);
   AL(w_theta, nw1);
   AL(w_shell, nw1);
-  AL(w_rank, nw1);
   AL(sh_list, (size_t)QNB_MAXSH * nw1);
   AL(sh_lth, (size_t)QNB_MAXSH * nw1);
   AL(sh_n, QNB_MAXSH);
-  AL(wp_part, (size_t)(1 + QNB_MAXSH) * ((nw1 + WP_THREADS - 1) / WP_THREADS));
+  AL(wp_rank, 2 * (size_t)QNB_MAXSH * nw1);
 
 #undef AL
   double sh0[3 * QNB_MAXSH] = {0};
@@ -694,7 +691,7 @@ static void launch_eval(qnb_handle* h, uint32_t mask) {
   const int with_qq = S.nqat > 0 && (mask & (QNB_T_QQ | QNB_T_QQP));
   const int with_pol = S.nwat > 0 && S.wpol && S.nshell > 0 && (mask & QNB_T_POL);
   if (with_qq) hipLaunchKernelGGL((k_qq<R, NS>), dim3(1), dim3(QQ_THREADS), 0, h->stream, h->dsys, mask);
-  if (with_pol) launch_watpol(h->stream, (S.nwat + WP_THREADS - 1) / WP_THREADS, 1, h->dsys, (const int*)h->d_istep);
+  if (with_pol) launch_watpol(h->stream, S.nwat, 1, h->dsys, (const int*)h->d_istep, false);
   hipLaunchKernelGGL(k_reduce_part, dim3(QNB_RED_BLOCKS, 1), dim3(256), 0, h->stream, h->dsys);
   hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(256), 0, h->stream, h->dsys, with_qq, with_pol);
 }

@@ -164,11 +164,10 @@ struct DevSys {
   double* sh_state;  // [3*QNB_MAXSH]: theta_corr, avtheta, avn_insh
   double* w_theta;   // [nwat]
   int* w_shell;      // [nwat]
-  int* w_rank;       // [nwat] rank of the water in its shell
   int* sh_list;      // [QNB_MAXSH][nwat] members of each shell
   double* sh_lth;    // [QNB_MAXSH][nwat] their theta
   int* sh_n;         // [QNB_MAXSH] members per shell
-  double* wp_part;   // [ceil(nwat / WP_THREADS)][1 + QNB_MAXSH] per-block sums
+  double* wp_rank;   // [QNB_MAXSH][nwat][2] restraint energy and theta of each member, by rank
   // energy sampling: energies are accumulated when ene_every <= 0 or when
   // the instance's step counter is a multiple of ene_every
   const int* step_ptr;
@@ -421,6 +420,37 @@ __device__ __forceinline__ void store_energy_record(double* ep, const double (&p
   if (lane < QNB_NE) *(__attribute__((address_space(1))) double*)(ep + lane) = v;
 }
 
+// shell members per block of the polarisation-restraint force kernel
+#define WP_WATERS 64
+__device__ __forceinline__ bool has_pol(const DevSys& S) { return S.nwat > 0 && S.wpol && S.nshell > 0; }
+// restraint energy (c = 0) or theta (c = 1) of shell is, added over its n
+// members by one wave (every lane active): lane l takes ranks l, l + 64, ...,
+// then a fixed tree
+__device__ __forceinline__ double watpol_sum(const DevSys& S, int is, int n, int c) {
+  const auto p = gp(S.wp_rank + 2 * (size_t)is * S.nwat);
+  double v = 0.0;
+#pragma unroll 4
+  for (int k = threadIdx.x % QNB_WAVE; k < n; k += QNB_WAVE) v += p[2 * (size_t)k + c];
+  return wave_sum(v);
+}
+
+// Last phase of the polarisation restraint, one wave per system: accumulates
+// avtheta and avn_insh and clears the shell counts for the
+// next step's angle kernel.
+__device__ __forceinline__ void watpol_finish(const DevSys& S) {
+  if (!has_pol(S)) return;
+  for (int is = 0; is < S.nshell; is++) {
+    const int n = ldg(S.sh_n + is);
+    if (n == 0) continue;
+    const double s = watpol_sum(S, is, n, 1);
+    if (threadIdx.x % QNB_WAVE == 0) {
+      S.sh_n[is] = 0;
+      S.sh_state[QNB_MAXSH + is] += s / (double)n;
+      S.sh_state[2 * QNB_MAXSH + is] += (double)n;
+    }
+  }
+}
+
 // Second pass of the energy reduction, one block of 256 threads: lane k of
 // wave c adds energy k of every fourth partial from c on, wave 0 adds the four
 // sums, the Q-Q record and the polarisation record, and writes ered.
@@ -434,11 +464,17 @@ __device__ __forceinline__ void reduce_final(const DevSys& S, int with_qq, int w
     for (int g = 0; g < QNB_RED_BLOCKS / 4; g++) s += p[(size_t)(c + 4 * g) * QNB_NE + k];
   }
   part[c][k] = s;
+  __shared__ double pol;
+  if (c == 1 && with_pol && has_pol(S)) {
+    double e = 0.0;
+    for (int is = 0; is < S.nshell; is++) e += watpol_sum(S, is, ldg(S.sh_n + is), 0);
+    if (k == 0) pol = e;
+  }
   __syncthreads();
   if (c == 0 && k < QNB_NE) {
     double t = ((part[0][k] + part[1][k]) + part[2][k]) + part[3][k];
     if (with_qq && S.nqat > 0) t += S.epart[(size_t)S.ncgp * QNB_NE + k];
-    if (with_pol && S.nwat > 0 && S.wpol && S.nshell > 0) t += S.epart[(size_t)(S.ncgp + 1) * QNB_NE + k];
+    if (k == E_POL && with_pol && has_pol(S)) t += pol;
     S.ered[k] = t;
   }
   __syncthreads();
@@ -752,13 +788,10 @@ inline int qforces_blocks(int nq, int chunks, int W) { return 8 * ((chunks + W -
 
 // threads of the Q-Q kernel's block (one block per system)
 #define QQ_THREADS 1024
-// threads per block of the polarisation-restraint kernels (one per water)
+// polarisation restraint: threads per block of the angle kernel (one per
+// water); shell members staged in LDS at a time by the force kernel
 #define WP_THREADS 256
-// threads of a polarisation-shell rank block (k_watpol_rank loops over any
-// shell size with this stride; the launch uses the same value)
-#ifndef WP_RANK_THREADS
-#define WP_RANK_THREADS 1024
-#endif
+#define WP_CHUNK 1024
 
 #define FC_WPB 8
 #ifndef FC_CAP

@@ -1726,14 +1726,12 @@ __device__ __forceinline__ void wat_vectors(const DevSys& S, int i, double* rmu,
   for (int c = 0; c < 3; c++) rcu[c] = v[c] / rc;
 }
 
-__device__ __forceinline__ bool has_pol(const DevSys& S) { return S.nwat > 0 && S.wpol && S.nshell > 0; }
-
 // Phase 1, one thread per water: theta and shell (-1: inside the innermost
 // shell, or excluded); the members of each shell are appended to its list
 // (slot order is immaterial: ranks are counted by value).  Block 0 first
 // applies the theta_corr feedback of the steps that are multiples of itdis
 // (nonbondene.f90:6653-6666).  The shell counts start at zero (set at
-// creation and cleared by phase 4).
+// creation and cleared by watpol_finish).
 __global__ __launch_bounds__(WP_THREADS) void k_watpol_theta(const DevSys* __restrict__ systems,
                                                              const int* __restrict__ istep) {
   const DevSys& S = systems[blockIdx.y];
@@ -1775,8 +1773,8 @@ __global__ __launch_bounds__(WP_THREADS) void k_watpol_theta(const DevSys* __res
   stg(S.w_theta + w, th);
   stg(S.w_shell + w, sh);
   // append to the shell lists with one atomic per (wave, shell): the lanes of
-  // a shell take consecutive places (k_watpol_rank orders each shell by
-  // (theta, water index), so the order of appending does not matter)
+  // a shell take consecutive places (ranks are counted by (theta, water index),
+  // so the order of appending does not matter)
   const int lane = t % QNB_WAVE;
   int pending = sh;
   for (;;) {
@@ -1797,165 +1795,99 @@ __global__ __launch_bounds__(WP_THREADS) void k_watpol_theta(const DevSys* __res
   }
 }
 
-// Phase 2, one block per (shell, system): the rank of every member in the
-// shell's stable ascending order of theta (the reference's selection sort;
-// ties by water index).  Shells of up to WP_SORT members are sorted by
-// (theta, water index) with a bitonic network in LDS and the rank is the
-// sorted position; larger shells count, for every member, the members
-// before it (staged through LDS in chunks of WP_SORT).
-#define WP_SORT 4096
-__global__ __launch_bounds__(WP_RANK_THREADS) void k_watpol_rank(const DevSys* __restrict__ systems) {
+// Phase 2, WP_WATERS members of one shell per block, four waves on the same
+// members: each member's rank in its shell's stable ascending order of theta
+// (the reference's selection sort; ties by water index) is the number of
+// members before it, counted against the shell's list staged in LDS, a quarter
+// of it per wave; wave 0 then forms the target angle from the rank, the
+// restraint energy and the forces (adds to d), and writes energy and theta at
+// the member's rank (wp_rank), so the sums over a shell do not depend on the
+// order the angle kernel appended its members in.  Counting is n^2 compares,
+// but over all blocks it is a few microseconds of latency at n = 700, where
+// one block per shell running a bitonic network over its 55 steps took 14-23
+// us and was a launch of its own.  Blocks take the members of one shell, not
+// the waters in index order, so a wave counts one list: the index order, where
+// every block holds every shell, cost 51 windows of 2,352 waters 22 us per
+// step more.
+__global__ __launch_bounds__(256) void k_watpol_force(const DevSys* __restrict__ systems) {
   const DevSys& S = systems[blockIdx.y];
-  const int sh = blockIdx.x;
-  if (!has_pol(S) || sh >= S.nshell) return;
-  __shared__ double c_th[WP_SORT];
-  __shared__ int c_w[WP_SORT];
-  const int t = threadIdx.x, nw = S.nwat;
-  const int n = S.sh_n[sh];
-  const int* L = S.sh_list + (size_t)sh * nw;
-  const double* Lth = S.sh_lth + (size_t)sh * nw;
-  if (n <= WP_SORT) {
-    int N = 2;
-    while (N < n) N <<= 1;
-    for (int k = t; k < N; k += WP_RANK_THREADS) {
-      c_th[k] = k < n ? ldg(Lth + k) : __builtin_inf();
-      c_w[k] = k < n ? ldg(L + k) : 0x7fffffff;
-    }
-    __syncthreads();
-    for (int k = 2; k <= N; k <<= 1)
-      for (int j = k >> 1; j > 0; j >>= 1) {
-        for (int i = t; i < N; i += WP_RANK_THREADS) {
-          const int l = i ^ j;
-          if (l > i) {
-            const double ti = c_th[i], tl = c_th[l];
-            const int wi = c_w[i], wl = c_w[l];
-            const bool gt = ti > tl || (ti == tl && wi > wl);  // (i) after (l)
-            if (((i & k) == 0) == gt) {
-              c_th[i] = tl;
-              c_th[l] = ti;
-              c_w[i] = wl;
-              c_w[l] = wi;
-            }
-          }
-        }
-        __syncthreads();
-      }
-    for (int p = t; p < n; p += WP_RANK_THREADS) stg(S.w_rank + c_w[p], p);
-    return;
-  }
-  for (int m0 = 0; m0 < n; m0 += WP_RANK_THREADS) {
-    const int m = m0 + t;
-    const int w = m < n ? ldg(L + m) : -1;
-    const double th = m < n ? ldg(Lth + m) : 0.0;
-    int r = 0;
-    for (int k0 = 0; k0 < n; k0 += WP_SORT) {
-      const int nk = min(WP_SORT, n - k0);
-      __syncthreads();
-      for (int k = t; k < nk; k += WP_RANK_THREADS) {
-        c_w[k] = ldg(L + k0 + k);
-        c_th[k] = ldg(Lth + k0 + k);
-      }
-      __syncthreads();
-      if (m < n)
-        for (int k = 0; k < nk; k++) {
-          const double t2 = c_th[k];
-          r += (t2 < th) || (t2 == th && c_w[k] < w);
-        }
-    }
-    if (m < n) stg(S.w_rank + w, r);
-  }
-}
-
-// Phase 3, one thread per water of a shell: target angle from the rank, the
-// restraint energy and forces (adds to d), and per-block sums of the energy
-// and of theta per shell into wp_part.
-__global__ __launch_bounds__(WP_THREADS) void k_watpol_force(const DevSys* __restrict__ systems) {
-  const DevSys& S = systems[blockIdx.y];
-  const int t = threadIdx.x, lane = t % QNB_WAVE, wid = t / QNB_WAVE;
+  const int lane = threadIdx.x % QNB_WAVE, wid = threadIdx.x / QNB_WAVE;
   if (!has_pol(S)) return;
   const int nsh = S.nshell, nw = S.nwat;
-  // blocks of this system (the grid is sized for the batch's largest)
-  const int nblk = (nw + WP_THREADS - 1) / WP_THREADS;
-  if ((int)blockIdx.x >= nblk) return;
-  const double pi = 3.141592653589793;
-  const int w = blockIdx.x * WP_THREADS + t;
-  const int sh = w < nw ? ldg(S.w_shell + w) : -1;
-  double epol = 0.0, th = 0.0;
-  if (sh >= 0) {
-    const double* st = S.sh_state;
-    const int n = S.sh_n[sh];
-    const int il = ldg(S.w_rank + w) + 1;
-    th = ldg(S.w_theta + w);
-    const double tc = st[sh];
-    double arg = 1.0 + (1.0 - 2.0 * (double)il) / (double)n;
-    double th0 = acos(arg);
-    th0 = th0 - 3.0 * sin(th0) * S.sh_cstb[sh] / 2.0;
-    if (th0 < 0.0) th0 = 0.0;
-    if (th0 > pi) th0 = pi;
-    const double dth = th - th0 + tc;
-    epol = 0.5 * S.fkwpol * (dth * dth);
-    const double dv = S.fkwpol * dth;
-    const int i = S.nat_solute + S.sa * w;
-    double rmu[3], rcu[3], rm, rc;
-    wat_vectors(S, i, rmu, rm, rcu, rc);
-    double scp = rmu[0] * rcu[0] + rmu[1] * rcu[1] + rmu[2] * rcu[2];
-    scp = scp > 1.0 ? 1.0 : (scp < -1.0 ? -1.0 : scp);
-    double f0 = sin(acos(scp));
-    if (fabs(f0) < 1.0e-10) f0 = 1.0e-10;
-    f0 = -1.0 / f0;
-    f0 = dv * f0;
-    const auto d = gpm(S.d);
-    for (int c = 0; c < 3; c++) {
-      const double av = rcu[c] - rmu[c] * scp;
-      const double f1 = (av * (-2.0)) / rm, f3 = av / rm, f2 = (rmu[c] - rcu[c] * scp) / rc;
-      d[3 * i + c] += (f1 + f2) * f0;
-      for (int k = 1; k < S.sa; k++) d[3 * (i + k) + c] += f3 * f0;
+  // block x of the system takes members 64 x' .. of shell sh, the blocks of
+  // the shells laid end to end
+  int sh = 0, xb = blockIdx.x, n = 0;
+  for (; sh < nsh; sh++) {
+    n = ldg(S.sh_n + sh);
+    const int nb = (n + WP_WATERS - 1) / WP_WATERS;
+    if (xb < nb) break;
+    xb -= nb;
+  }
+  if (sh >= nsh) return;
+  __shared__ double c_th[WP_CHUNK];
+  __shared__ int c_w[WP_CHUNK];
+  __shared__ int s_cnt[4][QNB_WAVE];
+  const int m = xb * WP_WATERS + lane;
+  const double* L_th = S.sh_lth + (size_t)sh * nw;
+  const int* L_w = S.sh_list + (size_t)sh * nw;
+  const int w = m < n ? ldg(L_w + m) : 0;
+  const double th = m < n ? ldg(L_th + m) : 0.0;
+  int before = 0;
+  for (int k0 = 0; k0 < n; k0 += WP_CHUNK) {
+    const int nk = min(WP_CHUNK, n - k0);
+    __syncthreads();
+    for (int k = threadIdx.x; k < nk; k += blockDim.x) {
+      c_th[k] = ldg(L_th + k0 + k);
+      c_w[k] = ldg(L_w + k0 + k);
+    }
+    __syncthreads();
+    const int q0 = nk * wid / 4, q1 = nk * (wid + 1) / 4;
+#pragma unroll 4
+    for (int k = q0; k < q1; k++) {
+      const double t2 = c_th[k];
+      before += (t2 < th) || (t2 == th && c_w[k] < w);
     }
   }
-  // block sums: [0] energy, [1 + is] theta over the block's members of shell is
-  __shared__ double red[WP_THREADS / QNB_WAVE][1 + QNB_MAXSH];
-  double v = wave_sum(epol);
-  if (lane == 0) red[wid][0] = v;
-  for (int is = 0; is < nsh; is++) {
-    const double s2 = wave_sum(sh == is ? th : 0.0);
-    if (lane == 0) red[wid][1 + is] = s2;
-  }
+  s_cnt[wid][lane] = before;
   __syncthreads();
-  if (t == 0) {
-    double* part = S.wp_part + (size_t)blockIdx.x * (1 + QNB_MAXSH);
-    for (int c = 0; c <= nsh; c++) {
-      double s2 = 0.0;
-      for (int k = 0; k < WP_THREADS / QNB_WAVE; k++) s2 += red[k][c];
-      part[c] = s2;
-    }
+  if (wid != 0 || m >= n) return;
+  const double pi = 3.141592653589793;
+  const int il = s_cnt[0][lane] + s_cnt[1][lane] + s_cnt[2][lane] + s_cnt[3][lane] + 1;
+  const double tc = S.sh_state[sh];
+  double arg = 1.0 + (1.0 - 2.0 * (double)il) / (double)n;
+  double th0 = acos(arg);
+  th0 = th0 - 3.0 * sin(th0) * S.sh_cstb[sh] / 2.0;
+  if (th0 < 0.0) th0 = 0.0;
+  if (th0 > pi) th0 = pi;
+  const double dth = th - th0 + tc;
+  const double epol = 0.5 * S.fkwpol * (dth * dth);
+  const double dv = S.fkwpol * dth;
+  const int i = S.nat_solute + S.sa * w;
+  double rmu[3], rcu[3], rm, rc;
+  wat_vectors(S, i, rmu, rm, rcu, rc);
+  double scp = rmu[0] * rcu[0] + rmu[1] * rcu[1] + rmu[2] * rcu[2];
+  scp = scp > 1.0 ? 1.0 : (scp < -1.0 ? -1.0 : scp);
+  double f0 = sin(acos(scp));
+  if (fabs(f0) < 1.0e-10) f0 = 1.0e-10;
+  f0 = -1.0 / f0;
+  f0 = dv * f0;
+  const auto d = gpm(S.d);
+  for (int c = 0; c < 3; c++) {
+    const double av = rcu[c] - rmu[c] * scp;
+    const double f1 = (av * (-2.0)) / rm, f3 = av / rm, f2 = (rmu[c] - rcu[c] * scp) / rc;
+    d[3 * i + c] += (f1 + f2) * f0;
+    for (int k = 1; k < S.sa; k++) d[3 * (i + k) + c] += f3 * f0;
   }
+  double* o = S.wp_rank + 2 * ((size_t)sh * nw + il - 1);
+  stg(o, epol);
+  stg(o + 1, th);
 }
 
-// Phase 4, one thread per system: adds the block sums in block order,
-// accumulates avtheta and avn_insh, writes the energy slot and clears the
-// shell counts for the next step's phase 1.
+// Phase 3 on its own, one wave per system (watpol_finish): the minimiser's
+// step; the MD step runs it in k_thermo, a single evaluation in
+// k_reduce_final.
 __global__ __launch_bounds__(64) void k_watpol_finish(const DevSys* __restrict__ systems) {
-  const DevSys& S = systems[blockIdx.x];
-  if (threadIdx.x != 0) return;
-  double* ep = S.epart + (size_t)(S.ncgp + 1) * QNB_NE;
-  for (int k = 0; k < QNB_NE; k++) ep[k] = 0.0;
-  if (!has_pol(S)) return;
-  const int nsh = S.nshell, nblk = (S.nwat + WP_THREADS - 1) / WP_THREADS;
-  double sum[1 + QNB_MAXSH];
-  for (int k = 0; k <= nsh; k++) sum[k] = 0.0;
-  for (int blk = 0; blk < nblk; blk++) {
-    const double* pb = S.wp_part + (size_t)blk * (1 + QNB_MAXSH);
-    for (int k = 0; k <= nsh; k++) sum[k] += pb[k];
-  }
-  double* st = S.sh_state;
-  for (int is = 0; is < nsh; is++) {
-    const int n = S.sh_n[is];
-    S.sh_n[is] = 0;
-    if (n == 0) continue;
-    st[QNB_MAXSH + is] += sum[1 + is] / (double)n;
-    st[2 * QNB_MAXSH + is] += (double)n;
-  }
-  ep[E_POL] = sum[0];
+  watpol_finish(systems[blockIdx.x]);
 }
 
 // ---------------------------------------------------------------------------
@@ -2005,6 +1937,7 @@ __global__ __launch_bounds__(256) void k_reduce_part(const DevSys* __restrict__ 
 __global__ __launch_bounds__(256) void k_reduce_final(const DevSys* __restrict__ systems, int with_qq, int with_pol) {
   const DevSys& S = systems[blockIdx.x];
   if (want_energies(S)) reduce_final(S, with_qq, with_pol);
+  if (with_pol && threadIdx.x < QNB_WAVE) watpol_finish(S);
 }
 
 // explicit instantiations used by the host code
