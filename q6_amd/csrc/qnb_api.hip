@@ -19,33 +19,42 @@ namespace qnb {
 template <typename R, bool ANY>
 __global__ void k_lists_lrf(const DevSys*);
 __global__ void k_qlists(const DevSys*);
-template <typename R, int NS, bool E, int CAP>
+template <typename R, int NS, bool E>
 __global__ void k_wforces(const DevSys*, uint32_t, int, int, int);
 template <typename R, int NS>
 __global__ void k_gforces(const DevSys*, uint32_t, int, int, int);
-template <typename R, int NS, bool E, int CAP>
+template <typename R, int NS, bool E>
 __global__ void k_sforces(const DevSys*, uint32_t, int, int, int);
 template <typename R, int NS>
-__global__ void k_qforces(const DevSys*, uint32_t, int, double*, int);
+__global__ void k_qforces(const DevSys*, uint32_t, int, int);
 template <typename R, int NS>
 __global__ void k_qq(const DevSys*, uint32_t);
 __global__ void k_pack_xq(const DevSys*);
 __global__ void k_pw_first(const DevSys*);
+__global__ void k_expand(const DevSys*);
 __global__ void k_watpol_theta(const DevSys*, const int*);
 __global__ void k_watpol_force(const DevSys*);
 __global__ void k_watpol_finish(const DevSys*);
 
-// SCAAS polarisation restraint: angles and shells, then ranks and forces
-// (grid.y the instance); `finish`: the per-system sums too, where no later
-// kernel of the caller runs them
-void launch_watpol(hipStream_t st, int nwat, int B, const DevSys* dsys, const int* istep, bool finish) {
-  hipLaunchKernelGGL(k_watpol_theta, dim3((nwat + WP_THREADS - 1) / WP_THREADS, B), dim3(WP_THREADS), 0, st, dsys, istep);
+void launch_watpol(hipStream_t st, int nwat, int B, const DevSys* dsys, const int* istep, bool theta, bool finish) {
+  if (theta)
+    hipLaunchKernelGGL(k_watpol_theta, dim3((nwat + WP_THREADS - 1) / WP_THREADS, B), dim3(WP_THREADS), 0, st, dsys,
+                       istep);
   hipLaunchKernelGGL(k_watpol_force, dim3(nwat / WP_WATERS + QNB_MAXSH, B), dim3(256), 0, st, dsys);
   if (finish) hipLaunchKernelGGL(k_watpol_finish, dim3(B), dim3(64), 0, st, dsys);
 }
+
+// Up to this many receiver waves (four per solute group, one per solvent
+// molecule) a force pass is one launch of k_forces_small: 256 CUs hold 3,072
+// of its waves at a time.  Measured per MD step, that kernel against the
+// separate ones on two streams: 62 against 78 us at 1,160 waves, 92 / 97 at
+// 3,950 (FP64: 111 / 122), 87 / 99 at 9,300 of few solute groups, but 116 / 110
+// at 7,900 with 800 solute groups (FP64: 157 / 149).
+bool small_launch(long solute_groups, long solvent) { return 4 * solute_groups + solvent <= 6144; }
+
 __global__ void k_reduce_part(const DevSys*);
 __global__ void k_reduce_final(const DevSys*, int, int);
-__global__ void k_atom_terms(const DevSys*, uint32_t, const double*);
+__global__ void k_atom_terms(const DevSys*, uint32_t, const double*, int);
 
 static thread_local std::string g_err;
 
@@ -272,6 +281,18 @@ int topo_build(DevSys& S, const qnb_system* s, HostTopo& T, DevAlloc& M) {
   UP(cgpatom, s->cgpatom, ncgpat);
   UP(atom_group, atom_group.data(), nat);
   UP(gslot, gslot.data(), ncgpat);
+  {
+    std::vector<int> off(1, 0), atoms;
+    for (int g = 0; g < s->ncgp_solute; g++) {
+      for (int k = s->cgp_first[g]; k <= s->cgp_last[g]; k++)
+        if (s->iqatom[s->cgpatom[k]] == 0) atoms.push_back(s->cgpatom[k]);
+      off.push_back((int)atoms.size());
+      T.max_nq_group = std::max(T.max_nq_group, off[g + 1] - off[g]);
+    }
+    T.n_nq = (int)atoms.size();
+    UP(nqoff, off.data(), off.size());
+    UP(nqatom, atoms.data(), atoms.size());
+  }
 
   UP(avdw, s->avdw, 3 * s->ntypes);
   UP(bvdw, s->bvdw, 3 * s->ntypes);
@@ -299,15 +320,17 @@ int topo_build(DevSys& S, const qnb_system* s, HostTopo& T, DevAlloc& M) {
     bool code1 = s->ivdw_rule == 1;
     for (int k = 0; k < s->ntypes * s->ntypes && code1; k++) code1 = s->ljcod[k] == 1;
     S.ppfast = code1 ? 1 : 0;
-    std::vector<double> pd(4 * (size_t)nsol1, 0.0);
-    std::vector<float> pf(4 * (size_t)nsol1, 0.0f);
+    std::vector<double> pd(PP_REC * (size_t)nsol1, 0.0);
     for (int i = 0; i < nsol; i++) {
       const int t = s->iac[i];
-      pd[4 * i] = s->avdw[3 * t];
-      pd[4 * i + 1] = s->bvdw[3 * t];
-      pd[4 * i + 2] = s->crg[i];
-      for (int c = 0; c < 3; c++) pf[4 * i + c] = (float)pd[4 * i + c];
+      double* r = pd.data() + PP_REC * (size_t)i;
+      r[0] = s->avdw[3 * t];
+      r[1] = s->bvdw[3 * t];
+      r[2] = s->crg[i];
+      r[4] = s->avdw[3 * t + 2];
+      r[5] = s->bvdw[3 * t + 2];
     }
+    const std::vector<float> pf(pd.begin(), pd.end());
     UP(ppd, pd.data(), pd.size());
     UP(ppf, pf.data(), pf.size());
   }
@@ -365,6 +388,22 @@ int topo_build(DevSys& S, const qnb_system* s, HostTopo& T, DevAlloc& M) {
       UP(qwB, s->qw_B, n);
       UP(qwEl, s->qw_el, n);
       UP(qwSc, s->qw_sc, n);
+      std::vector<double> pd(4 * n);
+      for (int iq = 0; iq < nq; iq++)
+        for (int k = 0; k < sa; k++)
+          for (int st = 0; st < ns; st++) {
+            const size_t a = (size_t)iq + nq * ((size_t)k + (size_t)sa * st), b = 4 * ((size_t)(iq * sa + k) * ns + st);
+            pd[b] = s->qw_A[a];
+            pd[b + 1] = s->qw_B[a];
+            pd[b + 2] = s->qw_el[a];
+            pd[b + 3] = s->qw_sc[a];
+          }
+      if (S.prec == QNB_PREC_MIXED) {
+        const std::vector<float> pf(pd.begin(), pd.end());
+        UP(qw_f, pf.data(), pf.size());
+      } else {
+        UP(qw_d, pd.data(), pd.size());
+      }
     }
     S.nqq = (int)qq_iq.size();
     UP(qq_iq, qq_iq.data(), qq_iq.size());
@@ -419,12 +458,27 @@ int topo_build(DevSys& S, const qnb_system* s, HostTopo& T, DevAlloc& M) {
     UP(qe_atom, ent_atom.data(), ent_atom.size());
     UP(qe_off, off.data(), off.size());
     UP(qe_item, item.data(), item.size());
+    std::vector<int> qe_of(nsol1, -1);
+    for (int e = 0; e < nent; e++) qe_of[ent_atom[e]] = e;
+    UP(qe_of, qe_of.data(), qe_of.size());
   }
 #undef UP
   return 0;
 }
 
-int instance_alloc(DevSys& S, DevAlloc& M, const qnb_params* p, int nslots) {
+int row_alloc(DevSys& S, const HostTopo& T, DevAlloc& M, int cap) {
+  M.release(S.nbr);
+  M.release(S.alist);
+  S.nbr = S.alist = nullptr;
+  S.cap = cap;
+  // a row of cap groups and the receiver's own holds at most this many atoms
+  const long atoms = std::min((long)T.n_nq, ((long)cap + 1) * T.max_nq_group);
+  S.acap = (int)((std::max(atoms, 1L) + 63) / 64 * 64);
+  int rc = M.alloc(&S.nbr, (size_t)S.cap * S.ncgp);
+  return rc ? rc : M.alloc(&S.alist, (size_t)S.acap * S.ncgp);
+}
+
+int instance_alloc(DevSys& S, const HostTopo& T, DevAlloc& M, const qnb_params* p, int nslots) {
   int rc = 0;
 #define AL(field, n)                                          \
   do {                                                        \
@@ -436,10 +490,14 @@ int instance_alloc(DevSys& S, DevAlloc& M, const qnb_params* p, int nslots) {
   else AL(xqgd, 4 * (size_t)S.ncgpat);
   AL(gref, 4 * (size_t)S.ncgp);
   AL(d, 3 * nat);
+  AL(dq, 3 * (size_t)std::max(S.nqat, 1));
+  AL(dqq, 3 * (size_t)std::max(S.nqe, 1));
   AL(lrf, (size_t)QNB_NLRF * S.ncgp);
-  if (S.cap <= 0) S.cap = 256;
-  AL(nbr, (size_t)S.cap * S.ncgp);
+  S.nbr = S.alist = nullptr;
+  if (int rc2 = row_alloc(S, T, M, S.cap > 0 ? S.cap : 256)) return rc2;
+  AL(alist_n, 2 * (size_t)S.ncgp);
   AL(nnbr, S.ncgp);
+  AL(nnsol, S.ncgp);
   AL(pw_first, std::max(S.ncgp_solute, 1));
   AL(need, 1);
   AL(qw_in, nw1);
@@ -465,9 +523,12 @@ int instance_alloc(DevSys& S, DevAlloc& M, const qnb_params* p, int nslots) {
   for (int k = 0; k < S.nshell; k++) sh0[k] = p->wshell_theta_corr[k];
   HIPCHK(hipMemcpy(S.sh_state, sh0, sizeof sh0, hipMemcpyHostToDevice));
   HIPCHK(hipMemset(S.nq_lists, 0, 2 * sizeof(int)));
+  HIPCHK(hipMemset(S.dq, 0, sizeof(double) * 3 * std::max(S.nqat, 1)));
   HIPCHK(hipMemset(S.need, 0, sizeof(int)));
   HIPCHK(hipMemset(S.sh_n, 0, sizeof(int) * QNB_MAXSH));
   HIPCHK(hipMemset(S.nnbr, 0, sizeof(int) * S.ncgp));
+  HIPCHK(hipMemset(S.nnsol, 0, sizeof(int) * S.ncgp));
+  HIPCHK(hipMemset(S.alist_n, 0, sizeof(int) * 2 * S.ncgp));
   HIPCHK(hipMemset(S.ered, 0, sizeof(double) * QNB_NE));
   return 0;
 }
@@ -505,7 +566,6 @@ static int scratch_lookup(int dev) {
 
 struct qnb_handle {
   int device = 0;  // the device current at qnb_create
-  bool small_groups = true;  // every solute group fits the water kernel's small staging
   DevSys hs;  // host copy of the device record (device pointers)
   DevSys* dsys = nullptr;
   DevAlloc mem;
@@ -585,11 +645,10 @@ extern "C" int32_t qnb_create(const qnb_system* s, const qnb_params* p, qnb_hand
   if ((rc = scratch_lookup(dev))) return rc;
   qnb_handle* h = new qnb_handle();
   h->device = dev;
-  h->small_groups = max_solute_group(s->cgp_first, s->cgp_last, s->ncgp_solute) <= WF_CAP_SMALL;
   DevSys& S = h->hs;
   memset(&S, 0, sizeof S);
   fill_params(S, s, p);
-  if ((rc = topo_build(S, s, h->T, h->mem)) || (rc = instance_alloc(S, h->mem, p, s->ncgp + 2)) ||
+  if ((rc = topo_build(S, s, h->T, h->mem)) || (rc = instance_alloc(S, h->T, h->mem, p, s->ncgp + qq_slots(S))) ||
       (rc = h->mem.alloc(&h->d_tfree, 1)) || (rc = h->mem.alloc(&h->d_istep, 1)) || (rc = h->mem.alloc(&h->dsys, 1))) {
     delete h;
     return rc;
@@ -617,6 +676,7 @@ static void launch_lists(qnb_handle* h) {
     hipLaunchKernelGGL(k_pw_first, dim3((h->hs.ncgp_solute + 3) / 4, 1), dim3(256), 0, h->stream, h->dsys);
   if (h->hs.any_atom) hipLaunchKernelGGL((k_lists_lrf<R, true>), grid, dim3(64 * wpb), 0, h->stream, h->dsys);
   else hipLaunchKernelGGL((k_lists_lrf<R, false>), grid, dim3(64 * wpb), 0, h->stream, h->dsys);
+  hipLaunchKernelGGL(k_expand, grid, dim3(64 * wpb), 0, h->stream, h->dsys);
 }
 
 extern "C" int32_t qnb_make_pair_lists(qnb_handle* h, const double* x) {
@@ -634,11 +694,7 @@ extern "C" int32_t qnb_make_pair_lists(qnb_handle* h, const double* x) {
     if (need <= h->hs.cap) break;
     // reallocate_nonbondlist_* (qalloc.f90:370-605): grow and rebuild
     int ncap = ((need * 5 / 4) + 63) / 64 * 64;
-    h->mem.release(h->hs.nbr);
-    h->hs.nbr = nullptr;
-    rc = h->mem.alloc(&h->hs.nbr, (size_t)ncap * h->hs.ncgp);
-    if (rc) return rc;
-    h->hs.cap = ncap;
+    if ((rc = row_alloc(h->hs, h->T, h->mem, ncap))) return rc;
     HIPCHK(hipMemcpy(h->dsys, &h->hs, sizeof(DevSys), hipMemcpyHostToDevice));
     if (attempt == 3) return fail(QNB_EOVERFLOW, "neighbour list capacity");
   }
@@ -658,42 +714,44 @@ template <typename R, int NS>
 static void launch_eval(qnb_handle* h, uint32_t mask) {
   const DevSys& S = h->hs;
   const int wpb = 4;
+  const bool with_pol = has_pol(S) && (mask & QNB_T_POL);
+  if (small_launch(S.ncgp_solute, S.nwat)) {
+    const SmallGrid G = small_grid(S.ncgp_solute, S.nwat, S.sa, S.nqat, S.nat_solute, S.nqe, mask, with_pol);
+    launch_forces_small(h->stream, S.prec, S.nstates, true, G, 1, h->dsys, mask, h->d_istep);
+    hipLaunchKernelGGL(k_atom_terms, dim3((S.natom + 255) / 256, 1), dim3(256), 0, h->stream, h->dsys, mask,
+                       (const double*)h->d_tfree, (G.qside ? QROWS_SIDE : 0) | (G.qq ? QROWS_QQ : 0));
+    if (with_pol) launch_watpol(h->stream, S.nwat, 1, h->dsys, h->d_istep, false, false);
+    hipLaunchKernelGGL(k_reduce_part, dim3(QNB_RED_BLOCKS, 1), dim3(256), 0, h->stream, h->dsys);
+    hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(256), 0, h->stream, h->dsys,
+                       G.qq ? (int)QQ_RECORD_PER_BLOCK : 0, (int)with_pol);
+    return;
+  }
   if (S.nwat > 0 && S.sa != 3) {
     const int nb = (S.nwat + FC_WPB - 1) / FC_WPB;
     hipLaunchKernelGGL((k_gforces<R, NS>), dim3(nb, 1), dim3(64 * FC_WPB), 0, h->stream, h->dsys, mask, 0, nb, 1);
   } else if (S.nwat > 0) {
     const int nb = (S.nwat + wpb - 1) / wpb;
-    if (h->small_groups)
-      hipLaunchKernelGGL((k_wforces<R, NS, true, WF_CAP_SMALL>), dim3(nb, 1), dim3(64 * wpb),
-                         (wf_wave_bytes<R, WF_CAP_SMALL>() * wpb), h->stream, h->dsys, mask, 0, nb, 1);
-    else
-      hipLaunchKernelGGL((k_wforces<R, NS, true, FC_CAP>), dim3(nb, 1), dim3(64 * wpb),
-                         (wf_wave_bytes<R, FC_CAP>() * wpb), h->stream, h->dsys, mask, 0, nb, 1);
+    hipLaunchKernelGGL((k_wforces<R, NS, true>), dim3(nb, 1), dim3(64 * wpb), 0, h->stream, h->dsys, mask, 0, nb, 1);
   }
   if (S.ncgp_solute > 0) {
     const int nb = (S.ncgp_solute + wpb - 1) / wpb;
-    if (h->small_groups)
-      hipLaunchKernelGGL((k_sforces<R, NS, true, WF_CAP_SMALL>), dim3(nb, 1), dim3(64 * wpb),
-                         (sf_wave_bytes<R, WF_CAP_SMALL>() * wpb), h->stream, h->dsys, mask, 0, nb, 1);
-    else
-      hipLaunchKernelGGL((k_sforces<R, NS, true, FC_CAP>), dim3(nb, 1), dim3(64 * wpb), (sf_wave_bytes<R, FC_CAP>() * wpb),
-                         h->stream, h->dsys, mask, 0, nb, 1);
+    hipLaunchKernelGGL((k_sforces<R, NS, true>), dim3(nb, 1), dim3(64 * wpb), wpb * so_wave_bytes<R>(), h->stream,
+                       h->dsys, mask, 0, nb, 1);
   }
   hipLaunchKernelGGL(k_atom_terms, dim3((S.natom + 255) / 256, 1), dim3(256), 0, h->stream, h->dsys, mask,
-                     (const double*)h->d_tfree);
+                     (const double*)h->d_tfree, 0);
   if (S.nqat > 0 && (mask & (QNB_T_QW | QNB_T_QP))) {
     // partners per Q-atom: at most nwat + nat_solute; about QF_PART / 64 per lane
     int maxp = S.nwat + S.nat_solute;
     int chunks = std::max(1, std::min((maxp + QF_PART - 1) / QF_PART, 64));
     hipLaunchKernelGGL((k_qforces<R, NS>), dim3(qforces_blocks(S.nqat, chunks, wpb), 1), dim3(64 * wpb), 0,
-                       h->stream, h->dsys, mask, chunks, (double*)nullptr, 0);
+                       h->stream, h->dsys, mask, chunks, 0);
   }
-  const int with_qq = S.nqat > 0 && (mask & (QNB_T_QQ | QNB_T_QQP));
-  const int with_pol = S.nwat > 0 && S.wpol && S.nshell > 0 && (mask & QNB_T_POL);
+  const int with_qq = S.nqat > 0 && (mask & (QNB_T_QQ | QNB_T_QQP)) ? QQ_ONE_RECORD : 0;
   if (with_qq) hipLaunchKernelGGL((k_qq<R, NS>), dim3(1), dim3(QQ_THREADS), 0, h->stream, h->dsys, mask);
-  if (with_pol) launch_watpol(h->stream, S.nwat, 1, h->dsys, (const int*)h->d_istep, false);
+  if (with_pol) launch_watpol(h->stream, S.nwat, 1, h->dsys, (const int*)h->d_istep, true, false);
   hipLaunchKernelGGL(k_reduce_part, dim3(QNB_RED_BLOCKS, 1), dim3(256), 0, h->stream, h->dsys);
-  hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(256), 0, h->stream, h->dsys, with_qq, with_pol);
+  hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(256), 0, h->stream, h->dsys, with_qq, (int)with_pol);
 }
 
 template <typename R>

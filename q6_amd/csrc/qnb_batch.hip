@@ -20,17 +20,17 @@ __global__ void k_lists_lrf(const DevSys*);
 __global__ void k_qlists(const DevSys*);
 __global__ void k_pack_xq(const DevSys*);
 __global__ void k_pw_first(const DevSys*);
-template <typename R, int NS, bool E, int CAP>
+__global__ void k_expand(const DevSys*);
+template <typename R, int NS, bool E>
 __global__ void k_wforces(const DevSys*, uint32_t, int, int, int);
-template <typename R, int NS, bool E, int CAP>
+template <typename R, int NS, bool E>
 __global__ void k_sforces(const DevSys*, uint32_t, int, int, int);
 template <typename R, int NS>
-__global__ void k_qforces(const DevSys*, uint32_t, int, double*, int);
+__global__ void k_qforces(const DevSys*, uint32_t, int, int);
 template <typename R, int NS>
 __global__ void k_qq(const DevSys*, uint32_t);
-void launch_watpol(hipStream_t st, int nwat, int B, const DevSys* dsys, const int* istep, bool finish);
 __global__ void k_reduce_part(const DevSys*);
-__global__ void k_atom_terms(const DevSys*, uint32_t, const double*);
+__global__ void k_atom_terms(const DevSys*, uint32_t, const double*, int);
 
 // per-instance MD record
 struct MdDev {
@@ -176,8 +176,7 @@ __global__ __launch_bounds__(256) void k_bonded(const DevSys* __restrict__ syste
 // the SCAAS radial restraint (as k_atom_terms with every term on) and the
 // solute bonds and angles, added to the atom's gradient in one update.
 __global__ __launch_bounds__(256) void k_atom_step(const DevSys* __restrict__ systems, const MdDev* __restrict__ mds,
-                                                   const double* __restrict__ tfree, double* __restrict__ dq,
-                                                   int dq_stride) {
+                                                   const double* __restrict__ tfree, int rows) {
   const DevSys& S = systems[blockIdx.y];
   const MdDev& M = mds[blockIdx.y];
   __shared__ double red[4];
@@ -194,15 +193,7 @@ __global__ __launch_bounds__(256) void k_atom_step(const DevSys* __restrict__ sy
       radial_restraint(S, src, shift, f, er);
     }
     if (i < M.nbat) bonded_atom(S, M, i, f, eb, ea);
-    // the Q-atom side's rows of this step, cleared for the next one
-    const int iq = i < S.nat_solute ? ldg(S.iqatom + i) : 0;
-    if (iq > 0) {
-      double* q = dq + (size_t)blockIdx.y * dq_stride + 3 * (iq - 1);
-      for (int c = 0; c < 3; c++) {
-        f[c] += q[c];
-        q[c] = 0.0;
-      }
-    }
+    add_qrows(S, i, rows, f);
     store_atom_gradient(S, i, f);
     if (want_energies(S)) {
       stg(S.eatom + 2 * i, el);
@@ -540,12 +531,11 @@ struct qnb_batch {
   int maxg = 0, maxat = 0, maxsw = 0, maxw = 0, maxs = 0, ns_max = 1, prec = 0;
   int nbblk = 1;  // k_bonded blocks per instance
   bool anyq = false, anypol = false, static_q = true;
-  int qchunks = 1, nq_max = 0;
-  double* dq = nullptr;  // [n][nq_max][3]: the Q-atom side's gradient rows of the MD step
+  int qchunks = 1, nq_max = 0, nqe_max = 0, nsol_max = 0;
+  long sum_solute = 0, sum_solvent = 0;  // receiver groups of all instances
   int wpb_lists = 4, wpb_forces = 4;  // waves per block, picked by qnb_batch_autotune
   int imap_water = 1;                 // block placement of the water-receiver kernel (map_block), autotuned
   int imap_solute = 0;                // block placement of the solute-receiver kernel, autotuned
-  bool small_groups = true;           // every solute group fits the water kernel's small staging
   std::vector<int> nbcycle;
   std::vector<int> ene_every;  // per instance energy sampling interval
   // Q bonded terms per instance
@@ -592,17 +582,10 @@ static void launch_lists(qnb_batch* b, int wpb) {
     if (any) hipLaunchKernelGGL((k_lists_lrf<double, true>), g, t, 0, b->stream, b->dsys);
     else hipLaunchKernelGGL((k_lists_lrf<double, false>), g, t, 0, b->stream, b->dsys);
   }
+  hipLaunchKernelGGL(k_expand, dim3((b->maxg + 3) / 4, b->n), dim3(256), 0, b->stream, b->dsys);
 }
 
 static const uint32_t kStepMask = QNB_T_NONBONDED | QNB_T_QQ | QNB_T_QQP | QNB_T_RAD | QNB_T_POL;
-
-// waves per block of the force kernel, kept within 64 KiB of LDS per block
-// (the per-wave partner slots plus the solute launch's type-pair tables)
-template <typename R>
-static int forces_wpb(int wpb) {
-  const int cap = (int)((65536 - fc_static_bytes<R>()) / fc_wave_bytes<R>());
-  return std::max(1, std::min(std::min(wpb, FC_WPB), cap));
-}
 
 // Blocks are dealt to the 8 XCDs round-robin in linear block order
 // (blockIdx.y * gridDim.x + blockIdx.x); with gridDim.x a multiple of 8 the
@@ -611,30 +594,22 @@ static int forces_wpb(int wpb) {
 // the same XCD and find them in its L2.  The padding blocks exit at once.
 static unsigned xcd_cols(int blocks) { return (unsigned)((blocks + 7) / 8 * 8); }
 
-// water receivers (k_wforces) with the block placement imap (map_block)
-template <typename R, int NS, bool E, int CAP>
-static void launch_water(qnb_batch* b, int wpb, int imap, hipStream_t st) {
-  const int nb = (b->maxw + wpb - 1) / wpb;
-  const dim3 grid = imap == 0 ? dim3(xcd_cols(nb), b->n) : dim3((unsigned)(8 * (((long)nb * b->n + 7) / 8)), 1);
-  hipLaunchKernelGGL((k_wforces<R, NS, E, CAP>), grid, dim3(64 * wpb), (wf_wave_bytes<R, CAP>() * wpb), st, b->dsys,
-                     kStepMask, imap, nb, b->n);
-}
-
+// water receivers (parts 1) and solute receivers (parts 2) with their block
+// placements (map_block)
 template <typename R, int NS, bool E>
 static void launch_forces_e(qnb_batch* b, int wpb, int parts, hipStream_t wst) {
+  auto grid = [&](int nb, int imap) {
+    return imap == 0 ? dim3(xcd_cols(nb), b->n) : dim3((unsigned)(8 * (((long)nb * b->n + 7) / 8)), 1);
+  };
   if (b->maxw > 0 && (parts & 1)) {
-    if (b->small_groups) launch_water<R, NS, E, WF_CAP_SMALL>(b, wpb, b->imap_water, wst);
-    else launch_water<R, NS, E, FC_CAP>(b, wpb, b->imap_water, wst);
+    const int nb = (b->maxw + wpb - 1) / wpb;
+    hipLaunchKernelGGL((k_wforces<R, NS, E>), grid(nb, b->imap_water), dim3(64 * wpb), 0, wst, b->dsys, kStepMask,
+                       b->imap_water, nb, b->n);
   }
   if (b->maxs > 0 && (parts & 2)) {
-    const int nb = (b->maxs + wpb - 1) / wpb, imap = b->imap_solute;
-    const dim3 grid = imap == 0 ? dim3(xcd_cols(nb), b->n) : dim3((unsigned)(8 * (((long)nb * b->n + 7) / 8)), 1);
-    if (b->small_groups)
-      hipLaunchKernelGGL((k_sforces<R, NS, E, WF_CAP_SMALL>), grid, dim3(64 * wpb),
-                         (sf_wave_bytes<R, WF_CAP_SMALL>() * wpb), b->stream, b->dsys, kStepMask, imap, nb, b->n);
-    else
-      hipLaunchKernelGGL((k_sforces<R, NS, E, FC_CAP>), grid, dim3(64 * wpb), (sf_wave_bytes<R, FC_CAP>() * wpb),
-                         b->stream, b->dsys, kStepMask, imap, nb, b->n);
+    const int nb = (b->maxs + wpb - 1) / wpb;
+    hipLaunchKernelGGL((k_sforces<R, NS, E>), grid(nb, b->imap_solute), dim3(64 * wpb), wpb * so_wave_bytes<R>(),
+                       b->stream, b->dsys, kStepMask, b->imap_solute, nb, b->n);
   }
 }
 
@@ -644,13 +619,12 @@ static void launch_forces_e(qnb_batch* b, int wpb, int parts, hipStream_t wst) {
 template <typename R, int NS>
 static void launch_forces_t(qnb_batch* b, int wpb, bool energy = true, bool atom_terms = true, int parts = 3,
                             hipStream_t wst = nullptr) {
-  wpb = forces_wpb<R>(wpb);
   if (!wst) wst = b->stream;
   if (energy) launch_forces_e<R, NS, true>(b, wpb, parts, wst);
   else launch_forces_e<R, NS, false>(b, wpb, parts, wst);
   if (atom_terms)
     hipLaunchKernelGGL(k_atom_terms, dim3((b->maxat + 255) / 256, b->n), dim3(256), 0, b->stream, b->dsys, kStepMask,
-                       (const double*)b->tfree);
+                       (const double*)b->tfree, 0);
 }
 
 static void launch_forces(qnb_batch* b, int wpb, bool energy = true, bool atom_terms = true, int parts = 3) {
@@ -675,10 +649,8 @@ static void launch_qforces(qnb_batch* b) {
   const dim3 grid(qforces_blocks(b->nq_max, b->qchunks, wpb), b->n), block(64 * wpb);
 #define QNB_LQ(NS)                                                                                     \
   if (mixed)                                                                                                  \
-    hipLaunchKernelGGL((k_qforces<float, NS>), grid, block, 0, b->stream, b->dsys, kStepMask, b->qchunks,     \
-                       (double*)nullptr, 0);                                                                  \
-  else hipLaunchKernelGGL((k_qforces<double, NS>), grid, block, 0, b->stream, b->dsys, kStepMask, b->qchunks, \
-                          (double*)nullptr, 0)
+    hipLaunchKernelGGL((k_qforces<float, NS>), grid, block, 0, b->stream, b->dsys, kStepMask, b->qchunks, 0); \
+  else hipLaunchKernelGGL((k_qforces<double, NS>), grid, block, 0, b->stream, b->dsys, kStepMask, b->qchunks, 0)
   switch (b->ns_max) {
     case 1: QNB_LQ(1); break;
     case 2: QNB_LQ(2); break;
@@ -705,14 +677,24 @@ static void enqueue_forces_forked(qnb_batch* b, bool energy) {
   (void)hipStreamWaitEvent(b->side, b->ev_fork, 0);
   if (b->anyq)
     hipLaunchKernelGGL((k_qforces<R, NS>), dim3(qforces_blocks(b->nq_max, b->qchunks, wpb), B), dim3(64 * wpb), 0,
-                       b->side, b->dsys, kStepMask, b->qchunks, b->dq, 3 * b->nq_max);
+                       b->side, b->dsys, kStepMask, b->qchunks, (int)QROWS_SIDE);
   if (b->maxw > 0) launch_forces_t<R, NS>(b, b->wpb_forces, energy, false, 1, b->side);
   if (b->anypol)
-    launch_watpol(b->side, b->maxw, B, b->dsys, (const int*)b->istep, false);
+    launch_watpol(b->side, b->maxw, B, b->dsys, (const int*)b->istep, true, false);
   launch_forces_t<R, NS>(b, b->wpb_forces, energy, false, 2);
   if (b->anyq) hipLaunchKernelGGL((k_qq<R, NS>), dim3(B), dim3(QQ_THREADS), 0, b->stream, b->dsys, kStepMask);
   (void)hipEventRecord(b->ev_join, b->side);
   (void)hipStreamWaitEvent(b->stream, b->ev_join, 0);
+}
+
+// the MD step's force pass of a batch too small to fill the chip: everything
+// in one launch, then the polarisation forces
+static bool small_step(const qnb_batch* b) { return small_launch(b->sum_solute, b->sum_solvent); }
+
+static void enqueue_forces_small(qnb_batch* b, bool energy) {
+  const SmallGrid G = small_grid(b->maxs, b->maxw, 3, b->nq_max, b->nsol_max, b->nqe_max, kStepMask, b->anypol);
+  launch_forces_small(b->stream, b->prec, b->ns_max, energy, G, b->n, b->dsys, kStepMask, b->istep);
+  if (b->anypol) launch_watpol(b->stream, b->maxw, b->n, b->dsys, b->istep, false, false);
 }
 
 template <typename R, int NS>
@@ -722,10 +704,10 @@ static void enqueue_forces(qnb_batch* b, bool energy = true, bool atom_terms = t
   launch_forces_t<R, NS>(b, b->wpb_forces, energy, atom_terms);
   if (b->anyq) {
     hipLaunchKernelGGL((k_qforces<R, NS>), dim3(qforces_blocks(b->nq_max, b->qchunks, wpb), B), dim3(64 * wpb), 0,
-                       b->stream, b->dsys, mask, b->qchunks, (double*)nullptr, 0);
+                       b->stream, b->dsys, mask, b->qchunks, 0);
     hipLaunchKernelGGL((k_qq<R, NS>), dim3(B), dim3(QQ_THREADS), 0, b->stream, b->dsys, mask);
   }
-  if (b->anypol) launch_watpol(b->stream, b->maxw, B, b->dsys, (const int*)b->istep, true);
+  if (b->anypol) launch_watpol(b->stream, b->maxw, B, b->dsys, (const int*)b->istep, true, true);
 }
 
 // leap-frog + SHAKE + new velocities, then the temperatures and Berendsen
@@ -742,7 +724,9 @@ static void enqueue_step(qnb_batch* b, bool lists, bool energy) {
     launch_lists(b, b->wpb_lists);
     if (b->anyq && !b->static_q) hipLaunchKernelGGL(k_qlists, dim3(B), dim3(1024), 0, b->stream, b->dsys);
   }
-  switch (b->ns_max) {
+  const bool small = small_step(b);
+  if (small) enqueue_forces_small(b, energy);
+  else switch (b->ns_max) {
     case 1: enqueue_forces_forked<R, 1>(b, energy); break;
     case 2: enqueue_forces_forked<R, 2>(b, energy); break;
     case 3:
@@ -750,7 +734,8 @@ static void enqueue_step(qnb_batch* b, bool lists, bool energy) {
     default: enqueue_forces_forked<R, 8>(b, energy); break;
   }
   hipLaunchKernelGGL(k_atom_step, dim3((b->maxat + 255) / 256, B), dim3(256), 0, b->stream, b->dsys, b->dmd,
-                     (const double*)b->tfree, b->dq, 3 * b->nq_max);
+                     (const double*)b->tfree,
+                     !b->anyq ? 0 : (int)(small ? QROWS_SIDE | QROWS_QQ : QROWS_SIDE));
   if (b->anyqb) launch_qbonded(b->stream, B, b->dsys, b->dqb);
   // the reduction and the record do nothing on a step no instance samples
   // (energy is false only then); the record also counts stored snapshots
@@ -758,8 +743,8 @@ static void enqueue_step(qnb_batch* b, bool lists, bool energy) {
   if (b->anysnap)
     hipLaunchKernelGGL(k_snap, dim3((3 * b->maxat + 255) / 256, B), dim3(256), 0, b->stream, b->dsys, b->dmd);
   if (energy || b->anysnap)
-    hipLaunchKernelGGL(k_record, dim3(B), dim3(256), 0, b->stream, b->dsys, b->dmd, (int)energy, (int)b->anyq,
-                       (int)b->anypol);
+    hipLaunchKernelGGL(k_record, dim3(B), dim3(256), 0, b->stream, b->dsys, b->dmd, (int)energy,
+                       !b->anyq ? 0 : (int)(small ? QQ_RECORD_PER_BLOCK : QQ_ONE_RECORD), (int)b->anypol);
   if (energy && b->exc_threads > 0)
     hipLaunchKernelGGL(k_exc_record, dim3((b->exc_threads + 63) / 64, B), dim3(64), 0, b->stream, b->dsys, b->dmd,
                        (const ExcDev*)b->dexc);
@@ -838,13 +823,15 @@ extern "C" int32_t qnb_batch_create(int32_t n, const qnb_system* const* sys, con
       b->topo_of.push_back(b->topo_of[it->second]);
     }
     S.cap = 0;
-    if ((rc = instance_alloc(S, b->mem, par[k], sys[k]->ncgp + 2))) return rc;
+    if ((rc = instance_alloc(S, *b->topos[b->topo_of[k]], b->mem, par[k], sys[k]->ncgp + qq_slots(S)))) return rc;
     HIPCHK(hipMemcpy(S.x, x0[k], sizeof(double) * 3 * S.natom, hipMemcpyHostToDevice));
     b->maxg = std::max(b->maxg, S.ncgp);
     b->maxw = std::max(b->maxw, S.nwat);
     b->maxs = std::max(b->maxs, S.ncgp_solute);
-    b->small_groups = b->small_groups &&
-                      max_solute_group(sys[k]->cgp_first, sys[k]->cgp_last, sys[k]->ncgp_solute) <= WF_CAP_SMALL;
+    b->nqe_max = std::max(b->nqe_max, S.nqe);
+    b->nsol_max = std::max(b->nsol_max, S.nat_solute);
+    b->sum_solute += S.ncgp_solute;
+    b->sum_solvent += S.nwat;
     b->maxat = std::max(b->maxat, S.natom);
     b->maxsw = std::max(b->maxsw, S.nwat + S.nat_solute);
     b->ns_max = std::max(b->ns_max, S.nstates);
@@ -863,8 +850,6 @@ extern "C" int32_t qnb_batch_create(int32_t n, const qnb_system* const* sys, con
   HIPCHK(hipEventCreateWithFlags(&b->ev_join, hipEventDisableTiming));
   if ((rc = b->mem.alloc(&b->tfree, n)) || (rc = b->mem.alloc(&b->istep, n))) return rc;
   HIPCHK(hipMemset(b->istep, 0, sizeof(int) * n));
-  if ((rc = b->mem.alloc(&b->dq, (size_t)n * 3 * std::max(b->nq_max, 1)))) return rc;
-  HIPCHK(hipMemset(b->dq, 0, sizeof(double) * n * 3 * std::max(b->nq_max, 1)));
   // MD records
   for (int k = 0; k < n; k++) {
     const qnb_md_params* m = md[k];
@@ -984,9 +969,7 @@ extern "C" int32_t qnb_batch_create(int32_t n, const qnb_system* const* sys, con
   // during a run is reported by qnb_batch_sync)
   for (int k = 0; k < n; k++) {
     DevSys& S = b->hs[k];
-    b->mem.release(S.nbr);
-    S.cap = std::min(((S.ncgp + 63) / 64) * 64, 1024);
-    if ((rc = b->mem.alloc(&S.nbr, (size_t)S.cap * S.ncgp))) return rc;
+    if ((rc = row_alloc(S, *b->topos[b->topo_of[k]], b->mem, std::min(((S.ncgp + 63) / 64) * 64, 1024)))) return rc;
   }
   for (int attempt = 0;; attempt++) {
     HIPCHK(hipMemcpy(b->dsys, b->hs.data(), sizeof(DevSys) * n, hipMemcpyHostToDevice));
@@ -1001,9 +984,7 @@ extern "C" int32_t qnb_batch_create(int32_t n, const qnb_system* const* sys, con
       int need = 0;
       HIPCHK(hipMemcpy(&need, S.need, sizeof(int), hipMemcpyDeviceToHost));
       if (need > S.cap) {
-        b->mem.release(S.nbr);
-        S.cap = ((need + 63) / 64) * 64;
-        if ((rc = b->mem.alloc(&S.nbr, (size_t)S.cap * S.ncgp))) return rc;
+        if ((rc = row_alloc(S, *b->topos[b->topo_of[k]], b->mem, ((need + 63) / 64) * 64))) return rc;
         again = true;
       }
     }
@@ -1019,9 +1000,7 @@ extern "C" int32_t qnb_batch_create(int32_t n, const qnb_system* const* sys, con
     const int cap = ((mx * 3 / 2 + 64) + 63) / 64 * 64;
     if (cap < S.cap) {
       // shrink: rebuild happens at the first step of the run
-      b->mem.release(S.nbr);
-      S.cap = cap;
-      if ((rc = b->mem.alloc(&S.nbr, (size_t)S.cap * S.ncgp))) return rc;
+      if ((rc = row_alloc(S, *b->topos[b->topo_of[k]], b->mem, cap))) return rc;
     }
     HIPCHK(hipMemset(S.need, 0, sizeof(int)));
   }

@@ -62,6 +62,9 @@ struct DevSys {
   // the atom's group modulo 64, its bit in the far-group ballot word of the
   // list sweep's 64-group chunk
   const int* gslot;
+  // the solute groups' atoms without Q-atoms: group b's at nqatom[nqoff[b]] ..
+  const int* nqoff;
+  const int* nqatom;
   int ncgpat;
   const double* avdw;  // [t*3+k]
   const double* bvdw;
@@ -80,8 +83,8 @@ struct DevSys {
   const int* gspan;       // [ncgp_solute][2]: smallest and largest atom index of the group
   const uint8_t* glong;   // [ncgp_solute]: an atom of the group has long-range exclusion / 1-4 partners
   int ppfast;             // geometric rule and ljcod = 1 throughout
-  const double* ppd;      // [nat_solute][4]: avdw(t, 1), bvdw(t, 1), charge, 0 (FP64 path)
-  const float* ppf;       // [nat_solute][4]: the same in FP32 (mixed path)
+  const double* ppd;      // [nat_solute][PP_REC]: avdw(t, 1), bvdw(t, 1), charge, 0, avdw(t, 3), bvdw(t, 3), 0, 0 (FP64 path)
+  const float* ppf;       // the same in FP32 (mixed path)
   const double* pwA;       // [i + j*nat_solute]
   const double* pwB;
   const double* pwEl;
@@ -104,6 +107,10 @@ struct DevSys {
   const float* qpB_f;
   const float* qpEl_f;
   const float* qpSc_f;
+  // the Q-solvent table packed for the force kernels, [iq][k][s] {A, B, el,
+  // soft-core score}; FP64 path / mixed path
+  const double* qw_d;
+  const float* qw_f;
   const double* qwA;  // [iq + nq*(j + sa*s)]
   const double* qwB;
   const double* qwEl;
@@ -127,6 +134,7 @@ struct DevSys {
   const int* qe_off;
   const int* qe_item;  // [4 * items]
   int nqe;
+  const int* qe_of;    // [nat_solute] the atom's entity, -1 where it has none
 
   // per-instance state
   double* x;
@@ -140,9 +148,20 @@ struct DevSys {
   // excluded, else 0
   double* gref;
   double* d;
+  // gradient rows of the Q-atom side [nqat][3] and of the Q-Q entities
+  // [nqe][3] where these run beside the solute receivers (QROWS_*), added to
+  // d by the per-atom pass; dq is zero between steps, dqq stored anew
+  double* dq;
+  double* dqq;
   double* lrf;
   int* nbr;
   int* nnbr;
+  // partner atoms of each receiver (k_expand): rows of acap entries, counts
+  // [ncgp][2] from the front and from the back
+  int* alist;
+  int* alist_n;
+  int acap;
+  int* nnsol;  // [ncgp] length of the row's solute prefix (rows are sorted)
   // reference test-point reuse of the LRF-off switch-atom solute-water list
   // (quirk bit 0 with use_lrf = 0): per solute group, the first water within
   // the cut-off of the switch atom (nwat when none); later waters are tested
@@ -229,6 +248,9 @@ template <typename T>
 __device__ __forceinline__ __attribute__((address_space(1))) T* gpm(T* p) {
   return (__attribute__((address_space(1))) T*)p;
 }
+// a value that is the same in every lane, in a scalar register: loop bounds
+// and branches on it are the wave's and not each lane's
+__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
 template <typename T>
 __device__ __forceinline__ void stg(T* p, T v) {
   *(__attribute__((address_space(1))) T*)p = v;
@@ -404,13 +426,10 @@ __host__ __device__ constexpr int wave_sum_tr_lane(int j) {
 }
 
 // A wave's energy record ep[0 .. QNB_NE) in one coalesced store from lanes
-// 0 .. QNB_NE-1: the N per-lane partials are summed with one transposed
-// reduction, each sum is read from its lane, and entry slot[j] takes sum j,
-// every other entry 0.
+// 0 .. QNB_NE-1: `sum` holds wave_sum_tr<N>'s sums of the N partials, each is
+// read from its lane, and entry slot[j] takes sum j, every other entry 0.
 template <int N>
-__device__ __forceinline__ void store_energy_record(double* ep, const double (&part)[N], const int (&slot)[N],
-                                                    int lane) {
-  const double sum = wave_sum_tr(part, lane);
+__device__ __forceinline__ void store_energy_record(double* ep, double sum, const int (&slot)[N], int lane) {
   double v = 0.0;
 #pragma unroll
   for (int j = 0; j < N; j++) {
@@ -419,10 +438,14 @@ __device__ __forceinline__ void store_energy_record(double* ep, const double (&p
   }
   if (lane < QNB_NE) *(__attribute__((address_space(1))) double*)(ep + lane) = v;
 }
+// energy records of the Q-Q pairs after the charge groups' ones: one when k_qq
+// wrote them, one per four entities when k_forces_small did
+__host__ __device__ __forceinline__ int qq_slots(const DevSys& S) { return S.nqe > 4 ? (S.nqe + 3) / 4 : 1; }
+enum { QQ_ONE_RECORD = 1, QQ_RECORD_PER_BLOCK = 2 };
 
 // shell members per block of the polarisation-restraint force kernel
 #define WP_WATERS 64
-__device__ __forceinline__ bool has_pol(const DevSys& S) { return S.nwat > 0 && S.wpol && S.nshell > 0; }
+__host__ __device__ __forceinline__ bool has_pol(const DevSys& S) { return S.nwat > 0 && S.wpol && S.nshell > 0; }
 // restraint energy (c = 0) or theta (c = 1) of shell is, added over its n
 // members by one wave (every lane active): lane l takes ranks l, l + 64, ...,
 // then a fixed tree
@@ -473,7 +496,9 @@ __device__ __forceinline__ void reduce_final(const DevSys& S, int with_qq, int w
   __syncthreads();
   if (c == 0 && k < QNB_NE) {
     double t = ((part[0][k] + part[1][k]) + part[2][k]) + part[3][k];
-    if (with_qq && S.nqat > 0) t += S.epart[(size_t)S.ncgp * QNB_NE + k];
+    if (with_qq && S.nqat > 0)
+      for (int m = 0, nm = with_qq == QQ_ONE_RECORD ? 1 : qq_slots(S); m < nm; m++)
+        t += ldg(S.epart + (size_t)(S.ncgp + m) * QNB_NE + k);
     if (k == E_POL && with_pol && has_pol(S)) t += pol;
     S.ered[k] = t;
   }
@@ -588,6 +613,24 @@ __device__ __forceinline__ void store_atom_gradient(const DevSys& S, int i, cons
     d[3 * i + 1] += f[1];
     d[3 * i + 2] += f[2];
   }
+}
+
+// which gradient rows of the Q kernels hold this step's sums
+enum { QROWS_SIDE = 1, QROWS_QQ = 2 };
+// adds atom i's rows to f; the Q-atom side's row is cleared for the next step
+__device__ __forceinline__ void add_qrows(const DevSys& S, int i, int rows, double* f) {
+  if (rows == 0 || i >= S.nat_solute || S.nqat <= 0) return;
+  const int iq = (rows & QROWS_SIDE) ? ldg(S.iqatom + i) : 0;
+  if (iq > 0) {
+    const auto q = gpm(S.dq) + 3 * (iq - 1);
+    for (int c = 0; c < 3; c++) {
+      f[c] += q[c];
+      q[c] = 0.0;
+    }
+  }
+  const int e = (rows & QROWS_QQ) ? ldg(S.qe_of + i) : -1;
+  if (e >= 0)
+    for (int c = 0; c < 3; c++) f[c] += ldg(S.dqq + 3 * e + c);
 }
 
 // LRF Taylor application for one atom (lrf_taylor, nonbondene.f90:507-571)
@@ -757,25 +800,27 @@ struct PairMath {
   // nbe_qx (nonbonded.f90:200-222), soft-core score sc, state weight lam
   static __device__ __forceinline__ R nbe_qx(R r2, R r, R r6in, R A, R B, R q, R sc, R lam, double& el,
                                              double& vdw, bool want = true) {
-    R r6_hc = recip(r6in);
-    R r6 = recip(r6_hc + sc);
+    R r6 = r6in, soft = R(1);
+    if (sc != R(0)) {
+      const R r6_hc = recip(r6in);
+      r6 = recip(r6_hc + sc);
+      soft = r6 * r6_hc;
+    }
     R r12 = r6 * r6;
     R Vel = q * r, Va = A * r12, Vb = B * r6;
     if (want) {
       el += (double)Vel;
       vdw += (double)Va - (double)Vb;
     }
-    return r2 * (-Vel - (R(12) * Va - R(6) * Vb) * r6 * r6_hc) * lam;
+    return r2 * (-Vel - (R(12) * Va - R(6) * Vb) * soft) * lam;
   }
 };
 
-// Receiver-side force kernel: at most FC_WPB wavefronts per block, FC_CAP
-// staged partner atoms and FC_CH receiver atoms per sweep; per-wave LDS:
-// partner offsets and receiver offsets (R x 3), partner index and tag,
-// receiver index
 // floats per solute atom in the FP32 solute-water table (3 sites x A, B, el,
 // padded to 16-byte records)
 #define PW_REC 12
+// values per solute atom in the solute-solute factor tables (ppd, ppf)
+#define PP_REC 8
 
 // partners per wave of the Q-atom force kernel (the Q-atom's partners are
 // split into chunks of about this many)
@@ -786,6 +831,16 @@ struct PairMath {
 // the blocks of one Q-atom's chunks (W waves per block)
 inline int qforces_blocks(int nq, int chunks, int W) { return 8 * ((chunks + W - 1) / W) * ((nq + 7) / 8); }
 
+// the same inside k_forces_small: more, shorter waves (as launches of their own
+// the Q-atom side took 11-13 us at 8 partners per lane)
+#define QF_PART_SMALL 192
+
+// blocks of each role of k_forces_small, and the chunks of a Q-atom's partners
+struct SmallGrid {
+  int solute, solvent, qside, qq, theta, qchunks;
+  int blocks() const { return solute + solvent + qside + qq + theta; }
+};
+
 // threads of the Q-Q kernel's block (one block per system)
 #define QQ_THREADS 1024
 // polarisation restraint: threads per block of the angle kernel (one per
@@ -793,40 +848,21 @@ inline int qforces_blocks(int nq, int chunks, int W) { return 8 * ((chunks + W -
 #define WP_THREADS 256
 #define WP_CHUNK 1024
 
+// at most FC_WPB wavefronts per block of the solvent-receiver kernels
 #define FC_WPB 8
+// largest charge group (atoms)
 #ifndef FC_CAP
 #define FC_CAP 384
 #endif
-#ifndef FC_CH
-#define FC_CH 10
-#endif
-// solute receivers: at most 168 VGPRs, so three waves fit a SIMD (the
-// no-energy FP32 form fits; the energy-sampling and FP64 forms spill a few
-// bytes to scratch)
-#ifndef FC_OCC_ATTR
-#define FC_OCC_ATTR __attribute__((amdgpu_waves_per_eu(3)))
-#endif
+// partner-atom entries (DevSys::alist): atom index and flags
+enum : int { AL_ATOM = (1 << 28) - 1, AL_OWN = 1 << 28, AL_SELF = 1 << 29 };
+// Solute-receiver force kernel (k_sforces): receiver atoms per sweep, at most
+// as many as the scalar registers hold (6 values of R each), and per-wave LDS
 template <typename R>
-__host__ __device__ constexpr size_t fc_wave_bytes() {
-  return ((sizeof(R) * (3 * (2 * FC_CAP + FC_CH) + 9 * FC_CH) + sizeof(double) * FC_CH +
-           sizeof(int) * (2 * FC_CAP + 4 * FC_CH)) + 15) / 16 * 16;
-}
-// type tables of the solute-solute parameters held in LDS up to this many types
-// Water-receiver force kernel (k_wforces): solute partner atoms are staged in
-// rounds of at most CAP slots per wave (WF_CAP_SMALL when every solute group
-// of the launch fits, else FC_CAP); partner waters need no staging.
-#define WF_CAP_SMALL 128
-// per-wave LDS of the solute-receiver kernel (k_sforces) with CAP partner
-// slots: partner offsets, the sweep's receiver data, the partners' LJ and
-// charge factors, then partner indices and tags and receiver records
-template <typename R, int CAP>
-__host__ __device__ constexpr size_t sf_wave_bytes() {
-  return ((sizeof(R) * (3 * (2 * CAP + FC_CH) + 9 * FC_CH) + sizeof(double) * FC_CH +
-           sizeof(int) * (2 * CAP + 4 * FC_CH)) + 15) / 16 * 16;
-}
-template <typename R, int CAP>
-__host__ __device__ constexpr size_t wf_wave_bytes() {
-  return (sizeof(R) * 3 * CAP + sizeof(int) * 2 * CAP + 15) / 16 * 16;
+__host__ __device__ constexpr int so_ch() { return sizeof(R) == 4 ? 10 : 5; }
+template <typename R>
+__host__ __device__ constexpr size_t so_wave_bytes() {
+  return (so_ch<R>() * (sizeof(double) + 11 * sizeof(R) + 3 * sizeof(int)) + 15) / 16 * 16;
 }
 
 // Placement of a batch's blocks on the XCDs.  Blocks are dealt to the 8 XCDs
@@ -855,14 +891,6 @@ inline int max_solute_group(const int* gfirst, const int* glast, int ncgp_solute
   int m = 0;
   for (int g = 0; g < ncgp_solute; g++) m = glast[g] - gfirst[g] + 1 > m ? glast[g] - gfirst[g] + 1 : m;
   return m;
-}
-
-#define FC_MAXT 64
-// static LDS of the solute-receiver force kernel: the LJ factors and the
-// ljcod table of up to FC_MAXT types
-template <typename R>
-__host__ __device__ constexpr size_t fc_static_bytes() {
-  return 2 * 3 * FC_MAXT * sizeof(double) + FC_MAXT * FC_MAXT;
 }
 
 // Adjoint of the per-state Q-atom energies over a set of frames: tangent

@@ -45,6 +45,7 @@ struct DevAlloc {
     return 0;
   }
   void release(void* p) {
+    if (!p) return;
     auto it = std::find(ptrs.begin(), ptrs.end(), p);
     if (it != ptrs.end()) {
       (void)hipFree(p);
@@ -56,6 +57,7 @@ struct DevAlloc {
 // host copies of the topology kept for list export
 struct HostTopo {
   int ntypes = 0, ivdw_rule = 1;
+  int n_nq = 0, max_nq_group = 0;  // non-Q atoms of the solute groups: all, most in one group
   std::vector<int> gfirst, glast, gswitch, cgpatom, iqatom, iac, ljcod, lx_off, lx_j, iqseq;
   std::vector<uint8_t> excl, qconn3, lx_kind;
   std::vector<uint32_t> exmask, m14mask;
@@ -70,8 +72,22 @@ void fill_params(DevSys& S, const qnb_system* s, const qnb_params* p);
 int topo_build(DevSys& S, const qnb_system* s, HostTopo& T, DevAlloc& M);
 // host twin of the device solute-solute filter (pp_param), for list export
 bool host_pp_param(const HostTopo& T, int i, int j);
+// the force pass of a small launch as one kernel (k_forces_small): the grid
+// for systems of at most these sizes (pol: the polarisation angles too), and
+// the launch
+SmallGrid small_grid(int solute_groups, int nwat, int sa, int nqat, int nat_solute, int nqe, uint32_t mask, bool pol);
+void launch_forces_small(hipStream_t st, int prec, int ns_max, bool energy, const SmallGrid& G, int B,
+                         const DevSys* dsys, uint32_t mask, const int* istep);
+// whether a force pass over so many receivers (of all instances) takes that
+// kernel
+bool small_launch(long solute_groups, long solvent);
+// polarisation restraint: angles and shells (theta), ranks and forces, and
+// the per-system sums (finish) where no later kernel of the caller runs them
+void launch_watpol(hipStream_t st, int nwat, int B, const DevSys* dsys, const int* istep, bool theta, bool finish);
 // per-instance device state (coordinates, gradient, lists, LRF, energies)
-int instance_alloc(DevSys& S, DevAlloc& M, const qnb_params* p, int nslots);
+int instance_alloc(DevSys& S, const HostTopo& T, DevAlloc& M, const qnb_params* p, int nslots);
+// neighbour rows of `cap` groups and the partner-atom rows that hold them
+int row_alloc(DevSys& S, const HostTopo& T, DevAlloc& M, int cap);
 // group contributions (qnb_exc.hip): the pair lists of each energy array
 // and state, built on the host from the system's Q tables
 struct ExcHost {

@@ -9,7 +9,7 @@
 // pair is exported in.  Q-atoms, whose partners are all waters and solute
 // atoms within Rcq, are the one many-to-one case: their forces are summed per
 // wavefront and added with one atomic per wave and component.
-#include "qnb_dev.h"
+#include "qnb_host.h"
 
 namespace qnb {
 
@@ -334,7 +334,7 @@ __global__ __launch_bounds__(512) void k_lists_lrf(const DevSys* __restrict__ sy
   double acc[20];
 #pragma unroll
   for (int k = 0; k < 20; k++) acc[k] = 0.0;
-  int count = 0;
+  int count = 0, count_sol = 0;
   int* __restrict__ row = S.nbr + (size_t)a * S.cap;
   // mixed path: the lane's raw FP32 sums since the last flush to the FP64
   // expansion, flushed after a chunk once a lane has been offered LRF_FLUSH
@@ -384,6 +384,7 @@ __global__ __launch_bounds__(512) void k_lists_lrf(const DevSys* __restrict__ sy
       const int pos = count + __popcll(m & ((1ull << lane) - 1ull));
       if (in && pos < S.cap) stg(row + pos, b);
       count += __popcll(m);
+      if (b0 < S.ncgp_solute) count_sol += __popcll(__ballot(in && b < S.ncgp_solute));
       const uint64_t fw = __ballot(far);
       if (fw != 0) {
         // the chunk's atoms: the run from b0's first to its last group's last
@@ -424,6 +425,7 @@ __global__ __launch_bounds__(512) void k_lists_lrf(const DevSys* __restrict__ sy
   for (int k = 0; k < 20; k++) acc[k] = wave_sum_all(acc[k]);
   if (lane == 0) {
     S.nnbr[a] = count;
+    S.nnsol[a] = count_sol;
     if (count > S.cap) atomicMax(S.need, count);
     double* L = S.lrf + (size_t)QNB_NLRF * a;
     L[0] = cx;
@@ -524,22 +526,9 @@ enum : uint32_t { T_WW = QNB_T_WW, T_QW = QNB_T_QW, T_PW = QNB_T_PW, T_PP = QNB_
 // pp_param (nonbond_pp 4694-4760).  Writes (not adds) d for every atom of a,
 // and the wave's energy partials into epart[a] on the sampled steps.
 
-// Partner staging: the wave takes up to 64 neighbour groups whose atoms fit
-// in FC_CAP slots (wave prefix sum over the groups' atom counts; groups
-// larger than FC_CAP are refused at set-up) and writes, per partner atom,
-// its index, its position relative to the receiver's reference atom (formed
-// in FP64, rounded to R) and a tag: bits 0-1 the atom's rank in its group,
-// bit 2 solute partner, bit 3 the receiver owns the group pair's energy,
-// bit 4 a Q-atom (its pairs belong to the Q kernels).  Returns the number of
-// staged atoms; *ngroups receives the number of groups consumed.
-#define FT_SOL 4
-#define FT_OWN 8
-#define FT_Q 16
-#define FT_FAR 32  // solute partner group that holds no excluded or 1-4 pair with the receiver group
 // pp_param from data at hand: the two atoms' types, charges and exclusion
 // masks (bit 31: partners beyond the 25-atom window, looked up in the long
-// list) and the type tables (LJ factors, ljcod) in LDS.  Same result as
-// pp_param.
+// list).  Same result as pp_param.
 // the pair (lo, hi) in lo's long exclusion / 1-4 list: 1 excluded, 2 1-4,
 // 0 neither (kept out of line: rare, and its loop would stop the callers'
 // receiver-atom loops from unrolling)
@@ -553,38 +542,40 @@ __device__ __noinline__ int long_pair_kind(const DevSys& S, int lo, int hi) {
   return ex ? 1 : (is14 ? 2 : 0);
 }
 
+// the pair (i, j) from the atoms' exclusion and 1-4 masks: 1 excluded, 2 1-4,
+// 0 neither
+__device__ __forceinline__ int pair_kind(const DevSys& S, int i, uint32_t xi, uint32_t mi, int j, uint32_t xj,
+                                         uint32_t mj) {
+  const bool il = i < j;
+  const int dk = il ? j - i : i - j;
+  const uint32_t xm = il ? xi : xj, m14 = il ? mi : mj;
+  if (dk <= 25) {
+    const uint32_t bit = 1u << (dk - 1);
+    return (xm & bit) ? 1 : ((m14 & bit) ? 2 : 0);
+  }
+  return (xm >> 31) ? long_pair_kind(S, il ? i : j, il ? j : i) : 0;
+}
+
 struct PPAtom {
   int i, t;
   uint32_t xm, m14;
   double q;
 };
-__device__ __forceinline__ bool pp_param_fast(const DevSys& S, const PPAtom& P, const PPAtom& Q,
-                                              const double* __restrict__ avdw, const double* __restrict__ bvdw,
-                                              const uint8_t* __restrict__ ljc, double& A, double& B, double& el) {
-  const bool pl = P.i < Q.i;
-  const int dk = pl ? Q.i - P.i : P.i - Q.i;
-  const uint32_t xm = pl ? P.xm : Q.xm, m14 = pl ? P.m14 : Q.m14;
-  bool is14 = false;
-  if (dk <= 25) {
-    const uint32_t bit = 1u << (dk - 1);
-    if (xm & bit) return false;
-    is14 = (m14 & bit) != 0;
-  } else if (xm >> 31) {
-    const int lo = pl ? P.i : Q.i, hi = pl ? Q.i : P.i;
-    const int kind = long_pair_kind(S, lo, hi);
-    if (kind == 1) return false;
-    is14 = kind == 2;
-  }
-  const int vdw = is14 ? 3 : ljc[P.t + Q.t * S.ntypes];
-  const int k = vdw - 1;
+__device__ __forceinline__ bool pp_pair(const DevSys& S, const PPAtom& P, const PPAtom& Q, double& A, double& B,
+                                        double& el) {
+  const int kind = pair_kind(S, P.i, P.xm, P.m14, Q.i, Q.xm, Q.m14);
+  if (kind == 1) return false;
+  const bool is14 = kind == 2;
+  const int vdw = is14 ? 3 : ldg(S.ljcod + (P.t + Q.t * S.ntypes));
+  const int kp = P.t * 3 + vdw - 1, kq = Q.t * 3 + vdw - 1;
   if (S.ivdw_rule == 1) {
-    A = avdw[P.t * 3 + k] * avdw[Q.t * 3 + k];
-    B = bvdw[P.t * 3 + k] * bvdw[Q.t * 3 + k];
+    A = ldg(S.avdw + kp) * ldg(S.avdw + kq);
+    B = ldg(S.bvdw + kp) * ldg(S.bvdw + kq);
   } else {
-    double tA = avdw[P.t * 3 + k] + avdw[Q.t * 3 + k];
+    double tA = ldg(S.avdw + kp) + ldg(S.avdw + kq);
     tA = tA * tA;
     tA = tA * tA * tA;
-    double tB = bvdw[P.t * 3 + k] * bvdw[Q.t * 3 + k];
+    double tB = ldg(S.bvdw + kp) * ldg(S.bvdw + kq);
     A = (tA * tA) * tB;
     B = 2.0 * tA * tB;
   }
@@ -594,448 +585,428 @@ __device__ __forceinline__ bool pp_param_fast(const DevSys& S, const PPAtom& P, 
   return set;
 }
 
-template <typename R, int CAP = FC_CAP, bool PPF = false>
-__device__ __forceinline__ int stage_partners(const DevSys& S, int a, const int* __restrict__ row, int p0, int nn,
-                                              uint32_t use_sol, uint32_t use_wat, double xr0, double xr1,
-                                              double xr2, int* s_j, R (*s_d)[3], int* s_t, int* ngroups,
-                                              R (*s_f)[3] = nullptr) {
-  const int lane = threadIdx.x % QNB_WAVE;
-  const int p = p0 + lane;
-  int b = -1, cnt = 0, f0 = 0;
-  if (p < nn) {
-    b = ldg(row + p);
-    if (b < S.ncgp_solute ? use_sol : use_wat) {
-      f0 = ldg(S.gfirst + b);
-      cnt = ldg(S.glast + b) - f0 + 1;
-    }
+// ---------------------------------------------------------------------------
+// The lambda-weighted dv of a Q pair over its states (nbe_qx per state,
+// nonbonded.f90:200-222): `par(s)` gives state s's A, B, el and soft-core score.
+// Without a soft core the force is linear in A, B and el, so on the steps that
+// sample no energies the states' parameters are weighted and summed first and
+// the pair is evaluated once.
+template <typename R>
+struct QPar {
+  R A, B, q, sc;
+};
+template <typename R, int NS, typename F>
+__device__ __forceinline__ R qx_states(const DevSys& S, R r2, R r, int ns, double* eq, bool want, F par) {
+  const R r6 = r2 * r2 * r2;
+  QPar<R> p[NS];
+  R A = R(0), B = R(0), q = R(0);
+  bool soft = false;
+#pragma unroll
+  for (int s = 0; s < NS; s++) {
+    if (s >= ns) break;
+    p[s] = par(s);
+    const R lam = (R)S.lambda[s];
+    A += lam * p[s].A;
+    B += lam * p[s].B;
+    q += lam * p[s].q;
+    soft = soft || p[s].sc != R(0);
   }
-  int incl = cnt;
+  if (!want && !soft) return r2 * (r6 * (R(6) * B - R(12) * A * r6) - q * r);
+  R dvs = R(0);
 #pragma unroll
-  for (int o2 = 1; o2 < QNB_WAVE; o2 <<= 1) {
-    const int v = __shfl_up(incl, o2, QNB_WAVE);
-    if (lane >= o2) incl += v;
+  for (int s = 0; s < NS; s++) {
+    if (s >= ns) break;
+    dvs += PairMath<R>::nbe_qx(r2, r, r6, p[s].A, p[s].B, p[s].q, p[s].sc, (R)S.lambda[s], eq[2 * s], eq[2 * s + 1],
+                               want);
   }
-  // inclusive sums never decrease, so the groups that fit are a prefix
-  const int ng = __popcll(__ballot(incl <= CAP));
-  *ngroups = ng;
-  if (ng == 0) return 0;
-  const int total = __shfl(incl, ng - 1, QNB_WAVE);
-  // every group of the batch skipped by the term mask: nothing staged (the
-  // slots below hold nothing of this batch)
-  if (total == 0) return 0;
-  // the group lanes lay out their slots (LDS only): position in cgpatom and
-  // the group part of the tag (FT_FAR for a solute group whose atoms are all
-  // more than 25 indices from the solute receiver's, neither group having
-  // long-range exclusion / 1-4 partners)
-  if (lane < ng && cnt > 0) {
-    int tag0 = (b < S.ncgp_solute ? FT_SOL : 0) | (owns(a, b) ? FT_OWN : 0);
-    if (b < S.ncgp_solute && a < S.ncgp_solute && !ldg(S.glong + a) && !ldg(S.glong + b)) {
-      const int alo = ldg(S.gspan + 2 * a), ahi = ldg(S.gspan + 2 * a + 1);
-      const int blo = ldg(S.gspan + 2 * b), bhi = ldg(S.gspan + 2 * b + 1);
-      if (blo - ahi > 25 || alo - bhi > 25) tag0 |= FT_FAR;
-    }
-    for (int m = 0, slot = incl - cnt; m < cnt; m++, slot++) {
-      s_j[slot] = f0 + m;
-      s_t[slot] = tag0 | (m & 3);
-    }
+  return dvs;
+}
+// Coulomb only (nbe_qspc, nonbonded.f90:226-243: an SPC hydrogen)
+template <typename R, int NS, typename F>
+__device__ __forceinline__ R qspc_states(const DevSys& S, R r2, R r, int ns, double* eq, bool want, F el) {
+  R q = R(0);
+#pragma unroll
+  for (int s = 0; s < NS; s++) {
+    if (s >= ns) break;
+    const R e = el(s);
+    if (want) eq[2 * s] += (double)(e * r);
+    q += (R)S.lambda[s] * e;
   }
-  __builtin_amdgcn_wave_barrier();
-  // every lane then fills slots lane, lane + 64, ...: FC_SPR slots per round,
-  // all atom-index loads of the round first, then all position loads, so the
-  // loads of a round are in flight together (slots past the end load the
-  // receiver's first atom, a valid index, and store nothing)
-  constexpr int FC_SPL = (CAP + QNB_WAVE - 1) / QNB_WAVE;
-  constexpr int FC_SPR = FC_SPL % 3 == 0 ? 3 : (FC_SPL % 2 == 0 ? 2 : 1);
-  static_assert(FC_SPL % FC_SPR == 0, "staging rounds must cover the slots");
-  const int pos_pad = ldg(S.gfirst + a);
-#pragma unroll
-  for (int u0 = 0; u0 < FC_SPL; u0 += FC_SPR) {
-    int jj[FC_SPR], tg[FC_SPR], qa[FC_SPR];
-    double px[FC_SPR][3];
-#pragma unroll
-    for (int u = 0; u < FC_SPR; u++) {
-      const int k = lane + (u0 + u) * QNB_WAVE;
-      const bool in = k < total;
-      tg[u] = in ? s_t[k] : 0;
-      jj[u] = ldg(S.cgpatom + (in ? s_j[k] : pos_pad));
-    }
-    R pf[FC_SPR][3];
-#pragma unroll
-    for (int u = 0; u < FC_SPR; u++) {
-      const int j = jj[u];
-      px[u][0] = ldg(S.x + 3 * j);
-      px[u][1] = ldg(S.x + 3 * j + 1);
-      px[u][2] = ldg(S.x + 3 * j + 2);
-      qa[u] = ldg(S.iqatom + j);
-      if constexpr (PPF) {
-        // the solute partner's LJ factors and charge (ppf / ppd rows); the
-        // row of the receiver's first atom stands in for a solvent atom
-        const int jp = j < S.nat_solute ? j : ldg(S.cgpatom + pos_pad);
-        const R* t = qp_tab<R>(S.ppd, S.ppf) + 4 * (size_t)jp;
-        pf[u][0] = ldg(t);
-        pf[u][1] = ldg(t + 1);
-        pf[u][2] = ldg(t + 2);
-      }
-    }
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-    for (int u = 0; u < FC_SPR; u++) {
-      const int k = lane + (u0 + u) * QNB_WAVE;
-      if (k < total) {
-        s_j[k] = jj[u];
-        s_d[k][0] = (R)(px[u][0] - xr0);
-        s_d[k][1] = (R)(px[u][1] - xr1);
-        s_d[k][2] = (R)(px[u][2] - xr2);
-        s_t[k] = tg[u] | (((tg[u] & FT_SOL) && qa[u] != 0) ? FT_Q : 0);
-        if constexpr (PPF) {
-          s_f[k][0] = pf[u][0];
-          s_f[k][1] = pf[u][1];
-          s_f[k][2] = pf[u][2];
-        }
-      }
-    }
-  }
-  __builtin_amdgcn_wave_barrier();
-  return total;
+  return -r2 * r * q;
+}
+// entry (iq, k, s) of the Q-solvent table in the pair arithmetic's type
+template <typename R>
+__device__ __forceinline__ QPar<R> qw_par(const DevSys& S, int iq, int k, int s) {
+  const R* t = qp_tab<R>(S.qw_d, S.qw_f) + 4 * ((size_t)(iq * S.sa + k) * S.nstates + s);
+  return QPar<R>{ldg(t), ldg(t + 1), ldg(t + 2), ldg(t + 3)};
+}
+template <typename R>
+__device__ __forceinline__ R qw_el(const DevSys& S, int iq, int k, int s) {
+  return ldg(qp_tab<R>(S.qw_d, S.qw_f) + 4 * ((size_t)(iq * S.sa + k) * S.nstates + s) + 2);
 }
 
 // ---------------------------------------------------------------------------
-// Solute receivers: one wavefront per solute charge group a, its atoms taken
-// in sweeps of up to CH (receiver data in LDS and registers).  The row is
-// sorted, so the partner solute groups come first and the waters after them.
-// Per sweep:
-//  * partner solute groups through the staged atom expansion, one partner
-//    atom per lane against the sweep's receiver atoms (nonbond_pp,
-//    nonbondene.f90:4694-4760).  A group that can hold no excluded or 1-4
-//    pair with a (FT_FAR) takes A, B and qq as products of per-atom factors
-//    when the system uses the geometric rule with LJ code 1 throughout
-//    (ppfast): the products pp_param forms for such a pair, same operands;
-//    every other pair goes through pp_param (exclusions, 1-4, ljcod, rule);
-//  * partner waters with the fixed mapping of k_wforces (lane l takes site
-//    l % 3 of water l / 3 of the round), the pw parameters of that site for
-//    every receiver atom held in registers (nonbond_pw 4856-4916);
-//  * the pairs inside the group (ig == jgr, i < j, nonbondene.f90:1610) and
-//    the receiver side of the Q-atom - solute pairs (nonbond_qp 5157-5230).
-// Writes d of the group's atoms, and the wave's pp, pw and qp energy
-// partials on the sampled steps (a pp pair's energy on its owner side).
-template <typename R, int NS, bool E, int CAP>
-__global__ __launch_bounds__(64 * FC_WPB) FC_OCC_ATTR void k_sforces(const DevSys* __restrict__ systems, uint32_t mask,
-                                                                     int imap, int nb, int ninst) {
-  int inst, blk;
-  if (!map_block(imap, nb, ninst, inst, blk)) return;
-  const DevSys& S = systems[inst];
-  const int wib = threadIdx.x / QNB_WAVE;
-  const int a = __builtin_amdgcn_readfirstlane(blk * (int)(blockDim.x / QNB_WAVE) + wib);
-  // LJ factor and ljcod tables in LDS (every thread of the block takes part
-  // before any wave leaves)
-  __shared__ double s_avdw[3 * FC_MAXT], s_bvdw[3 * FC_MAXT];
-  __shared__ uint8_t s_ljc[FC_MAXT * FC_MAXT];
-  const bool lds_types = S.ntypes <= FC_MAXT;
-  if (lds_types) {
-    const int nt = S.ntypes;
-    for (int k = threadIdx.x; k < 3 * nt; k += blockDim.x) {
-      s_avdw[k] = ldg(S.avdw + k);
-      s_bvdw[k] = ldg(S.bvdw + k);
+// Partner atoms of every receiver group, written after each list update and
+// read by the force kernels of every step until the next one: the row's solute
+// groups (and, for a solute receiver, the group itself) as atoms, Q-atoms left
+// out (their pairs belong to the Q kernels).  One wavefront per receiver, lane
+// = partner group.  Row a of S.alist holds from its front the atoms of groups
+// that can hold an excluded or 1-4 pair with a solute receiver (an index
+// within 25 of the receiver's, long-range partners in either group, or the
+// group itself), from its back downwards the others; the counts go to
+// alist_n.  An entry is the atom's index with AL_OWN (the receiver owns the
+// energy of the two groups' pairs) and AL_SELF (the receiver's own group).
+// The force kernels then read one coalesced list per receiver instead of
+// walking group -> atoms -> positions through LDS at every step.
+__global__ __launch_bounds__(256) void k_expand(const DevSys* __restrict__ systems) {
+  const DevSys& S = systems[blockIdx.y];
+  const int a = uni(blockIdx.x * (blockDim.x / QNB_WAVE) + threadIdx.x / QNB_WAVE);
+  if (a >= S.ncgp) return;
+  const int lane = threadIdx.x % QNB_WAVE, ncs = S.ncgp_solute;
+  const bool a_sol = a < ncs;
+  const int nsr = uni(min(ldg(S.nnsol + a), S.cap));
+  const int* __restrict__ row = S.nbr + (size_t)a * S.cap;
+  int* __restrict__ out = S.alist + (size_t)a * S.acap;
+  const bool along = a_sol && ldg(S.glong + a);
+  const int alo = a_sol ? ldg(S.gspan + 2 * a) : 0, ahi = a_sol ? ldg(S.gspan + 2 * a + 1) : 0;
+  int near = 0, far = 0;
+  // index nsr stands for the receiver itself
+  const int nv = nsr + (a_sol && !ldg(S.excl + ldg(S.gswitch + a)) ? 1 : 0);
+  for (int v0 = 0; v0 < nv; v0 += QNB_WAVE) {
+    const int v = v0 + lane;
+    int off = 0, cnt = 0, tag = 0;
+    bool isnear = false;
+    if (v < nv) {
+      const int b = v < nsr ? ldg(row + v) : a;
+      off = ldg(S.nqoff + b);
+      cnt = ldg(S.nqoff + b + 1) - off;
+      tag = owns(a, b) ? AL_OWN : 0;
+      if (b == a) {
+        tag = AL_SELF;
+        isnear = true;
+      } else if (a_sol) {
+        const int blo = ldg(S.gspan + 2 * b), bhi = ldg(S.gspan + 2 * b + 1);
+        isnear = along || ldg(S.glong + b) || !(blo - ahi > 25 || alo - bhi > 25);
+      }
     }
-    for (int k = threadIdx.x; k < nt * nt; k += blockDim.x) s_ljc[k] = (uint8_t)ldg(S.ljcod + k);
+    int in = isnear ? cnt : 0, fa = isnear ? 0 : cnt;
+#pragma unroll
+    for (int o = 1; o < QNB_WAVE; o <<= 1) {
+      const int u = __shfl_up(in, o, QNB_WAVE), w = __shfl_up(fa, o, QNB_WAVE);
+      if (lane >= o) {
+        in += u;
+        fa += w;
+      }
+    }
+    int pos = isnear ? near + in - cnt : S.acap - 1 - (far + fa - cnt);
+    const int step = isnear ? 1 : -1;
+    for (int m = 0; m < cnt; m++, pos += step) stg(out + pos, ldg(S.nqatom + off + m) | tag);
+    near += __shfl(in, QNB_WAVE - 1, QNB_WAVE);
+    far += __shfl(fa, QNB_WAVE - 1, QNB_WAVE);
   }
+  if (lane == 0) {
+    S.alist_n[2 * a] = near;
+    S.alist_n[2 * a + 1] = far;
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Solute receivers: one wavefront per solute charge group a, or, in a small
+// launch (SPLIT), the four waves of a block, each with a quarter of a's
+// partners.  a's atoms are taken in sweeps of up to SO_CH; they are the same
+// for every lane and live in scalar registers, and a lane takes one partner at
+// a time against them, the next partner's data in flight meanwhile:
+//  * solute partners from the receiver's atom list (k_expand; nonbond_pp,
+//    nonbondene.f90:4694-4760): the atoms of groups without an excluded or 1-4
+//    pair take A, B and qq as products of per-atom factors when the system
+//    uses the geometric rule with LJ code 1 throughout (ppfast): the products
+//    pp_param forms for such a pair, same operands; every other pair, those
+//    inside a included (ig == jgr, i < j, nonbondene.f90:1610), goes through
+//    pp_param (exclusions, 1-4, ljcod, rule);
+//  * solvent partners, a lane per molecule, its sites in turn (nonbond_pw
+//    4856-4916; a site without LJ parameters takes Coulomb only);
+//  * the receiver side of the Q-atom - solute pairs (nonbond_qp 5157-5230).
+// Writes d of the group's atoms, and the pp, pw and qp energy partials on the
+// sampled steps (a pp pair's energy on its owner side).
+//
+// Bound by VALU issue at 51 windows and by the latency of one row in a small
+// launch.  Staging 128 partners at a time through LDS, with ten receiver atoms
+// in vector registers (167 of them, three waves per SIMD), took 213 us at 51
+// windows of 400 ten-atom groups and 52 us for one FP64 window; staging by
+// blocks of four waves 310 us at 51 windows (its barriers wait on four chains
+// of loads); from the atom lists it takes 156 us, and 20 us split four ways.
+
+// per-pair LJ + Coulomb with the factors 12 and 6 already in A and B: returns
+// nbe's dv
+template <typename R>
+__device__ __forceinline__ R pair_dv(R ux, R uy, R uz, R A12, R B6, R q, R& el, R& vdw, bool want) {
+  R r2, r;
+  rinv(ux * ux + uy * uy + uz * uz, r2, r);
+  const R r6 = r2 * r2 * r2;
+  const R Vel = q * r;
+  if (want) {
+    el += Vel;
+    vdw += A12 * (r6 * r6) * R(1.0 / 12.0) - B6 * r6 * R(1.0 / 6.0);
+  }
+  return r2 * (r6 * (B6 - A12 * r6) - Vel);
+}
+
+__device__ __forceinline__ float lane_get(float v, int lane) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+__device__ __forceinline__ double lane_get(double v, int lane) { return lane_value(v, lane); }
+__device__ __forceinline__ int lane_get(int v, int lane) { return __builtin_amdgcn_readlane(v, lane); }
+
+// the sum of each lane's value over waves w0 .. w0 + n - 1 of the block, in
+// wave order; every wave of the block takes part
+__device__ __forceinline__ double waves_sum(double (*comb)[QNB_WAVE], double v, int w0, int n, int lane) {
   __syncthreads();
-  if (a >= S.ncgp_solute) return;
+  comb[threadIdx.x / QNB_WAVE][lane] = v;
+  __syncthreads();
+  double s = comb[w0][lane];
+  for (int w = 1; w < n; w++) s += comb[w0 + w][lane];
+  return s;
+}
+
+template <typename R, int NS, bool E, bool SPLIT>
+__device__ __forceinline__ void solute_receiver(const DevSys& S, uint32_t mask, int a, int wave, int waves,
+                                                unsigned char* wbase, double (*comb)[QNB_WAVE]) {
+  constexpr int CH = so_ch<R>();
   const int lane = threadIdx.x % QNB_WAVE;
-  extern __shared__ __align__(16) unsigned char fc_smem[];
-  unsigned char* wbase = fc_smem + (size_t)wib * sf_wave_bytes<R, CAP>();
-  R(*s_pd)[3] = reinterpret_cast<R(*)[3]>(wbase);
-  R(*s_o)[3] = reinterpret_cast<R(*)[3]>(wbase + sizeof(R) * 3 * CAP);
-  R(*s_pw)[3][3] = reinterpret_cast<R(*)[3][3]>(wbase + sizeof(R) * 3 * (CAP + FC_CH));
-  R(*s_pf)[3] = reinterpret_cast<R(*)[3]>(wbase + sizeof(R) * (3 * (CAP + FC_CH) + 9 * FC_CH));
-  double* s_rq = reinterpret_cast<double*>(wbase + sizeof(R) * (3 * (2 * CAP + FC_CH) + 9 * FC_CH));
-  int* s_pj = reinterpret_cast<int*>(s_rq + FC_CH);
-  int* s_pt = s_pj + CAP;
-  int* s_ia = s_pt + CAP;
-  int* s_rt = s_ia + FC_CH;
-  uint32_t* s_rx = reinterpret_cast<uint32_t*>(s_rt + FC_CH);
-  uint32_t* s_rm = s_rx + FC_CH;
+  // the sweep's receiver data that only the rarer pairs need, in LDS: charge,
+  // solute-solvent parameters of the three water sites, LJ factors of code 3,
+  // type, masks
+  double* s_rq = reinterpret_cast<double*>(wbase);
+  R(*s_pw)[11] = reinterpret_cast<R(*)[11]>(s_rq + CH);
+  int* s_rt = reinterpret_cast<int*>(s_pw + CH);
+  uint32_t* s_rx = reinterpret_cast<uint32_t*>(s_rt + CH);
+  uint32_t* s_rm = s_rx + CH;
   const double* __restrict__ x = S.x;
   const auto d = gpm(S.d);
-  const int nn = min(ldg(S.nnbr + a), S.cap);
+  const int nn = uni(min(ldg(S.nnbr + a), S.cap)), nsr = uni(min(ldg(S.nnsol + a), nn));
   const int* __restrict__ row = S.nbr + (size_t)a * S.cap;
+  const int* __restrict__ al = S.alist + (size_t)a * S.acap;
+  const int acap = S.acap;
   const bool want_e = E && want_energies(S);
   const int nsol = S.nat_solute, sa = S.sa, ncs = S.ncgp_solute;
-  const int ra = ldg(S.gswitch + a);
-  const bool aexcl = ldg(S.excl + ra);
-  const bool fast = S.ppfast != 0;
+  const int ra = uni(ldg(S.gswitch + a));
+  const bool aexcl = uni(ldg(S.excl + ra));
+  const bool fast = S.ppfast != 0, coul_h = S.pw_coul_h != 0;
   double e_ppel = 0.0, e_ppvdw = 0.0, e_pwel = 0.0, e_pwvdw = 0.0;
   double eq[2 * NS];  // per state: qp_el, qp_vdw
 #pragma unroll
   for (int k = 0; k < 2 * NS; k++) eq[k] = 0.0;
-  const double xr0 = ldg(x + (3 * ra)), xr1 = ldg(x + (3 * ra + 1)), xr2 = ldg(x + (3 * ra + 2));
-  const int g0 = ldg(S.gfirst + a), na = ldg(S.glast + a) - g0 + 1;
+  const double xr0 = ldg(x + 3 * ra), xr1 = ldg(x + 3 * ra + 1), xr2 = ldg(x + 3 * ra + 2);
+  const int g0 = uni(ldg(S.gfirst + a)), na = uni(ldg(S.glast + a)) - g0 + 1;
   const int nq = S.nqat, ns = S.nstates;
-  // length of the row's solute prefix
-  int nsr = 0;
-  for (int p0 = 0; p0 < nn; p0 += QNB_WAVE) {
-    const int p = p0 + lane;
-    const uint64_t m = __ballot(p < nn && ldg(row + p) < ncs);
-    nsr += __popcll(m);
-    if (m != ~0ull) break;
-  }
-  const bool qin = (mask & T_QP) && nq > 0 && ldg(S.qp_in + a);
-  constexpr int CH = sizeof(R) == 4 ? FC_CH : FC_CH / 2;
-  for (int c0 = 0; c0 < na; c0 += CH) {
-    const int nk = min(CH, na - c0);
-    // receiver atoms of this sweep in LDS: index (-1: takes no pair terms)
-    // and offset from the reference atom
+  const bool qin = (mask & T_QP) && nq > 0 && uni(ldg(S.qp_in + a));
+  const bool pp = (mask & T_PP) && !aexcl;
+  const int n_near = pp ? uni(ldg(S.alist_n + 2 * a)) : 0, n_far = pp ? uni(ldg(S.alist_n + 2 * a + 1)) : 0;
+  const bool pw = (mask & T_PW) && !aexcl && nsr < nn;
+  // SPLIT: sets of waves with receiver atoms of their own (nset), the waves of
+  // a set sharing the partners
+  const int nset = !SPLIT || na <= CH ? 1 : (na <= 2 * CH ? 2 : 4), parts = SPLIT ? waves / nset : 1;
+  const int set = SPLIT ? wave / parts : 0, part = SPLIT ? wave % parts : 0;
+  // the first far partners' entries, and the first of their positions, are
+  // requested before the receiver's own chain of loads
+  const int t0 = lane + QNB_WAVE * part;
+  auto far_entry = [&](int t) { return t < n_far ? ldg(al + (acap - 1 - t)) : ra; };
+  const int e0 = fast ? far_entry(t0) : ra, e1 = fast ? far_entry(t0 + QNB_WAVE * parts) : ra;
+  for (int cb = 0; cb < na; cb += nset * CH) {
+    const int c0 = cb + set * CH, nk = max(0, min(CH, na - c0));
+    // receiver atoms: lane k loads atom c0 + k (index -1: takes no pair
+    // terms), then each value is read into scalar registers
+    int il = -1, i_own = 0;
+    R ol0 = R(0), ol1 = R(0), ol2 = R(0), fa = R(0), fb = R(0), fc = R(0);
     if (lane < nk) {
       const int i = ldg(S.cgpatom + (g0 + c0 + lane));
-      s_ia[lane] = (!aexcl && ldg(S.iqatom + i) == 0) ? i : -1;
-      s_o[lane][0] = (R)(ldg(x + (3 * i)) - xr0);
-      s_o[lane][1] = (R)(ldg(x + (3 * i + 1)) - xr1);
-      s_o[lane][2] = (R)(ldg(x + (3 * i + 2)) - xr2);
+      i_own = i;
+      il = (!aexcl && ldg(S.iqatom + i) == 0) ? i : -1;
+      ol0 = (R)(ldg(x + 3 * i) - xr0);
+      ol1 = (R)(ldg(x + 3 * i + 1) - xr1);
+      ol2 = (R)(ldg(x + 3 * i + 2) - xr2);
+      const R* pf = qp_tab<R>(S.ppd, S.ppf) + PP_REC * (size_t)i;
+      fa = R(12) * ldg(pf);
+      fb = R(6) * ldg(pf + 1);
+      fc = ldg(pf + 2);
       s_rt[lane] = ldg(S.iac + i);
       s_rx[lane] = ldg(S.exmask + i);
       s_rm[lane] = ldg(S.m14mask + i);
       s_rq[lane] = ldg(S.crg + i);
-      // the atom's solute-water parameters against the 3 water sites
-      if (S.nwat > 0 && sa == 3)
+      s_pw[lane][9] = R(12) * ldg(pf + 4);
+      s_pw[lane][10] = R(6) * ldg(pf + 5);
+      if (pw && sa == 3)
+#pragma unroll
         for (int kb = 0; kb < 3; kb++) {
           const size_t tt = (size_t)i + (size_t)nsol * kb;
-          s_pw[lane][kb][0] = (R)ldg(S.pwA + tt);
-          s_pw[lane][kb][1] = (R)ldg(S.pwB + tt);
-          s_pw[lane][kb][2] = (R)ldg(S.pwEl + tt);
+          s_pw[lane][3 * kb] = R(12) * (R)ldg(S.pwA + tt);
+          s_pw[lane][3 * kb + 1] = R(6) * (R)ldg(S.pwB + tt);
+          s_pw[lane][3 * kb + 2] = (R)ldg(S.pwEl + tt);
         }
     }
     __builtin_amdgcn_wave_barrier();
-    // the sweep's receiver data in registers: usable flag, offset, per-atom
-    // LJ factors and charge of the fast path
-    bool rok[CH];
-    R ro[CH][3], rA[CH], rB[CH], rQ[CH];
+    int ri[CH];
+    R ro[CH][3], rA[CH], rB[CH], rQ[CH], f[CH][3];
 #pragma unroll
     for (int k = 0; k < CH; k++) {
-      const int i = k < nk ? s_ia[k] : -1;
-      rok[k] = i >= 0;
-      ro[k][0] = s_o[k][0];
-      ro[k][1] = s_o[k][1];
-      ro[k][2] = s_o[k][2];
-      if constexpr (sizeof(R) == 4) {
-        rA[k] = rok[k] ? ldg(S.ppf + 4 * i) : 0.0f;
-        rB[k] = rok[k] ? ldg(S.ppf + 4 * i + 1) : 0.0f;
-        rQ[k] = rok[k] ? ldg(S.ppf + 4 * i + 2) : 0.0f;
-      } else {
-        rA[k] = rok[k] ? ldg(S.ppd + 4 * i) : 0.0;
-        rB[k] = rok[k] ? ldg(S.ppd + 4 * i + 1) : 0.0;
-        rQ[k] = rok[k] ? ldg(S.ppd + 4 * i + 2) : 0.0;
+      ri[k] = lane_get(il, k);
+      ro[k][0] = lane_get(ol0, k);
+      ro[k][1] = lane_get(ol1, k);
+      ro[k][2] = lane_get(ol2, k);
+      rA[k] = lane_get(fa, k);
+      rB[k] = lane_get(fb, k);
+      rQ[k] = lane_get(fc, k);
+      f[k][0] = f[k][1] = f[k][2] = R(0);
+    }
+    // ---- solute partners that may be excluded or 1-4 (all, if !fast)
+    for (int t = t0, n = nk == 0 ? 0 : (fast ? n_near : n_near + n_far); t < n; t += QNB_WAVE * parts) {
+      const int e = ldg(al + (t < n_near ? t : acap - 1 - (t - n_near))), j = e & AL_ATOM;
+      const R dx = (R)(ldg(x + 3 * j) - xr0), dy = (R)(ldg(x + 3 * j + 1) - xr1), dz = (R)(ldg(x + 3 * j + 2) - xr2);
+      const PPAtom Q{j, ldg(S.iac + j), ldg(S.exmask + j), ldg(S.m14mask + j), ldg(S.crg + j)};
+      const R* pf = qp_tab<R>(S.ppd, S.ppf) + PP_REC * (size_t)j;
+      const R qA = ldg(pf), qB = ldg(pf + 1), qQ = ldg(pf + 2), qA3 = ldg(pf + 4), qB3 = ldg(pf + 5);
+      R pel = R(0), pvdw = R(0);
+#pragma unroll
+      for (int k = 0; k < CH; k++) {
+        const int i = ri[k];
+        if (i < 0 || i == j) continue;
+        R A, B, el;
+        if (fast) {
+          // code 1, or 3 for a 1-4 pair: products of per-atom factors again
+          const int kind = pair_kind(S, i, s_rx[k], s_rm[k], j, Q.xm, Q.m14);
+          if (kind == 1) continue;
+          const bool is14 = kind == 2;
+          A = is14 ? s_pw[k][9] * qA3 : rA[k] * qA;
+          B = is14 ? s_pw[k][10] * qB3 : rB[k] * qB;
+          el = rQ[k] * qQ;
+          if constexpr (sizeof(R) == 8)
+            if (!(fabs(A) > R(12.0e-10) || fabs(B) > R(6.0e-10) || fabs(el) > R(1.0e-10))) continue;
+          if (is14) el = el * (R)S.el14;
+        } else {
+          const PPAtom P{i, s_rt[k], s_rx[k], s_rm[k], s_rq[k]};
+          double Ad, Bd, eld;
+          if (!pp_pair(S, P, Q, Ad, Bd, eld)) continue;
+          A = R(12) * (R)Ad;
+          B = R(6) * (R)Bd;
+          el = (R)eld;
+        }
+        const bool acc = want_e && ((e & AL_SELF) ? i < j : (e & AL_OWN) != 0);
+        const R ux = dx - ro[k][0], uy = dy - ro[k][1], uz = dz - ro[k][2];
+        const R dv = pair_dv(ux, uy, uz, A, B, el, pel, pvdw, acc);
+        f[k][0] += ux * dv;
+        f[k][1] += uy * dv;
+        f[k][2] += uz * dv;
+      }
+      if (want_e) {
+        e_ppel += (double)pel;
+        e_ppvdw += (double)pvdw;
       }
     }
-    R f[CH][3];
-#pragma unroll
-    for (int k = 0; k < CH; k++) f[k][0] = f[k][1] = f[k][2] = R(0);
-    if (!aexcl) {
-      // ---- partner solute groups, one staged atom per lane
-      if (mask & T_PP) {
-        for (int p0 = 0, ng = 0; p0 < nsr; p0 += ng) {
-          const int total = stage_partners<R, CAP, true>(S, a, row, p0, nsr, 1u, 0u, xr0, xr1, xr2, s_pj, s_pd, s_pt,
-                                                         &ng, s_pf);
-          if (ng == 0) break;
-          for (int t = lane; t < total; t += QNB_WAVE) {
-            const int tag = s_pt[t], j = s_pj[t];
-            if (tag & FT_Q) continue;
-            const bool acc = want_e && (tag & FT_OWN);
-            const R dx = s_pd[t][0], dy = s_pd[t][1], dz = s_pd[t][2];
-            R pel = R(0), pvdw = R(0);
-            if (fast && (tag & FT_FAR)) {
-              // no exclusion or 1-4 pair possible: A, B, qq from the factors
-              // (staged with the partner)
-              const R pA = s_pf[t][0], pB = s_pf[t][1], pQ = s_pf[t][2];
-#pragma unroll
-              for (int k = 0; k < CH; k++) {
-                if (!rok[k]) continue;
-                const R A = rA[k] * pA, B = rB[k] * pB, el = rQ[k] * pQ;
-                // pp_param's `set` test (QREAL_EPS, src/sizes.f90:50); in FP32
-                // a pair of zero parameters adds exactly zero, so it is skipped
-                // only on the FP64 path
-                if constexpr (sizeof(R) == 8)
-                  if (!(fabs(A) > R(1.0e-10) || fabs(B) > R(1.0e-10) || fabs(el) > R(1.0e-10))) continue;
-                const R ux = dx - ro[k][0], uy = dy - ro[k][1], uz = dz - ro[k][2];
-                const R dv = PairMath<R>::nbe(ux, uy, uz, A, B, el, pel, pvdw, acc);
-                f[k][0] += ux * dv;
-                f[k][1] += uy * dv;
-                f[k][2] += uz * dv;
-              }
-            } else {
-              PPAtom Q{j, 0, 0u, 0u, 0.0};
-              if (lds_types) {
-                Q.t = ldg(S.iac + j);
-                Q.xm = ldg(S.exmask + j);
-                Q.m14 = ldg(S.m14mask + j);
-                Q.q = ldg(S.crg + j);
-              }
-#pragma unroll
-              for (int k = 0; k < CH; k++) {
-                if (!rok[k]) continue;
-                const int i = s_ia[k];
-                double Ad, Bd, eld;
-                bool ok;
-                if (lds_types) {
-                  const PPAtom P{i, s_rt[k], s_rx[k], s_rm[k], s_rq[k]};
-                  ok = pp_param_fast(S, P, Q, s_avdw, s_bvdw, s_ljc, Ad, Bd, eld);
-                } else {
-                  ok = pp_param(S, i, j, Ad, Bd, eld);
-                }
-                if (!ok) continue;
-                const R ux = dx - ro[k][0], uy = dy - ro[k][1], uz = dz - ro[k][2];
-                const R dv = PairMath<R>::nbe(ux, uy, uz, (R)Ad, (R)Bd, (R)eld, pel, pvdw, acc);
-                f[k][0] += ux * dv;
-                f[k][1] += uy * dv;
-                f[k][2] += uz * dv;
-              }
-            }
-            if (acc) {
-              e_ppel += (double)pel;
-              e_ppvdw += (double)pvdw;
-            }
-          }
-          __builtin_amdgcn_wave_barrier();
-        }
-      }
-      // ---- partner waters: lane l takes site kb = l % 3 of water l / 3 of the round
-      if ((mask & T_PW) && nsr < nn && sa == 3 && lane < 3 * (QNB_WAVE / 3)) {
-        const int kb = lane % 3;
-        R pw[CH][3];
+    // ---- the other solute partners: A, B, qq from the factors; the next
+    // partner's position and factors load while this one is evaluated
+    if (fast && nk > 0) {
+      int t = t0, e = e0, en = e1;
+      double px, py, pz;
+      R pA, pB, pQ;
+      auto fetch = [&](int entry) {
+        const int j = entry & AL_ATOM;
+        px = ldg(x + 3 * j);
+        py = ldg(x + 3 * j + 1);
+        pz = ldg(x + 3 * j + 2);
+        const R* pf = qp_tab<R>(S.ppd, S.ppf) + PP_REC * (size_t)j;
+        pA = ldg(pf);
+        pB = ldg(pf + 1);
+        pQ = ldg(pf + 2);
+      };
+      fetch(e);
+      for (; t < n_far; t += QNB_WAVE * parts) {
+        const R dx = (R)(px - xr0), dy = (R)(py - xr1), dz = (R)(pz - xr2);
+        const R qA = pA, qB = pB, qQ = pQ;
+        const bool acc = want_e && (e & AL_OWN);
+        e = en;
+        fetch(e);
+        en = far_entry(t + 2 * QNB_WAVE * parts);
+        R pel = R(0), pvdw = R(0);
 #pragma unroll
         for (int k = 0; k < CH; k++) {
-          pw[k][0] = rok[k] ? s_pw[k][kb][0] : R(0);
-          pw[k][1] = rok[k] ? s_pw[k][kb][1] : R(0);
-          pw[k][2] = rok[k] ? s_pw[k][kb][2] : R(0);
+          if (ri[k] < 0) continue;
+          const R A = rA[k] * qA, B = rB[k] * qB, el = rQ[k] * qQ;
+          // pp_param's `set` test (QREAL_EPS, src/sizes.f90:50); in FP32
+          // a pair of zero parameters adds exactly zero, so it is skipped
+          // only on the FP64 path
+          if constexpr (sizeof(R) == 8)
+            if (!(fabs(A) > R(12.0e-10) || fabs(B) > R(6.0e-10) || fabs(el) > R(1.0e-10))) continue;
+          const R ux = dx - ro[k][0], uy = dy - ro[k][1], uz = dz - ro[k][2];
+          const R dv = pair_dv(ux, uy, uz, A, B, el, pel, pvdw, acc);
+          f[k][0] += ux * dv;
+          f[k][1] += uy * dv;
+          f[k][2] += uz * dv;
         }
-        for (int p = nsr + lane / 3; p < nn; p += QNB_WAVE / 3) {
-          const int b = ldg(row + p);
-          const int j = nsol + sa * (b - ncs) + kb;
+        if (acc) {
+          e_ppel += (double)pel;
+          e_ppvdw += (double)pvdw;
+        }
+      }
+    }
+    // ---- solvent partners: a lane per molecule, its sites in turn
+    if (pw && nk > 0) {
+      for (int p = nsr + lane + QNB_WAVE * part; p < nn; p += QNB_WAVE * parts) {
+        const int j0 = nsol + sa * (ldg(row + p) - ncs);
+        R pel = R(0), pvdw = R(0);
+        for (int kb = 0; kb < sa; kb++) {
+          const int j = j0 + kb;
           const R dx = (R)(ldg(x + 3 * j) - xr0), dy = (R)(ldg(x + 3 * j + 1) - xr1),
                   dz = (R)(ldg(x + 3 * j + 2) - xr2);
-          R pel = R(0), pvdw = R(0);
+          const bool coul = kb > 0 && coul_h;
 #pragma unroll
           for (int k = 0; k < CH; k++) {
-            if (!rok[k]) continue;
+            if (ri[k] < 0) continue;
+            R A, B, el;
+            if (sa == 3) {
+              A = s_pw[k][3 * kb];
+              B = s_pw[k][3 * kb + 1];
+              el = s_pw[k][3 * kb + 2];
+            } else {
+              const size_t tt = (size_t)ri[k] + (size_t)nsol * kb;
+              A = R(12) * (R)ldg(S.pwA + tt);
+              B = R(6) * (R)ldg(S.pwB + tt);
+              el = (R)ldg(S.pwEl + tt);
+            }
             const R ux = dx - ro[k][0], uy = dy - ro[k][1], uz = dz - ro[k][2];
-            const R dv = PairMath<R>::nbe(ux, uy, uz, pw[k][0], pw[k][1], pw[k][2], pel, pvdw, want_e);
+            const R dv = coul ? PairMath<R>::nbe_spc(ux, uy, uz, el, pel, want_e)
+                              : pair_dv(ux, uy, uz, A, B, el, pel, pvdw, want_e);
             f[k][0] += ux * dv;
             f[k][1] += uy * dv;
             f[k][2] += uz * dv;
           }
-          if (want_e) {
-            e_pwel += (double)pel;
-            e_pwvdw += (double)pvdw;
-          }
         }
-      }
-      // ---- partner molecules of any other solvent: lane l takes site
-      // kb = l % sa of molecule l / sa of the round, 64 / sa molecules per
-      // round, the parameters read per receiver atom
-      if ((mask & T_PW) && nsr < nn && sa != 3 && lane < sa * (QNB_WAVE / sa)) {
-        const int kb = lane % sa, M = QNB_WAVE / sa;
-        for (int p = nsr + lane / sa; p < nn; p += M) {
-          const int b = ldg(row + p);
-          const int j = nsol + sa * (b - ncs) + kb;
-          const R dx = (R)(ldg(x + 3 * j) - xr0), dy = (R)(ldg(x + 3 * j + 1) - xr1),
-                  dz = (R)(ldg(x + 3 * j + 2) - xr2);
-          R pel = R(0), pvdw = R(0);
-#pragma unroll
-          for (int k = 0; k < CH; k++) {
-            if (!rok[k]) continue;
-            const size_t tt = (size_t)s_ia[k] + (size_t)nsol * kb;
-            const R ux = dx - ro[k][0], uy = dy - ro[k][1], uz = dz - ro[k][2];
-            const R dv = PairMath<R>::nbe(ux, uy, uz, (R)ldg(S.pwA + tt), (R)ldg(S.pwB + tt), (R)ldg(S.pwEl + tt),
-                                          pel, pvdw, want_e);
-            f[k][0] += ux * dv;
-            f[k][1] += uy * dv;
-            f[k][2] += uz * dv;
-          }
-          if (want_e) {
-            e_pwel += (double)pel;
-            e_pwvdw += (double)pvdw;
-          }
+        if (want_e) {
+          e_pwel += (double)pel;
+          e_pwvdw += (double)pvdw;
         }
-      }
-      __builtin_amdgcn_wave_barrier();
-      // ---- pairs inside the group: lane (g, kq) = (lane / nk, lane % nk)
-      // takes receiver atom kq against group atoms q = g, g + G, ...
-      // (G = 64 / nk); an atom of this sweep has its data in LDS, others
-      // (groups larger than one sweep) are read from memory
-      if (mask & T_PP) {
-        const int G = QNB_WAVE / nk, kq = lane % nk, g = lane / nk;
-        const int i = s_ia[kq];
-        R fq[3] = {R(0), R(0), R(0)};
-        if (g < G && i >= 0) {
-          const R ox = s_o[kq][0], oy = s_o[kq][1], oz = s_o[kq][2];
-          for (int q = g; q < na; q += G) {
-            const int ql = q - c0;
-            const bool in_sweep = ql >= 0 && ql < nk;
-            int j;
-            R dx, dy, dz;
-            if (in_sweep) {
-              j = s_ia[ql];  // -1: a Q-atom, whose pairs belong to the Q kernels
-              dx = s_o[ql][0];
-              dy = s_o[ql][1];
-              dz = s_o[ql][2];
-            } else {
-              j = ldg(S.cgpatom + (g0 + q));
-              if (ldg(S.iqatom + j) != 0) continue;
-              dx = (R)(ldg(x + 3 * j) - xr0);
-              dy = (R)(ldg(x + 3 * j + 1) - xr1);
-              dz = (R)(ldg(x + 3 * j + 2) - xr2);
-            }
-            if (j < 0 || j == i) continue;
-            double A, B, el;
-            bool ok;
-            if (in_sweep && lds_types) {
-              const PPAtom P{i, s_rt[kq], s_rx[kq], s_rm[kq], s_rq[kq]};
-              const PPAtom Q{j, s_rt[ql], s_rx[ql], s_rm[ql], s_rq[ql]};
-              ok = pp_param_fast(S, P, Q, s_avdw, s_bvdw, s_ljc, A, B, el);
-            } else {
-              ok = pp_param(S, i, j, A, B, el);
-            }
-            if (!ok) continue;
-            const R ux = dx - ox, uy = dy - oy, uz = dz - oz;
-            const R dv = PairMath<R>::nbe(ux, uy, uz, (R)A, (R)B, (R)el, e_ppel, e_ppvdw, want_e && i < j);
-            fq[0] += ux * dv;
-            fq[1] += uy * dv;
-            fq[2] += uz * dv;
-          }
-        }
-#pragma unroll
-        for (int k = 0; k < CH; k++)
-          if (k == kq) {
-            f[k][0] += fq[0];
-            f[k][1] += fq[1];
-            f[k][2] += fq[2];
-          }
       }
     }
     // ---- Q-atom - solute atom, receiver side: lane (g, kq) = (lane / nk,
-    // lane % nk) takes receiver atom kq against Q-atoms g, g + G, ...
-    if (qin) {
+    // lane % nk) takes receiver atom kq against Q-atoms g, g + G, ... (G = 64
+    // / nk)
+    if (qin && nk > 0) {
       const R *qtA = qp_tab<R>(S.qpA, S.qpA_f), *qtB = qp_tab<R>(S.qpB, S.qpB_f);
       const R *qtE = qp_tab<R>(S.qpEl, S.qpEl_f), *qtS = qp_tab<R>(S.qpSc, S.qpSc_f);
       const int G = QNB_WAVE / nk, kq = lane % nk, g = lane / nk;
-      const int i = s_ia[kq];
+      const int i = __shfl(il, kq, QNB_WAVE);
+      const R ox = __shfl(ol0, kq, QNB_WAVE), oy = __shfl(ol1, kq, QNB_WAVE), oz = __shfl(ol2, kq, QNB_WAVE);
       R fq[3] = {R(0), R(0), R(0)};
       if (g < G && i >= 0 && !ldg(S.qconn3 + i)) {
-        const R ox = s_o[kq][0], oy = s_o[kq][1], oz = s_o[kq][2];
-        for (int iq = g; iq < nq; iq += G) {
+        for (int iq = g + G * part; iq < nq; iq += G * parts) {
           const int q = ldg(S.iqseq + iq);
           const R ux = (R)(ldg(x + 3 * q) - xr0) - ox, uy = (R)(ldg(x + 3 * q + 1) - xr1) - oy,
                   uz = (R)(ldg(x + 3 * q + 2) - xr2) - oz;
           R r2, r;
           rinv(ux * ux + uy * uy + uz * uz, r2, r);
-          const R r6 = r2 * r2 * r2;
-          R dvs = R(0);
-#pragma unroll
-          for (int s = 0; s < NS; s++) {
-            if (s >= ns) break;
+          const R dvs = qx_states<R, NS>(S, r2, r, ns, eq, want_e, [&](int s) {
             const size_t t = (size_t)i + (size_t)nsol * ((size_t)iq + (size_t)nq * s);
-            dvs += PairMath<R>::nbe_qx(r2, r, r6, ldg(qtA + t), ldg(qtB + t), ldg(qtE + t), ldg(qtS + t),
-                                       (R)S.lambda[s], eq[2 * s], eq[2 * s + 1], want_e);
-          }
+            return QPar<R>{ldg(qtA + t), ldg(qtB + t), ldg(qtE + t), ldg(qtS + t)};
+          });
           fq[0] += ux * dvs;
           fq[1] += uy * dvs;
           fq[2] += uz * dvs;
@@ -1049,44 +1020,56 @@ __global__ __launch_bounds__(64 * FC_WPB) FC_OCC_ATTR void k_sforces(const DevSy
           f[k][2] += fq[2];
         }
     }
-    // reduce all 3 CH force components at once (the per-atom LRF Taylor term
-    // follows in k_atom_terms); component c of sweep atom k is value 3k + c
-    {
-      R fv[3 * CH];
+    // reduce all 3 CH force components of the wave at once; component c of
+    // sweep atom k is value 3k + c
+    R fv[3 * CH];
 #pragma unroll
-      for (int k = 0; k < CH; k++)
+    for (int k = 0; k < CH; k++)
 #pragma unroll
-        for (int c = 0; c < 3; c++) fv[3 * k + c] = f[k][c];
-      const double fs = wave_sum_tr(fv, lane);
-      const int j = wave_sum_tr_index<3 * CH>(lane);
-      if (wave_sum_tr_writer<3 * CH>(lane) && j / 3 < nk) {
-        const int i = ldg(S.cgpatom + (g0 + c0 + j / 3));
-        d[3 * i + j % 3] = -fs;
-      }
-    }
+      for (int c = 0; c < 3; c++) fv[3 * k + c] = f[k][c];
+    double fs = wave_sum_tr(fv, lane);
+    if constexpr (SPLIT) fs = waves_sum(comb, fs, set * parts, parts, lane);
+    const int j = wave_sum_tr_index<3 * CH>(lane);
+    const int iw = __shfl(i_own, j / 3, QNB_WAVE);
+    if (part == 0 && wave_sum_tr_writer<3 * CH>(lane) && j / 3 < nk) d[3 * iw + j % 3] = -fs;
     __builtin_amdgcn_wave_barrier();
   }
   if (!want_e) return;
   // pp and pw energies, then each state's qp el and vdW
-  double part[4 + 2 * NS];
+  double en[4 + 2 * NS];
   int slot[4 + 2 * NS];
-  part[0] = e_ppel, slot[0] = E_PP_EL;
-  part[1] = e_ppvdw, slot[1] = E_PP_VDW;
-  part[2] = e_pwel, slot[2] = E_PW_EL;
-  part[3] = e_pwvdw, slot[3] = E_PW_VDW;
+  en[0] = e_ppel, slot[0] = E_PP_EL;
+  en[1] = e_ppvdw, slot[1] = E_PP_VDW;
+  en[2] = e_pwel, slot[2] = E_PW_EL;
+  en[3] = e_pwvdw, slot[3] = E_PW_VDW;
 #pragma unroll
   for (int s = 0; s < NS; s++) {
-    part[4 + 2 * s] = eq[2 * s], slot[4 + 2 * s] = E_Q0 + 6 * s + 2;
-    part[5 + 2 * s] = eq[2 * s + 1], slot[5 + 2 * s] = E_Q0 + 6 * s + 3;
+    en[4 + 2 * s] = eq[2 * s], slot[4 + 2 * s] = E_Q0 + 6 * s + 2;
+    en[5 + 2 * s] = eq[2 * s + 1], slot[5 + 2 * s] = E_Q0 + 6 * s + 3;
   }
-  store_energy_record(S.epart + (size_t)a * QNB_NE, part, slot, lane);
+  double sum = wave_sum_tr(en, lane);
+  if constexpr (SPLIT) sum = waves_sum(comb, sum, 0, waves, lane);
+  if (!SPLIT || wave == 0) store_energy_record<4 + 2 * NS>(S.epart + (size_t)a * QNB_NE, sum, slot, lane);
+}
+
+template <typename R, int NS, bool E>
+__global__ __launch_bounds__(64 * FC_WPB) void k_sforces(const DevSys* __restrict__ systems, uint32_t mask, int imap,
+                                                         int nb, int ninst) {
+  int inst, blk;
+  if (!map_block(imap, nb, ninst, inst, blk)) return;
+  const DevSys& S = systems[inst];
+  const int wib = threadIdx.x / QNB_WAVE;
+  const int a = uni(blk * (int)(blockDim.x / QNB_WAVE) + wib);
+  if (a >= S.ncgp_solute) return;
+  extern __shared__ __align__(16) unsigned char so_smem[];
+  solute_receiver<R, NS, E, false>(S, mask, a, 0, 1, so_smem + (size_t)wib * so_wave_bytes<R>(), nullptr);
 }
 
 // ---------------------------------------------------------------------------
 // Water receivers (rigid 3-site solvent): one wavefront per water a.  Its
 // neighbour row is sorted, so the solute groups (indices below ncgp_solute)
-// come first, then the waters.  Solute partners go through the staged atom
-// expansion, one partner atom per lane against the three receiver atoms with
+// come first, then the waters.  Solute partners come from the receiver's atom
+// list (k_expand), one partner atom per lane against the three receiver atoms with
 // the pw parameters (nonbond_pw, nonbondene.f90:4856-4916; energy counted on
 // the solute side).  Partner waters need no staging: their atoms are
 // consecutive, so in each round lane l takes atom l % 3 of the row's water
@@ -1096,29 +1079,17 @@ __global__ __launch_bounds__(64 * FC_WPB) FC_OCC_ATTR void k_sforces(const DevSy
 // other pairs Coulomb only; nonbond_ww 5509-5573 for other solvents).  Then
 // the receiver side of the Q-atom - water pairs.  Writes d of the three
 // atoms, and the wave's ww and qw energy partials on the sampled steps.
-template <typename R, int NS, bool E, int CAP>
-__global__ __launch_bounds__(64 * FC_WPB) void k_wforces(const DevSys* __restrict__ systems, uint32_t mask,
-                                                         int imap, int nb, int ninst) {
-  int inst, blk;
-  if (!map_block(imap, nb, ninst, inst, blk)) return;
-  const DevSys& S = systems[inst];
-  const int wib = threadIdx.x / QNB_WAVE;
-  const int a = __builtin_amdgcn_readfirstlane(S.ncgp_solute + blk * (int)(blockDim.x / QNB_WAVE) + wib);
-  if (a >= S.ncgp) return;
+template <typename R, int NS, bool E>
+__device__ __forceinline__ void water_receiver(const DevSys& S, uint32_t mask, int a) {
   const int lane = threadIdx.x % QNB_WAVE;
-  extern __shared__ __align__(16) unsigned char wf_smem[];
-  unsigned char* wbase = wf_smem + (size_t)wib * wf_wave_bytes<R, CAP>();
-  R(*s_pd)[3] = reinterpret_cast<R(*)[3]>(wbase);
-  int* s_pj = reinterpret_cast<int*>(wbase + sizeof(R) * 3 * CAP);
-  int* s_pt = s_pj + CAP;
   const double* __restrict__ x = S.x;
   const auto d = gpm(S.d);
-  const int nn = min(ldg(S.nnbr + a), S.cap);
+  const int nn = uni(min(ldg(S.nnbr + a), S.cap));
   const int* __restrict__ row = S.nbr + (size_t)a * S.cap;
   const bool want_e = E && want_energies(S);
   const int nsol = S.nat_solute, sa = S.sa, ncs = S.ncgp_solute;
   const int ra = nsol + sa * (a - ncs);
-  const bool aexcl = ldg(S.excl + ra);
+  const bool aexcl = uni(ldg(S.excl + ra));
   const int nq = S.nqat, ns = S.nstates;
   double e_el = 0.0, e_vdw = 0.0;
   double eq[2 * NS];  // per state: qw_el, qw_vdw
@@ -1134,51 +1105,55 @@ __global__ __launch_bounds__(64 * FC_WPB) void k_wforces(const DevSys* __restric
     f[k][0] = f[k][1] = f[k][2] = R(0);
   }
   if (!aexcl) {
-    // length of the row's solute prefix
-    int nsr = 0;
-    for (int p0 = 0; p0 < nn; p0 += QNB_WAVE) {
-      const int p = p0 + lane;
-      const uint64_t m = __ballot(p < nn && ldg(row + p) < ncs);
-      nsr += __popcll(m);
-      if (m != ~0ull) break;
-    }
-    // solute partners, one staged atom per lane
+    const int nsr = uni(min(ldg(S.nnsol + a), nn));  // length of the row's solute prefix
+    // solute partners from the receiver's atom list, one per lane, the next
+    // one's data in flight
     if (mask & T_PW) {
-      for (int p0 = 0, ng = 0; p0 < nsr; p0 += ng) {
-        const int total = stage_partners<R, CAP>(S, a, row, p0, nsr, 1u, 0u, xr0, xr1, xr2, s_pj, s_pd, s_pt, &ng);
-        if (ng == 0) break;
-        for (int t = lane; t < total; t += QNB_WAVE) {
-          if (s_pt[t] & FT_Q) continue;
-          const int j = s_pj[t];
-          const R dx = s_pd[t][0], dy = s_pd[t][1], dz = s_pd[t][2];
-          R pw[9];
+      const int* __restrict__ al = S.alist + (size_t)a * S.acap + S.acap - 1;
+      const int n = uni(ldg(S.alist_n + 2 * a + 1));
+      int j = lane < n ? ldg(al - lane) & AL_ATOM : 0;
+      int jn = lane + QNB_WAVE < n ? ldg(al - lane - QNB_WAVE) & AL_ATOM : 0;
+      double px = 0.0, py = 0.0, pz = 0.0;
+      R pl[9];
+      auto fetch = [&](int i) {
+        px = ldg(x + 3 * i);
+        py = ldg(x + 3 * i + 1);
+        pz = ldg(x + 3 * i + 2);
 #pragma unroll
-          for (int k = 0; k < 3; k++) {
-            if constexpr (sizeof(R) == 4) {
-              pw[3 * k] = ldg(S.pw_f + PW_REC * j + 3 * k);
-              pw[3 * k + 1] = ldg(S.pw_f + PW_REC * j + 3 * k + 1);
-              pw[3 * k + 2] = ldg(S.pw_f + PW_REC * j + 3 * k + 2);
-            } else {
-              const size_t tt = (size_t)j + (size_t)nsol * k;
-              pw[3 * k] = (R)ldg(S.pwA + tt);
-              pw[3 * k + 1] = (R)ldg(S.pwB + tt);
-              pw[3 * k + 2] = (R)ldg(S.pwEl + tt);
-            }
-          }
-#pragma unroll
-          for (int k = 0; k < 3; k++) {
-            const R ux = dx - o[k][0], uy = dy - o[k][1], uz = dz - o[k][2];
-            R ee = R(0), ev = R(0);
-            // sites without LJ: nbe with A = B = 0 is nbe_spc exactly
-            const R dv = (k > 0 && S.pw_coul_h)
-                             ? PairMath<R>::nbe_spc(ux, uy, uz, pw[3 * k + 2], ee, false)
-                             : PairMath<R>::nbe(ux, uy, uz, pw[3 * k], pw[3 * k + 1], pw[3 * k + 2], ee, ev, false);
-            f[k][0] += ux * dv;
-            f[k][1] += uy * dv;
-            f[k][2] += uz * dv;
+        for (int k = 0; k < 3; k++) {
+          if constexpr (sizeof(R) == 4) {
+            pl[3 * k] = ldg(S.pw_f + PW_REC * i + 3 * k);
+            pl[3 * k + 1] = ldg(S.pw_f + PW_REC * i + 3 * k + 1);
+            pl[3 * k + 2] = ldg(S.pw_f + PW_REC * i + 3 * k + 2);
+          } else {
+            const size_t tt = (size_t)i + (size_t)nsol * k;
+            pl[3 * k] = (R)ldg(S.pwA + tt);
+            pl[3 * k + 1] = (R)ldg(S.pwB + tt);
+            pl[3 * k + 2] = (R)ldg(S.pwEl + tt);
           }
         }
-        __builtin_amdgcn_wave_barrier();
+      };
+      if (n > 0) fetch(j);
+      for (int t = lane; t < n; t += QNB_WAVE) {
+        const R dx = (R)(px - xr0), dy = (R)(py - xr1), dz = (R)(pz - xr2);
+        R pw[9];
+#pragma unroll
+        for (int k = 0; k < 9; k++) pw[k] = pl[k];
+        j = jn;
+        fetch(j);
+        jn = t + 2 * QNB_WAVE < n ? ldg(al - t - 2 * QNB_WAVE) & AL_ATOM : 0;
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+          const R ux = dx - o[k][0], uy = dy - o[k][1], uz = dz - o[k][2];
+          R ee = R(0), ev = R(0);
+          // sites without LJ: nbe with A = B = 0 is nbe_spc exactly
+          const R dv = (k > 0 && S.pw_coul_h)
+                           ? PairMath<R>::nbe_spc(ux, uy, uz, pw[3 * k + 2], ee, false)
+                           : PairMath<R>::nbe(ux, uy, uz, pw[3 * k], pw[3 * k + 1], pw[3 * k + 2], ee, ev, false);
+          f[k][0] += ux * dv;
+          f[k][1] += uy * dv;
+          f[k][2] += uz * dv;
+        }
       }
     }
     // partner waters: lane l takes atom kb = l % 3 of water (l / 3) of the round
@@ -1237,26 +1212,9 @@ __global__ __launch_bounds__(64 * FC_WPB) void k_wforces(const DevSys* __restric
         const R ux = qx - o[k][0], uy = qy - o[k][1], uz = qz - o[k][2];
         R r2, r;
         rinv(ux * ux + uy * uy + uz * uz, r2, r);
-        R dvs = R(0);
-        if (k == 0 || !S.spc) {
-          const R r6 = r2 * r2 * r2;
-#pragma unroll
-          for (int s = 0; s < NS; s++) {
-            if (s >= ns) break;
-            const size_t t = (size_t)iq + (size_t)nq * ((size_t)k + (size_t)sa * s);
-            dvs += PairMath<R>::nbe_qx(r2, r, r6, (R)ldg(S.qwA + t), (R)ldg(S.qwB + t), (R)ldg(S.qwEl + t),
-                                       (R)ldg(S.qwSc + t), (R)S.lambda[s], eq[2 * s], eq[2 * s + 1], want_e);
-          }
-        } else {
-#pragma unroll
-          for (int s = 0; s < NS; s++) {
-            if (s >= ns) break;
-            const size_t t = (size_t)iq + (size_t)nq * ((size_t)k + (size_t)sa * s);
-            const R Vel = (R)ldg(S.qwEl + t) * r;
-            if (want_e) eq[2 * s] += (double)Vel;
-            dvs += -r2 * Vel * (R)S.lambda[s];
-          }
-        }
+        const R dvs = k == 0 || !S.spc
+                          ? qx_states<R, NS>(S, r2, r, ns, eq, want_e, [&](int s) { return qw_par<R>(S, iq, k, s); })
+                          : qspc_states<R, NS>(S, r2, r, ns, eq, want_e, [&](int s) { return qw_el<R>(S, iq, k, s); });
         f[k][0] += ux * dvs;
         f[k][1] += uy * dvs;
         f[k][2] += uz * dvs;
@@ -1285,7 +1243,18 @@ __global__ __launch_bounds__(64 * FC_WPB) void k_wforces(const DevSys* __restric
     part[2 + 2 * s] = eq[2 * s], slot[2 + 2 * s] = E_Q0 + 6 * s + 4;
     part[3 + 2 * s] = eq[2 * s + 1], slot[3 + 2 * s] = E_Q0 + 6 * s + 5;
   }
-  store_energy_record(S.epart + (size_t)a * QNB_NE, part, slot, lane);
+  store_energy_record<2 + 2 * NS>(S.epart + (size_t)a * QNB_NE, wave_sum_tr(part, lane), slot, lane);
+}
+
+template <typename R, int NS, bool E>
+__global__ __launch_bounds__(64 * FC_WPB) void k_wforces(const DevSys* __restrict__ systems, uint32_t mask,
+                                                         int imap, int nb, int ninst) {
+  int inst, blk;
+  if (!map_block(imap, nb, ninst, inst, blk)) return;
+  const DevSys& S = systems[inst];
+  const int wib = threadIdx.x / QNB_WAVE;
+  const int a = __builtin_amdgcn_readfirstlane(S.ncgp_solute + blk * (int)(blockDim.x / QNB_WAVE) + wib);
+  if (a < S.ncgp) water_receiver<R, NS, E>(S, mask, a);
 }
 
 // ---------------------------------------------------------------------------
@@ -1306,15 +1275,7 @@ __global__ __launch_bounds__(64 * FC_WPB) void k_wforces(const DevSys* __restric
 // of the molecule's atoms and the wave's ww and qw energy partials on the
 // sampled steps.
 template <typename R, int NS>
-__global__ __launch_bounds__(64 * FC_WPB) void k_gforces(const DevSys* __restrict__ systems, uint32_t mask,
-                                                         int imap, int nb, int ninst) {
-  int inst, blk;
-  if (!map_block(imap, nb, ninst, inst, blk)) return;
-  const DevSys& S = systems[inst];
-  const int wib = threadIdx.x / QNB_WAVE;
-  const int a = __builtin_amdgcn_readfirstlane(S.ncgp_solute + blk * (int)(blockDim.x / QNB_WAVE) + wib);
-  if (a >= S.ncgp) return;
-  __shared__ double s_f[FC_WPB][QNB_WAVE][3];
+__device__ __forceinline__ void solvent_receiver(const DevSys& S, uint32_t mask, int a, double (*s_f)[3]) {
   const int lane = threadIdx.x % QNB_WAVE;
   const int sa = S.sa, M = QNB_WAVE / sa;
   const int k = lane % sa, m = lane / sa;
@@ -1324,7 +1285,7 @@ __global__ __launch_bounds__(64 * FC_WPB) void k_gforces(const DevSys* __restric
   const int base = nsol + sa * (a - ncs), ia = base + k;
   const bool aexcl = ldg(S.excl + base);
   const bool want_e = want_energies(S);
-  const int nn = min(ldg(S.nnbr + a), S.cap);
+  const int nn = uni(min(ldg(S.nnbr + a), S.cap));
   const int* __restrict__ row = S.nbr + (size_t)a * S.cap;
   const double xi0 = ldg(x + 3 * ia), xi1 = ldg(x + 3 * ia + 1), xi2 = ldg(x + 3 * ia + 2);
   double f[3] = {0.0, 0.0, 0.0};
@@ -1381,26 +1342,9 @@ __global__ __launch_bounds__(64 * FC_WPB) void k_gforces(const DevSys* __restric
         const R ux = (R)(ldg(x + 3 * q) - xi0), uy = (R)(ldg(x + 3 * q + 1) - xi1), uz = (R)(ldg(x + 3 * q + 2) - xi2);
         R r2, r;
         rinv(ux * ux + uy * uy + uz * uz, r2, r);
-        R dvs = R(0);
-        if (k == 0 || !S.spc) {
-          const R r6 = r2 * r2 * r2;
-#pragma unroll
-          for (int st = 0; st < NS; st++) {
-            if (st >= ns) break;
-            const size_t t = (size_t)iq + (size_t)nq * ((size_t)k + (size_t)sa * st);
-            dvs += PairMath<R>::nbe_qx(r2, r, r6, (R)ldg(S.qwA + t), (R)ldg(S.qwB + t), (R)ldg(S.qwEl + t),
-                                       (R)ldg(S.qwSc + t), (R)S.lambda[st], eq[2 * st], eq[2 * st + 1], want_e);
-          }
-        } else {
-#pragma unroll
-          for (int st = 0; st < NS; st++) {
-            if (st >= ns) break;
-            const size_t t = (size_t)iq + (size_t)nq * ((size_t)k + (size_t)sa * st);
-            const R Vel = (R)ldg(S.qwEl + t) * r;
-            if (want_e) eq[2 * st] += (double)Vel;
-            dvs += -r2 * Vel * (R)S.lambda[st];
-          }
-        }
+        const R dvs = k == 0 || !S.spc
+                          ? qx_states<R, NS>(S, r2, r, ns, eq, want_e, [&](int s) { return qw_par<R>(S, iq, k, s); })
+                          : qspc_states<R, NS>(S, r2, r, ns, eq, want_e, [&](int s) { return qw_el<R>(S, iq, k, s); });
         f[0] += (double)(ux * dvs);
         f[1] += (double)(uy * dvs);
         f[2] += (double)(uz * dvs);
@@ -1433,17 +1377,17 @@ __global__ __launch_bounds__(64 * FC_WPB) void k_gforces(const DevSys* __restric
       }
     }
   }
-  s_f[wib][lane][0] = f[0];
-  s_f[wib][lane][1] = f[1];
-  s_f[wib][lane][2] = f[2];
+  s_f[lane][0] = f[0];
+  s_f[lane][1] = f[1];
+  s_f[lane][2] = f[2];
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
   if (lane < sa) {
     double t0 = 0.0, t1 = 0.0, t2 = 0.0;
     for (int mm = 0; mm < M; mm++) {
-      t0 += s_f[wib][lane + sa * mm][0];
-      t1 += s_f[wib][lane + sa * mm][1];
-      t2 += s_f[wib][lane + sa * mm][2];
+      t0 += s_f[lane + sa * mm][0];
+      t1 += s_f[lane + sa * mm][1];
+      t2 += s_f[lane + sa * mm][2];
     }
     const auto d = gpm(S.d);
     d[3 * ia] = -t0;
@@ -1460,7 +1404,20 @@ __global__ __launch_bounds__(64 * FC_WPB) void k_gforces(const DevSys* __restric
     part[2 + 2 * st] = eq[2 * st], slot[2 + 2 * st] = E_Q0 + 6 * st + 4;
     part[3 + 2 * st] = eq[2 * st + 1], slot[3 + 2 * st] = E_Q0 + 6 * st + 5;
   }
-  store_energy_record(S.epart + (size_t)a * QNB_NE, part, slot, lane);
+  store_energy_record<2 + 2 * NS>(S.epart + (size_t)a * QNB_NE, wave_sum_tr(part, lane), slot, lane);
+}
+
+template <typename R, int NS>
+__global__ __launch_bounds__(64 * FC_WPB) void k_gforces(const DevSys* __restrict__ systems, uint32_t mask,
+                                                         int imap, int nb, int ninst) {
+  int inst, blk;
+  if (!map_block(imap, nb, ninst, inst, blk)) return;
+  const DevSys& S = systems[inst];
+  const int wib = threadIdx.x / QNB_WAVE;
+  const int a = __builtin_amdgcn_readfirstlane(S.ncgp_solute + blk * (int)(blockDim.x / QNB_WAVE) + wib);
+  if (a >= S.ncgp) return;
+  __shared__ double s_f[FC_WPB][QNB_WAVE][3];
+  solvent_receiver<R, NS>(S, mask, a, s_f[wib]);
 }
 
 // ---------------------------------------------------------------------------
@@ -1471,7 +1428,7 @@ __global__ __launch_bounds__(64 * FC_WPB) void k_gforces(const DevSys* __restric
 // sampled steps the atom's two energies go to eatom[2i], eatom[2i+1] for the
 // fixed-order reduction.
 __global__ __launch_bounds__(256) void k_atom_terms(const DevSys* __restrict__ systems, uint32_t mask,
-                                                    const double* __restrict__ tfree) {
+                                                    const double* __restrict__ tfree, int rows) {
   const DevSys& S = systems[blockIdx.y];
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= S.natom) return;
@@ -1484,6 +1441,7 @@ __global__ __launch_bounds__(256) void k_atom_terms(const DevSys* __restrict__ s
     const double shift = S.fk_wsphere != 0.0 ? sqrt(S.Boltz * T / S.fk_wsphere) : 0.0;
     radial_restraint(S, src, shift, f, er);
   }
+  add_qrows(S, i, rows, f);
   store_atom_gradient(S, i, f);
   if (want_energies(S)) {
     stg(S.eatom + 2 * i, el);
@@ -1492,25 +1450,14 @@ __global__ __launch_bounds__(256) void k_atom_terms(const DevSys* __restrict__ s
 }
 
 // ---------------------------------------------------------------------------
-// Q-atom side of the Q-water and Q-solute pairs: wave = (Q-atom, chunk of its
-// partners, 64 at a time); the wave's sum is added to the Q-atom's gradient
-// with atomics (a few per Q-atom), or, with dq, to the system's row
-// dq[blockIdx.y * dq_stride + 3 iq ..] (the MD step runs this beside the
-// solute receivers, which store the same atoms' rows, and adds dq in its
-// per-atom pass).
+// Q-atom side of the Q-water and Q-solute pairs: wave = (Q-atom iq, every
+// chunks-th 64 of its partners from 64 ch on); the wave's sum is added with
+// atomics (a few per Q-atom) to the Q-atom's gradient, or, with rows, to its
+// row of S.dq (launches that run beside or inside the solute receivers' one,
+// which store the same atoms' gradients; the per-atom pass adds dq).
 template <typename R, int NS>
-__global__ __launch_bounds__(256) void k_qforces(const DevSys* __restrict__ systems, uint32_t mask,
-                                                 int chunks_per_q, double* __restrict__ dq, int dq_stride) {
-  const DevSys& S = systems[blockIdx.y];
-  // block x runs on XCD x % 8 and takes Q-atom iq = x % 8 + 8 * (x / 8 / bq),
-  // chunks (x / 8 % bq) * W .. + W - 1 (W waves per block, bq blocks per
-  // Q-atom): an XCD serves only the Q-atoms iq = its index mod 8, so the rows
-  // of the Q tables it reads stay in its L2 across the instances
-  const int W = blockDim.x / QNB_WAVE, bq = (chunks_per_q + W - 1) / W;
-  const int m = blockIdx.x / 8;
-  const int iq = blockIdx.x % 8 + 8 * (m / bq), ch = (m % bq) * W + threadIdx.x / QNB_WAVE;
+__device__ __forceinline__ void qatom_side(const DevSys& S, uint32_t mask, int iq, int ch, int chunks, int rows) {
   const int lane = threadIdx.x % QNB_WAVE;
-  if (iq >= S.nqat || ch >= chunks_per_q) return;
   const int nqw = ldg(S.nq_lists + 0), nqp = ldg(S.nq_lists + 1);
   const int nw_ch = (mask & T_QW) ? (nqw + QNB_WAVE - 1) / QNB_WAVE : 0;
   const int np_ch = (mask & T_QP) ? (nqp + QNB_WAVE - 1) / QNB_WAVE : 0;
@@ -1521,10 +1468,10 @@ __global__ __launch_bounds__(256) void k_qforces(const DevSys* __restrict__ syst
   // per-lane partials in R (a lane takes one partner per chunk), summed over
   // the wave in FP64
   R f[3] = {R(0), R(0), R(0)};
-  double dummy_e = 0.0, dummy_v = 0.0;
+  double dummy[2 * NS];
   const R *qtA = qp_tab<R>(S.qpA, S.qpA_f), *qtB = qp_tab<R>(S.qpB, S.qpB_f);
   const R *qtE = qp_tab<R>(S.qpEl, S.qpEl_f), *qtS = qp_tab<R>(S.qpSc, S.qpSc_f);
-  for (int c = ch; c < nw_ch + np_ch; c += chunks_per_q) {
+  for (int c = ch; c < nw_ch + np_ch; c += chunks) {
     const int p = c * QNB_WAVE + lane;
     if (c < nw_ch) {
       if (p >= nqw) continue;
@@ -1535,25 +1482,9 @@ __global__ __launch_bounds__(256) void k_qforces(const DevSys* __restrict__ syst
         const R rux = (R)ux, ruy = (R)uy, ruz = (R)uz;
         R r2, r;
         rinv(rux * rux + ruy * ruy + ruz * ruz, r2, r);
-        R dvs = R(0);
-        if (k == 0 || !S.spc) {
-          R r6 = r2 * r2 * r2;
-#pragma unroll
-          for (int s = 0; s < NS; s++) {
-            if (s >= ns) break;
-            const size_t t = (size_t)iq + (size_t)nq * ((size_t)k + (size_t)sa * s);
-            dvs += PairMath<R>::nbe_qx(r2, r, r6, (R)ldg(S.qwA + t), (R)ldg(S.qwB + t), (R)ldg(S.qwEl + t),
-                                       (R)ldg(S.qwSc + t),
-                                       (R)S.lambda[s], dummy_e, dummy_v, false);
-          }
-        } else {
-#pragma unroll
-          for (int s = 0; s < NS; s++) {
-            if (s >= ns) break;
-            const size_t t = (size_t)iq + (size_t)nq * ((size_t)k + (size_t)sa * s);
-            dvs += -r2 * ((R)ldg(S.qwEl + t) * r) * (R)S.lambda[s];
-          }
-        }
+        const R dvs = k == 0 || !S.spc
+                          ? qx_states<R, NS>(S, r2, r, ns, dummy, false, [&](int s) { return qw_par<R>(S, iq, k, s); })
+                          : qspc_states<R, NS>(S, r2, r, ns, dummy, false, [&](int s) { return qw_el<R>(S, iq, k, s); });
         f[0] -= rux * dvs;
         f[1] -= ruy * dvs;
         f[2] -= ruz * dvs;
@@ -1566,31 +1497,40 @@ __global__ __launch_bounds__(256) void k_qforces(const DevSys* __restrict__ syst
       const R rux = (R)ux, ruy = (R)uy, ruz = (R)uz;
       R r2, r;
       rinv(rux * rux + ruy * ruy + ruz * ruz, r2, r);
-      R r6 = r2 * r2 * r2;
-#pragma unroll
-      for (int s = 0; s < NS; s++) {
-        if (s >= ns) break;
+      const R dvs = qx_states<R, NS>(S, r2, r, ns, dummy, false, [&](int s) {
         const size_t t = (size_t)j + (size_t)S.nat_solute * ((size_t)iq + (size_t)nq * s);
-        R dv = PairMath<R>::nbe_qx(r2, r, r6, ldg(qtA + t), ldg(qtB + t), ldg(qtE + t), ldg(qtS + t),
-                                   (R)S.lambda[s], dummy_e, dummy_v, false);
-        f[0] -= rux * dv;
-        f[1] -= ruy * dv;
-        f[2] -= ruz * dv;
-      }
+        return QPar<R>{ldg(qtA + t), ldg(qtB + t), ldg(qtE + t), ldg(qtS + t)};
+      });
+      f[0] -= rux * dvs;
+      f[1] -= ruy * dvs;
+      f[2] -= ruz * dvs;
     }
   }
   const double fs = wave_sum_tr(f, lane);
   const int c = wave_sum_tr_index<3>(lane);
   if (wave_sum_tr_writer<3>(lane) && fs != 0.0)
-    unsafeAtomicAdd(dq ? dq + (size_t)blockIdx.y * dq_stride + 3 * iq + c : &S.d[3 * i + c], fs);
+    unsafeAtomicAdd(rows ? S.dq + 3 * iq + c : S.d + 3 * i + c, fs);
+}
+
+template <typename R, int NS>
+__global__ __launch_bounds__(256) void k_qforces(const DevSys* __restrict__ systems, uint32_t mask,
+                                                 int chunks_per_q, int rows) {
+  const DevSys& S = systems[blockIdx.y];
+  // block x runs on XCD x % 8 and takes Q-atom iq = x % 8 + 8 * (x / 8 / bq),
+  // chunks (x / 8 % bq) * W .. + W - 1 (W waves per block, bq blocks per
+  // Q-atom): an XCD serves only the Q-atoms iq = its index mod 8, so the rows
+  // of the Q tables it reads stay in its L2 across the instances
+  const int W = blockDim.x / QNB_WAVE, bq = (chunks_per_q + W - 1) / W;
+  const int m = blockIdx.x / 8;
+  const int iq = blockIdx.x % 8 + 8 * (m / bq), ch = uni((m % bq) * W + threadIdx.x / QNB_WAVE);
+  if (iq < S.nqat && ch < chunks_per_q) qatom_side<R, NS>(S, mask, iq, ch, chunks_per_q, rows);
 }
 
 // ---------------------------------------------------------------------------
 // Static Q-Q (nonbond_qq, nonbondene.f90:5013-5082, pair kernel nbe_qq
 // nonbonded.f90:111-150) and Q-bonded-neighbour (nonbond_qqp, 5085-5153)
-// lists: one block of QQ_THREADS per system, a wavefront per atom of the
-// lists (entity) whose lanes evaluate the pairs the atom belongs to; the
-// wave's sum goes to the atom's gradient once (no atomics; each pair is
+// lists: a wavefront per atom of the lists (entity) whose lanes evaluate the
+// pairs the atom belongs to; the wave's sum goes to the atom's gradient once (no atomics; each pair is
 // evaluated from both sides).  A pair's energy is counted by its first atom;
 // per state the energies are summed per wave and then over the waves in
 // order.
@@ -1604,20 +1544,20 @@ __device__ __forceinline__ void qq_add(double (&eq)[NS][4], int s, int c0, doubl
     }
 }
 
+// Wave `wave` takes entities wave, wave + stride, ..., its lanes the entity's
+// pairs; the block's energies go to record `slot`.  rows: the sums go to the
+// entities' rows of S.dqq (stored, not added), which the per-atom pass adds.
 template <typename R, int NS>
-__global__ __launch_bounds__(QQ_THREADS) void k_qq(const DevSys* __restrict__ systems, uint32_t mask) {
-  const DevSys& S = systems[blockIdx.x];
-  const int slot = S.ncgp;
-  const int t = threadIdx.x, lane = t % QNB_WAVE, wid = t / QNB_WAVE;
-  constexpr int NW = QQ_THREADS / QNB_WAVE;
+__device__ __forceinline__ void qq_pairs(const DevSys& S, uint32_t mask, int wave, int stride, int slot, int rows,
+                                         double* red) {
+  const int lane = threadIdx.x % QNB_WAVE, wid = threadIdx.x / QNB_WAVE;
   const auto x = gp(S.x);
   const auto d = gpm(S.d);
   const bool want_e = want_energies(S);
   double eq[NS][4];
 #pragma unroll
   for (int s = 0; s < NS; s++) eq[s][0] = eq[s][1] = eq[s][2] = eq[s][3] = 0.0;
-  // wave wid takes entities wid, wid + NW, ...; its lanes take the entity's pairs
-  for (int e = wid; e < S.nqe; e += NW) {
+  for (int e = wave; e < S.nqe; e += stride) {
     const int me = ldg(S.qe_atom + e);
     double f[3] = {0.0, 0.0, 0.0};
     for (int it = ldg(S.qe_off + e) + lane, end = ldg(S.qe_off + e + 1); it < end; it += QNB_WAVE) {
@@ -1664,30 +1604,45 @@ __global__ __launch_bounds__(QQ_THREADS) void k_qq(const DevSys* __restrict__ sy
     f[1] = wave_sum(f[1]);
     f[2] = wave_sum(f[2]);
     if (lane == 0) {
-      d[3 * me] += f[0];
-      d[3 * me + 1] += f[1];
-      d[3 * me + 2] += f[2];
+      if (rows) {
+        const auto o = gpm(S.dqq) + 3 * e;
+        o[0] = f[0];
+        o[1] = f[1];
+        o[2] = f[2];
+      } else {
+        d[3 * me] += f[0];
+        d[3 * me + 1] += f[1];
+        d[3 * me + 2] += f[2];
+      }
     }
   }
   if (!want_e) return;
-  __shared__ double red[NW][NS][4];
 #pragma unroll
   for (int s = 0; s < NS; s++)
 #pragma unroll
     for (int c = 0; c < 4; c++) {
       const double v = wave_sum(eq[s][c]);
-      if (lane == 0) red[wid][s][c] = v;
+      if (lane == 0) red[4 * (wid * NS + s) + c] = v;
     }
   __syncthreads();
-  if (t != 0) return;
+  if (threadIdx.x != 0) return;
+  const int nw = blockDim.x / QNB_WAVE;
   double* ep = S.epart + (size_t)slot * QNB_NE;
   for (int k = 0; k < QNB_NE; k++) ep[k] = 0.0;
   for (int s = 0; s < NS; s++)
     for (int c = 0; c < 4; c++) {
       double v = 0.0;
-      for (int w = 0; w < NW; w++) v += red[w][s][c];
+      for (int w = 0; w < nw; w++) v += red[4 * (w * NS + s) + c];
       ep[E_Q0 + 6 * s + c] = v;
     }
+}
+
+template <typename R, int NS>
+__global__ __launch_bounds__(QQ_THREADS) void k_qq(const DevSys* __restrict__ systems, uint32_t mask) {
+  const DevSys& S = systems[blockIdx.x];
+  constexpr int NW = QQ_THREADS / QNB_WAVE;
+  __shared__ double red[NW * NS * 4];
+  qq_pairs<R, NS>(S, mask, threadIdx.x / QNB_WAVE, NW, S.ncgp, 0, red);
 }
 
 // ---------------------------------------------------------------------------
@@ -1732,14 +1687,11 @@ __device__ __forceinline__ void wat_vectors(const DevSys& S, int i, double* rmu,
 // applies the theta_corr feedback of the steps that are multiples of itdis
 // (nonbondene.f90:6653-6666).  The shell counts start at zero (set at
 // creation and cleared by watpol_finish).
-__global__ __launch_bounds__(WP_THREADS) void k_watpol_theta(const DevSys* __restrict__ systems,
-                                                             const int* __restrict__ istep) {
-  const DevSys& S = systems[blockIdx.y];
+__device__ __forceinline__ void watpol_theta(const DevSys& S, int blk, int step) {
   if (!has_pol(S)) return;
   const int t = threadIdx.x, nsh = S.nshell, nw = S.nwat;
-  if (blockIdx.x == 0 && t == 0) {
+  if (blk == 0 && t == 0) {
     double* st = S.sh_state;  // theta_corr[8], avtheta[8], avn_insh[8]
-    const int step = istep[blockIdx.y];
     const int itd = (int)llround(S.itdis);
     if (step > 0 && itd > 0 && step % itd == 0) {
       for (int is = 0; is < nsh; is++) {
@@ -1751,7 +1703,7 @@ __global__ __launch_bounds__(WP_THREADS) void k_watpol_theta(const DevSys* __res
       }
     }
   }
-  const int w = blockIdx.x * WP_THREADS + t;
+  const int w = blk * WP_THREADS + t;
   if (w >= nw) return;
   const int i = S.nat_solute + S.sa * w;
   int sh = -1;
@@ -1793,6 +1745,60 @@ __global__ __launch_bounds__(WP_THREADS) void k_watpol_theta(const DevSys* __res
       pending = -1;
     }
   }
+}
+
+__global__ __launch_bounds__(WP_THREADS) void k_watpol_theta(const DevSys* __restrict__ systems,
+                                                             const int* __restrict__ istep) {
+  watpol_theta(systems[blockIdx.y], blockIdx.x, istep[blockIdx.y]);
+}
+
+// ---------------------------------------------------------------------------
+// All force kernels of a step in one launch, for launches too small to fill
+// the chip (small_launch): blocks of four waves take, in this order, one
+// solute receiver (its row split over the four waves), four solvent receivers,
+// four chunks of a Q-atom's partners, four Q-Q entities, or WP_THREADS waters'
+// polarisation angles.  Everything they read is there before the launch and
+// they write disjoint rows (the Q kernels' sums go to dq and dqq), so no order
+// between them is needed.  What bounds such a step is the latency of each
+// launch and of one wave walking one row: as launches of their own on two
+// streams a step of one 3,342-atom window took 78 us and one of an FP64 window
+// of 11,056 atoms 122 us, with this kernel 62 and 111.
+template <typename R, int NS, bool E>
+__global__ __launch_bounds__(256) void k_forces_small(const DevSys* __restrict__ systems, uint32_t mask,
+                                                                  SmallGrid G, const int* __restrict__ istep) {
+  const DevSys& S = systems[blockIdx.y];
+  const int wib = threadIdx.x / QNB_WAVE;
+  extern __shared__ __align__(16) unsigned char small_smem[];
+  int b = blockIdx.x;
+  if (b < G.solute) {
+    __shared__ double comb[4][QNB_WAVE];
+    if (b < S.ncgp_solute)
+      solute_receiver<R, NS, E, true>(S, mask, b, uni(wib), 4, small_smem + (size_t)wib * so_wave_bytes<R>(), comb);
+    return;
+  }
+  b -= G.solute;
+  if (b < G.solvent) {
+    const int a = __builtin_amdgcn_readfirstlane(S.ncgp_solute + 4 * b + wib);
+    if (a >= S.ncgp) return;
+    if (S.sa == 3)
+      water_receiver<R, NS, E>(S, mask, a);
+    else
+      solvent_receiver<R, NS>(S, mask, a, reinterpret_cast<double(*)[3]>(small_smem) + QNB_WAVE * wib);
+    return;
+  }
+  b -= G.solvent;
+  if (b < G.qside) {
+    const int bq = (G.qchunks + 3) / 4, iq = b / bq, ch = uni(4 * (b % bq) + wib);
+    if (iq < S.nqat && ch < G.qchunks) qatom_side<R, NS>(S, mask, iq, ch, G.qchunks, 1);
+    return;
+  }
+  b -= G.qside;
+  if (b < G.qq) {
+    if (b < qq_slots(S))
+      qq_pairs<R, NS>(S, mask, 4 * b + wib, 4 * qq_slots(S), S.ncgp + b, 1, reinterpret_cast<double*>(small_smem));
+    return;
+  }
+  watpol_theta(S, b - G.qq, istep[blockIdx.y]);
 }
 
 // Phase 2, WP_WATERS members of one shell per block, four waves on the same
@@ -1940,21 +1946,59 @@ __global__ __launch_bounds__(256) void k_reduce_final(const DevSys* __restrict__
   if (with_pol && threadIdx.x < QNB_WAVE) watpol_finish(S);
 }
 
+SmallGrid small_grid(int solute_groups, int nwat, int sa, int nqat, int nat_solute, int nqe, uint32_t mask, bool pol) {
+  SmallGrid G{};
+  G.solute = solute_groups;
+  G.solvent = (nwat + 3) / 4;
+  if (nqat > 0 && (mask & (QNB_T_QW | QNB_T_QP))) {
+    G.qchunks = std::max(1, std::min((nwat + nat_solute + QF_PART_SMALL - 1) / QF_PART_SMALL, 64));
+    G.qside = nqat * ((G.qchunks + 3) / 4);
+  }
+  if (nqat > 0 && (mask & (QNB_T_QQ | QNB_T_QQP))) G.qq = (std::max(nqe, 1) + 3) / 4;
+  if (pol) G.theta = (nwat + WP_THREADS - 1) / WP_THREADS;
+  return G;
+}
+
+template <typename R, int NS, bool E>
+static void launch_small(hipStream_t st, const SmallGrid& G, int B, const DevSys* dsys, uint32_t mask,
+                         const int* istep) {
+  const size_t lds = std::max(4 * so_wave_bytes<R>(),
+                              std::max(sizeof(double) * 4 * NS * 4, sizeof(double) * 3 * 4 * QNB_WAVE));
+  hipLaunchKernelGGL((k_forces_small<R, NS, E>), dim3(G.blocks(), B), dim3(256), lds, st, dsys, mask, G, istep);
+}
+
+template <typename R, bool E>
+static void launch_small_ns(int ns, hipStream_t st, const SmallGrid& G, int B, const DevSys* dsys, uint32_t mask,
+                            const int* istep) {
+  if (ns <= 1) launch_small<R, 1, E>(st, G, B, dsys, mask, istep);
+  else if (ns <= 2) launch_small<R, 2, E>(st, G, B, dsys, mask, istep);
+  else if (ns <= 4) launch_small<R, 4, E>(st, G, B, dsys, mask, istep);
+  else launch_small<R, 8, E>(st, G, B, dsys, mask, istep);
+}
+
+void launch_forces_small(hipStream_t st, int prec, int ns_max, bool energy, const SmallGrid& G, int B,
+                         const DevSys* dsys, uint32_t mask, const int* istep) {
+  if (G.blocks() <= 0) return;
+  if (prec == QNB_PREC_MIXED) {
+    if (energy) launch_small_ns<float, true>(ns_max, st, G, B, dsys, mask, istep);
+    else launch_small_ns<float, false>(ns_max, st, G, B, dsys, mask, istep);
+  } else {
+    if (energy) launch_small_ns<double, true>(ns_max, st, G, B, dsys, mask, istep);
+    else launch_small_ns<double, false>(ns_max, st, G, B, dsys, mask, istep);
+  }
+}
+
 // explicit instantiations used by the host code
 template __global__ void k_lists_lrf<double, false>(const DevSys*);
 template __global__ void k_lists_lrf<float, false>(const DevSys*);
 template __global__ void k_lists_lrf<double, true>(const DevSys*);
 template __global__ void k_lists_lrf<float, true>(const DevSys*);
 #define QNB_INST(R, NS)                                                            \
-  template __global__ void k_qforces<R, NS>(const DevSys*, uint32_t, int, double*, int);                       \
-  template __global__ void k_sforces<R, NS, true, WF_CAP_SMALL>(const DevSys*, uint32_t, int, int, int); \
-  template __global__ void k_sforces<R, NS, false, WF_CAP_SMALL>(const DevSys*, uint32_t, int, int, int); \
-  template __global__ void k_sforces<R, NS, true, FC_CAP>(const DevSys*, uint32_t, int, int, int);       \
-  template __global__ void k_sforces<R, NS, false, FC_CAP>(const DevSys*, uint32_t, int, int, int);      \
-  template __global__ void k_wforces<R, NS, true, WF_CAP_SMALL>(const DevSys*, uint32_t, int, int, int); \
-  template __global__ void k_wforces<R, NS, false, WF_CAP_SMALL>(const DevSys*, uint32_t, int, int, int); \
-  template __global__ void k_wforces<R, NS, true, FC_CAP>(const DevSys*, uint32_t, int, int, int);       \
-  template __global__ void k_wforces<R, NS, false, FC_CAP>(const DevSys*, uint32_t, int, int, int);       \
+  template __global__ void k_qforces<R, NS>(const DevSys*, uint32_t, int, int);                       \
+  template __global__ void k_sforces<R, NS, true>(const DevSys*, uint32_t, int, int, int); \
+  template __global__ void k_sforces<R, NS, false>(const DevSys*, uint32_t, int, int, int); \
+  template __global__ void k_wforces<R, NS, true>(const DevSys*, uint32_t, int, int, int); \
+  template __global__ void k_wforces<R, NS, false>(const DevSys*, uint32_t, int, int, int); \
   template __global__ void k_gforces<R, NS>(const DevSys*, uint32_t, int, int, int);
 QNB_INST(double, 1)
 QNB_INST(double, 2)
