@@ -282,17 +282,15 @@ int topo_build(DevSys& S, const qnb_system* s, HostTopo& T, DevAlloc& M) {
   UP(atom_group, atom_group.data(), nat);
   UP(gslot, gslot.data(), ncgpat);
   {
-    std::vector<int> off(1, 0), atoms;
-    for (int g = 0; g < s->ncgp_solute; g++) {
-      for (int k = s->cgp_first[g]; k <= s->cgp_last[g]; k++)
-        if (s->iqatom[s->cgpatom[k]] == 0) atoms.push_back(s->cgpatom[k]);
-      off.push_back((int)atoms.size());
-      T.max_nq_group = std::max(T.max_nq_group, off[g + 1] - off[g]);
-    }
-    T.n_nq = (int)atoms.size();
-    UP(nqoff, off.data(), off.size());
-    UP(nqatom, atoms.data(), atoms.size());
+    std::vector<int> entry(T.cgpatom);
+    for (int& e : entry)
+      if (s->iqatom[e] != 0) e |= AL_SKIP;
+    UP(cgentry, entry.data(), entry.size());
   }
+  T.n_group_atoms = s->ncgp_solute > 0 ? s->cgp_last[s->ncgp_solute - 1] + 1 : 0;
+  for (int g = 0; g < s->ncgp_solute; g++)
+    T.max_group = std::max(T.max_group, s->cgp_last[g] - s->cgp_first[g] + 1);
+  S.al_batch = T.max_group <= AL_BATCH ? AL_BATCH : FC_CAP;
 
   UP(avdw, s->avdw, 3 * s->ntypes);
   UP(bvdw, s->bvdw, 3 * s->ntypes);
@@ -466,42 +464,57 @@ int topo_build(DevSys& S, const qnb_system* s, HostTopo& T, DevAlloc& M) {
   return 0;
 }
 
-int row_alloc(DevSys& S, const HostTopo& T, DevAlloc& M, int cap) {
-  M.release(S.nbr);
-  M.release(S.alist);
-  S.nbr = S.alist = nullptr;
-  S.cap = cap;
-  // a row of cap groups and the receiver's own holds at most this many atoms
-  const long atoms = std::min((long)T.n_nq, ((long)cap + 1) * T.max_nq_group);
-  S.acap = (int)((std::max(atoms, 1L) + 63) / 64 * 64);
-  int rc = M.alloc(&S.nbr, (size_t)S.cap * S.ncgp);
-  return rc ? rc : M.alloc(&S.alist, (size_t)S.acap * S.ncgp);
+// A row of S.cap groups holds at most `atoms` atoms.  Of two batches in a row
+// the first ends because the next group would pass al_batch >= 128 slots, or
+// holds 64 groups, so batches hold 64 atoms on average and their padding (at
+// most 63 slots each, one batch more at the end) at most doubles the row.
+int atom_row_cap(const DevSys& S, const HostTopo& T) {
+  const long atoms = std::min((long)T.n_group_atoms, (long)S.cap * T.max_group);
+  return (int)((2 * atoms + 64 + 63) / 64 * 64);
 }
 
-int instance_alloc(DevSys& S, const HostTopo& T, DevAlloc& M, const qnb_params* p, int nslots) {
-  int rc = 0;
-#define AL(field, n)                                          \
-  do {                                                        \
-    if ((rc = M.alloc(&S.field, (size_t)(n)))) return rc;     \
-  } while (0)
+int atom_rows_alloc(DevSys& S, const HostTopo& T, DevAlloc& M) {
+  M.release(S.alist);
+  S.alist = nullptr;
+  S.acap = atom_row_cap(S, T);
+  return M.alloc(&S.alist, (size_t)S.acap * S.ncgp);
+}
+
+int row_alloc(DevSys& S, DevAlloc& M, int cap) {
+  M.release(S.nbr);
+  S.nbr = nullptr;
+  S.cap = cap;
+  return M.alloc(&S.nbr, (size_t)S.cap * S.ncgp);
+}
+
+int instance_alloc(DevSys& S, DevAlloc& M, const qnb_params* p, int nslots) {
+  // one allocation for all of the instance's buffers but the rows, which are
+  // sized and resized on their own
+  std::vector<std::pair<void**, size_t>> want;
+  size_t total = 0;
+  auto add = [&](auto** field, size_t n) {
+    want.push_back({(void**)field, total});
+    total += (std::max(n, (size_t)1) * sizeof(**field) + 255) & ~(size_t)255;
+  };
+#define AL(field, n) add(&S.field, (size_t)(n))
   const int nat = S.natom, nsol1 = std::max(S.nat_solute, 1), nw1 = std::max(S.nwat, 1);
   AL(x, 3 * nat);
+  S.xqg = nullptr;
+  S.xqgd = nullptr;
   if (p->precision == QNB_PREC_MIXED) AL(xqg, 4 * (size_t)S.ncgpat);
   else AL(xqgd, 4 * (size_t)S.ncgpat);
   AL(gref, 4 * (size_t)S.ncgp);
   AL(d, 3 * nat);
-  AL(dq, 3 * (size_t)std::max(S.nqat, 1));
-  AL(dqq, 3 * (size_t)std::max(S.nqe, 1));
+  AL(dq, 3 * (size_t)S.nqat);
+  AL(dqq, 3 * (size_t)S.nqe);
   AL(lrf, (size_t)QNB_NLRF * S.ncgp);
-  S.nbr = S.alist = nullptr;
-  if (int rc2 = row_alloc(S, T, M, S.cap > 0 ? S.cap : 256)) return rc2;
-  AL(alist_n, 2 * (size_t)S.ncgp);
+  AL(alist_n, S.ncgp);
   AL(nnbr, S.ncgp);
   AL(nnsol, S.ncgp);
-  AL(pw_first, std::max(S.ncgp_solute, 1));
+  AL(pw_first, S.ncgp_solute);
   AL(need, 1);
   AL(qw_in, nw1);
-  AL(qp_in, std::max(S.ncgp_solute, 1));
+  AL(qp_in, S.ncgp_solute);
   AL(qw_list, nw1);
   AL(qp_list, nsol1);
   AL(nq_lists, 2);
@@ -517,20 +530,17 @@ int instance_alloc(DevSys& S, const HostTopo& T, DevAlloc& M, const qnb_params* 
   AL(sh_lth, (size_t)QNB_MAXSH * nw1);
   AL(sh_n, QNB_MAXSH);
   AL(wp_rank, 2 * (size_t)QNB_MAXSH * nw1);
-
 #undef AL
+  unsigned char* base = nullptr;
+  if (int rc = M.alloc(&base, total)) return rc;
+  for (auto& w : want) *w.first = base + w.second;
+  // counts, flags, energies and the Q-atom rows start at zero
+  HIPCHK(hipMemset(base, 0, total));
   double sh0[3 * QNB_MAXSH] = {0};
   for (int k = 0; k < S.nshell; k++) sh0[k] = p->wshell_theta_corr[k];
   HIPCHK(hipMemcpy(S.sh_state, sh0, sizeof sh0, hipMemcpyHostToDevice));
-  HIPCHK(hipMemset(S.nq_lists, 0, 2 * sizeof(int)));
-  HIPCHK(hipMemset(S.dq, 0, sizeof(double) * 3 * std::max(S.nqat, 1)));
-  HIPCHK(hipMemset(S.need, 0, sizeof(int)));
-  HIPCHK(hipMemset(S.sh_n, 0, sizeof(int) * QNB_MAXSH));
-  HIPCHK(hipMemset(S.nnbr, 0, sizeof(int) * S.ncgp));
-  HIPCHK(hipMemset(S.nnsol, 0, sizeof(int) * S.ncgp));
-  HIPCHK(hipMemset(S.alist_n, 0, sizeof(int) * 2 * S.ncgp));
-  HIPCHK(hipMemset(S.ered, 0, sizeof(double) * QNB_NE));
-  return 0;
+  S.nbr = S.alist = nullptr;
+  return row_alloc(S, M, S.cap > 0 ? S.cap : 256);
 }
 
 }  // namespace qnb
@@ -648,7 +658,8 @@ extern "C" int32_t qnb_create(const qnb_system* s, const qnb_params* p, qnb_hand
   DevSys& S = h->hs;
   memset(&S, 0, sizeof S);
   fill_params(S, s, p);
-  if ((rc = topo_build(S, s, h->T, h->mem)) || (rc = instance_alloc(S, h->T, h->mem, p, s->ncgp + qq_slots(S))) ||
+  if ((rc = topo_build(S, s, h->T, h->mem)) || (rc = instance_alloc(S, h->mem, p, s->ncgp + qq_slots(S))) ||
+      (rc = atom_rows_alloc(S, h->T, h->mem)) ||
       (rc = h->mem.alloc(&h->d_tfree, 1)) || (rc = h->mem.alloc(&h->d_istep, 1)) || (rc = h->mem.alloc(&h->dsys, 1))) {
     delete h;
     return rc;
@@ -694,7 +705,7 @@ extern "C" int32_t qnb_make_pair_lists(qnb_handle* h, const double* x) {
     if (need <= h->hs.cap) break;
     // reallocate_nonbondlist_* (qalloc.f90:370-605): grow and rebuild
     int ncap = ((need * 5 / 4) + 63) / 64 * 64;
-    if ((rc = row_alloc(h->hs, h->T, h->mem, ncap))) return rc;
+    if ((rc = row_alloc(h->hs, h->mem, ncap)) || (rc = atom_rows_alloc(h->hs, h->T, h->mem))) return rc;
     HIPCHK(hipMemcpy(h->dsys, &h->hs, sizeof(DevSys), hipMemcpyHostToDevice));
     if (attempt == 3) return fail(QNB_EOVERFLOW, "neighbour list capacity");
   }

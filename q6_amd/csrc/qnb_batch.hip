@@ -564,7 +564,8 @@ __global__ void k_exc_record(const DevSys* __restrict__ systems, const MdDev* __
                              const ExcDev* __restrict__ excs);
 
 // launchers shared by the step, the minimiser, the timer and the autotuner
-static void launch_lists(qnb_batch* b, int wpb) {
+// `rows`: expand the neighbour rows into partner atoms too
+static void launch_lists(qnb_batch* b, int wpb, bool rows = true) {
   dim3 g((b->maxg + wpb - 1) / wpb, b->n), t(64 * wpb);
   bool any = false, quirk = false;
   int maxsg = 0;
@@ -582,7 +583,7 @@ static void launch_lists(qnb_batch* b, int wpb) {
     if (any) hipLaunchKernelGGL((k_lists_lrf<double, true>), g, t, 0, b->stream, b->dsys);
     else hipLaunchKernelGGL((k_lists_lrf<double, false>), g, t, 0, b->stream, b->dsys);
   }
-  hipLaunchKernelGGL(k_expand, dim3((b->maxg + 3) / 4, b->n), dim3(256), 0, b->stream, b->dsys);
+  if (rows) hipLaunchKernelGGL(k_expand, dim3((b->maxg + 3) / 4, b->n), dim3(256), 0, b->stream, b->dsys);
 }
 
 static const uint32_t kStepMask = QNB_T_NONBONDED | QNB_T_QQ | QNB_T_QQP | QNB_T_RAD | QNB_T_POL;
@@ -823,7 +824,7 @@ extern "C" int32_t qnb_batch_create(int32_t n, const qnb_system* const* sys, con
       b->topo_of.push_back(b->topo_of[it->second]);
     }
     S.cap = 0;
-    if ((rc = instance_alloc(S, *b->topos[b->topo_of[k]], b->mem, par[k], sys[k]->ncgp + qq_slots(S)))) return rc;
+    if ((rc = instance_alloc(S, b->mem, par[k], sys[k]->ncgp + qq_slots(S)))) return rc;
     HIPCHK(hipMemcpy(S.x, x0[k], sizeof(double) * 3 * S.natom, hipMemcpyHostToDevice));
     b->maxg = std::max(b->maxg, S.ncgp);
     b->maxw = std::max(b->maxw, S.nwat);
@@ -969,13 +970,13 @@ extern "C" int32_t qnb_batch_create(int32_t n, const qnb_system* const* sys, con
   // during a run is reported by qnb_batch_sync)
   for (int k = 0; k < n; k++) {
     DevSys& S = b->hs[k];
-    if ((rc = row_alloc(S, *b->topos[b->topo_of[k]], b->mem, std::min(((S.ncgp + 63) / 64) * 64, 1024)))) return rc;
+    if ((rc = row_alloc(S, b->mem, std::min(((S.ncgp + 63) / 64) * 64, 1024)))) return rc;
   }
   for (int attempt = 0;; attempt++) {
     HIPCHK(hipMemcpy(b->dsys, b->hs.data(), sizeof(DevSys) * n, hipMemcpyHostToDevice));
     for (int k = 0; k < n; k++) HIPCHK(hipMemset(b->hs[k].need, 0, sizeof(int)));
     const int wpb = 4;
-    launch_lists(b.get(), wpb);
+    launch_lists(b.get(), wpb, false);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(b->stream));
     bool again = false;
@@ -984,7 +985,7 @@ extern "C" int32_t qnb_batch_create(int32_t n, const qnb_system* const* sys, con
       int need = 0;
       HIPCHK(hipMemcpy(&need, S.need, sizeof(int), hipMemcpyDeviceToHost));
       if (need > S.cap) {
-        if ((rc = row_alloc(S, *b->topos[b->topo_of[k]], b->mem, ((need + 63) / 64) * 64))) return rc;
+        if ((rc = row_alloc(S, b->mem, ((need + 63) / 64) * 64))) return rc;
         again = true;
       }
     }
@@ -1000,9 +1001,24 @@ extern "C" int32_t qnb_batch_create(int32_t n, const qnb_system* const* sys, con
     const int cap = ((mx * 3 / 2 + 64) + 63) / 64 * 64;
     if (cap < S.cap) {
       // shrink: rebuild happens at the first step of the run
-      if ((rc = row_alloc(S, *b->topos[b->topo_of[k]], b->mem, cap))) return rc;
+      if ((rc = row_alloc(S, b->mem, cap))) return rc;
     }
     HIPCHK(hipMemset(S.need, 0, sizeof(int)));
+  }
+  // the partner-atom rows of all instances in one allocation
+  {
+    size_t total = 0;
+    for (int k = 0; k < n; k++) {
+      DevSys& S = b->hs[k];
+      S.acap = atom_row_cap(S, *b->topos[b->topo_of[k]]);
+      total += (size_t)S.acap * S.ncgp;
+    }
+    int* rows = nullptr;
+    if ((rc = b->mem.alloc(&rows, total))) return rc;
+    for (int k = 0; k < n; k++) {
+      b->hs[k].alist = rows;
+      rows += (size_t)b->hs[k].acap * b->hs[k].ncgp;
+    }
   }
   HIPCHK(hipMemcpy(b->dsys, b->hs.data(), sizeof(DevSys) * n, hipMemcpyHostToDevice));
   {

@@ -62,10 +62,8 @@ struct DevSys {
   // the atom's group modulo 64, its bit in the far-group ballot word of the
   // list sweep's 64-group chunk
   const int* gslot;
-  // the solute groups' atoms without Q-atoms: group b's at nqatom[nqoff[b]] ..
-  const int* nqoff;
-  const int* nqatom;
   int ncgpat;
+  const int* cgentry;  // per group-ordered atom: its index, with AL_SKIP for a Q-atom (k_expand)
   const double* avdw;  // [t*3+k]
   const double* bvdw;
   const int* ljcod;    // [ti + tj*ntypes], 1-based code
@@ -156,11 +154,11 @@ struct DevSys {
   double* lrf;
   int* nbr;
   int* nnbr;
-  // partner atoms of each receiver (k_expand): rows of acap entries, counts
-  // [ncgp][2] from the front and from the back
+  // partner atoms of each receiver (k_expand): rows of acap slots, the slots in
+  // use [ncgp], slots per batch of groups
   int* alist;
   int* alist_n;
-  int acap;
+  int acap, al_batch;
   int* nnsol;  // [ncgp] length of the row's solute prefix (rows are sorted)
   // reference test-point reuse of the LRF-off switch-atom solute-water list
   // (quirk bit 0 with use_lrf = 0): per solute group, the first water within
@@ -763,6 +761,12 @@ __device__ __forceinline__ void rinv(float d2, float& r2, float& r) {
   r = __builtin_amdgcn_rsqf(d2);
   r2 = r * r;
 }
+// |u|^2; in FP32 with the multiply-adds written out, so that its rounding does
+// not depend on which of them the compiler would fuse at a call site
+__device__ __forceinline__ double norm2(double x, double y, double z) { return x * x + y * y + z * z; }
+__device__ __forceinline__ float norm2(float x, float y, float z) {
+  return __builtin_fmaf(z, z, __builtin_fmaf(x, x, y * y));
+}
 // 1/v: IEEE in FP64, hardware reciprocal (v_rcp_f32, 1 ulp) in FP32
 __device__ __forceinline__ double recip(double v) { return 1.0 / v; }
 __device__ __forceinline__ float recip(float v) { return __builtin_amdgcn_rcpf(v); }
@@ -778,7 +782,7 @@ struct PairMath {
   template <typename T>
   static __device__ __forceinline__ R nbe(R ux, R uy, R uz, R A, R B, R q, T& el, T& vdw, bool want = true) {
     R r2, r;
-    rinv(ux * ux + uy * uy + uz * uz, r2, r);
+    rinv(norm2(ux, uy, uz), r2, r);
     R r6 = r2 * r2 * r2;
     R r12 = r6 * r6;
     R Vel = q * r, Va = A * r12, Vb = B * r6;
@@ -792,7 +796,7 @@ struct PairMath {
   template <typename T>
   static __device__ __forceinline__ R nbe_spc(R ux, R uy, R uz, R q, T& el, bool want = true) {
     R r2, r;
-    rinv(ux * ux + uy * uy + uz * uz, r2, r);
+    rinv(norm2(ux, uy, uz), r2, r);
     R Vel = q * r;
     if (want) el += (T)Vel;
     return -r2 * Vel;
@@ -800,11 +804,12 @@ struct PairMath {
   // nbe_qx (nonbonded.f90:200-222), soft-core score sc, state weight lam
   static __device__ __forceinline__ R nbe_qx(R r2, R r, R r6in, R A, R B, R q, R sc, R lam, double& el,
                                              double& vdw, bool want = true) {
-    R r6 = r6in, soft = R(1);
-    if (sc != R(0)) {
-      const R r6_hc = recip(r6in);
+    R r6_hc = R(1), r6 = r6in;
+    // FP64: without a soft core 1/(1/r6) and r6/r6 are r6 and 1; FP32 keeps the
+    // rounding of the two reciprocals
+    if (sizeof(R) == 4 || sc != R(0)) {
+      r6_hc = recip(r6in);
       r6 = recip(r6_hc + sc);
-      soft = r6 * r6_hc;
     }
     R r12 = r6 * r6;
     R Vel = q * r, Va = A * r12, Vb = B * r6;
@@ -812,7 +817,8 @@ struct PairMath {
       el += (double)Vel;
       vdw += (double)Va - (double)Vb;
     }
-    return r2 * (-Vel - (R(12) * Va - R(6) * Vb) * soft) * lam;
+    if (sizeof(R) == 8 && sc == R(0)) return r2 * (-Vel - (R(12) * Va - R(6) * Vb)) * lam;
+    return r2 * (-Vel - (R(12) * Va - R(6) * Vb) * r6 * r6_hc) * lam;
   }
 };
 
@@ -854,15 +860,17 @@ struct SmallGrid {
 #ifndef FC_CAP
 #define FC_CAP 384
 #endif
-// partner-atom entries (DevSys::alist): atom index and flags
-enum : int { AL_ATOM = (1 << 28) - 1, AL_OWN = 1 << 28, AL_SELF = 1 << 29 };
+// partner-atom entries (DevSys::alist): atom index and flags; slots per batch
+// of groups where every solute group fits in them, else FC_CAP
+enum : int { AL_ATOM = (1 << 28) - 1, AL_OWN = 1 << 28, AL_FAR = 1 << 29, AL_SKIP = 1 << 30 };
+#define AL_BATCH 128
 // Solute-receiver force kernel (k_sforces): receiver atoms per sweep, at most
 // as many as the scalar registers hold (6 values of R each), and per-wave LDS
 template <typename R>
 __host__ __device__ constexpr int so_ch() { return sizeof(R) == 4 ? 10 : 5; }
 template <typename R>
 __host__ __device__ constexpr size_t so_wave_bytes() {
-  return (so_ch<R>() * (sizeof(double) + 11 * sizeof(R) + 3 * sizeof(int)) + 15) / 16 * 16;
+  return (so_ch<R>() * (5 * sizeof(double) + 12 * sizeof(R) + 4 * sizeof(int)) + 15) / 16 * 16;
 }
 
 // Placement of a batch's blocks on the XCDs.  Blocks are dealt to the 8 XCDs

@@ -57,7 +57,7 @@ struct DevAlloc {
 // host copies of the topology kept for list export
 struct HostTopo {
   int ntypes = 0, ivdw_rule = 1;
-  int n_nq = 0, max_nq_group = 0;  // non-Q atoms of the solute groups: all, most in one group
+  int n_group_atoms = 0, max_group = 0;  // atoms of the solute groups: all, most in one group
   std::vector<int> gfirst, glast, gswitch, cgpatom, iqatom, iac, ljcod, lx_off, lx_j, iqseq;
   std::vector<uint8_t> excl, qconn3, lx_kind;
   std::vector<uint32_t> exmask, m14mask;
@@ -85,9 +85,12 @@ bool small_launch(long solute_groups, long solvent);
 // the per-system sums (finish) where no later kernel of the caller runs them
 void launch_watpol(hipStream_t st, int nwat, int B, const DevSys* dsys, const int* istep, bool theta, bool finish);
 // per-instance device state (coordinates, gradient, lists, LRF, energies)
-int instance_alloc(DevSys& S, const HostTopo& T, DevAlloc& M, const qnb_params* p, int nslots);
-// neighbour rows of `cap` groups and the partner-atom rows that hold them
-int row_alloc(DevSys& S, const HostTopo& T, DevAlloc& M, int cap);
+int instance_alloc(DevSys& S, DevAlloc& M, const qnb_params* p, int nslots);
+// neighbour rows of `cap` groups; entries per partner-atom row that always
+// hold such a row's atoms (k_expand), and the rows themselves
+int row_alloc(DevSys& S, DevAlloc& M, int cap);
+int atom_row_cap(const DevSys& S, const HostTopo& T);
+int atom_rows_alloc(DevSys& S, const HostTopo& T, DevAlloc& M);
 // group contributions (qnb_exc.hip): the pair lists of each energy array
 // and state, built on the host from the system's Q tables
 struct ExcHost {

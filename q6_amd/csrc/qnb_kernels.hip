@@ -589,8 +589,11 @@ __device__ __forceinline__ bool pp_pair(const DevSys& S, const PPAtom& P, const 
 // The lambda-weighted dv of a Q pair over its states (nbe_qx per state,
 // nonbonded.f90:200-222): `par(s)` gives state s's A, B, el and soft-core score.
 // Without a soft core the force is linear in A, B and el, so on the steps that
-// sample no energies the states' parameters are weighted and summed first and
-// the pair is evaluated once.
+// sample no energies the FP64 path weights and sums the states' parameters
+// first and evaluates the pair once.  The mixed path keeps the states apart,
+// as every FP32 sum of these kernels keeps its terms and their order: a run of
+// many windows meets a group pair at its cut-off at every list update, and
+// another rounding of the forces would take such a pair the other way.
 template <typename R>
 struct QPar {
   R A, B, q, sc;
@@ -598,6 +601,16 @@ struct QPar {
 template <typename R, int NS, typename F>
 __device__ __forceinline__ R qx_states(const DevSys& S, R r2, R r, int ns, double* eq, bool want, F par) {
   const R r6 = r2 * r2 * r2;
+  if constexpr (sizeof(R) == 4) {
+    R dvs = R(0);
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+      if (s >= ns) break;
+      const QPar<R> p = par(s);
+      dvs += PairMath<R>::nbe_qx(r2, r, r6, p.A, p.B, p.q, p.sc, (R)S.lambda[s], eq[2 * s], eq[2 * s + 1], want);
+    }
+    return dvs;
+  }
   QPar<R> p[NS];
   R A = R(0), B = R(0), q = R(0);
   bool soft = false;
@@ -624,15 +637,15 @@ __device__ __forceinline__ R qx_states(const DevSys& S, R r2, R r, int ns, doubl
 // Coulomb only (nbe_qspc, nonbonded.f90:226-243: an SPC hydrogen)
 template <typename R, int NS, typename F>
 __device__ __forceinline__ R qspc_states(const DevSys& S, R r2, R r, int ns, double* eq, bool want, F el) {
-  R q = R(0);
+  R dvs = R(0);
 #pragma unroll
   for (int s = 0; s < NS; s++) {
     if (s >= ns) break;
-    const R e = el(s);
-    if (want) eq[2 * s] += (double)(e * r);
-    q += (R)S.lambda[s] * e;
+    const R Vel = el(s) * r;
+    if (want) eq[2 * s] += (double)Vel;
+    dvs += -r2 * Vel * (R)S.lambda[s];
   }
-  return -r2 * r * q;
+  return dvs;
 }
 // entry (iq, k, s) of the Q-solvent table in the pair arithmetic's type
 template <typename R>
@@ -647,67 +660,76 @@ __device__ __forceinline__ R qw_el(const DevSys& S, int iq, int k, int s) {
 
 // ---------------------------------------------------------------------------
 // Partner atoms of every receiver group, written after each list update and
-// read by the force kernels of every step until the next one: the row's solute
-// groups (and, for a solute receiver, the group itself) as atoms, Q-atoms left
-// out (their pairs belong to the Q kernels).  One wavefront per receiver, lane
-// = partner group.  Row a of S.alist holds from its front the atoms of groups
-// that can hold an excluded or 1-4 pair with a solute receiver (an index
-// within 25 of the receiver's, long-range partners in either group, or the
-// group itself), from its back downwards the others; the counts go to
-// alist_n.  An entry is the atom's index with AL_OWN (the receiver owns the
-// energy of the two groups' pairs) and AL_SELF (the receiver's own group).
+// read by the force kernels of every step until the next one: the solute
+// groups of the row's prefix as atoms.  One wavefront per receiver, lane =
+// partner group; the groups are taken in batches of up to 64 whose atoms fit
+// in `batch` slots (al_batch) and every batch ends at a multiple of 64 slots,
+// so lane l of the force kernels, taking slots l, l + 64, ..., always adds the
+// same partners in the same order.  An entry is the atom's index with AL_OWN
+// (the receiver owns the energy of the two groups' pairs) and AL_FAR (a solute
+// receiver and a group that can hold no excluded or 1-4 pair with it: every
+// index more than 25 from the receiver's, no long-range partners in either);
+// AL_SKIP marks Q-atoms (their pairs belong to the Q kernels) and the padding.
 // The force kernels then read one coalesced list per receiver instead of
 // walking group -> atoms -> positions through LDS at every step.
 __global__ __launch_bounds__(256) void k_expand(const DevSys* __restrict__ systems) {
   const DevSys& S = systems[blockIdx.y];
   const int a = uni(blockIdx.x * (blockDim.x / QNB_WAVE) + threadIdx.x / QNB_WAVE);
   if (a >= S.ncgp) return;
-  const int lane = threadIdx.x % QNB_WAVE, ncs = S.ncgp_solute;
-  const bool a_sol = a < ncs;
+  const int lane = threadIdx.x % QNB_WAVE, batch = S.al_batch;
+  const bool a_sol = a < S.ncgp_solute;
   const int nsr = uni(min(ldg(S.nnsol + a), S.cap));
   const int* __restrict__ row = S.nbr + (size_t)a * S.cap;
   int* __restrict__ out = S.alist + (size_t)a * S.acap;
   const bool along = a_sol && ldg(S.glong + a);
   const int alo = a_sol ? ldg(S.gspan + 2 * a) : 0, ahi = a_sol ? ldg(S.gspan + 2 * a + 1) : 0;
-  int near = 0, far = 0;
-  // index nsr stands for the receiver itself
-  const int nv = nsr + (a_sol && !ldg(S.excl + ldg(S.gswitch + a)) ? 1 : 0);
-  for (int v0 = 0; v0 < nv; v0 += QNB_WAVE) {
-    const int v = v0 + lane;
-    int off = 0, cnt = 0, tag = 0;
-    bool isnear = false;
-    if (v < nv) {
-      const int b = v < nsr ? ldg(row + v) : a;
-      off = ldg(S.nqoff + b);
-      cnt = ldg(S.nqoff + b + 1) - off;
+  __shared__ int s_incl[4][QNB_WAVE], s_src[4][QNB_WAVE], s_tag[4][QNB_WAVE];
+  const int w = threadIdx.x / QNB_WAVE;
+  int n = 0;
+  for (int p0 = 0, ng = 0; p0 < nsr; p0 += ng) {
+    const int p = p0 + lane;
+    int f0 = 0, cnt = 0, tag = 0;
+    if (p < nsr) {
+      const int b = ldg(row + p);
+      f0 = ldg(S.gfirst + b);
+      cnt = ldg(S.glast + b) - f0 + 1;
       tag = owns(a, b) ? AL_OWN : 0;
-      if (b == a) {
-        tag = AL_SELF;
-        isnear = true;
-      } else if (a_sol) {
+      if (a_sol && !along && !ldg(S.glong + b)) {
         const int blo = ldg(S.gspan + 2 * b), bhi = ldg(S.gspan + 2 * b + 1);
-        isnear = along || ldg(S.glong + b) || !(blo - ahi > 25 || alo - bhi > 25);
+        if (blo - ahi > 25 || alo - bhi > 25) tag |= AL_FAR;
       }
     }
-    int in = isnear ? cnt : 0, fa = isnear ? 0 : cnt;
+    int incl = cnt;
 #pragma unroll
     for (int o = 1; o < QNB_WAVE; o <<= 1) {
-      const int u = __shfl_up(in, o, QNB_WAVE), w = __shfl_up(fa, o, QNB_WAVE);
-      if (lane >= o) {
-        in += u;
-        fa += w;
-      }
+      const int u = __shfl_up(incl, o, QNB_WAVE);
+      if (lane >= o) incl += u;
     }
-    int pos = isnear ? near + in - cnt : S.acap - 1 - (far + fa - cnt);
-    const int step = isnear ? 1 : -1;
-    for (int m = 0; m < cnt; m++, pos += step) stg(out + pos, ldg(S.nqatom + off + m) | tag);
-    near += __shfl(in, QNB_WAVE - 1, QNB_WAVE);
-    far += __shfl(fa, QNB_WAVE - 1, QNB_WAVE);
+    // inclusive sums never decrease, so the groups that fit are a prefix (a
+    // group always fits)
+    ng = min(__popcll(__ballot(incl <= batch)), nsr - p0);
+    const int total = __shfl(incl, ng - 1, QNB_WAVE);
+    // lane = slot: its group is the first whose inclusive count passes it
+    s_incl[w][lane] = incl;
+    s_src[w][lane] = f0 - (incl - cnt);
+    s_tag[w][lane] = tag;
+    __builtin_amdgcn_wave_barrier();
+    const int end = (total + QNB_WAVE - 1) / QNB_WAVE * QNB_WAVE;
+    for (int s = lane; s < end; s += QNB_WAVE) {
+      int e = AL_SKIP;
+      if (s < total) {
+        int g = 0;
+#pragma unroll
+        for (int h = 32; h > 0; h >>= 1)
+          if (s_incl[w][g + h - 1] <= s) g += h;
+        e = ldg(S.cgentry + s_src[w][g] + s) | s_tag[w][g];
+      }
+      stg(out + n + s, e);
+    }
+    __builtin_amdgcn_wave_barrier();
+    n += end;
   }
-  if (lane == 0) {
-    S.alist_n[2 * a] = near;
-    S.alist_n[2 * a + 1] = far;
-  }
+  if (lane == 0) S.alist_n[a] = n;
 }
 
 // ---------------------------------------------------------------------------
@@ -717,15 +739,15 @@ __global__ __launch_bounds__(256) void k_expand(const DevSys* __restrict__ syste
 // for every lane and live in scalar registers, and a lane takes one partner at
 // a time against them, the next partner's data in flight meanwhile:
 //  * solute partners from the receiver's atom list (k_expand; nonbond_pp,
-//    nonbondene.f90:4694-4760): the atoms of groups without an excluded or 1-4
-//    pair take A, B and qq as products of per-atom factors when the system
-//    uses the geometric rule with LJ code 1 throughout (ppfast): the products
-//    pp_param forms for such a pair, same operands; every other pair, those
-//    inside a included (ig == jgr, i < j, nonbondene.f90:1610), goes through
-//    pp_param (exclusions, 1-4, ljcod, rule);
-//  * solvent partners, a lane per molecule, its sites in turn (nonbond_pw
-//    4856-4916; a site without LJ parameters takes Coulomb only);
-//  * the receiver side of the Q-atom - solute pairs (nonbond_qp 5157-5230).
+//    nonbondene.f90:4694-4760): those of a group without an excluded or 1-4
+//    pair (AL_FAR) take A, B and qq as products of per-atom factors when the
+//    system uses the geometric rule with LJ code 1 throughout (ppfast): the
+//    products pp_param forms for such a pair, same operands; every other pair
+//    goes through the exclusion masks and pp_param's rules;
+//  * partner waters with the fixed mapping of k_wforces (lane l takes site
+//    l % 3 of water l / 3 of the round; nonbond_pw 4856-4916);
+//  * the pairs inside the group (ig == jgr, i < j, nonbondene.f90:1610) and
+//    the receiver side of the Q-atom - solute pairs (nonbond_qp 5157-5230).
 // Writes d of the group's atoms, and the pp, pw and qp energy partials on the
 // sampled steps (a pp pair's energy on its owner side).
 //
@@ -734,22 +756,8 @@ __global__ __launch_bounds__(256) void k_expand(const DevSys* __restrict__ syste
 // in vector registers (167 of them, three waves per SIMD), took 213 us at 51
 // windows of 400 ten-atom groups and 52 us for one FP64 window; staging by
 // blocks of four waves 310 us at 51 windows (its barriers wait on four chains
-// of loads); from the atom lists it takes 156 us, and 20 us split four ways.
-
-// per-pair LJ + Coulomb with the factors 12 and 6 already in A and B: returns
-// nbe's dv
-template <typename R>
-__device__ __forceinline__ R pair_dv(R ux, R uy, R uz, R A12, R B6, R q, R& el, R& vdw, bool want) {
-  R r2, r;
-  rinv(ux * ux + uy * uy + uz * uz, r2, r);
-  const R r6 = r2 * r2 * r2;
-  const R Vel = q * r;
-  if (want) {
-    el += Vel;
-    vdw += A12 * (r6 * r6) * R(1.0 / 12.0) - B6 * r6 * R(1.0 / 6.0);
-  }
-  return r2 * (r6 * (B6 - A12 * r6) - Vel);
-}
+// of loads); from the atom lists it takes 151 us, and about 20
+// us split four ways.
 
 __device__ __forceinline__ float lane_get(float v, int lane) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
@@ -773,12 +781,15 @@ __device__ __forceinline__ void solute_receiver(const DevSys& S, uint32_t mask, 
                                                 unsigned char* wbase, double (*comb)[QNB_WAVE]) {
   constexpr int CH = so_ch<R>();
   const int lane = threadIdx.x % QNB_WAVE;
-  // the sweep's receiver data that only the rarer pairs need, in LDS: charge,
-  // solute-solvent parameters of the three water sites, LJ factors of code 3,
-  // type, masks
+  // the sweep's receiver data in LDS for the pairs that take it by lane:
+  // charge, LJ factors of codes 1 and 3, solute-solvent parameters of the
+  // three water sites, offset, index, type, masks
   double* s_rq = reinterpret_cast<double*>(wbase);
-  R(*s_pw)[11] = reinterpret_cast<R(*)[11]>(s_rq + CH);
-  int* s_rt = reinterpret_cast<int*>(s_pw + CH);
+  double(*s_r3)[4] = reinterpret_cast<double(*)[4]>(s_rq + CH);
+  R(*s_pw)[3][3] = reinterpret_cast<R(*)[3][3]>(s_r3 + CH);
+  R(*s_o)[3] = reinterpret_cast<R(*)[3]>(s_pw + CH);
+  int* s_ia = reinterpret_cast<int*>(s_o + CH);
+  int* s_rt = s_ia + CH;
   uint32_t* s_rx = reinterpret_cast<uint32_t*>(s_rt + CH);
   uint32_t* s_rm = s_rx + CH;
   const double* __restrict__ x = S.x;
@@ -786,7 +797,6 @@ __device__ __forceinline__ void solute_receiver(const DevSys& S, uint32_t mask, 
   const int nn = uni(min(ldg(S.nnbr + a), S.cap)), nsr = uni(min(ldg(S.nnsol + a), nn));
   const int* __restrict__ row = S.nbr + (size_t)a * S.cap;
   const int* __restrict__ al = S.alist + (size_t)a * S.acap;
-  const int acap = S.acap;
   const bool want_e = E && want_energies(S);
   const int nsol = S.nat_solute, sa = S.sa, ncs = S.ncgp_solute;
   const int ra = uni(ldg(S.gswitch + a));
@@ -801,17 +811,17 @@ __device__ __forceinline__ void solute_receiver(const DevSys& S, uint32_t mask, 
   const int nq = S.nqat, ns = S.nstates;
   const bool qin = (mask & T_QP) && nq > 0 && uni(ldg(S.qp_in + a));
   const bool pp = (mask & T_PP) && !aexcl;
-  const int n_near = pp ? uni(ldg(S.alist_n + 2 * a)) : 0, n_far = pp ? uni(ldg(S.alist_n + 2 * a + 1)) : 0;
+  const int nsl = pp ? uni(ldg(S.alist_n + a)) : 0;
   const bool pw = (mask & T_PW) && !aexcl && nsr < nn;
   // SPLIT: sets of waves with receiver atoms of their own (nset), the waves of
   // a set sharing the partners
   const int nset = !SPLIT || na <= CH ? 1 : (na <= 2 * CH ? 2 : 4), parts = SPLIT ? waves / nset : 1;
   const int set = SPLIT ? wave / parts : 0, part = SPLIT ? wave % parts : 0;
-  // the first far partners' entries, and the first of their positions, are
-  // requested before the receiver's own chain of loads
-  const int t0 = lane + QNB_WAVE * part;
-  auto far_entry = [&](int t) { return t < n_far ? ldg(al + (acap - 1 - t)) : ra; };
-  const int e0 = fast ? far_entry(t0) : ra, e1 = fast ? far_entry(t0 + QNB_WAVE * parts) : ra;
+  // the first two rounds' entries are requested before the receiver's own
+  // chain of loads
+  const int t0 = lane + QNB_WAVE * part, ts = QNB_WAVE * parts;
+  auto entry = [&](int t) { return t < nsl ? ldg(al + t) : (int)AL_SKIP; };
+  const int e0 = entry(t0), e1 = entry(t0 + ts);
   for (int cb = 0; cb < na; cb += nset * CH) {
     const int c0 = cb + set * CH, nk = max(0, min(CH, na - c0));
     // receiver atoms: lane k loads atom c0 + k (index -1: takes no pair
@@ -825,23 +835,29 @@ __device__ __forceinline__ void solute_receiver(const DevSys& S, uint32_t mask, 
       ol0 = (R)(ldg(x + 3 * i) - xr0);
       ol1 = (R)(ldg(x + 3 * i + 1) - xr1);
       ol2 = (R)(ldg(x + 3 * i + 2) - xr2);
+      s_ia[lane] = il;
+      s_o[lane][0] = ol0;
+      s_o[lane][1] = ol1;
+      s_o[lane][2] = ol2;
       const R* pf = qp_tab<R>(S.ppd, S.ppf) + PP_REC * (size_t)i;
-      fa = R(12) * ldg(pf);
-      fb = R(6) * ldg(pf + 1);
+      fa = ldg(pf);
+      fb = ldg(pf + 1);
       fc = ldg(pf + 2);
       s_rt[lane] = ldg(S.iac + i);
       s_rx[lane] = ldg(S.exmask + i);
       s_rm[lane] = ldg(S.m14mask + i);
       s_rq[lane] = ldg(S.crg + i);
-      s_pw[lane][9] = R(12) * ldg(pf + 4);
-      s_pw[lane][10] = R(6) * ldg(pf + 5);
+      s_r3[lane][0] = ldg(S.ppd + PP_REC * (size_t)i);
+      s_r3[lane][1] = ldg(S.ppd + PP_REC * (size_t)i + 1);
+      s_r3[lane][2] = ldg(S.ppd + PP_REC * (size_t)i + 4);
+      s_r3[lane][3] = ldg(S.ppd + PP_REC * (size_t)i + 5);
       if (pw && sa == 3)
 #pragma unroll
         for (int kb = 0; kb < 3; kb++) {
           const size_t tt = (size_t)i + (size_t)nsol * kb;
-          s_pw[lane][3 * kb] = R(12) * (R)ldg(S.pwA + tt);
-          s_pw[lane][3 * kb + 1] = R(6) * (R)ldg(S.pwB + tt);
-          s_pw[lane][3 * kb + 2] = (R)ldg(S.pwEl + tt);
+          s_pw[lane][kb][0] = (R)ldg(S.pwA + tt);
+          s_pw[lane][kb][1] = (R)ldg(S.pwB + tt);
+          s_pw[lane][kb][2] = (R)ldg(S.pwEl + tt);
         }
     }
     __builtin_amdgcn_wave_barrier();
@@ -858,54 +874,34 @@ __device__ __forceinline__ void solute_receiver(const DevSys& S, uint32_t mask, 
       rQ[k] = lane_get(fc, k);
       f[k][0] = f[k][1] = f[k][2] = R(0);
     }
-    // ---- solute partners that may be excluded or 1-4 (all, if !fast)
-    for (int t = t0, n = nk == 0 ? 0 : (fast ? n_near : n_near + n_far); t < n; t += QNB_WAVE * parts) {
-      const int e = ldg(al + (t < n_near ? t : acap - 1 - (t - n_near))), j = e & AL_ATOM;
-      const R dx = (R)(ldg(x + 3 * j) - xr0), dy = (R)(ldg(x + 3 * j + 1) - xr1), dz = (R)(ldg(x + 3 * j + 2) - xr2);
-      const PPAtom Q{j, ldg(S.iac + j), ldg(S.exmask + j), ldg(S.m14mask + j), ldg(S.crg + j)};
-      const R* pf = qp_tab<R>(S.ppd, S.ppf) + PP_REC * (size_t)j;
-      const R qA = ldg(pf), qB = ldg(pf + 1), qQ = ldg(pf + 2), qA3 = ldg(pf + 4), qB3 = ldg(pf + 5);
-      R pel = R(0), pvdw = R(0);
-#pragma unroll
-      for (int k = 0; k < CH; k++) {
-        const int i = ri[k];
-        if (i < 0 || i == j) continue;
-        R A, B, el;
-        if (fast) {
-          // code 1, or 3 for a 1-4 pair: products of per-atom factors again
-          const int kind = pair_kind(S, i, s_rx[k], s_rm[k], j, Q.xm, Q.m14);
-          if (kind == 1) continue;
-          const bool is14 = kind == 2;
-          A = is14 ? s_pw[k][9] * qA3 : rA[k] * qA;
-          B = is14 ? s_pw[k][10] * qB3 : rB[k] * qB;
-          el = rQ[k] * qQ;
-          if constexpr (sizeof(R) == 8)
-            if (!(fabs(A) > R(12.0e-10) || fabs(B) > R(6.0e-10) || fabs(el) > R(1.0e-10))) continue;
-          if (is14) el = el * (R)S.el14;
-        } else {
-          const PPAtom P{i, s_rt[k], s_rx[k], s_rm[k], s_rq[k]};
-          double Ad, Bd, eld;
-          if (!pp_pair(S, P, Q, Ad, Bd, eld)) continue;
-          A = R(12) * (R)Ad;
-          B = R(6) * (R)Bd;
-          el = (R)eld;
-        }
-        const bool acc = want_e && ((e & AL_SELF) ? i < j : (e & AL_OWN) != 0);
-        const R ux = dx - ro[k][0], uy = dy - ro[k][1], uz = dz - ro[k][2];
-        const R dv = pair_dv(ux, uy, uz, A, B, el, pel, pvdw, acc);
-        f[k][0] += ux * dv;
-        f[k][1] += uy * dv;
-        f[k][2] += uz * dv;
+    // A, B and qq of sweep atom k with atom j (pp_param); false: no pair
+    auto general = [&](int k, int i, int j, const double* qf, double qc, uint32_t qx, uint32_t qm, R& A, R& B,
+                       R& el) {
+      double Ad, Bd, eld;
+      if (fast) {
+        // code 1, or 3 for a 1-4 pair
+        const int kind = pair_kind(S, i, s_rx[k], s_rm[k], j, qx, qm);
+        if (kind == 1) return false;
+        const bool is14 = kind == 2;
+        Ad = is14 ? s_r3[k][2] * qf[2] : s_r3[k][0] * qf[0];
+        Bd = is14 ? s_r3[k][3] * qf[3] : s_r3[k][1] * qf[1];
+        eld = s_rq[k] * qc;
+        if (!(fabs(Ad) > 1.0e-10 || fabs(Bd) > 1.0e-10 || fabs(eld) > 1.0e-10)) return false;
+        if (is14) eld = eld * S.el14;
+      } else {
+        const PPAtom P{i, s_rt[k], s_rx[k], s_rm[k], s_rq[k]};
+        const PPAtom Q{j, ldg(S.iac + j), qx, qm, qc};
+        if (!pp_pair(S, P, Q, Ad, Bd, eld)) return false;
       }
-      if (want_e) {
-        e_ppel += (double)pel;
-        e_ppvdw += (double)pvdw;
-      }
-    }
-    // ---- the other solute partners: A, B, qq from the factors; the next
-    // partner's position and factors load while this one is evaluated
-    if (fast && nk > 0) {
-      int t = t0, e = e0, en = e1;
+      A = (R)Ad;
+      B = (R)Bd;
+      el = (R)eld;
+      return true;
+    };
+    // ---- partner solute atoms, one list slot per lane; the next slot's
+    // position and factors load while this one is evaluated
+    if (nk > 0 && nsl > 0) {
+      int e = e0, en = e1;
       double px, py, pz;
       R pA, pB, pQ;
       auto fetch = [&](int entry) {
@@ -919,25 +915,46 @@ __device__ __forceinline__ void solute_receiver(const DevSys& S, uint32_t mask, 
         pQ = ldg(pf + 2);
       };
       fetch(e);
-      for (; t < n_far; t += QNB_WAVE * parts) {
+      for (int t = t0; t < nsl; t += ts) {
         const R dx = (R)(px - xr0), dy = (R)(py - xr1), dz = (R)(pz - xr2);
         const R qA = pA, qB = pB, qQ = pQ;
-        const bool acc = want_e && (e & AL_OWN);
+        const int ec = e;
         e = en;
         fetch(e);
-        en = far_entry(t + 2 * QNB_WAVE * parts);
+        en = entry(t + 2 * ts);
+        if (ec & AL_SKIP) continue;
+        const bool acc = want_e && (ec & AL_OWN);
         R pel = R(0), pvdw = R(0);
+        // AL_FAR: no exclusion or 1-4 pair possible, A, B, qq from the factors
+        const bool far = fast && (ec & AL_FAR);
+        const int j = ec & AL_ATOM;
+        double qf[4], qc = 0.0;
+        uint32_t qx = 0u, qm = 0u;
+        // the receiver data in LDS is read where it is used: hoisted out of the
+        // loop it would fill the registers that the other partners need
+        __asm__ volatile("" ::: "memory");
+        if (!far) {
+          const double* pf = S.ppd + PP_REC * (size_t)j;
+          qf[0] = ldg(pf), qf[1] = ldg(pf + 1), qf[2] = ldg(pf + 4), qf[3] = ldg(pf + 5);
+          qc = ldg(S.crg + j);
+          qx = ldg(S.exmask + j);
+          qm = ldg(S.m14mask + j);
+        }
 #pragma unroll
         for (int k = 0; k < CH; k++) {
           if (ri[k] < 0) continue;
-          const R A = rA[k] * qA, B = rB[k] * qB, el = rQ[k] * qQ;
-          // pp_param's `set` test (QREAL_EPS, src/sizes.f90:50); in FP32
-          // a pair of zero parameters adds exactly zero, so it is skipped
-          // only on the FP64 path
-          if constexpr (sizeof(R) == 8)
-            if (!(fabs(A) > R(12.0e-10) || fabs(B) > R(6.0e-10) || fabs(el) > R(1.0e-10))) continue;
+          R A = rA[k] * qA, B = rB[k] * qB, el = rQ[k] * qQ;
+          if (far) {
+            // pp_param's `set` test (QREAL_EPS, src/sizes.f90:50); in FP32
+            // a pair of zero parameters adds exactly zero, so it is skipped
+            // only on the FP64 path
+            if constexpr (sizeof(R) == 8)
+              if (!(fabs(A) > R(1.0e-10) || fabs(B) > R(1.0e-10) || fabs(el) > R(1.0e-10))) continue;
+          } else if (!general(k, ri[k], j, qf, qc, qx, qm, A, B, el)) {
+            continue;
+          }
           const R ux = dx - ro[k][0], uy = dy - ro[k][1], uz = dz - ro[k][2];
-          const R dv = pair_dv(ux, uy, uz, A, B, el, pel, pvdw, acc);
+          const R dv = PairMath<R>::nbe(ux, uy, uz, A, B, el, pel, pvdw, acc);
           f[k][0] += ux * dv;
           f[k][1] += uy * dv;
           f[k][2] += uz * dv;
@@ -948,43 +965,96 @@ __device__ __forceinline__ void solute_receiver(const DevSys& S, uint32_t mask, 
         }
       }
     }
-    // ---- solvent partners: a lane per molecule, its sites in turn
+    // ---- partner solvent molecules: lane l takes site kb = l % sa of molecule
+    // l / sa of the round, M = 64 / sa molecules per round
     if (pw && nk > 0) {
-      for (int p = nsr + lane + QNB_WAVE * part; p < nn; p += QNB_WAVE * parts) {
-        const int j0 = nsol + sa * (ldg(row + p) - ncs);
-        R pel = R(0), pvdw = R(0);
-        for (int kb = 0; kb < sa; kb++) {
-          const int j = j0 + kb;
+      const int M = sa == 3 ? QNB_WAVE / 3 : QNB_WAVE / sa;
+      const int kb = sa == 3 ? lane % 3 : lane % sa, m = sa == 3 ? lane / 3 : lane / sa;
+      if (m < M)
+        for (int p = nsr + m + M * part; p < nn; p += M * parts) {
+          const int j = nsol + sa * (ldg(row + p) - ncs) + kb;
           const R dx = (R)(ldg(x + 3 * j) - xr0), dy = (R)(ldg(x + 3 * j + 1) - xr1),
                   dz = (R)(ldg(x + 3 * j + 2) - xr2);
-          const bool coul = kb > 0 && coul_h;
+          R pel = R(0), pvdw = R(0);
+          __asm__ volatile("" ::: "memory");
 #pragma unroll
           for (int k = 0; k < CH; k++) {
             if (ri[k] < 0) continue;
             R A, B, el;
             if (sa == 3) {
-              A = s_pw[k][3 * kb];
-              B = s_pw[k][3 * kb + 1];
-              el = s_pw[k][3 * kb + 2];
+              A = s_pw[k][kb][0];
+              B = s_pw[k][kb][1];
+              el = s_pw[k][kb][2];
             } else {
               const size_t tt = (size_t)ri[k] + (size_t)nsol * kb;
-              A = R(12) * (R)ldg(S.pwA + tt);
-              B = R(6) * (R)ldg(S.pwB + tt);
+              A = (R)ldg(S.pwA + tt);
+              B = (R)ldg(S.pwB + tt);
               el = (R)ldg(S.pwEl + tt);
             }
             const R ux = dx - ro[k][0], uy = dy - ro[k][1], uz = dz - ro[k][2];
-            const R dv = coul ? PairMath<R>::nbe_spc(ux, uy, uz, el, pel, want_e)
-                              : pair_dv(ux, uy, uz, A, B, el, pel, pvdw, want_e);
+            const R dv = PairMath<R>::nbe(ux, uy, uz, A, B, el, pel, pvdw, want_e);
             f[k][0] += ux * dv;
             f[k][1] += uy * dv;
             f[k][2] += uz * dv;
           }
+          if (want_e) {
+            e_pwel += (double)pel;
+            e_pwvdw += (double)pvdw;
+          }
         }
-        if (want_e) {
-          e_pwel += (double)pel;
-          e_pwvdw += (double)pvdw;
+    }
+    // ---- pairs inside the group: lane (g, kq) = (lane / nk, lane % nk)
+    // takes receiver atom kq against group atoms q = g, g + G, ...
+    // (G = 64 / nk); an atom of this sweep has its data in LDS, others
+    // (groups larger than one sweep) are read from memory
+    if (pp && nk > 0) {
+      const int G = QNB_WAVE / nk, kq = lane % nk, g = lane / nk;
+      const int i = s_ia[kq];
+      R fq[3] = {R(0), R(0), R(0)};
+      if (g < G && i >= 0) {
+        const R ox = s_o[kq][0], oy = s_o[kq][1], oz = s_o[kq][2];
+        for (int q = g + G * part; q < na; q += G * parts) {
+          const int ql = q - c0;
+          const bool in_sweep = ql >= 0 && ql < nk;
+          int j;
+          R dx, dy, dz;
+          if (in_sweep) {
+            j = s_ia[ql];  // -1: a Q-atom, whose pairs belong to the Q kernels
+            dx = s_o[ql][0];
+            dy = s_o[ql][1];
+            dz = s_o[ql][2];
+          } else {
+            j = ldg(S.cgpatom + (g0 + q));
+            if (ldg(S.iqatom + j) != 0) continue;
+            dx = (R)(ldg(x + 3 * j) - xr0);
+            dy = (R)(ldg(x + 3 * j + 1) - xr1);
+            dz = (R)(ldg(x + 3 * j + 2) - xr2);
+          }
+          if (j < 0 || j == i) continue;
+          R A, B, el;
+          bool ok;
+          if (in_sweep) {
+            ok = general(kq, i, j, s_r3[ql], s_rq[ql], s_rx[ql], s_rm[ql], A, B, el);
+          } else {
+            const double* pf = S.ppd + PP_REC * (size_t)j;
+            const double qf[4] = {ldg(pf), ldg(pf + 1), ldg(pf + 4), ldg(pf + 5)};
+            ok = general(kq, i, j, qf, ldg(S.crg + j), ldg(S.exmask + j), ldg(S.m14mask + j), A, B, el);
+          }
+          if (!ok) continue;
+          const R ux = dx - ox, uy = dy - oy, uz = dz - oz;
+          const R dv = PairMath<R>::nbe(ux, uy, uz, A, B, el, e_ppel, e_ppvdw, want_e && i < j);
+          fq[0] += ux * dv;
+          fq[1] += uy * dv;
+          fq[2] += uz * dv;
         }
       }
+#pragma unroll
+      for (int k = 0; k < CH; k++)
+        if (k == kq) {
+          f[k][0] += fq[0];
+          f[k][1] += fq[1];
+          f[k][2] += fq[2];
+        }
     }
     // ---- Q-atom - solute atom, receiver side: lane (g, kq) = (lane / nk,
     // lane % nk) takes receiver atom kq against Q-atoms g, g + G, ... (G = 64
@@ -1002,7 +1072,7 @@ __device__ __forceinline__ void solute_receiver(const DevSys& S, uint32_t mask, 
           const R ux = (R)(ldg(x + 3 * q) - xr0) - ox, uy = (R)(ldg(x + 3 * q + 1) - xr1) - oy,
                   uz = (R)(ldg(x + 3 * q + 2) - xr2) - oz;
           R r2, r;
-          rinv(ux * ux + uy * uy + uz * uz, r2, r);
+          rinv(norm2(ux, uy, uz), r2, r);
           const R dvs = qx_states<R, NS>(S, r2, r, ns, eq, want_e, [&](int s) {
             const size_t t = (size_t)i + (size_t)nsol * ((size_t)iq + (size_t)nq * s);
             return QPar<R>{ldg(qtA + t), ldg(qtB + t), ldg(qtE + t), ldg(qtS + t)};
@@ -1109,10 +1179,10 @@ __device__ __forceinline__ void water_receiver(const DevSys& S, uint32_t mask, i
     // solute partners from the receiver's atom list, one per lane, the next
     // one's data in flight
     if (mask & T_PW) {
-      const int* __restrict__ al = S.alist + (size_t)a * S.acap + S.acap - 1;
-      const int n = uni(ldg(S.alist_n + 2 * a + 1));
-      int j = lane < n ? ldg(al - lane) & AL_ATOM : 0;
-      int jn = lane + QNB_WAVE < n ? ldg(al - lane - QNB_WAVE) & AL_ATOM : 0;
+      const int* __restrict__ al = S.alist + (size_t)a * S.acap;
+      const int n = uni(ldg(S.alist_n + a));
+      int e = lane < n ? ldg(al + lane) : 0;
+      int en = lane + QNB_WAVE < n ? ldg(al + lane + QNB_WAVE) : 0;
       double px = 0.0, py = 0.0, pz = 0.0;
       R pl[9];
       auto fetch = [&](int i) {
@@ -1133,15 +1203,17 @@ __device__ __forceinline__ void water_receiver(const DevSys& S, uint32_t mask, i
           }
         }
       };
-      if (n > 0) fetch(j);
+      if (n > 0) fetch(e & AL_ATOM);
       for (int t = lane; t < n; t += QNB_WAVE) {
         const R dx = (R)(px - xr0), dy = (R)(py - xr1), dz = (R)(pz - xr2);
         R pw[9];
 #pragma unroll
         for (int k = 0; k < 9; k++) pw[k] = pl[k];
-        j = jn;
-        fetch(j);
-        jn = t + 2 * QNB_WAVE < n ? ldg(al - t - 2 * QNB_WAVE) & AL_ATOM : 0;
+        const int ec = e;
+        e = en;
+        fetch(e & AL_ATOM);
+        en = t + 2 * QNB_WAVE < n ? ldg(al + t + 2 * QNB_WAVE) : 0;
+        if (ec & AL_SKIP) continue;
 #pragma unroll
         for (int k = 0; k < 3; k++) {
           const R ux = dx - o[k][0], uy = dy - o[k][1], uz = dz - o[k][2];
@@ -1211,7 +1283,7 @@ __device__ __forceinline__ void water_receiver(const DevSys& S, uint32_t mask, i
       for (int k = 0; k < 3; k++) {
         const R ux = qx - o[k][0], uy = qy - o[k][1], uz = qz - o[k][2];
         R r2, r;
-        rinv(ux * ux + uy * uy + uz * uz, r2, r);
+        rinv(norm2(ux, uy, uz), r2, r);
         const R dvs = k == 0 || !S.spc
                           ? qx_states<R, NS>(S, r2, r, ns, eq, want_e, [&](int s) { return qw_par<R>(S, iq, k, s); })
                           : qspc_states<R, NS>(S, r2, r, ns, eq, want_e, [&](int s) { return qw_el<R>(S, iq, k, s); });
@@ -1341,7 +1413,7 @@ __device__ __forceinline__ void solvent_receiver(const DevSys& S, uint32_t mask,
         const int q = ldg(S.iqseq + iq);
         const R ux = (R)(ldg(x + 3 * q) - xi0), uy = (R)(ldg(x + 3 * q + 1) - xi1), uz = (R)(ldg(x + 3 * q + 2) - xi2);
         R r2, r;
-        rinv(ux * ux + uy * uy + uz * uz, r2, r);
+        rinv(norm2(ux, uy, uz), r2, r);
         const R dvs = k == 0 || !S.spc
                           ? qx_states<R, NS>(S, r2, r, ns, eq, want_e, [&](int s) { return qw_par<R>(S, iq, k, s); })
                           : qspc_states<R, NS>(S, r2, r, ns, eq, want_e, [&](int s) { return qw_el<R>(S, iq, k, s); });
@@ -1481,7 +1553,7 @@ __device__ __forceinline__ void qatom_side(const DevSys& S, uint32_t mask, int i
         const double ux = ldg(x + 3 * j) - xi0, uy = ldg(x + 3 * j + 1) - xi1, uz = ldg(x + 3 * j + 2) - xi2;
         const R rux = (R)ux, ruy = (R)uy, ruz = (R)uz;
         R r2, r;
-        rinv(rux * rux + ruy * ruy + ruz * ruz, r2, r);
+        rinv(norm2(rux, ruy, ruz), r2, r);
         const R dvs = k == 0 || !S.spc
                           ? qx_states<R, NS>(S, r2, r, ns, dummy, false, [&](int s) { return qw_par<R>(S, iq, k, s); })
                           : qspc_states<R, NS>(S, r2, r, ns, dummy, false, [&](int s) { return qw_el<R>(S, iq, k, s); });
@@ -1496,14 +1568,28 @@ __device__ __forceinline__ void qatom_side(const DevSys& S, uint32_t mask, int i
       const double ux = ldg(x + 3 * j) - xi0, uy = ldg(x + 3 * j + 1) - xi1, uz = ldg(x + 3 * j + 2) - xi2;
       const R rux = (R)ux, ruy = (R)uy, ruz = (R)uz;
       R r2, r;
-      rinv(rux * rux + ruy * ruy + ruz * ruz, r2, r);
-      const R dvs = qx_states<R, NS>(S, r2, r, ns, dummy, false, [&](int s) {
+      rinv(norm2(rux, ruy, ruz), r2, r);
+      auto par = [&](int s) {
         const size_t t = (size_t)j + (size_t)S.nat_solute * ((size_t)iq + (size_t)nq * s);
         return QPar<R>{ldg(qtA + t), ldg(qtB + t), ldg(qtE + t), ldg(qtS + t)};
-      });
-      f[0] -= rux * dvs;
-      f[1] -= ruy * dvs;
-      f[2] -= ruz * dvs;
+      };
+      if constexpr (sizeof(R) == 8) {
+        const R dvs = qx_states<R, NS>(S, r2, r, ns, dummy, false, par);
+        f[0] -= rux * dvs;
+        f[1] -= ruy * dvs;
+        f[2] -= ruz * dvs;
+      } else {
+        const R r6 = r2 * r2 * r2;
+#pragma unroll
+        for (int s = 0; s < NS; s++) {
+          if (s >= ns) break;
+          const QPar<R> p = par(s);
+          const R dv = PairMath<R>::nbe_qx(r2, r, r6, p.A, p.B, p.q, p.sc, (R)S.lambda[s], dummy[0], dummy[1], false);
+          f[0] -= rux * dv;
+          f[1] -= ruy * dv;
+          f[2] -= ruz * dv;
+        }
+      }
     }
   }
   const double fs = wave_sum_tr(f, lane);
@@ -1569,7 +1655,7 @@ __device__ __forceinline__ void qq_pairs(const DevSys& S, uint32_t mask, int wav
       const double ux = x[3 * j] - x[3 * i], uy = x[3 * j + 1] - x[3 * i + 1], uz = x[3 * j + 2] - x[3 * i + 2];
       const R rux = (R)ux, ruy = (R)uy, ruz = (R)uz;
       R r2, r;
-      rinv(rux * rux + ruy * ruy + ruz * ruz, r2, r);
+      rinv(norm2(rux, ruy, ruz), r2, r);
       const R pA = (R)ldg(pr), pB = (R)ldg(pr + 1), pel = (R)ldg(pr + 2), psc = (R)ldg(pr + 3);
       const R lam = (R)S.lambda[s];
       R dv;
