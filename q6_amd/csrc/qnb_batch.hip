@@ -37,12 +37,6 @@ struct MdDev {
   double dt, dt_over_tau, T0, Boltz;
   int nbcycle, ene_every, max_frames;
   int nbonds, nangles;
-  const int* bond_ij;
-  const double* bond_r0;
-  const double* bond_k;
-  const int* angle_ijk;
-  const double* angle_t0;
-  const double* angle_k;
   const double* winv;
   double roh2, rhh2;
   // temperature groups (temperature, src/md.f90:1379-1447): with separate
@@ -63,14 +57,6 @@ struct MdDev {
   int xs_every, xs_max;
   double* bpart;  // [nbpart][2] bond and angle energy per k_bonded block
   int nbpart;
-  // atom-centred bonded terms: for atom i, items boff[i]..boff[i+1]-1 of
-  // bitem (2 * bond + role) and aoff[i]..aoff[i+1]-1 of aitem (3 * angle +
-  // role); atoms [0, nbat) carry all of them
-  const int* boff;
-  const int* bitem;
-  const int* aoff;
-  const int* aitem;
-  int nbat;
   // fused integrator: per-block kinetic energy sums
   double* tpart;  // [ceil((nwat + nat_solute) / 256)][4]: Ekin, free Ekin of groups 0 and 1
   // EVB off-diagonal elements sampled with the energies
@@ -94,61 +80,6 @@ __device__ __forceinline__ double block_sum(double v, double* red) {
   return s;
 }
 
-// harmonic bonds and angles of the solute (bond, angle: src/bondene.f90:41-246)
-// One thread per atom sums the terms of every bond and angle it belongs to
-// (each term is evaluated once per member atom), so the gradient needs no
-// atomics and does not depend on scheduling.  A bond's energy is counted by
-// its first atom, an angle's by its vertex; each block's energy sums go to
-// bpart[block] and k_record adds them in block order.  bonded_atom is the
-// per-atom part, used by k_bonded (the minimiser) and k_atom_step (MD).
-__device__ __forceinline__ void bonded_atom(const DevSys& S, const MdDev& M, int i, double* f, double& eb,
-                                            double& ea) {
-  const auto x = gp(S.x);
-  for (int it = ldg(M.boff + i), e = ldg(M.boff + i + 1); it < e; it++) {
-    const int item = ldg(M.bitem + it), b = item >> 1, role = item & 1;
-    const int bi = ldg(M.bond_ij + 2 * b), bj = ldg(M.bond_ij + 2 * b + 1);
-    const double ax = x[3 * bj] - x[3 * bi], ay = x[3 * bj + 1] - x[3 * bi + 1], az = x[3 * bj + 2] - x[3 * bi + 2];
-    const double r = sqrt(ax * ax + ay * ay + az * az);
-    const double kb = ldg(M.bond_k + b), db = r - ldg(M.bond_r0 + b);
-    const double dv = kb * db / r;
-    const double sg = role == 0 ? -dv : dv;
-    f[0] += ax * sg;
-    f[1] += ay * sg;
-    f[2] += az * sg;
-    if (role == 0) eb += 0.5 * kb * db * db;
-  }
-  for (int it = ldg(M.aoff + i), e = ldg(M.aoff + i + 1); it < e; it++) {
-    const int item = ldg(M.aitem + it), a = item / 3, role = item - 3 * a;
-    const int ai = ldg(M.angle_ijk + 3 * a), aj = ldg(M.angle_ijk + 3 * a + 1), ak = ldg(M.angle_ijk + 3 * a + 2);
-    double u[3], w[3];
-    for (int c = 0; c < 3; c++) {
-      u[c] = x[3 * ai + c] - x[3 * aj + c];
-      w[c] = x[3 * ak + c] - x[3 * aj + c];
-    }
-    const double ru = sqrt(u[0] * u[0] + u[1] * u[1] + u[2] * u[2]);
-    const double rw = sqrt(w[0] * w[0] + w[1] * w[1] + w[2] * w[2]);
-    double ct = (u[0] * w[0] + u[1] * w[1] + u[2] * w[2]) / (ru * rw);
-    ct = fmin(1.0, fmax(-1.0, ct));
-    const double th = acos(ct);
-    // sin(theta) from the cross product, consistent with the numerator of
-    // the derivative below even for nearly linear angles, where
-    // sin(acos(ct)) loses all digits; at a linear angle the derivative has
-    // no direction
-    const double cx = u[1] * w[2] - u[2] * w[1], cy = u[2] * w[0] - u[0] * w[2], cz = u[0] * w[1] - u[1] * w[0];
-    const double st = sqrt(cx * cx + cy * cy + cz * cz) / (ru * rw);
-    const double ka = ldg(M.angle_k + a), da = th - ldg(M.angle_t0 + a);
-    if (role == 1) ea += 0.5 * ka * da * da;
-    if (!(st > 1.0e-8)) continue;
-    const double dv = ka * da;
-    // dtheta/dx_i = -(w/(ru rw) - ct u/ru^2)/sin(theta), likewise for k; j balances
-    for (int c = 0; c < 3; c++) {
-      const double gi = -(w[c] / (ru * rw) - ct * u[c] / (ru * ru)) / st;
-      const double gk = -(u[c] / (ru * rw) - ct * w[c] / (rw * rw)) / st;
-      f[c] += dv * (role == 0 ? gi : (role == 2 ? gk : -(gi + gk)));
-    }
-  }
-}
-
 // solute bonds and angles alone (the minimiser's step)
 __global__ __launch_bounds__(256) void k_bonded(const DevSys* __restrict__ systems, const MdDev* __restrict__ mds) {
   const DevSys& S = systems[blockIdx.y];
@@ -156,9 +87,9 @@ __global__ __launch_bounds__(256) void k_bonded(const DevSys* __restrict__ syste
   __shared__ double red[4];
   double eb = 0.0, ea = 0.0;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < M.nbat) {
+  if (i < S.nbat) {
     double f[3] = {0.0, 0.0, 0.0};
-    bonded_atom(S, M, i, f, eb, ea);
+    bonded_atom(S, i, f, eb, ea);
     const auto d = gpm(S.d);
     d[3 * i] += f[0];
     d[3 * i + 1] += f[1];
@@ -185,14 +116,14 @@ __global__ __launch_bounds__(256) void k_atom_step(const DevSys* __restrict__ sy
   if (i < S.natom) {
     double f[3] = {0.0, 0.0, 0.0};
     double el = 0.0, er = 0.0;
-    if (S.use_lrf && !ldg(S.excl + i) && ldg(S.iqatom + i) == 0) lrf_taylor_atom(S, i, f, el);
+    if (S.use_lrf && !ldg(S.excl + i) && ldg(S.iqatom + i) == 0) lrf_taylor_atom(S, i, ldg(S.atom_group + i), f, el);
     const int src = radial_source(S, i);
     if (src >= 0) {
       const double T = tfree[blockIdx.y];
       const double shift = S.fk_wsphere != 0.0 ? sqrt(S.Boltz * T / S.fk_wsphere) : 0.0;
       radial_restraint(S, src, shift, f, er);
     }
-    if (i < M.nbat) bonded_atom(S, M, i, f, eb, ea);
+    if (i < S.nbat) bonded_atom(S, i, f, eb, ea);
     add_qrows(S, i, rows, f);
     store_atom_gradient(S, i, f);
     if (want_energies(S)) {
@@ -208,13 +139,69 @@ __global__ __launch_bounds__(256) void k_atom_step(const DevSys* __restrict__ sy
   }
 }
 
-// One MD step's integration of every atom, fused: leap-frog with the
-// Berendsen factor of the previous step (newvel_ber, src/md.f90:1451-1466),
-// SHAKE of each rigid water (src/bondene.f90:1069-1151), v = (x - x_old)/dt
-// for every atom (src/md.f90:1787-1793) and per-block sums of the kinetic
-// energy (k_thermo adds them).  Thread t < nwat takes water t (3 atoms), the
-// next nat_solute threads one solute atom each.
-__global__ __launch_bounds__(256) void k_integrate(const DevSys* __restrict__ systems, const MdDev* __restrict__ mds) {
+// Temperatures and Berendsen factors from the kinetic energies of the
+// temperature groups (temperature, src/md.f90:1412-1443): Temp and Tfree over
+// all atoms, each group's free temperature, and sfact = sqrt(1 + dt/tau
+// (T0/tfree - 1)); a group with tfree = 0 keeps its previous sfact inside the
+// square root, as the reference's update does.
+__device__ void thermo_update(const MdDev& M, const double* ek, const double* ekf) {
+  const double eks = M.ngroup == 2 ? ek[0] + ek[1] : ek[0];
+  const double ekfs = M.ngroup == 2 ? ekf[0] + ekf[1] : ekf[0];
+  const double T = 2.0 * eks / M.Boltz / M.ndegf;
+  const double Tf = 2.0 * ekfs / M.Boltz / M.ndegfree;
+  M.st[1] = Tf;
+  M.st[2] = T;
+  M.st[3] = eks;
+  *M.tfree = Tf;
+  for (int g = 0; g < M.ngroup; g++) {
+    const double tf = 2.0 * ekf[g] / M.Boltz / M.gndegfree[g];
+    double sf = M.st[g == 0 ? 0 : 6];
+    if (tf != 0.0) sf = M.T0 / tf - 1.0;
+    M.st[g == 0 ? 0 : 6] = sqrt(1.0 + M.dt_over_tau * sf);
+    M.st[4 + g] = tf;
+  }
+}
+
+// Closes an MD step, four waves of the last block of k_integrate.  Wave 0: the
+// kinetic energy from the block sums (lane l takes blocks l, l + 64, ..., then
+// a fixed tree), the temperature, Tfree and the Berendsen factor of the next
+// step (temperature, src/md.f90:1379-1447), the step counter and the errors;
+// the others close the polarisation restraint's step (watpol_finish).  A
+// launch of its own took 7 us for this.
+__device__ __forceinline__ void thermo(const DevSys& S, const MdDev& M, int nblk, int wid, int lane) {
+  if (wid != 0) {
+    watpol_finish(S, wid - 1, 3);
+    return;
+  }
+  double s[4] = {0.0, 0.0, 0.0, 0.0};
+  for (int k = lane; k < nblk; k += QNB_WAVE)
+    for (int c = 0; c < 4; c++)
+      s[c] += __longlong_as_double((long long)__hip_atomic_load(
+          reinterpret_cast<unsigned long long*>(M.tpart) + 4 * k + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+  for (int c = 0; c < 4; c++) s[c] = wave_sum(s[c]);
+  if (lane != 0) return;
+  const double ek[2] = {s[0], s[2]}, ekf[2] = {s[1], s[3]};
+  thermo_update(M, ek, ekf);
+  const double T = M.st[2];
+  if (!isfinite(T) || !isfinite(S.ered[E_PP_EL] + S.ered[E_WW_EL])) atomicOr(&M.ctr[1], ERR_NONFINITE);
+  if (*S.need > S.cap) atomicOr(&M.ctr[1], ERR_OVERFLOW);
+  M.ctr[3] = 0;
+  *M.istep = *M.istep + 1;
+}
+
+// One MD step's integration of every atom: leap-frog with the Berendsen factor
+// of the previous step (newvel_ber, src/md.f90:1451-1466), SHAKE of each rigid
+// water (src/bondene.f90:1069-1151), v = (x - x_old)/dt for every atom
+// (src/md.f90:1787-1793) and per-block sums of the kinetic energy; the block
+// that ends last adds them (thermo).  Thread t < nwat takes water t (3 atoms),
+// the next nat_solute threads one solute atom each.  FUSED: the per-atom terms
+// of the step (LRF Taylor term, radial restraint, the rows of the bonded terms
+// and of the Q kernels: what k_atom_step adds) are formed here and not written,
+// on steps that neither record energies nor run the Q bonded terms in between:
+// a launch and a pass over the gradients less.
+template <bool FUSED>
+__global__ __launch_bounds__(256) void k_integrate(const DevSys* __restrict__ systems, const MdDev* __restrict__ mds,
+                                                   int rows) {
   const DevSys& S = systems[blockIdx.y];
   const MdDev& M = mds[blockIdx.y];
   const int nthr = S.nwat + S.nat_solute;
@@ -229,14 +216,27 @@ __global__ __launch_bounds__(256) void k_integrate(const DevSys* __restrict__ sy
   double ek = 0.0, ekf = 0.0;
   const bool solvent = t < S.nwat;
   const double s = (solvent && M.ngroup == 2) ? M.st[6] : M.st[0];
+  double el = 0.0, er = 0.0;  // energies: not kept on these steps
   if (t < S.nwat) {
     const int o = S.nat_solute + 3 * t;
     double xo[3][3], xn[3][3], wi[3];
     for (int k = 0; k < 3; k++) {
       wi[k] = ldg(M.winv + o + k);
+      double f[3] = {0.0, 0.0, 0.0};
+      if constexpr (FUSED) {
+        if (S.use_lrf && !ldg(S.excl + o + k)) lrf_taylor_atom(S, o + k, S.ncgp_solute + t, f, el);
+        if (k == 0 && !ldg(S.excl + o)) {
+          const double shift = S.fk_wsphere != 0.0 ? sqrt(S.Boltz * *M.tfree / S.fk_wsphere) : 0.0;
+          radial_restraint(S, o, shift, f, er);
+        }
+        if (o + k < S.nbat)
+          for (int c = 0; c < 3; c++) f[c] += ldg(S.brow + 3 * (o + k) + c);
+      }
       for (int c = 0; c < 3; c++) {
         const int q = 3 * (o + k) + c;
-        const double v = (vg[q] - dg[q] * wi[k] * dt) * s;
+        double g = dg[q];
+        if constexpr (FUSED) g += f[c];
+        const double v = (vg[q] - g * wi[k] * dt) * s;
         xo[k][c] = xg[q];
         xn[k][c] = xo[k][c] + v * dt;
       }
@@ -281,10 +281,24 @@ __global__ __launch_bounds__(256) void k_integrate(const DevSys* __restrict__ sy
   } else if (t < nthr) {
     const int i = t - S.nwat;
     const double wi = ldg(M.winv + i);
+    double f[3] = {0.0, 0.0, 0.0};
+    const bool excl = ldg(S.excl + i);
+    // an excluded atom in no charge group has no pair gradient (store_atom_gradient)
+    bool grouped = true;
+    if constexpr (FUSED) {
+      const int g = ldg(S.atom_group + i);
+      grouped = g >= 0;
+      if (S.use_lrf && !excl && ldg(S.iqatom + i) == 0) lrf_taylor_atom(S, i, g, f, el);
+      if (i < S.nbat)
+        for (int c = 0; c < 3; c++) f[c] += ldg(S.brow + 3 * i + c);
+      add_qrows(S, i, rows, f);
+    }
     double v2 = 0.0;
     for (int c = 0; c < 3; c++) {
       const int q = 3 * i + c;
-      const double v0 = (vg[q] - dg[q] * wi * dt) * s;
+      double g = dg[q];
+      if constexpr (FUSED) g = grouped ? g + f[c] : f[c];
+      const double v0 = (vg[q] - g * wi * dt) * s;
       const double xo = xg[q], xn = xo + v0 * dt;
       const double v = (xn - xo) / dt;
       xg[q] = xn;
@@ -293,67 +307,36 @@ __global__ __launch_bounds__(256) void k_integrate(const DevSys* __restrict__ sy
     }
     const double e = 0.5 * (1.0 / wi) * v2;
     ek += e;
-    if (!ldg(S.excl + i)) ekf += e;
+    if (!excl) ekf += e;
   }
-  __shared__ double red[4];
+  // the four sums of the block, in wave order
   const bool g1 = solvent && M.ngroup == 2;
-  const double ek0 = block_sum(g1 ? 0.0 : ek, red);
-  const double ekf0 = block_sum(g1 ? 0.0 : ekf, red);
-  const double ek1 = block_sum(g1 ? ek : 0.0, red);
-  const double ekf1 = block_sum(g1 ? ekf : 0.0, red);
-  if (threadIdx.x == 0) {
-    M.tpart[4 * blockIdx.x] = ek0;
-    M.tpart[4 * blockIdx.x + 1] = ekf0;
-    M.tpart[4 * blockIdx.x + 2] = ek1;
-    M.tpart[4 * blockIdx.x + 3] = ekf1;
+  const int lane = threadIdx.x % QNB_WAVE, wid = threadIdx.x / QNB_WAVE;
+  __shared__ double red[4][4];
+  __shared__ bool last;
+  const double sums[4] = {wave_sum_all(g1 ? 0.0 : ek), wave_sum_all(g1 ? 0.0 : ekf), wave_sum_all(g1 ? ek : 0.0),
+                          wave_sum_all(g1 ? ekf : 0.0)};
+  if (lane == 0)
+    for (int c = 0; c < 4; c++) red[wid][c] = sums[c];
+  __syncthreads();
+  if (wid == 0) {
+    // The sums are exchanged into memory at device scope, and their old values
+    // waited for, before the block counts itself: the block that counts last
+    // finds every block's sums there.  A release fence would do as much, but
+    // writes the whole L2 back.
+    if (lane < 4) {
+      const double s4 = ((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane];
+      const unsigned long long old =
+          __hip_atomic_exchange(reinterpret_cast<unsigned long long*>(M.tpart) + 4 * blockIdx.x + lane,
+                                (unsigned long long)__double_as_longlong(s4), __ATOMIC_RELAXED,
+                                __HIP_MEMORY_SCOPE_AGENT);
+      __asm__ volatile("" ::"v"(old) : "memory");
+    }
+    if (lane == 0)
+      last = __hip_atomic_fetch_add(&M.ctr[3], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nblk - 1;
   }
-}
-
-// Temperatures and Berendsen factors from the kinetic energies of the
-// temperature groups (temperature, src/md.f90:1412-1443): Temp and Tfree over
-// all atoms, each group's free temperature, and sfact = sqrt(1 + dt/tau
-// (T0/tfree - 1)); a group with tfree = 0 keeps its previous sfact inside the
-// square root, as the reference's update does.
-__device__ void thermo_update(const MdDev& M, const double* ek, const double* ekf) {
-  const double eks = M.ngroup == 2 ? ek[0] + ek[1] : ek[0];
-  const double ekfs = M.ngroup == 2 ? ekf[0] + ekf[1] : ekf[0];
-  const double T = 2.0 * eks / M.Boltz / M.ndegf;
-  const double Tf = 2.0 * ekfs / M.Boltz / M.ndegfree;
-  M.st[1] = Tf;
-  M.st[2] = T;
-  M.st[3] = eks;
-  *M.tfree = Tf;
-  for (int g = 0; g < M.ngroup; g++) {
-    const double tf = 2.0 * ekf[g] / M.Boltz / M.gndegfree[g];
-    double sf = M.st[g == 0 ? 0 : 6];
-    if (tf != 0.0) sf = M.T0 / tf - 1.0;
-    M.st[g == 0 ? 0 : 6] = sqrt(1.0 + M.dt_over_tau * sf);
-    M.st[4 + g] = tf;
-  }
-}
-
-// After k_integrate, one wave per system: the kinetic energy from the block
-// sums (lane l takes blocks l, l + 64, ..., then a fixed tree), the
-// temperature, Tfree and the Berendsen factor of the next step (temperature,
-// src/md.f90:1379-1447); closes the polarisation restraint's step
-// (watpol_finish), advances the step counter and records errors.  Latency
-// only: one lane walking the block sums took 2.5 to 6.5 us at 9 to 27 blocks.
-__global__ __launch_bounds__(64) void k_thermo(const DevSys* __restrict__ systems, const MdDev* __restrict__ mds) {
-  const DevSys& S = systems[blockIdx.x];
-  const MdDev& M = mds[blockIdx.x];
-  const int lane = threadIdx.x, nblk = (S.nwat + S.nat_solute + 255) / 256;
-  double s[4] = {0.0, 0.0, 0.0, 0.0};
-  for (int k = lane; k < nblk; k += QNB_WAVE)
-    for (int c = 0; c < 4; c++) s[c] += ldg(M.tpart + 4 * k + c);
-  for (int c = 0; c < 4; c++) s[c] = wave_sum(s[c]);
-  watpol_finish(S);
-  if (lane != 0) return;
-  const double ek[2] = {s[0], s[2]}, ekf[2] = {s[1], s[3]};
-  thermo_update(M, ek, ekf);
-  const double T = M.st[2];
-  if (!isfinite(T) || !isfinite(S.ered[E_PP_EL] + S.ered[E_WW_EL])) atomicOr(&M.ctr[1], ERR_NONFINITE);
-  if (*S.need > S.cap) atomicOr(&M.ctr[1], ERR_OVERFLOW);
-  *M.istep = *M.istep + 1;
+  __syncthreads();
+  if (last) thermo(S, M, nblk, wid, lane);
 }
 
 // shake (src/bondene.f90:1069-1151) on each rigid water (O-H1, O-H2, H1-H2),
@@ -672,16 +655,16 @@ static void launch_qforces(qnb_batch* b) {
 // atoms) and disjoint energy slots; the batch stream waits for the side
 // branch before the per-atom terms, which add dq to the Q-atoms' gradients.
 template <typename R, int NS>
-static void enqueue_forces_forked(qnb_batch* b, bool energy) {
+static void enqueue_forces_forked(qnb_batch* b, bool energy, bool bonded) {
   const int wpb = 4, B = b->n;
   (void)hipEventRecord(b->ev_fork, b->stream);
   (void)hipStreamWaitEvent(b->side, b->ev_fork, 0);
+  if (bonded) launch_watpol(b->side, 0, B, b->dsys, (const int*)b->istep, false, false, b->nbblk);
   if (b->anyq)
     hipLaunchKernelGGL((k_qforces<R, NS>), dim3(qforces_blocks(b->nq_max, b->qchunks, wpb), B), dim3(64 * wpb), 0,
                        b->side, b->dsys, kStepMask, b->qchunks, (int)QROWS_SIDE);
   if (b->maxw > 0) launch_forces_t<R, NS>(b, b->wpb_forces, energy, false, 1, b->side);
-  if (b->anypol)
-    launch_watpol(b->side, b->maxw, B, b->dsys, (const int*)b->istep, true, false);
+  if (b->anypol) launch_watpol(b->side, b->maxw, B, b->dsys, (const int*)b->istep, true, false, 0);
   launch_forces_t<R, NS>(b, b->wpb_forces, energy, false, 2);
   if (b->anyq) hipLaunchKernelGGL((k_qq<R, NS>), dim3(B), dim3(QQ_THREADS), 0, b->stream, b->dsys, kStepMask);
   (void)hipEventRecord(b->ev_join, b->side);
@@ -692,10 +675,10 @@ static void enqueue_forces_forked(qnb_batch* b, bool energy) {
 // in one launch, then the polarisation forces
 static bool small_step(const qnb_batch* b) { return small_launch(b->sum_solute, b->sum_solvent); }
 
-static void enqueue_forces_small(qnb_batch* b, bool energy) {
+static void enqueue_forces_small(qnb_batch* b, bool energy, bool bonded) {
   const SmallGrid G = small_grid(b->maxs, b->maxw, 3, b->nq_max, b->nsol_max, b->nqe_max, kStepMask, b->anypol);
   launch_forces_small(b->stream, b->prec, b->ns_max, energy, G, b->n, b->dsys, kStepMask, b->istep);
-  if (b->anypol) launch_watpol(b->stream, b->maxw, b->n, b->dsys, b->istep, false, false);
+  launch_watpol(b->stream, b->anypol ? b->maxw : 0, b->n, b->dsys, b->istep, false, false, bonded ? b->nbblk : 0);
 }
 
 template <typename R, int NS>
@@ -708,14 +691,15 @@ static void enqueue_forces(qnb_batch* b, bool energy = true, bool atom_terms = t
                        b->stream, b->dsys, mask, b->qchunks, 0);
     hipLaunchKernelGGL((k_qq<R, NS>), dim3(B), dim3(QQ_THREADS), 0, b->stream, b->dsys, mask);
   }
-  if (b->anypol) launch_watpol(b->stream, b->maxw, B, b->dsys, (const int*)b->istep, true, true);
+  if (b->anypol) launch_watpol(b->stream, b->maxw, B, b->dsys, (const int*)b->istep, true, true, 0);
 }
 
-// leap-frog + SHAKE + new velocities, then the temperatures and Berendsen
-// factors of the next step
-static void launch_integrate(qnb_batch* b) {
-  hipLaunchKernelGGL(k_integrate, dim3((b->maxsw + 255) / 256, b->n), dim3(256), 0, b->stream, b->dsys, b->dmd);
-  hipLaunchKernelGGL(k_thermo, dim3(b->n), dim3(64), 0, b->stream, b->dsys, b->dmd);
+// leap-frog + SHAKE + new velocities, the temperatures and Berendsen factors
+// of the next step; fused: with the per-atom terms
+static void launch_integrate(qnb_batch* b, bool fused, int rows) {
+  const dim3 grid((b->maxsw + 255) / 256, b->n);
+  if (fused) hipLaunchKernelGGL((k_integrate<true>), grid, dim3(256), 0, b->stream, b->dsys, b->dmd, rows);
+  else hipLaunchKernelGGL((k_integrate<false>), grid, dim3(256), 0, b->stream, b->dsys, b->dmd, rows);
 }
 
 template <typename R>
@@ -725,18 +709,21 @@ static void enqueue_step(qnb_batch* b, bool lists, bool energy) {
     launch_lists(b, b->wpb_lists);
     if (b->anyq && !b->static_q) hipLaunchKernelGGL(k_qlists, dim3(B), dim3(1024), 0, b->stream, b->dsys);
   }
-  const bool small = small_step(b);
-  if (small) enqueue_forces_small(b, energy);
+  // the per-atom terms: in the integrator where nothing reads the whole
+  // gradient or the terms' energies before it, else in k_atom_step
+  const bool small = small_step(b), fused = !energy && !b->anyqb;
+  const int rows = !b->anyq ? 0 : (int)(small ? QROWS_SIDE | QROWS_QQ : QROWS_SIDE);
+  if (small) enqueue_forces_small(b, energy, fused);
   else switch (b->ns_max) {
-    case 1: enqueue_forces_forked<R, 1>(b, energy); break;
-    case 2: enqueue_forces_forked<R, 2>(b, energy); break;
+    case 1: enqueue_forces_forked<R, 1>(b, energy, fused); break;
+    case 2: enqueue_forces_forked<R, 2>(b, energy, fused); break;
     case 3:
-    case 4: enqueue_forces_forked<R, 4>(b, energy); break;
-    default: enqueue_forces_forked<R, 8>(b, energy); break;
+    case 4: enqueue_forces_forked<R, 4>(b, energy, fused); break;
+    default: enqueue_forces_forked<R, 8>(b, energy, fused); break;
   }
-  hipLaunchKernelGGL(k_atom_step, dim3((b->maxat + 255) / 256, B), dim3(256), 0, b->stream, b->dsys, b->dmd,
-                     (const double*)b->tfree,
-                     !b->anyq ? 0 : (int)(small ? QROWS_SIDE | QROWS_QQ : QROWS_SIDE));
+  if (!fused)
+    hipLaunchKernelGGL(k_atom_step, dim3((b->maxat + 255) / 256, B), dim3(256), 0, b->stream, b->dsys, b->dmd,
+                       (const double*)b->tfree, rows);
   if (b->anyqb) launch_qbonded(b->stream, B, b->dsys, b->dqb);
   // the reduction and the record do nothing on a step no instance samples
   // (energy is false only then); the record also counts stored snapshots
@@ -749,7 +736,7 @@ static void enqueue_step(qnb_batch* b, bool lists, bool energy) {
   if (energy && b->exc_threads > 0)
     hipLaunchKernelGGL(k_exc_record, dim3((b->exc_threads + 63) / 64, B), dim3(64), 0, b->stream, b->dsys, b->dmd,
                        (const ExcDev*)b->dexc);
-  launch_integrate(b);
+  launch_integrate(b, fused, rows);
 }
 
 template <typename R>
@@ -856,7 +843,7 @@ extern "C" int32_t qnb_batch_create(int32_t n, const qnb_system* const* sys, con
     const qnb_md_params* m = md[k];
     MdDev& M = b->hm[k];
     memset(&M, 0, sizeof M);
-    const DevSys& S = b->hs[k];
+    DevSys& S = b->hs[k];
     M.dt = 0.020462 * m->dt_fs;
     M.dt_over_tau = M.dt / (0.020462 * m->tau_T_fs);  // dt / tau_T in internal units (src/md.f90:207, 231)
     M.T0 = m->T0;
@@ -892,17 +879,14 @@ extern "C" int32_t qnb_batch_create(int32_t n, const qnb_system* const* sys, con
       M.ndegf = 3.0 * S.natom - 3.0 * S.nwat;
       M.ndegfree = (double)(long long)(M.ndegf - 3.0 * (nex[0] + nex[1]) + (exsh[0] + exsh[1]));
     }
-    if ((rc = b->mem.upload(&M.bond_ij, m->bond_ij, 2 * (size_t)m->nbonds)) ||
-        (rc = b->mem.upload(&M.bond_r0, m->bond_r0, m->nbonds)) || (rc = b->mem.upload(&M.bond_k, m->bond_k, m->nbonds)) ||
-        (rc = b->mem.upload(&M.angle_ijk, m->angle_ijk, 3 * (size_t)m->nangles)) ||
-        (rc = b->mem.upload(&M.angle_t0, m->angle_t0, m->nangles)) ||
-        (rc = b->mem.upload(&M.angle_k, m->angle_k, m->nangles)) || (rc = b->mem.upload(&M.winv, m->winv, S.natom)) ||
+    if ((rc = b->mem.upload(&M.winv, m->winv, S.natom)) ||
         (rc = b->mem.alloc(&M.v, 3 * (size_t)S.natom)) || (rc = b->mem.alloc(&M.xx, 3 * (size_t)S.natom)) ||
         (rc = b->mem.alloc(&M.hist, (size_t)std::max(m->max_frames, 1) * QNB_FRAME_LEN)) ||
         (rc = b->mem.alloc(&M.st, 8)) || (rc = b->mem.alloc(&M.ctr, 4)))
       return rc;
     // atom-centred incidence lists of the bonds and angles (k_bonded)
-    if (m->nbonds < 0 || m->nangles < 0 || (m->nbonds > 0 && !m->bond_ij) || (m->nangles > 0 && !m->angle_ijk))
+    if (m->nbonds < 0 || m->nangles < 0 || (m->nbonds > 0 && (!m->bond_ij || !m->bond_r0 || !m->bond_k)) ||
+        (m->nangles > 0 && (!m->angle_ijk || !m->angle_t0 || !m->angle_k)))
       return fail(QNB_EINVAL, "instance %d: bad bond/angle arrays", k);
     {
       std::vector<int> boff(S.natom + 1, 0), aoff(S.natom + 1, 0);
@@ -922,15 +906,24 @@ extern "C" int32_t qnb_batch_create(int32_t n, const qnb_system* const* sys, con
         boff[i + 1] += boff[i];
         aoff[i + 1] += aoff[i];
       }
-      std::vector<int> bitem(std::max(boff[S.natom], 1)), aitem(std::max(aoff[S.natom], 1));
+      std::vector<BondRec> brec(std::max(boff[S.natom], 1));
+      std::vector<AngleRec> arec(std::max(aoff[S.natom], 1));
       std::vector<int> bpos(boff.begin(), boff.end() - 1), apos(aoff.begin(), aoff.end() - 1);
-      for (int q = 0; q < 2 * m->nbonds; q++) bitem[bpos[m->bond_ij[q]]++] = q;  // q = 2 * bond + role
-      for (int q = 0; q < 3 * m->nangles; q++) aitem[apos[m->angle_ijk[q]]++] = q;  // q = 3 * angle + role
-      M.nbat = nbat;
-      if ((rc = b->mem.upload(&M.boff, boff.data(), boff.size())) ||
-          (rc = b->mem.upload(&M.bitem, bitem.data(), bitem.size())) ||
-          (rc = b->mem.upload(&M.aoff, aoff.data(), aoff.size())) ||
-          (rc = b->mem.upload(&M.aitem, aitem.data(), aitem.size())))
+      for (int q = 0; q < m->nbonds; q++)
+        for (int role = 0; role < 2; role++)
+          brec[bpos[m->bond_ij[2 * q + role]]++] =
+              BondRec{role, m->bond_ij[2 * q + 1 - role], m->bond_r0[q], m->bond_k[q]};
+      for (int q = 0; q < m->nangles; q++) {
+        const int32_t* p = m->angle_ijk + 3 * q;
+        for (int role = 0; role < 3; role++)
+          arec[apos[p[role]]++] = AngleRec{role, p[role == 0 ? 1 : 0], p[role == 2 ? 1 : 2], 0, m->angle_t0[q], m->angle_k[q]};
+      }
+      S.nbat = nbat;
+      if ((rc = b->mem.upload(&S.boff, boff.data(), boff.size())) ||
+          (rc = b->mem.upload(&S.brec, brec.data(), brec.size())) ||
+          (rc = b->mem.upload(&S.aoff, aoff.data(), aoff.size())) ||
+          (rc = b->mem.upload(&S.arec, arec.data(), arec.size())) ||
+          (rc = b->mem.alloc(&S.brow, 3 * (size_t)std::max(nbat, 1))))
         return rc;
       b->nbblk = std::max(b->nbblk, (nbat + 255) / 256);
       const int nib = (S.nwat + S.nat_solute + 255) / 256;
@@ -1085,7 +1078,7 @@ extern "C" int32_t qnb_batch_integrate(qnb_batch* b, const double* const* d) {
     if (!d[k]) return fail(QNB_EINVAL, "instance %d: null gradient", k);
   for (int k = 0; k < b->n; k++)
     HIPCHK(hipMemcpyAsync(b->hs[k].d, d[k], sizeof(double) * 3 * b->hs[k].natom, hipMemcpyHostToDevice, b->stream));
-  launch_integrate(b);
+  launch_integrate(b, false, 0);
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(b->stream));
   b->steps_done++;
@@ -1327,7 +1320,7 @@ extern "C" int32_t qnb_batch_adjoint(qnb_batch* b, const qnb_qtangent* const* ta
   for (int k = 0; k < b->n; k++) {
     int rc = frames_stored(b, k, &nf[k]);
     if (rc) return rc;
-    const DevSys& S = b->hs[k];
+    DevSys& S = b->hs[k];
     off[k + 1] = off[k] + (size_t)nf[k] * S.nstates * S.nqat * QNB_ADJ_NV;
     waves = std::max(waves, (long)nf[k] * S.nqat);
   }

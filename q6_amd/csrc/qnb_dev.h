@@ -30,6 +30,18 @@ enum {
 // blocks per system of the energy reduction's first pass (k_reduce_part)
 #define QNB_RED_BLOCKS 64
 
+// a bond or angle as one of its atoms sees it: its role (place in the term),
+// the other atoms in the term's order, and the parameters, so that an atom's
+// terms are one load away from their partners' positions
+struct alignas(8) BondRec {
+  int role, other;
+  double r0, k;
+};
+struct alignas(8) AngleRec {
+  int role, o1, o2, pad;
+  double t0, k;
+};
+
 struct DevSys {
   // sizes
   int natom, nat_solute, nwat, sa, ncgp, ncgp_solute, nqat, nstates, ntypes, ivdw_rule, spc;
@@ -184,6 +196,15 @@ struct DevSys {
   int* sh_list;      // [QNB_MAXSH][nwat] members of each shell
   double* sh_lth;    // [QNB_MAXSH][nwat] their theta
   int* sh_n;         // [QNB_MAXSH] members per shell
+  // atom-centred bonded terms of the MD path: for atom i, records
+  // boff[i]..boff[i+1]-1 of brec and aoff[i]..aoff[i+1]-1 of arec; atoms
+  // [0, nbat) carry all of them, with gradient rows brow (k_pol_bonded)
+  const int* boff;
+  const BondRec* brec;
+  const int* aoff;
+  const AngleRec* arec;
+  double* brow;
+  int nbat;
   double* wp_rank;   // [QNB_MAXSH][nwat][2] restraint energy and theta of each member, by rank
   // energy sampling: energies are accumulated when ene_every <= 0 or when
   // the instance's step counter is a multiple of ene_every
@@ -455,12 +476,12 @@ __device__ __forceinline__ double watpol_sum(const DevSys& S, int is, int n, int
   return wave_sum(v);
 }
 
-// Last phase of the polarisation restraint, one wave per system: accumulates
-// avtheta and avn_insh and clears the shell counts for the
-// next step's angle kernel.
-__device__ __forceinline__ void watpol_finish(const DevSys& S) {
+// Last phase of the polarisation restraint, `waves` waves of one block per
+// system (wave `w` takes shells w, w + waves, ...): accumulates avtheta and
+// avn_insh and clears the shell counts for the next step's angle kernel.
+__device__ __forceinline__ void watpol_finish(const DevSys& S, int w, int waves) {
   if (!has_pol(S)) return;
-  for (int is = 0; is < S.nshell; is++) {
+  for (int is = w; is < S.nshell; is += waves) {
     const int n = ldg(S.sh_n + is);
     if (n == 0) continue;
     const double s = watpol_sum(S, is, n, 1);
@@ -631,9 +652,102 @@ __device__ __forceinline__ void add_qrows(const DevSys& S, int i, int rows, doub
     for (int c = 0; c < 3; c++) f[c] += ldg(S.dqq + 3 * e + c);
 }
 
+// harmonic bonds and angles of the solute (bond, angle: src/bondene.f90:41-246)
+// One thread per atom sums the terms of every bond and angle it belongs to
+// (each term is evaluated once per member atom), so the gradient needs no
+// atomics and does not depend on scheduling.  A bond's energy is counted by
+// its first atom, an angle's by its vertex; each block's energy sums go to
+// bpart[block] and k_record adds them in block order.  bonded_atom is the
+// per-atom part, used by k_bonded (the minimiser), k_atom_step (MD steps that
+// record energies) and k_pol_bonded (the others).
+// An atom has a few terms, each a chain of loads: BA_U records and then their
+// partners' positions are requested together.
+#define BA_U 2
+__device__ __forceinline__ void bonded_atom(const DevSys& S, int i, double* f, double& eb, double& ea) {
+  const auto x = gp(S.x);
+  const int b0 = ldg(S.boff + i), b1 = ldg(S.boff + i + 1), a0 = ldg(S.aoff + i), a1 = ldg(S.aoff + i + 1);
+  const double xi[3] = {x[3 * i], x[3 * i + 1], x[3 * i + 2]};
+  for (int it = b0; it < b1; it += BA_U) {
+    BondRec r[BA_U];
+    double xo[BA_U][3];
+#pragma unroll
+    for (int u = 0; u < BA_U; u++) {
+      const auto p = gp(S.brec + min(it + u, b1 - 1));
+      r[u] = BondRec{p->role, p->other, p->r0, p->k};
+    }
+#pragma unroll
+    for (int u = 0; u < BA_U; u++)
+      for (int c = 0; c < 3; c++) xo[u][c] = x[3 * r[u].other + c];
+#pragma unroll
+    for (int u = 0; u < BA_U; u++) {
+      if (it + u >= b1) break;
+      const bool first = r[u].role == 0;
+      // from the bond's first atom to its second
+      double v[3];
+      for (int c = 0; c < 3; c++) v[c] = first ? xo[u][c] - xi[c] : xi[c] - xo[u][c];
+      const double d = sqrt(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
+      const double db = d - r[u].r0;
+      const double dv = r[u].k * db / d;
+      const double sg = first ? -dv : dv;
+      for (int c = 0; c < 3; c++) f[c] += v[c] * sg;
+      if (first) eb += 0.5 * r[u].k * db * db;
+    }
+  }
+  for (int it = a0; it < a1; it += BA_U) {
+    AngleRec r[BA_U];
+    double x1[BA_U][3], x2[BA_U][3];
+#pragma unroll
+    for (int u = 0; u < BA_U; u++) {
+      const auto p = gp(S.arec + min(it + u, a1 - 1));
+      r[u] = AngleRec{p->role, p->o1, p->o2, 0, p->t0, p->k};
+    }
+#pragma unroll
+    for (int u = 0; u < BA_U; u++)
+      for (int c = 0; c < 3; c++) {
+        x1[u][c] = x[3 * r[u].o1 + c];
+        x2[u][c] = x[3 * r[u].o2 + c];
+      }
+#pragma unroll
+    for (int u = 0; u < BA_U; u++) {
+      if (it + u >= a1) break;
+      const int role = r[u].role;
+      // the angle's atoms i, j (vertex), k
+      double v[3], w[3];
+      for (int c = 0; c < 3; c++) {
+        const double pi = role == 0 ? xi[c] : x1[u][c];
+        const double pj = role == 0 ? x1[u][c] : (role == 1 ? xi[c] : x2[u][c]);
+        const double pk = role == 2 ? xi[c] : x2[u][c];
+        v[c] = pi - pj;
+        w[c] = pk - pj;
+      }
+      const double ru = sqrt(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
+      const double rw = sqrt(w[0] * w[0] + w[1] * w[1] + w[2] * w[2]);
+      double ct = (v[0] * w[0] + v[1] * w[1] + v[2] * w[2]) / (ru * rw);
+      ct = fmin(1.0, fmax(-1.0, ct));
+      const double th = acos(ct);
+      // sin(theta) from the cross product, consistent with the numerator of
+      // the derivative below even for nearly linear angles, where
+      // sin(acos(ct)) loses all digits; at a linear angle the derivative has
+      // no direction
+      const double cx = v[1] * w[2] - v[2] * w[1], cy = v[2] * w[0] - v[0] * w[2], cz = v[0] * w[1] - v[1] * w[0];
+      const double st = sqrt(cx * cx + cy * cy + cz * cz) / (ru * rw);
+      const double da = th - r[u].t0;
+      if (role == 1) ea += 0.5 * r[u].k * da * da;
+      if (!(st > 1.0e-8)) continue;
+      const double dv = r[u].k * da;
+      // dtheta/dx_i = -(w/(ru rw) - ct u/ru^2)/sin(theta), likewise for k; j balances
+      for (int c = 0; c < 3; c++) {
+        const double gi = -(w[c] / (ru * rw) - ct * v[c] / (ru * ru)) / st;
+        const double gk = -(v[c] / (ru * rw) - ct * w[c] / (rw * rw)) / st;
+        f[c] += dv * (role == 0 ? gi : (role == 2 ? gk : -(gi + gk)));
+      }
+    }
+  }
+}
+
 // LRF Taylor application for one atom (lrf_taylor, nonbondene.f90:507-571)
-__device__ __forceinline__ void lrf_taylor_atom(const DevSys& S, int i, double* f, double& e) {
-  const auto L = gp(S.lrf + (size_t)QNB_NLRF * ldg(S.atom_group + i));
+__device__ __forceinline__ void lrf_taylor_atom(const DevSys& S, int i, int group, double* f, double& e) {
+  const auto L = gp(S.lrf + (size_t)QNB_NLRF * group);
   const auto x = gp(S.x);
   const double drx = L[0] - x[3 * i], dry = L[1] - x[3 * i + 1], drz = L[2] - x[3 * i + 2];
   const auto p1 = L + 4;

@@ -82,8 +82,10 @@ void launch_forces_small(hipStream_t st, int prec, int ns_max, bool energy, cons
 // kernel
 bool small_launch(long solute_groups, long solvent);
 // polarisation restraint: angles and shells (theta), ranks and forces, and
-// the per-system sums (finish) where no later kernel of the caller runs them
-void launch_watpol(hipStream_t st, int nwat, int B, const DevSys* dsys, const int* istep, bool theta, bool finish);
+// the per-system sums (finish) where no later kernel of the caller runs them;
+// beside the forces, bonded_blocks blocks of bonded terms (DevSys::brow)
+void launch_watpol(hipStream_t st, int nwat, int B, const DevSys* dsys, const int* istep, bool theta, bool finish,
+                   int bonded_blocks);
 // per-instance device state (coordinates, gradient, lists, LRF, energies)
 int instance_alloc(DevSys& S, DevAlloc& M, const qnb_params* p, int nslots);
 // neighbour rows of `cap` groups; entries per partner-atom row that always

@@ -1506,7 +1506,7 @@ __global__ __launch_bounds__(256) void k_atom_terms(const DevSys* __restrict__ s
   if (i >= S.natom) return;
   double f[3] = {0.0, 0.0, 0.0};
   double el = 0.0, er = 0.0;
-  if ((mask & T_LRF) && S.use_lrf && !ldg(S.excl + i) && ldg(S.iqatom + i) == 0) lrf_taylor_atom(S, i, f, el);
+  if ((mask & T_LRF) && S.use_lrf && !ldg(S.excl + i) && ldg(S.iqatom + i) == 0) lrf_taylor_atom(S, i, ldg(S.atom_group + i), f, el);
   const int src = (mask & T_RAD) ? radial_source(S, i) : -1;
   if (src >= 0) {
     const double T = tfree[blockIdx.y];
@@ -1901,21 +1901,44 @@ __global__ __launch_bounds__(256) void k_forces_small(const DevSys* __restrict__
 // the waters in index order, so a wave counts one list: the index order, where
 // every block holds every shell, cost 51 windows of 2,352 waters 22 us per
 // step more.
-__global__ __launch_bounds__(256) void k_watpol_force(const DevSys* __restrict__ systems) {
+//
+// BONDED: blocks from pol on form the bonded terms of 256 atoms each into their
+// rows, for k_integrate.  In a small step they share the launch with the
+// polarisation blocks, whose latency is the longer one; where the restraint
+// runs beside full force kernels the two are launches of their own, because
+// the 106 registers of the bonded terms (32 without) keep those from the CUs:
+// 51 windows of 11,056 atoms, 847 us per step in one launch, 834 in two.
+template <bool BONDED>
+__global__ __launch_bounds__(256) void k_pol_bonded(const DevSys* __restrict__ systems, int pol) {
   const DevSys& S = systems[blockIdx.y];
   const int lane = threadIdx.x % QNB_WAVE, wid = threadIdx.x / QNB_WAVE;
+  if constexpr (BONDED) {
+    if ((int)blockIdx.x >= pol) {
+      const int i = ((int)blockIdx.x - pol) * blockDim.x + threadIdx.x;
+      if (i >= S.nbat) return;
+      double f[3] = {0.0, 0.0, 0.0}, eb = 0.0, ea = 0.0;
+      bonded_atom(S, i, f, eb, ea);
+      for (int c = 0; c < 3; c++) stg(S.brow + 3 * i + c, f[c]);
+      return;
+    }
+  }
   if (!has_pol(S)) return;
   const int nsh = S.nshell, nw = S.nwat;
   // block x of the system takes members 64 x' .. of shell sh, the blocks of
   // the shells laid end to end
-  int sh = 0, xb = blockIdx.x, n = 0;
-  for (; sh < nsh; sh++) {
-    n = ldg(S.sh_n + sh);
-    const int nb = (n + WP_WATERS - 1) / WP_WATERS;
-    if (xb < nb) break;
-    xb -= nb;
+  int cnt[QNB_MAXSH];
+#pragma unroll
+  for (int is = 0; is < QNB_MAXSH; is++) cnt[is] = is < nsh ? ldg(S.sh_n + is) : 0;
+  int sh = -1, xb = blockIdx.x, n = 0;
+#pragma unroll
+  for (int is = 0; is < QNB_MAXSH; is++) {
+    const int nb = (cnt[is] + WP_WATERS - 1) / WP_WATERS;
+    if (sh < 0) {
+      if (xb < nb) sh = is, n = cnt[is];
+      else xb -= nb;
+    }
   }
-  if (sh >= nsh) return;
+  if (sh < 0) return;
   __shared__ double c_th[WP_CHUNK];
   __shared__ int c_w[WP_CHUNK];
   __shared__ int s_cnt[4][QNB_WAVE];
@@ -1948,7 +1971,8 @@ __global__ __launch_bounds__(256) void k_watpol_force(const DevSys* __restrict__
   const double tc = S.sh_state[sh];
   double arg = 1.0 + (1.0 - 2.0 * (double)il) / (double)n;
   double th0 = acos(arg);
-  th0 = th0 - 3.0 * sin(th0) * S.sh_cstb[sh] / 2.0;
+  // sin(acos(c)) = sqrt((1 - c)(1 + c)), here and below
+  th0 = th0 - 3.0 * sqrt((1.0 - arg) * (1.0 + arg)) * S.sh_cstb[sh] / 2.0;
   if (th0 < 0.0) th0 = 0.0;
   if (th0 > pi) th0 = pi;
   const double dth = th - th0 + tc;
@@ -1959,7 +1983,7 @@ __global__ __launch_bounds__(256) void k_watpol_force(const DevSys* __restrict__
   wat_vectors(S, i, rmu, rm, rcu, rc);
   double scp = rmu[0] * rcu[0] + rmu[1] * rcu[1] + rmu[2] * rcu[2];
   scp = scp > 1.0 ? 1.0 : (scp < -1.0 ? -1.0 : scp);
-  double f0 = sin(acos(scp));
+  double f0 = sqrt((1.0 - scp) * (1.0 + scp));
   if (fabs(f0) < 1.0e-10) f0 = 1.0e-10;
   f0 = -1.0 / f0;
   f0 = dv * f0;
@@ -1975,11 +1999,14 @@ __global__ __launch_bounds__(256) void k_watpol_force(const DevSys* __restrict__
   stg(o + 1, th);
 }
 
+template __global__ void k_pol_bonded<false>(const DevSys*, int);
+template __global__ void k_pol_bonded<true>(const DevSys*, int);
+
 // Phase 3 on its own, one wave per system (watpol_finish): the minimiser's
-// step; the MD step runs it in k_thermo, a single evaluation in
+// step; the MD step runs it in k_integrate, a single evaluation in
 // k_reduce_final.
 __global__ __launch_bounds__(64) void k_watpol_finish(const DevSys* __restrict__ systems) {
-  watpol_finish(systems[blockIdx.x]);
+  watpol_finish(systems[blockIdx.x], 0, 1);
 }
 
 // ---------------------------------------------------------------------------
@@ -2029,7 +2056,7 @@ __global__ __launch_bounds__(256) void k_reduce_part(const DevSys* __restrict__ 
 __global__ __launch_bounds__(256) void k_reduce_final(const DevSys* __restrict__ systems, int with_qq, int with_pol) {
   const DevSys& S = systems[blockIdx.x];
   if (want_energies(S)) reduce_final(S, with_qq, with_pol);
-  if (with_pol && threadIdx.x < QNB_WAVE) watpol_finish(S);
+  if (with_pol) watpol_finish(S, threadIdx.x / QNB_WAVE, 4);
 }
 
 SmallGrid small_grid(int solute_groups, int nwat, int sa, int nqat, int nat_solute, int nqe, uint32_t mask, bool pol) {
