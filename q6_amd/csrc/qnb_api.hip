@@ -196,11 +196,11 @@ int topo_build(DevSys& S, const qnb_system* s, HostTopo& T, DevAlloc& M) {
       return fail(QNB_EINVAL, "atom %d is in no charge group", i);
   // charge groups are consecutive runs of cgpatom, as the topology reader
   // lays them out
-  std::vector<int> gslot(ncgpat);
+  std::vector<uint64_t> gbit(ncgpat);
   for (int g = 0; g < s->ncgp; g++) {
     if (s->cgp_first[g] != (g == 0 ? 0 : s->cgp_last[g - 1] + 1) || s->cgp_last[g] < s->cgp_first[g])
       return fail(QNB_EINVAL, "charge group %d is not the run after group %d in cgpatom", g, g - 1);
-    for (int k = s->cgp_first[g]; k <= s->cgp_last[g]; k++) gslot[k] = g & 63;
+    for (int k = s->cgp_first[g]; k <= s->cgp_last[g]; k++) gbit[k] = 1ull << (g & 63);
   }
   S.ncgpat = ncgpat;
   const int nsol1 = std::max(nsol, 1);
@@ -285,7 +285,7 @@ int topo_build(DevSys& S, const qnb_system* s, HostTopo& T, DevAlloc& M) {
   UP(gswitch, s->cgp_iswitch, s->ncgp);
   UP(cgpatom, s->cgpatom, ncgpat);
   UP(atom_group, atom_group.data(), nat);
-  UP(gslot, gslot.data(), ncgpat);
+  UP(gbit, gbit.data(), ncgpat);
   {
     std::vector<int> entry(T.cgpatom);
     for (int& e : entry)

@@ -71,9 +71,9 @@ struct DevSys {
   const int* cgpatom;
   const int* atom_group;
   // per group-ordered atom k (cgpatom order; groups are consecutive runs):
-  // the atom's group modulo 64, its bit in the far-group ballot word of the
-  // list sweep's 64-group chunk
-  const int* gslot;
+  // the bit of the atom's group (its index modulo 64) in the far-group ballot
+  // word of the list sweep's 64-group chunk
+  const uint64_t* gbit;
   int ncgpat;
   const int* cgentry;  // per group-ordered atom: its index, with AL_SKIP for a Q-atom (k_expand)
   const double* avdw;  // [t*3+k]
@@ -867,9 +867,15 @@ __device__ __forceinline__ bool pp_param(const DevSys& S, int i, int j, double& 
 // 1/|u|^2 and 1/|u| from |u|^2: IEEE division and square root in FP64 (the
 // plain path evaluates them as q_dist does); in FP32 the hardware reciprocal
 // square root (v_rsq_f32, 1 ulp), the usual FP32 pair-kernel form
+// FP64: the hardware's reciprocal root (about 26 bits) with one third-order
+// step, y (1 + e/2 + 3 e^2/8) with e = 1 - d2 y^2, and 1/d2 from its square with
+// one Newton step: 15 slots and no branch, a division and a root took about 32
 __device__ __forceinline__ void rinv(double d2, double& r2, double& r) {
-  r2 = 1.0 / d2;
-  r = sqrt(r2);
+  const double y = __builtin_amdgcn_rsq(d2);
+  const double e = __builtin_fma(-d2 * y, y, 1.0);
+  r = __builtin_fma(y * e, __builtin_fma(0.375, e, 0.5), y);
+  const double s = r * r;
+  r2 = __builtin_fma(s, __builtin_fma(-d2, s, 1.0), s);
 }
 __device__ __forceinline__ void rinv(float d2, float& r2, float& r) {
   r = __builtin_amdgcn_rsqf(d2);

@@ -84,89 +84,41 @@ __device__ __forceinline__ bool owns(int a, int b) {
 }
 
 // ---------------------------------------------------------------------------
-// LRF expansion (lrf_update, nonbondene.f90:628-725), restated on the 20
-// independent components of the symmetric tensors: acc[0] phi0, acc[1..3]
-// phi1, acc[4..9] phi2 (xx xy xz yy yz zz), acc[10..19] phi3 (xxx xxy xxz xyy
-// xyz xzz yyy yyz yzz zzz).  dr = x_i - centre in FP64, terms in R; the
-// caller sums one source group's terms in R (at most a group's atoms) and
-// adds the group's partial to its FP64 accumulators.
-template <typename R>
-__device__ __forceinline__ void lrf_accumulate(R* acc, double drx, double dry, double drz, double q) {
-  R dx = (R)drx, dy = (R)dry, dz = (R)drz;
-  R r2 = dx * dx + dy * dy + dz * dz;
-  R f0, f1, f2;
-  if constexpr (sizeof(R) == 4) {
-    R ri2, ri;
-    rinv(r2, ri2, ri);
-    f0 = (R)q * ri * ri2;
-    f1 = R(3) * f0 * ri2;
-    f2 = -f1 * ri2;
-  } else {
-    f0 = (R)q / (r2 * sqrt(r2));
-    f1 = R(3) * f0 / r2;
-    f2 = -f1 / r2;
-  }
-  acc[0] += f0 * r2;
-  acc[1] -= dx * f0;
-  acc[2] -= dy * f0;
-  acc[3] -= dz * f0;
-  R xx = dx * dx, xy = dx * dy, xz = dx * dz, yy = dy * dy, yz = dy * dz, zz = dz * dz;
-  acc[4] += xx * f1 - f0;
-  acc[5] += xy * f1;
-  acc[6] += xz * f1;
-  acc[7] += yy * f1 - f0;
-  acc[8] += yz * f1;
-  acc[9] += zz * f1 - f0;
-  R g = R(5) * f2, h = f2 * r2;
-  R gx = g * dx, gy = g * dy, gz = g * dz;
-  acc[10] += gx * xx - R(3) * h * dx;
-  acc[11] += gx * xy - h * dy;
-  acc[12] += gx * xz - h * dz;
-  acc[13] += gx * yy - h * dx;
-  acc[14] += gx * yz;
-  acc[15] += gx * zz - h * dx;
-  acc[16] += gy * yy - R(3) * h * dy;
-  acc[17] += gy * yz - h * dz;
-  acc[18] += gy * zz - h * dy;
-  acc[19] += gz * zz - R(3) * h * dz;
-}
-
-// FP32 form for the mixed path: dr already formed in FP32 from the packed
-// positions (x_i and the centre each rounded once), q the atom's charge.
-// The lane keeps raw sums that need no per-atom constant or subtraction:
+// LRF expansion (lrf_update, nonbondene.f90:628-725), restated on raw sums that
+// need no per-atom constant or subtraction:
 //   p[0] = sum q/r,  p[1..3] = sum f0 d_a,  p[4..9] = sum w1 d_a d_b,
 //   p[10..19] = sum w2 d_a d_b d_c
-// with f0 = q/r^3, w1 = f0/r^2, w2 = w1/r^2 (component order as acc).
-// lrf_update's field1 = 3 f0/r^2 and its 5 field2 d d d term (field2 =
-// -field1/r^2) give phi2_ab = 3 p_ab - delta_ab sum f0 and
-// phi3_abc = -15 p_abc + 3 (delta_ab H_c + delta_ac H_b + delta_bc H_a),
-// H_a = sum w1 d_a; as w1 r^2 = f0 and w2 r^2 = w1, sum f0 is the trace of
-// p[4..9] and H_a the trace of p[10..19] over the other two indices, which
-// lrf_flush_f forms in FP64.
+// with d = x_i - centre, f0 = q/r^3, w1 = f0/r^2, w2 = w1/r^2; components xx xy
+// xz yy yz zz, then xxx xxy xxz xyy xyz xzz yyy yyz yzz zzz.  lrf_update's
+// field1 = 3 f0/r^2 and its 5 field2 d d d term (field2 = -field1/r^2) give
+// phi2_ab = 3 p_ab - delta_ab sum f0 and phi3_abc = -15 p_abc +
+// 3 (delta_ab H_c + delta_ac H_b + delta_bc H_a), H_a = sum w1 d_a; as
+// w1 r^2 = f0 and w2 r^2 = w1, sum f0 is the trace of p[4..9] and H_a the trace
+// of p[10..19] over the other two indices: lrf_tensors, once per receiver.
 #define LRF_NF 20
 typedef float f4v __attribute__((ext_vector_type(4)));
 typedef double d4v __attribute__((ext_vector_type(4)));
 typedef double d2v __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ void lrf_accumulate_f(float* p, float dx, float dy, float dz, float q) {
-  const float r2 = dx * dx + dy * dy + dz * dz;
-  float ri2, ri;
-  rinv(r2, ri2, ri);
-  const float qri = q * ri;
+template <typename R>
+__device__ __forceinline__ void lrf_accumulate(R* p, R dx, R dy, R dz, R q) {
+  R ri2, ri;
+  rinv(norm2(dx, dy, dz), ri2, ri);
+  const R qri = q * ri;
   p[0] += qri;
-  const float f0 = qri * ri2;
-  const float w1 = f0 * ri2;
-  const float w2 = w1 * ri2;
+  const R f0 = qri * ri2;
+  const R w1 = f0 * ri2;
+  const R w2 = w1 * ri2;
   p[1] += dx * f0;
   p[2] += dy * f0;
   p[3] += dz * f0;
-  const float xx = dx * dx, xy = dx * dy, xz = dx * dz, yy = dy * dy, yz = dy * dz, zz = dz * dz;
+  const R xx = dx * dx, xy = dx * dy, xz = dx * dz, yy = dy * dy, yz = dy * dz, zz = dz * dz;
   p[4] += xx * w1;
   p[5] += xy * w1;
   p[6] += xz * w1;
   p[7] += yy * w1;
   p[8] += yz * w1;
   p[9] += zz * w1;
-  const float gx = w2 * dx, gy = w2 * dy, gz = w2 * dz;
+  const R gx = w2 * dx, gy = w2 * dy, gz = w2 * dz;
   p[10] += gx * xx;
   p[11] += gx * xy;
   p[12] += gx * xz;
@@ -179,33 +131,30 @@ __device__ __forceinline__ void lrf_accumulate_f(float* p, float dx, float dy, f
   p[19] += gz * zz;
 }
 
-// adds a lane's raw FP32 sums to its FP64 expansion
-__device__ __forceinline__ void lrf_flush_f(double* acc, const float* p) {
-  double q[LRF_NF];
-#pragma unroll
-  for (int k = 0; k < LRF_NF; k++) q[k] = (double)p[k];
+// raw sums -> phi0, phi1[3], phi2[6], phi3[10] (lrf_update's tensors)
+__device__ __forceinline__ void lrf_tensors(double* acc, const double* q) {
   const double s0 = q[4] + q[7] + q[9];
   const double hx = q[10] + q[13] + q[15], hy = q[11] + q[16] + q[18], hz = q[12] + q[17] + q[19];
-  acc[0] += q[0];
-  acc[1] -= q[1];
-  acc[2] -= q[2];
-  acc[3] -= q[3];
-  acc[4] += 3.0 * q[4] - s0;
-  acc[5] += 3.0 * q[5];
-  acc[6] += 3.0 * q[6];
-  acc[7] += 3.0 * q[7] - s0;
-  acc[8] += 3.0 * q[8];
-  acc[9] += 3.0 * q[9] - s0;
-  acc[10] += 9.0 * hx - 15.0 * q[10];
-  acc[11] += 3.0 * hy - 15.0 * q[11];
-  acc[12] += 3.0 * hz - 15.0 * q[12];
-  acc[13] += 3.0 * hx - 15.0 * q[13];
-  acc[14] -= 15.0 * q[14];
-  acc[15] += 3.0 * hx - 15.0 * q[15];
-  acc[16] += 9.0 * hy - 15.0 * q[16];
-  acc[17] += 3.0 * hz - 15.0 * q[17];
-  acc[18] += 3.0 * hy - 15.0 * q[18];
-  acc[19] += 9.0 * hz - 15.0 * q[19];
+  acc[0] = q[0];
+  acc[1] = -q[1];
+  acc[2] = -q[2];
+  acc[3] = -q[3];
+  acc[4] = 3.0 * q[4] - s0;
+  acc[5] = 3.0 * q[5];
+  acc[6] = 3.0 * q[6];
+  acc[7] = 3.0 * q[7] - s0;
+  acc[8] = 3.0 * q[8];
+  acc[9] = 3.0 * q[9] - s0;
+  acc[10] = 9.0 * hx - 15.0 * q[10];
+  acc[11] = 3.0 * hy - 15.0 * q[11];
+  acc[12] = 3.0 * hz - 15.0 * q[12];
+  acc[13] = 3.0 * hx - 15.0 * q[13];
+  acc[14] = -15.0 * q[14];
+  acc[15] = 3.0 * hx - 15.0 * q[15];
+  acc[16] = 9.0 * hy - 15.0 * q[16];
+  acc[17] = 3.0 * hz - 15.0 * q[17];
+  acc[18] = 3.0 * hy - 15.0 * q[18];
+  acc[19] = 9.0 * hz - 15.0 * q[19];
 }
 
 // Raw buffer loads (32-bit byte offsets from a base in scalar registers; an
@@ -223,15 +172,21 @@ __device__ __forceinline__ d4v buf_d4(__amdgpu_buffer_rsrc_t r, uint32_t off) {
   const d2v hi = __builtin_bit_cast(d2v, __builtin_amdgcn_raw_buffer_load_b128(r, off + 16, 0, 0));
   return d4v{lo.x, lo.y, hi.x, hi.y};
 }
-__device__ __forceinline__ int buf_i(__amdgpu_buffer_rsrc_t r, uint32_t off) {
-  return (int)__builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0);
+typedef unsigned int u2v __attribute__((vector_size(8)));
+__device__ __forceinline__ u2v buf_u2(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+  return __builtin_bit_cast(u2v, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
+}
+// through the scalar cache: a table that no kernel writes, at an index that is
+// the same in every lane
+__device__ __forceinline__ int ldc(const int* p) {
+  return *(const __attribute__((address_space(4))) int*)(uintptr_t)p;
 }
 
 // Packs the LRF sources before a list update, one record per atom in
 // cgpatom order (a charge group's atoms are one run): x, y, z and the charge,
 // 0 for Q-atoms (lrf_update skips them); FP32 for the mixed path (each
 // coordinate rounded once), FP64 for the plain one.  Also packs each group's
-// reference atom and its exclusion flag for the group tests of the sweep.
+// reference atom for the group tests of the sweep, with 0 if it is excluded.
 __global__ __launch_bounds__(256) void k_pack_xq(const DevSys* __restrict__ systems) {
   const DevSys& S = systems[blockIdx.y];
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
@@ -259,7 +214,7 @@ __global__ __launch_bounds__(256) void k_pack_xq(const DevSys* __restrict__ syst
     o[4 * k] = x[3 * rb];
     o[4 * k + 1] = x[3 * rb + 1];
     o[4 * k + 2] = x[3 * rb + 2];
-    o[4 * k + 3] = ldg(S.excl + rb) ? 1.0 : 0.0;
+    o[4 * k + 3] = ldg(S.excl + rb) ? 0.0 : 1.0;
   }
 }
 
@@ -308,10 +263,22 @@ __device__ __forceinline__ double dist4v(const d4v& a, const d4v& b) {
 // nonbondene.f90:628-725), so every lane has an atom whatever the group sizes.
 // ANY: some system of the launch has iuse_switch_atom = 0 (any_atom), whose
 // group tests scan atom pairs; the switch-atom form is compiled without it.
+//
+// Bound by the vector unit: an atom costs 43 FP32 slots (about 55 FP64 ones)
+// for its 20 sums.  Around them: the run is read LRF_U records per lane at a
+// time (64 waters are three), the first before the group tests, from a base
+// that moves in scalar registers; FP32 has the next batch in flight while one
+// is summed, FP64 keeps the registers for a fourth wave.  A record's group is
+// one bit of a 64-bit word, so a test is two ANDs and reads past the run find
+// 0; FP64 takes the sums raw too, with rinv in place of a root and three
+// divisions.  Measured: 2,663 -> 2,270 us for 51 windows of 11,056 atoms
+// (FP32), 1,740 -> 870 us for 12 of them in FP64; a list update of 19,440 atoms
+// in FP64 775 -> 403 us.
+#define LRF_U 3
 template <typename R, bool ANY>
 __global__ __launch_bounds__(512) void k_lists_lrf(const DevSys* __restrict__ systems) {
   const DevSys& S = systems[blockIdx.y];
-  const int a = blockIdx.x * (blockDim.x / QNB_WAVE) + threadIdx.x / QNB_WAVE;
+  const int a = uni(blockIdx.x * (blockDim.x / QNB_WAVE) + threadIdx.x / QNB_WAVE);
   if (a >= S.ncgp) return;
   const int lane = threadIdx.x % QNB_WAVE;
   const double* __restrict__ x = S.x;
@@ -319,9 +286,9 @@ __global__ __launch_bounds__(512) void k_lists_lrf(const DevSys* __restrict__ sy
   const bool a_sol = a < S.ncgp_solute;
   // centre of a (cgp_centers, nonbondene.f90:43-78): sum in atom order, then divide
   double cx = 0.0, cy = 0.0, cz = 0.0;
-  const int ga0 = ldg(S.gfirst + a), ga1 = ldg(S.glast + a);
+  const int ga0 = ldc(S.gfirst + a), ga1 = ldc(S.glast + a);
   for (int k = ga0; k <= ga1; k++) {
-    int at = ldg(S.cgpatom + k);
+    int at = ldc(S.cgpatom + k);
     cx = cx + ldg(x + 3 * at);
     cy = cy + ldg(x + 3 * at + 1);
     cz = cz + ldg(x + 3 * at + 2);
@@ -330,45 +297,65 @@ __global__ __launch_bounds__(512) void k_lists_lrf(const DevSys* __restrict__ sy
   cx = cx / nat;
   cy = cy / nat;
   cz = cz / nat;
-  const float cxf = (float)cx, cyf = (float)cy, czf = (float)cz;
-  double acc[20];
+  const R cxr = (R)cx, cyr = (R)cy, czr = (R)cz;
+  double acc[LRF_NF];
 #pragma unroll
-  for (int k = 0; k < 20; k++) acc[k] = 0.0;
+  for (int k = 0; k < LRF_NF; k++) acc[k] = 0.0;
   int count = 0, count_sol = 0;
   int* __restrict__ row = S.nbr + (size_t)a * S.cap;
-  // mixed path: the lane's raw FP32 sums since the last flush to the FP64
-  // expansion, flushed after a chunk once a lane has been offered LRF_FLUSH
-  // atoms (at most LRF_FLUSH - 1 plus one chunk's share)
+  // mixed path: the lane's FP32 sums since the last flush to FP64, flushed
+  // after a chunk once a lane has been offered LRF_FLUSH atoms (at most
+  // LRF_FLUSH - 1 plus one chunk's share)
   constexpr int LRF_FLUSH = 16;
+  constexpr bool F32 = sizeof(R) == 4;
   float pf[LRF_NF];
 #pragma unroll
   for (int k = 0; k < LRF_NF; k++) pf[k] = 0.0f;
   int offered = 0;
   if (!ldg(S.excl + ra)) {
-    const auto grs = buf_rsrc(S.gref, (size_t)S.ncgp * 32);
+    const int ncgp = S.ncgp, nsol = S.ncgp_solute;
+    const auto grs = buf_rsrc(S.gref, (size_t)ncgp * 32);
     const d4v A = buf_d4(grs, (uint32_t)a * 32);
-    const auto rs = buf_rsrc(sizeof(R) == 4 ? (const void*)S.xqg : (const void*)S.xqgd,
-                             (size_t)S.ncgpat * (sizeof(R) == 4 ? 16 : 32));
-    const auto gs = buf_rsrc(S.gslot, (size_t)S.ncgpat * 4);
+    constexpr uint32_t RB = F32 ? 16 : 32;
+    const char* recs = F32 ? (const char*)S.xqg : (const char*)S.xqgd;
+    const char* bits = (const char*)S.gbit;
     // the cut-off of a pair with a solute group and with a water, given a
     const double cut_sol = a_sol ? S.rcpp2 : S.rcpw2, cut_wat = a_sol ? S.rcpw2 : S.rcww2;
-    const bool quirk = pw_quirk(S), any_atom = ANY && S.any_atom, use_lrf = S.use_lrf;
-    const double rclrf2 = S.rclrf2;
-    for (int b0 = 0; b0 < S.ncgp; b0 += QNB_WAVE) {
+    const bool quirk = pw_quirk(S), any_atom = ANY && S.any_atom;
+    const double rclrf2 = S.use_lrf ? S.rclrf2 : -1.0;
+    using Rec = decltype(lrf_rec<R>(grs, 0));
+    // the chunk's atoms: the run from b0's first to its last group's last
+    int k1 = ldc(S.gfirst);
+    for (int b0 = 0; b0 < ncgp; b0 += QNB_WAVE) {
       const int b = b0 + lane;
       const d4v G = buf_d4(grs, (uint32_t)b * 32);  // 0 past the last group
+      const int k0 = ldc(S.gfirst + b0);
+      k1 = ldc(S.glast + min(b0 + QNB_WAVE, ncgp) - 1) + 1;
+      Rec r[LRF_U];
+      u2v s[LRF_U];
+      auto fetch = [&](int k, Rec* rr, u2v* ss) {
+        // 0 past the end of the run
+        const auto rs = buf_rsrc(recs + (size_t)k * RB, (size_t)(k1 - k) * RB);
+        const auto bs = buf_rsrc(bits + (size_t)k * 8, (size_t)(k1 - k) * 8);
+#pragma unroll
+        for (int u = 0; u < LRF_U; u++) {
+          rr[u] = lrf_rec<R>(rs, (uint32_t)(lane + u * QNB_WAVE) * RB);
+          ss[u] = buf_u2(bs, (uint32_t)(lane + u * QNB_WAVE) * 8);
+        }
+      };
+      fetch(k0, r, s);
       bool in = false, far = false;
-      if (b < S.ncgp && b != a && G.w == 0.0) {
-        const bool b_sol = b < S.ncgp_solute;
+      if (G.w != 0.0 && b != a) {
+        const bool b_sol = b < nsol;
         const double cut2 = b_sol ? cut_sol : cut_wat;
         double r2;
         bool inside;
         if (any_atom && (a_sol || b_sol)) {
           inside = any_atom_pair(S, x, a, b, a_sol, b_sol, ra, group_ref_atom(S, b), cut2, r2);
-        } else if (a_sol != b_sol && quirk) {
+        } else if (quirk && a_sol != b_sol) {
           // nbpwlist's test point: the switch atom up to the group's first
           // water inside, atom glast + 1 after it (LRF off: r2 unused)
-          const int g = a_sol ? a : b, w = (a_sol ? b : a) - S.ncgp_solute;
+          const int g = a_sol ? a : b, w = (a_sol ? b : a) - nsol;
           const int wf = ldg(S.pw_first + g);
           r2 = 0.0;
           inside = w == wf ||
@@ -378,52 +365,65 @@ __global__ __launch_bounds__(512) void k_lists_lrf(const DevSys* __restrict__ sy
           inside = r2 <= cut2;
         }
         in = inside;
-        far = !inside && use_lrf && r2 <= rclrf2;
+        far = !inside && r2 <= rclrf2;
       }
       const uint64_t m = __ballot(in);
-      const int pos = count + __popcll(m & ((1ull << lane) - 1ull));
-      if (in && pos < S.cap) stg(row + pos, b);
-      count += __popcll(m);
-      if (b0 < S.ncgp_solute) count_sol += __popcll(__ballot(in && b < S.ncgp_solute));
-      const uint64_t fw = __ballot(far);
-      if (fw != 0) {
-        // the chunk's atoms: the run from b0's first to its last group's last
-        const int k0 = ldg(S.gfirst + b0), k1 = ldg(S.glast + min(b0 + QNB_WAVE, S.ncgp) - 1) + 1;
-        // one iteration ahead: the next record and its group slot are in
-        // flight while this one is evaluated (reads past the run are unused)
-        constexpr uint32_t RB = sizeof(R) == 4 ? 16 : 32;
-        int k = k0 + lane;
-        uint32_t off = (uint32_t)k * RB, offs = (uint32_t)k * 4;
-        auto r = lrf_rec<R>(rs, off);
-        int sl = buf_i(gs, offs);
-        for (; k - lane < k1; k += QNB_WAVE) {
-          off += QNB_WAVE * RB;
-          offs += QNB_WAVE * 4;
-          const auto rn = lrf_rec<R>(rs, off);
-          const int sn = buf_i(gs, offs);
-          if (k < k1 && ((fw >> sl) & 1ull)) {
-            if constexpr (sizeof(R) == 4) lrf_accumulate_f(pf, r.x - cxf, r.y - cyf, r.z - czf, r.w);
-            else lrf_accumulate<double>(acc, r.x - cx, r.y - cy, r.z - cz, r.w);
-          }
-          r = rn;
-          sl = sn;
-        }
-        offered += (k1 - k0 + QNB_WAVE - 1) / QNB_WAVE;
+      if (m != 0) {
+        const int pos = count + __popcll(m & ((1ull << lane) - 1ull));
+        if (in && pos < S.cap) stg(row + pos, b);
+        count += __popcll(m);
+        if (b0 < nsol) count_sol += __popcll(__ballot(in && b < nsol));
       }
-      if constexpr (sizeof(R) == 4) {
-        if (offered >= LRF_FLUSH) {
-          lrf_flush_f(acc, pf);
+      const uint64_t fw = __ballot(far);
+      if (fw == 0) continue;
+      const uint32_t f0 = (uint32_t)fw, f1 = (uint32_t)(fw >> 32);
+      auto sum = [&](const Rec* rr, const u2v* ss) {
 #pragma unroll
-          for (int c = 0; c < LRF_NF; c++) pf[c] = 0.0f;
+        for (int u = 0; u < LRF_U; u++)
+          if (((ss[u][0] & f0) | (ss[u][1] & f1)) != 0) {
+            if constexpr (F32) lrf_accumulate<float>(pf, rr[u].x - cxr, rr[u].y - cyr, rr[u].z - czr, rr[u].w);
+            else lrf_accumulate<double>(acc, rr[u].x - cxr, rr[u].y - cyr, rr[u].z - czr, rr[u].w);
+          }
+      };
+      if constexpr (F32) {
+        for (int k = k0 + LRF_U * QNB_WAVE; k < k1; k += LRF_U * QNB_WAVE) {
+          Rec rn[LRF_U];
+          u2v sn[LRF_U];
+          fetch(k, rn, sn);
+          sum(r, s);
+#pragma unroll
+          for (int u = 0; u < LRF_U; u++) r[u] = rn[u], s[u] = sn[u];
+        }
+        sum(r, s);
+      } else {
+        sum(r, s);
+        for (int k = k0 + LRF_U * QNB_WAVE; k < k1; k += LRF_U * QNB_WAVE) {
+          fetch(k, r, s);
+          sum(r, s);
+        }
+      }
+      if constexpr (F32) {
+        offered += (k1 - k0 + QNB_WAVE - 1) / QNB_WAVE;
+        if (offered >= LRF_FLUSH) {
+#pragma unroll
+          for (int c = 0; c < LRF_NF; c++) {
+            acc[c] += (double)pf[c];
+            pf[c] = 0.0f;
+          }
           offered = 0;
         }
       }
     }
   }
-  if constexpr (sizeof(R) == 4) lrf_flush_f(acc, pf);
+  if constexpr (F32)
 #pragma unroll
-  for (int k = 0; k < 20; k++) acc[k] = wave_sum_all(acc[k]);
+    for (int c = 0; c < LRF_NF; c++) acc[c] += (double)pf[c];
+  const double tr = wave_sum_tr<double, LRF_NF>(acc, lane);
+#pragma unroll
+  for (int k = 0; k < LRF_NF; k++) acc[k] = lane_value(tr, wave_sum_tr_lane<LRF_NF>(k));
   if (lane == 0) {
+    double t[LRF_NF];
+    lrf_tensors(t, acc);
     S.nnbr[a] = count;
     S.nnsol[a] = count_sol;
     if (count > S.cap) atomicMax(S.need, count);
@@ -431,16 +431,16 @@ __global__ __launch_bounds__(512) void k_lists_lrf(const DevSys* __restrict__ sy
     L[0] = cx;
     L[1] = cy;
     L[2] = cz;
-    L[3] = acc[0];
-    L[4] = acc[1];
-    L[5] = acc[2];
-    L[6] = acc[3];
+    L[3] = t[0];
+    L[4] = t[1];
+    L[5] = t[2];
+    L[6] = t[3];
     const int p2[3][3] = {{4, 5, 6}, {5, 7, 8}, {6, 8, 9}};
     for (int k = 0; k < 3; k++)
-      for (int c = 0; c < 3; c++) L[7 + 3 * k + c] = acc[p2[k][c]];
+      for (int c = 0; c < 3; c++) L[7 + 3 * k + c] = t[p2[k][c]];
     for (int n = 0; n < 3; n++)
       for (int j = 0; j < 3; j++)
-        for (int c = 0; c < 3; c++) L[16 + 3 * (j + 3 * n) + c] = acc[t3index(n, j, c)];
+        for (int c = 0; c < 3; c++) L[16 + 3 * (j + 3 * n) + c] = t[t3index(n, j, c)];
   }
 }
 
