@@ -15,8 +15,8 @@
 // State energies are formed from each frame as pot_energy forms EQ(s)%total
 // (src/potene.f90:224-231: Q bonded terms, then qx = qq + qp + qw, el and
 // vdW), plus the alpha shifts (qfep.f90:447-452).  Every sum runs over the
-// frames in order, as the reference's loops do (one thread per sum), with no
-// contraction of multiply-add pairs, so the results differ from Qfep6's only
+// frames in order, as the reference's loops do (its terms formed in parallel,
+// one thread per sum), with no contraction of multiply-add pairs, so the results differ from Qfep6's only
 // by the last bits of exp and log.
 #include <hip/hip_runtime.h>
 
@@ -68,140 +68,234 @@ __device__ double veff_of(const double* lam, const double* v, int ns) {
   return e;
 }
 
-// Part 1 sums and the gap range of window blockIdx.x: thread 0 the forward
-// average, thread 1 the reverse one, all threads the gap minimum and maximum
-__global__ __launch_bounds__(64) void k_fep_window(const FepWin* __restrict__ wins, int n, FepPar P, double* dgf,
-                                                   double* dgr, double* wmin, double* wmax) {
-  const int i = blockIdx.x;
+// Part 1 sums and the gap range of window blockIdx.x.  The Boltzmann factors
+// are formed by every thread, FW_CH frames at a time, and one thread per sum
+// adds them from LDS in frame order: 1,000 additions are 8 us of latency, where
+// one thread that also formed them took 586 us (51 windows of 1,000 frames),
+// 15 us now.
+#define FW_CH 1024
+__global__ __launch_bounds__(256) void k_fep_window(const FepWin* __restrict__ wins, int n, FepPar P, double* dgf,
+                                                    double* dgr, double* wmin, double* wmax) {
+  const int i = blockIdx.x, t = threadIdx.x;
   const FepWin& W = wins[i];
+  __shared__ double e[2][FW_CH];
+  __shared__ double ends[2][4];
   double v[QNB_MAX_STATES], vg, c1, gap, r;
-  const int t = threadIdx.x;
-  if (t < 2) {
-    const int o = t == 0 ? i + 1 : i - 1;
-    double out = NAN;
-    if (o >= 0 && o < n) {
-      double sum = 0.0;
-      for (int f = P.nskip; f < W.nf; f++) {
-        fep_frame(W, P, f, v, vg, c1, gap, r);
-        const double veff1 = veff_of(W.lam, v, P.ns);
-        const double veff2 = veff_of(wins[o].lam, v, P.ns);
-        const double dv = veff2 - veff1;
-        sum = sum + exp(-dv / P.kT);
+  double lo = INFINITY, hi = -INFINITY, sum = 0.0;
+  const bool fwd = i + 1 < n, rev = i > 0;
+  const int which = t / QNB_WAVE;  // wave 0 adds the forward sum, wave 1 the reverse one
+  for (int f0 = P.nskip; f0 < W.nf; f0 += FW_CH) {
+    const int nk = min(FW_CH, W.nf - f0);
+    __syncthreads();
+    for (int k = t; k < nk; k += blockDim.x) {
+      fep_frame(W, P, f0 + k, v, vg, c1, gap, r);
+      lo = fmin(lo, gap);
+      hi = fmax(hi, gap);
+      const double veff1 = veff_of(W.lam, v, P.ns);
+      if (fwd) {
+        const double dv = veff_of(wins[i + 1].lam, v, P.ns) - veff1;
+        e[0][k] = exp(-dv / P.kT);
       }
+      if (rev) {
+        const double dv = veff_of(wins[i - 1].lam, v, P.ns) - veff1;
+        e[1][k] = exp(-dv / P.kT);
+      }
+    }
+    __syncthreads();
+    if (t % QNB_WAVE == 0 && ((which == 0 && fwd) || (which == 1 && rev))) {
+#pragma unroll 16
+      for (int k = 0; k < nk; k++) sum = sum + e[which][k];
+    }
+  }
+  if (t % QNB_WAVE == 0 && which < 2) {
+    double out = NAN;
+    if (which == 0 ? fwd : rev) {
       sum = sum / (double)(W.nf - P.nskip);
       out = -P.kT * log(sum);
     }
-    (t == 0 ? dgf : dgr)[i] = out;
-  }
-  double lo = INFINITY, hi = -INFINITY;
-  for (int f = P.nskip + t; f < W.nf; f += blockDim.x) {
-    fep_frame(W, P, f, v, vg, c1, gap, r);
-    lo = fmin(lo, gap);
-    hi = fmax(hi, gap);
+    (which == 0 ? dgf : dgr)[i] = out;
   }
   for (int off = 32; off > 0; off >>= 1) {
     lo = fmin(lo, __shfl_xor(lo, off));
     hi = fmax(hi, __shfl_xor(hi, off));
   }
+  if (t % QNB_WAVE == 0) ends[0][which] = lo, ends[1][which] = hi;
+  __syncthreads();
   if (t == 0) {
-    wmin[i] = lo;
-    wmax[i] = hi;
+    wmin[i] = fmin(fmin(ends[0][0], ends[0][1]), fmin(ends[0][2], ends[0][3]));
+    wmax[i] = fmax(fmax(ends[1][0], ends[1][1]), fmax(ends[1][2], ends[1][3]));
   }
 }
 
-// dG chain and the overall gap range (sequential over windows)
-__global__ void k_fep_chain(int n, const double* dgf, const double* dgr, const double* wmin, const double* wmax,
-                            double* dG, double* range) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  dG[0] = 0.0;
-  for (int i = 1; i < n; i++) dG[i] = dG[i - 1] + 0.5 * (dgf[i - 1] - dgr[i]);
-  double lo = wmin[0], hi = wmax[0];
-  for (int i = 1; i < n; i++) {
-    lo = fmin(lo, wmin[i]);
-    hi = fmax(hi, wmax[i]);
+// dG chain and the overall gap range, one wave: the windows' values are read
+// 64 at a time, and lane 0 adds them up in order
+__global__ __launch_bounds__(64) void k_fep_chain(int n, const double* dgf, const double* dgr, const double* wmin,
+                                                  const double* wmax, double* dG, double* range) {
+  const int lane = threadIdx.x;
+  double lo = INFINITY, hi = -INFINITY, g = 0.0;
+  for (int i0 = 0; i0 < n; i0 += QNB_WAVE) {
+    const int i = i0 + lane;
+    double step = 0.0;
+    if (i < n) {
+      if (i > 0) step = 0.5 * (dgf[i - 1] - dgr[i]);
+      lo = fmin(lo, wmin[i]);
+      hi = fmax(hi, wmax[i]);
+    }
+    double mine = 0.0;
+    for (int k = 0; k < min(QNB_WAVE, n - i0); k++) {
+      if (i0 + k > 0) g = g + lane_value(step, k);
+      if (lane == k) mine = g;
+    }
+    if (i < n) dG[i] = mine;
   }
-  range[0] = lo;
-  range[1] = hi;
+  for (int off = 32; off > 0; off >>= 1) {
+    lo = fmin(lo, __shfl_xor(lo, off));
+    hi = fmax(hi, __shfl_xor(hi, off));
+  }
+  if (lane == 0) {
+    range[0] = lo;
+    range[1] = hi;
+  }
 }
 
-// Part 2 of window blockIdx.x: thread t owns bins t, t + blockDim.x, ...
-// and takes the window's frames in order for each of its bins.  Per (window,
-// bin) rec[] holds dGg, c1, c2, r, then dGv of each state; npts the points.
+// Part 2 of window blockIdx.x: thread t owns bin t of a tile of 256 bins and
+// takes the window's frames in order.  FB_CH frames at a time are formed by all
+// threads into LDS, with the frames of each bin as one bit mask per 64 frames
+// (lanes that hold the same bin, by ballots over the bits of its number); a
+// bin's thread then walks its masks.  A thread that formed every frame itself
+// to find its own took 2,040 us at 51 windows of 1,000 frames and 50 bins; 64
+// us now, the length of the walks.  Per (window, bin) rec[] holds dGg, c1, c2,
+// r, then dGv of each state; npts the points.  Two states (fep_params).
 #define FEP_REC (4 + QNB_MAX_STATES)
-__global__ __launch_bounds__(256) void k_fep_bins(const FepWin* __restrict__ wins, FepPar P, const double* dG,
-                                                  const double* range, double* rec, int* npts) {
-  const int i = blockIdx.x;
+#define FB_CH 512
+#define FB_BINS 256
+struct FepBinLds {
+  double val[6][FB_CH];
+  uint64_t frames[FB_CH / QNB_WAVE][FB_BINS];
+  double av[3][FB_BINS];
+};
+// adds the N staged values of bin t's frames, in order; clears the masks
+template <int N>
+__device__ __forceinline__ int fep_bin_walk(FepBinLds& L, int t, double (&s)[N]) {
+  int cnt = 0;
+  for (int g = 0; g < FB_CH / QNB_WAVE; g++) {
+    uint64_t m = L.frames[g][t];
+    if (m == 0) continue;
+    L.frames[g][t] = 0;
+    cnt += __popcll(m);
+    while (m != 0) {
+      const int f = g * QNB_WAVE + __ffsll((long long)m) - 1;
+      m &= m - 1;
+#pragma unroll
+      for (int c = 0; c < N; c++) s[c] = s[c] + L.val[c][f];
+    }
+  }
+  return cnt;
+}
+__global__ __launch_bounds__(FB_BINS) void k_fep_bins(const FepWin* __restrict__ wins, FepPar P, const double* dG,
+                                                      const double* range, double* rec, int* npts) {
+  const int i = blockIdx.x, t = threadIdx.x, lane = t % QNB_WAVE;
   const FepWin& W = wins[i];
   const int ns = P.ns;
   const double gapmin = range[0];
   const double xint = (range[1] - range[0]) / (double)P.nbins;
-  double v[QNB_MAX_STATES], vg, c1, gap, r;
-  for (int k = threadIdx.x; k < P.nbins; k += blockDim.x) {
+  __shared__ FepBinLds L;
+  for (int g = 0; g < FB_CH / QNB_WAVE; g++) L.frames[g][t] = 0;
+  for (int k0 = 0; k0 < P.nbins; k0 += FB_BINS) {
+    const int k = k0 + t, nk = min(FB_BINS, P.nbins - k0);
+    // the frames from f0 on into LDS: sums = false, the values to average;
+    // true, the exponentials about the averages
+    auto stage = [&](int f0, bool sums) {
+      for (int u = t; u < FB_CH; u += FB_BINS) {
+        const int f = f0 + u;
+        double v[QNB_MAX_STATES], vg, c1, gap, r;
+        int b = -1;
+        if (f < W.nf) {
+          fep_frame(W, P, f, v, vg, c1, gap, r);
+          const int bin = (int)((gap - gapmin) / xint);
+          if (bin >= k0 && bin < k0 + nk) b = bin - k0;
+        }
+        uint64_t same = __ballot(b >= 0);
+        for (int bit = 1; bit < nk; bit <<= 1) {
+          const uint64_t m = __ballot(b & bit);
+          same &= (b & bit) ? m : ~m;
+        }
+        if (b >= 0) {
+          if ((same & ((1ull << lane) - 1ull)) == 0) L.frames[u / QNB_WAVE][b] = same;
+          const double veff = veff_of(W.lam, v, ns);
+          if (sums) {
+            for (int s = 0; s < 2; s++) L.val[s][u] = exp(-(v[s] - veff - L.av[s][b]) / P.kT);
+            L.val[2][u] = exp(-(vg - veff - L.av[2][b]) / P.kT);
+          } else {
+            for (int s = 0; s < 2; s++) L.val[s][u] = v[s] - veff;
+            L.val[2][u] = vg - veff;
+            L.val[3][u] = c1;
+            L.val[4][u] = r;
+            L.val[5][u] = W.noffd > 0 ? 1.0 - c1 : 0.0;
+          }
+        }
+      }
+    };
+    // per bin: V_s - eps, E_g - eps, c1, r, c2
+    double av[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0}, sum[3] = {0.0, 0.0, 0.0};
     int cnt = 0;
-    double avdvv[QNB_MAX_STATES], sumv[QNB_MAX_STATES];
-    for (int s = 0; s < QNB_MAX_STATES; s++) avdvv[s] = sumv[s] = 0.0;
-    double avdvg = 0.0, avc1 = 0.0, avc2 = 0.0, avr = 0.0, sumg = 0.0;
-    for (int f = P.nskip; f < W.nf; f++) {
-      fep_frame(W, P, f, v, vg, c1, gap, r);
-      if ((int)((gap - gapmin) / xint) != k) continue;
-      const double veff = veff_of(W.lam, v, ns);
-      for (int s = 0; s < ns; s++) avdvv[s] = avdvv[s] + (v[s] - veff);
-      avdvg = avdvg + (vg - veff);
-      avc1 = avc1 + c1;
-      avc2 = avc2 + (W.noffd > 0 ? 1.0 - c1 : 0.0);
-      avr = avr + r;
-      cnt++;
+    for (int f0 = P.nskip; f0 < W.nf; f0 += FB_CH) {
+      __syncthreads();
+      stage(f0, false);
+      __syncthreads();
+      if (t < nk) cnt += fep_bin_walk(L, t, av);
     }
-    if (cnt != 0) {
-      avc1 = avc1 / (double)cnt;
-      avc2 = avc2 / (double)cnt;
-      avr = avr / (double)cnt;
-      for (int s = 0; s < ns; s++) avdvv[s] = avdvv[s] / (double)cnt;
-      avdvg = avdvg / (double)cnt;
+    if (cnt != 0)
+      for (int c = 0; c < 6; c++) av[c] = av[c] / (double)cnt;
+    for (int c = 0; c < 3; c++) L.av[c][t] = av[c];
+    for (int f0 = P.nskip; f0 < W.nf; f0 += FB_CH) {
+      __syncthreads();
+      stage(f0, true);
+      __syncthreads();
+      if (t < nk) fep_bin_walk(L, t, sum);
     }
-    for (int f = P.nskip; f < W.nf && cnt > 0; f++) {
-      fep_frame(W, P, f, v, vg, c1, gap, r);
-      if ((int)((gap - gapmin) / xint) != k) continue;
-      const double veff = veff_of(W.lam, v, ns);
-      for (int s = 0; s < ns; s++) sumv[s] = sumv[s] + exp(-(v[s] - veff - avdvv[s]) / P.kT);
-      sumg = sumg + exp(-(vg - veff - avdvg) / P.kT);
-    }
-    double* o = rec + ((size_t)i * P.nbins + k) * FEP_REC;
-    npts[(size_t)i * P.nbins + k] = cnt;
-    if (cnt > 0 && cnt >= P.nmin) {
-      for (int s = 0; s < ns; s++) o[4 + s] = dG[i] + (-P.kT * log(sumv[s] / (double)cnt) + avdvv[s]);
-      o[0] = dG[i] + (-P.kT * log(sumg / (double)cnt) + avdvg);
-      o[1] = avc1;
-      o[2] = avc2;
-      o[3] = avr;
-    } else {
-      for (int z = 0; z < FEP_REC; z++) o[z] = NAN;
+    if (t < nk) {
+      double* o = rec + ((size_t)i * P.nbins + k) * FEP_REC;
+      npts[(size_t)i * P.nbins + k] = cnt;
+      if (cnt > 0 && cnt >= P.nmin) {
+        for (int s = 0; s < 2; s++) o[4 + s] = dG[i] + (-P.kT * log(sum[s] / (double)cnt) + av[s]);
+        o[0] = dG[i] + (-P.kT * log(sum[2] / (double)cnt) + av[2]);
+        o[1] = av[3];
+        o[2] = av[5];
+        o[3] = av[4];
+      } else {
+        for (int z = 0; z < FEP_REC; z++) o[z] = NAN;
+      }
     }
   }
 }
 
-// Part 3: per bin, the windows in order
+// Part 3: per bin, the windows in order, FP3_U of them requested at a time
+#define FP3_U 8
 __global__ __launch_bounds__(256) void k_fep_part3(int n, FepPar P, const double* rec, const int* npts, double* bins,
                                                    int* ptsum) {
   for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < P.nbins; k += gridDim.x * blockDim.x) {
-    double b1 = 0.0, b2 = 0.0, b3 = 0.0, b4 = 0.0;
+    double b[4] = {0.0, 0.0, 0.0, 0.0};
     int pt = 0;
-    for (int i = 0; i < n; i++) {
-      const int c = npts[(size_t)i * P.nbins + k];
-      if (c == 0 || c < P.nmin) continue;
-      const double* o = rec + ((size_t)i * P.nbins + k) * FEP_REC;
-      b2 = b2 + o[1] * (double)c;
-      b3 = b3 + o[2] * (double)c;
-      b4 = b4 + o[3] * (double)c;
-      pt += c;
-      b1 = b1 + o[0] * (double)c;
+    for (int i0 = 0; i0 < n; i0 += FP3_U) {
+      int c[FP3_U];
+      double o[FP3_U][4];
+#pragma unroll
+      for (int u = 0; u < FP3_U; u++) {
+        const size_t w = (size_t)min(i0 + u, n - 1) * P.nbins + k;
+        c[u] = i0 + u < n ? npts[w] : 0;
+        for (int z = 0; z < 4; z++) o[u][z] = rec[w * FEP_REC + z];
+      }
+#pragma unroll
+      for (int u = 0; u < FP3_U; u++) {
+        if (c[u] == 0 || c[u] < P.nmin) continue;
+        pt += c[u];
+        for (int z = 0; z < 4; z++) b[z] = b[z] + o[u][z] * (double)c[u];
+      }
     }
     ptsum[k] = pt;
     const bool ok = pt > 0 && pt >= P.nmin;
-    bins[4 * k + 0] = ok ? b1 / (double)pt : NAN;
-    bins[4 * k + 1] = ok ? b2 / (double)pt : NAN;
-    bins[4 * k + 2] = ok ? b3 / (double)pt : NAN;
-    bins[4 * k + 3] = ok ? b4 / (double)pt : NAN;
+    for (int z = 0; z < 4; z++) bins[4 * k + z] = ok ? b[z] / (double)pt : NAN;
   }
 }
 
@@ -230,7 +324,7 @@ void launch_fep_part1(hipStream_t st, const FepWin* wins, int n, const FepPar& P
   size_t off[8];
   fep_layout(n, P.nbins, off);
   double* sd = scratch;
-  hipLaunchKernelGGL(k_fep_window, dim3(n), dim3(64), 0, st, wins, n, P, sd + off[0], sd + off[1], sd + off[3],
+  hipLaunchKernelGGL(k_fep_window, dim3(n), dim3(256), 0, st, wins, n, P, sd + off[0], sd + off[1], sd + off[3],
                      sd + off[3] + n);
   hipLaunchKernelGGL(k_fep_chain, dim3(1), dim3(64), 0, st, n, sd + off[0], sd + off[1], sd + off[3], sd + off[3] + n,
                      sd + off[2], sd + off[4]);
@@ -242,7 +336,7 @@ void launch_fep_bins(hipStream_t st, const FepWin* wins, int n, const FepPar& P,
   fep_layout(n, P.nbins, off);
   double* sd = scratch;
   int* npts = reinterpret_cast<int*>(sd + off[7]);
-  hipLaunchKernelGGL(k_fep_bins, dim3(n), dim3(256), 0, st, wins, P, sd + off[2], sd + off[4], sd + off[5], npts);
+  hipLaunchKernelGGL(k_fep_bins, dim3(n), dim3(FB_BINS), 0, st, wins, P, sd + off[2], sd + off[4], sd + off[5], npts);
   hipLaunchKernelGGL(k_fep_part3, dim3((P.nbins + 255) / 256), dim3(256), 0, st, n, P, sd + off[5], npts, sd + off[6],
                      npts + (size_t)n * P.nbins);
 }
