@@ -17,145 +17,187 @@
 
 namespace qnb {
 
-template <typename R, int NS>
-__device__ __forceinline__ void adj_pair(double (&g)[NS][QNB_ADJ_NV], int s, R r2, R r, R r6in, R A, R B, R el,
-                                         R sc, R tq, R tA, R tB, bool is14, bool lj, bool energy) {
-  R Vel = el * r;
-  R rq = tq * r;
+// one pair's parameters in one state: LJ and Coulomb, soft core, tangents
+template <typename R>
+struct AdjPar {
+  R A, B, el, sc, tq, tA, tB;
+};
+
+template <typename R>
+__device__ __forceinline__ void adj_pair(double (&g)[QNB_ADJ_NV], R r2, R r, const AdjPar<R>& p, bool is14, bool lj,
+                                         bool energy) {
   double e_vdw = 0.0, gA = 0.0, gB = 0.0;
   if (lj) {
-    R r6_hc = recip(r6in);
-    R r6 = recip(r6_hc + sc);
-    R r12 = r6 * r6;
-    R Va = A * r12, Vb = B * r6;
-    e_vdw = (double)Va - (double)Vb;
-    gA = (double)(tA * r12);
-    gB = -(double)(tB * r6);
+    R r6 = r2 * r2 * r2;
+    if (p.sc != R(0)) r6 = recip(recip(r6) + p.sc);
+    const R r12 = r6 * r6;
+    e_vdw = (double)(p.A * r12) - (double)(p.B * r6);
+    gA = (double)(p.tA * r12);
+    gB = -(double)(p.tB * r6);
   }
-#pragma unroll
-  for (int k = 0; k < NS; k++)
-    if (k == s) {
-      g[k][ADJ_DQ] += (double)rq;
-      g[k][is14 ? ADJ_DA14 : ADJ_DA] += gA;
-      g[k][is14 ? ADJ_DB14 : ADJ_DB] += gB;
-      if (energy) {
-        g[k][ADJ_EEL] += (double)Vel;
-        g[k][ADJ_EVDW] += e_vdw;
-      }
-    }
+  g[ADJ_DQ] += (double)(p.tq * r);
+  g[ADJ_DA] += is14 ? 0.0 : gA;
+  g[ADJ_DB] += is14 ? 0.0 : gB;
+  g[ADJ_DA14] += is14 ? gA : 0.0;
+  g[ADJ_DB14] += is14 ? gB : 0.0;
+  if (energy) {
+    g[ADJ_EEL] += (double)(p.el * r);
+    g[ADJ_EVDW] += e_vdw;
+  }
 }
 
-// one wavefront per (frame, Q-atom); grid.y = instance
+// One block per (frame, Q-atom), its four waves taking every fourth 64 waters,
+// solute atoms and Q pairs; grid.y = instance.  A wave's pass is a few dozen
+// iterations of dependent loads, so the kernel is bound by their latency until
+// the waves fill the chip: four waves per sum instead of one, the Q-water
+// tables of a site held over the waters, and each solute atom's list test from
+// its own word (qp_test) instead of through group, switch atom and exclusion
+// take 6 instances x 20 frames x 30 Q-atoms of 1,200 + 3,100 atoms from 175 to
+// 158 us (FP32 pairs), 24 frames x 18 Q-atoms from 50 to 20 us (FP64).
+#define ADJ_WPB 4
 template <typename R, int NS>
-__global__ __launch_bounds__(256) void k_adjoint(const DevSys* __restrict__ systems, const AdjDev* __restrict__ adjs) {
+__global__ __launch_bounds__(QNB_WAVE* ADJ_WPB) void k_adjoint(const DevSys* __restrict__ systems,
+                                                               const AdjDev* __restrict__ adjs) {
   const DevSys& S = systems[blockIdx.y];
   const AdjDev& A = adjs[blockIdx.y];
   const int nq = S.nqat, ns = S.nstates, sa = S.sa, nsol = S.nat_solute;
   if (nq <= 0) return;
-  const int wv = blockIdx.x * (blockDim.x / QNB_WAVE) + threadIdx.x / QNB_WAVE;
-  const int lane = threadIdx.x % QNB_WAVE;
-  const int f = wv / nq, iq = wv % nq;
+  const int t0 = threadIdx.x, lane = t0 % QNB_WAVE;
+  const int f = blockIdx.x / nq, iq = blockIdx.x % nq;
   if (f >= A.nframes) return;
-  const double* __restrict__ x = A.frames + (size_t)f * 3 * S.natom;
+  const auto x = gp(A.frames + (size_t)f * 3 * S.natom);
   const int i = S.iqseq[iq];
   const double xi0 = x[3 * i], xi1 = x[3 * i + 1], xi2 = x[3 * i + 2];
+  const double xp0 = S.xp[0], xp1 = S.xp[1], xp2 = S.xp[2], rcq2 = S.rcq2;
   double g[NS][QNB_ADJ_NV];
 #pragma unroll
   for (int s = 0; s < NS; s++)
 #pragma unroll
     for (int c = 0; c < QNB_ADJ_NV; c++) g[s][c] = 0.0;
+  auto inv = [&](double ax, double ay, double az, double bx, double by, double bz, R& r2, R& r) {
+    const R ux = (R)(ax - bx), uy = (R)(ay - by), uz = (R)(az - bz);
+    rinv(ux * ux + uy * uy + uz * uz, r2, r);
+  };
+  // dist4p's sum for the point (a, b, c) and the Q-list centre
+  auto inside = [&](double a, double b, double c) {
+#pragma clang fp contract(off)
+    const double dx = xp0 - a, dy = xp1 - b, dz = xp2 - c;
+    double d = dx * dx;
+    d = d + dy * dy;
+    d = d + dz * dz;
+    return d <= rcq2;
+  };
 
   // Q-water: every water whose oxygen lies within Rcq of the Q-list centre
-  for (int w = lane; w < S.nwat; w += QNB_WAVE) {
-    const int o = nsol + sa * w;
-    if (S.excl[o] || dist4p(x, o, S.xp) > S.rcq2) continue;
-    for (int k = 0; k < sa; k++) {
-      const int j = o + k;
-      const R ux = (R)(x[3 * j] - xi0), uy = (R)(x[3 * j + 1] - xi1), uz = (R)(x[3 * j + 2] - xi2);
+  for (int k = 0; k < sa; k++) {
+    AdjPar<R> p[NS];
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+      if (s >= ns || S.nwat <= 0) break;
+      const size_t t = (size_t)iq + (size_t)nq * ((size_t)k + (size_t)sa * s);
+      p[s] = AdjPar<R>{(R)S.qwA[t], (R)S.qwB[t], (R)S.qwEl[t], (R)S.qwSc[t],
+                       (R)A.qw_dq[t], (R)A.qw_dA[t], (R)A.qw_dB[t]};
+    }
+    const bool lj = k == 0 || !S.spc;
+#pragma unroll 2
+    for (int w = t0; w < S.nwat; w += QNB_WAVE * ADJ_WPB) {
+      const int o = nsol + sa * w, j = o + k;
+      const double ox = x[3 * o], oy = x[3 * o + 1], oz = x[3 * o + 2];
+      const double jx = x[3 * j], jy = x[3 * j + 1], jz = x[3 * j + 2];
+      if (ldg(S.excl + o) || !inside(ox, oy, oz)) continue;
       R r2, r;
-      rinv(ux * ux + uy * uy + uz * uz, r2, r);
-      const R r6in = r2 * r2 * r2;
-      const bool lj = k == 0 || !S.spc;
+      inv(jx, jy, jz, xi0, xi1, xi2, r2, r);
 #pragma unroll
       for (int s = 0; s < NS; s++) {
         if (s >= ns) break;
-        const size_t t = (size_t)iq + (size_t)nq * ((size_t)k + (size_t)sa * s);
-        adj_pair<R, NS>(g, s, r2, r, r6in, (R)S.qwA[t], (R)S.qwB[t], (R)S.qwEl[t], (R)S.qwSc[t], (R)A.qw_dq[t],
-                        (R)A.qw_dA[t], (R)A.qw_dB[t], false, lj, true);
+        adj_pair<R>(g[s], r2, r, p[s], false, lj, true);
       }
     }
   }
+  // the Q tables' entry t of the Q-solute pairs
+  auto qp_par = [&](size_t t) {
+    return AdjPar<R>{(R)ldg(S.qpA + t), (R)ldg(S.qpB + t), (R)ldg(S.qpEl + t), (R)ldg(S.qpSc + t),
+                     (R)ldg(A.qp_dq + t), (R)ldg(A.qp_dA + t), (R)ldg(A.qp_dB + t)};
+  };
   // Q-solute: atoms of solute groups inside Rcq (switch atom, or any atom
   // with iuse_switch_atom = 0), not 1-2/1-3 bonded to any Q-atom
-  for (int j = lane; j < nsol; j += QNB_WAVE) {
-    if (S.qconn3[j] || S.atom_group[j] < 0) continue;
-    if (!qp_group_in(S, x, S.atom_group[j])) continue;
-    const R ux = (R)(x[3 * j] - xi0), uy = (R)(x[3 * j + 1] - xi1), uz = (R)(x[3 * j + 2] - xi2);
+#pragma unroll 2
+  for (int j = t0; j < nsol; j += QNB_WAVE * ADJ_WPB) {
+    const int sw = ldg(S.qp_test + j);
+    if (sw < 0) continue;
+    if (S.any_atom) {
+      if (!qp_group_in(S, A.frames + (size_t)f * 3 * S.natom, ldg(S.atom_group + j))) continue;
+    } else if (!inside(x[3 * sw], x[3 * sw + 1], x[3 * sw + 2])) {
+      continue;
+    }
     R r2, r;
-    rinv(ux * ux + uy * uy + uz * uz, r2, r);
-    const R r6in = r2 * r2 * r2;
+    inv(x[3 * j], x[3 * j + 1], x[3 * j + 2], xi0, xi1, xi2, r2, r);
 #pragma unroll
     for (int s = 0; s < NS; s++) {
       if (s >= ns) break;
       const size_t t = (size_t)j + (size_t)nsol * ((size_t)iq + (size_t)nq * s);
-      adj_pair<R, NS>(g, s, r2, r, r6in, (R)S.qpA[t], (R)S.qpB[t], (R)S.qpEl[t], (R)S.qpSc[t], (R)A.qp_dq[t],
-                      (R)A.qp_dA[t], (R)A.qp_dB[t], A.qp_is14[t] != 0, true, true);
+      adj_pair<R>(g[s], r2, r, qp_par(t), ldg(A.qp_is14 + t) != 0, true, true);
     }
   }
   // Q-Q pairs with iq as either member; the energy is counted by the lower one
-  for (int p = lane; p < S.nqq; p += QNB_WAVE) {
-    const int ia = S.qq_iq[p], ja = S.qq_jq[p];
+  for (int q = t0; q < S.nqq; q += QNB_WAVE * ADJ_WPB) {
+    const int ia = S.qq_iq[q], ja = S.qq_jq[q];
     if (ia != iq && ja != iq) continue;
-    const int st = S.qq_st[p];
+    const int st = S.qq_st[q];
     const int a = S.iqseq[ia], b = S.iqseq[ja];
-    const R ux = (R)(x[3 * b] - x[3 * a]), uy = (R)(x[3 * b + 1] - x[3 * a + 1]), uz = (R)(x[3 * b + 2] - x[3 * a + 2]);
     R r2, r;
-    rinv(ux * ux + uy * uy + uz * uz, r2, r);
-    const double* pr = S.qq_par + 4 * p;
+    inv(x[3 * b], x[3 * b + 1], x[3 * b + 2], x[3 * a], x[3 * a + 1], x[3 * a + 2], r2, r);
+    const double* pr = S.qq_par + 4 * q;
     const size_t t = (size_t)ia + (size_t)nq * ((size_t)ja + (size_t)nq * st);
     const bool mine = ia == iq;
     const R tq = (R)(mine ? A.qq_dq_i[t] : A.qq_dq_j[t]);
-    if (S.qq_soft[p]) {
-      // exponential soft pair: its A, B are not LJ factors (no LJ tangent)
-      R Vel = (R)pr[2] * r;
-      R Va = (R)pr[0] * exp(-(R)pr[1] / r);
+    const bool soft = S.qq_soft[q], is14 = A.qq_is14[t] != 0;
+    const R tA = (R)(mine ? A.qq_dA_i[t] : A.qq_dA_j[t]);
+    const R tB = (R)(mine ? A.qq_dB_i[t] : A.qq_dB_j[t]);
 #pragma unroll
-      for (int k = 0; k < NS; k++)
-        if (k == st) {
-          g[k][ADJ_DQ] += (double)(tq * r);
-          if (mine) {
-            g[k][ADJ_EEL] += (double)Vel;
-            g[k][ADJ_EVDW] += (double)Va;
-          }
+    for (int k = 0; k < NS; k++) {
+      if (k != st) continue;
+      if (soft) {
+        // exponential soft pair: its A, B are not LJ factors (no LJ tangent)
+        g[k][ADJ_DQ] += (double)(tq * r);
+        if (mine) {
+          g[k][ADJ_EEL] += (double)((R)pr[2] * r);
+          g[k][ADJ_EVDW] += (double)((R)pr[0] * exp(-(R)pr[1] / r));
         }
-    } else {
-      const R tA = (R)(mine ? A.qq_dA_i[t] : A.qq_dA_j[t]);
-      const R tB = (R)(mine ? A.qq_dB_i[t] : A.qq_dB_j[t]);
-      adj_pair<R, NS>(g, st, r2, r, r2 * r2 * r2, (R)pr[0], (R)pr[1], (R)pr[2], (R)pr[3], tq, tA, tB,
-                      A.qq_is14[t] != 0, true, mine);
+      } else {
+        adj_pair<R>(g[k], r2, r, AdjPar<R>{(R)pr[0], (R)pr[1], (R)pr[2], (R)pr[3], tq, tA, tB}, is14, true, mine);
+      }
     }
   }
   // Q-bonded-neighbour pairs of iq (entries of the qp tables)
-  for (int p = lane; p < S.nqqp; p += QNB_WAVE) {
-    if (S.qqp_iq[p] != iq) continue;
-    const int j = S.qqp_j[p], st = S.qqp_st[p];
-    const R ux = (R)(x[3 * j] - xi0), uy = (R)(x[3 * j + 1] - xi1), uz = (R)(x[3 * j + 2] - xi2);
+  for (int q = t0; q < S.nqqp; q += QNB_WAVE * ADJ_WPB) {
+    if (S.qqp_iq[q] != iq) continue;
+    const int j = S.qqp_j[q], st = S.qqp_st[q];
     R r2, r;
-    rinv(ux * ux + uy * uy + uz * uz, r2, r);
-    const double* pr = S.qqp_par + 4 * p;
+    inv(x[3 * j], x[3 * j + 1], x[3 * j + 2], xi0, xi1, xi2, r2, r);
+    const double* pr = S.qqp_par + 4 * q;
     const size_t t = (size_t)j + (size_t)nsol * ((size_t)iq + (size_t)nq * st);
-    adj_pair<R, NS>(g, st, r2, r, r2 * r2 * r2, (R)pr[0], (R)pr[1], (R)pr[2], (R)pr[3], (R)A.qp_dq[t],
-                    (R)A.qp_dA[t], (R)A.qp_dB[t], A.qp_is14[t] != 0, true, true);
+    const AdjPar<R> p{(R)pr[0], (R)pr[1], (R)pr[2], (R)pr[3], (R)A.qp_dq[t], (R)A.qp_dA[t], (R)A.qp_dB[t]};
+#pragma unroll
+    for (int k = 0; k < NS; k++)
+      if (k == st) adj_pair<R>(g[k], r2, r, p, A.qp_is14[t] != 0, true, true);
   }
-  double* out = A.out + (size_t)f * ns * nq * QNB_ADJ_NV;
+  // the block's sums, in wave order
+  constexpr int NV = NS * QNB_ADJ_NV;
+  __shared__ double part[ADJ_WPB][64];
+  double v[NV];
 #pragma unroll
-  for (int s = 0; s < NS; s++) {
-    if (s >= ns) break;
+  for (int s = 0; s < NS; s++)
 #pragma unroll
-    for (int c = 0; c < QNB_ADJ_NV; c++) {
-      const double v = wave_sum(g[s][c]);
-      if (lane == 0) out[((size_t)s * nq + iq) * QNB_ADJ_NV + c] = v;
-    }
+    for (int c = 0; c < QNB_ADJ_NV; c++) v[s * QNB_ADJ_NV + c] = g[s][c];
+  const double sum = wave_sum_tr<double, NV>(v, lane);
+  if (wave_sum_tr_writer<NV>(lane)) part[t0 / QNB_WAVE][wave_sum_tr_index<NV>(lane)] = sum;
+  __syncthreads();
+  if (t0 < ns * QNB_ADJ_NV) {
+    const int s = t0 / QNB_ADJ_NV, c = t0 % QNB_ADJ_NV;
+    double e = part[0][t0];
+    for (int w = 1; w < ADJ_WPB; w++) e += part[w][t0];
+    A.out[(((size_t)f * ns + s) * nq + iq) * QNB_ADJ_NV + c] = e;
   }
 }
 
@@ -189,20 +231,19 @@ int adjoint_upload(DevAlloc& M, const DevSys& S, const qnb_qtangent* t, AdjDev& 
 }
 
 template <typename R>
-static void launch_adj_r(hipStream_t st, int ns_max, int waves, int B, const DevSys* dsys, const AdjDev* dadj) {
-  const int wpb = 4;
-  dim3 grid((waves + wpb - 1) / wpb, B), block(QNB_WAVE * wpb);
+static void launch_adj_r(hipStream_t st, int ns_max, int blocks, int B, const DevSys* dsys, const AdjDev* dadj) {
+  dim3 grid(blocks, B), block(QNB_WAVE * ADJ_WPB);
   if (ns_max <= 1) hipLaunchKernelGGL((k_adjoint<R, 1>), grid, block, 0, st, dsys, dadj);
   else if (ns_max <= 2) hipLaunchKernelGGL((k_adjoint<R, 2>), grid, block, 0, st, dsys, dadj);
   else if (ns_max <= 4) hipLaunchKernelGGL((k_adjoint<R, 4>), grid, block, 0, st, dsys, dadj);
   else hipLaunchKernelGGL((k_adjoint<R, 8>), grid, block, 0, st, dsys, dadj);
 }
 
-// waves = max over instances of nframes * nqat
-void launch_adjoint(hipStream_t st, int prec, int ns_max, long waves, int B, const DevSys* dsys, const AdjDev* dadj) {
-  if (waves <= 0 || B <= 0) return;
-  if (prec == QNB_PREC_MIXED) launch_adj_r<float>(st, ns_max, (int)waves, B, dsys, dadj);
-  else launch_adj_r<double>(st, ns_max, (int)waves, B, dsys, dadj);
+// blocks = max over instances of nframes * nqat
+void launch_adjoint(hipStream_t st, int prec, int ns_max, long blocks, int B, const DevSys* dsys, const AdjDev* dadj) {
+  if (blocks <= 0 || B <= 0) return;
+  if (prec == QNB_PREC_MIXED) launch_adj_r<float>(st, ns_max, (int)blocks, B, dsys, dadj);
+  else launch_adj_r<double>(st, ns_max, (int)blocks, B, dsys, dadj);
 }
 
 }  // namespace qnb

@@ -367,6 +367,12 @@ int topo_build(DevSys& S, const qnb_system* s, HostTopo& T, DevAlloc& M) {
     }
   }
   UP(qconn3, T.qconn3.data(), T.qconn3.size());
+  std::vector<int> qp_test(nsol1, -1);
+  for (int i = 0; i < nsol; i++) {
+    const int g = atom_group[i];
+    if (!T.qconn3[i] && g >= 0 && !s->excl[s->cgp_iswitch[g]]) qp_test[i] = s->cgp_iswitch[g];
+  }
+  UP(qp_test, qp_test.data(), qp_test.size());
   if (nq > 0) {
     UP(iqseq, s->iqseq, nq);
     if (nsol > 0) {

@@ -109,6 +109,10 @@ struct DevSys {
   const double* sint_par;
   const int* iqseq;
   const uint8_t* qconn3;
+  // per solute atom: the switch atom that decides whether its group is on the
+  // Q-solute list, or -1 where no group test can put it there (within two
+  // bonds of a Q-atom, in no group, excluded switch atom)
+  const int* qp_test;
   const double* qpA;  // [i + nsol*(iq + nq*s)]
   const double* qpB;
   const double* qpEl;

@@ -128,7 +128,7 @@ int fep_run(hipStream_t st, const std::vector<FepWin>& hw, const FepPar& P, qnb_
 
 // adjoint of the Q-atom energies: tangent upload and launch over frames
 int adjoint_upload(DevAlloc& M, const DevSys& S, const qnb_qtangent* t, AdjDev& A);
-void launch_adjoint(hipStream_t st, int prec, int ns_max, long waves, int B, const DevSys* dsys, const AdjDev* dadj);
+void launch_adjoint(hipStream_t st, int prec, int ns_max, long blocks, int B, const DevSys* dsys, const AdjDev* dadj);
 // Q-atom bonded terms: validation and device copies (buffers recorded in
 // `owned` so a later set can release them), and the per-instance launch
 int qbonded_build(const qnb_qbonded* q, int nstates, int natom, const double* lambda, DevAlloc& M,
