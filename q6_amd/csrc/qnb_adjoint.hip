@@ -201,16 +201,16 @@ __global__ __launch_bounds__(QNB_WAVE* ADJ_WPB) void k_adjoint(const DevSys* __r
   }
 }
 
-// Copies a caller's tangent tables to the device (sizes from the system).
-int adjoint_upload(DevAlloc& M, const DevSys& S, const qnb_qtangent* t, AdjDev& A) {
+// Adds a caller's tangent tables to a pack (sizes from the system); A, whose
+// pointers the pack sets, and the tables stay in place until it is copied.
+int adjoint_pack(DevPack& M, const DevSys& S, const qnb_qtangent* t, AdjDev& A) {
   if (!t) return fail(QNB_EINVAL, "null tangent tables");
   const size_t nq = S.nqat, ns = S.nstates, nsol = S.nat_solute, sa = S.sa;
   const size_t np = nsol * nq * ns, nw = S.nwat > 0 ? nq * sa * ns : 0, nqq = nq * nq * ns;
-  int rc = 0;
 #define UPT(field, n)                                                                     \
   do {                                                                                    \
     if ((n) > 0 && !t->field) return fail(QNB_EINVAL, "tangent table " #field " missing"); \
-    if ((rc = M.upload(&A.field, t->field, (n)))) return rc;                              \
+    M.add(&A.field, (n) > 0 ? t->field : nullptr, (n));                                   \
   } while (0)
   UPT(qp_dq, np);
   UPT(qp_dA, np);

@@ -927,23 +927,29 @@ extern "C" int32_t qnb_adjoint(qnb_handle* h, const qnb_qtangent* tan, int32_t n
   const DevSys& S = h->hs;
   if (S.nqat <= 0 || nframes == 0) return 0;
   DevAlloc tmp;
+  DevPack pack;
   AdjDev A{};
-  int rc = adjoint_upload(tmp, S, tan, A);
-  if (rc) return rc;
-  const int chunk = 256;
+  const int chunk = 256, most = std::min(nframes, chunk);
   const size_t fl = 3 * (size_t)S.natom, ol = (size_t)S.nstates * S.nqat * QNB_ADJ_NV;
   double *dfr = nullptr, *dout = nullptr;
-  AdjDev* dadj = nullptr;
-  if ((rc = tmp.alloc(&dfr, fl * std::min(nframes, chunk)))) return rc;
-  if ((rc = tmp.alloc(&dout, ol * std::min(nframes, chunk)))) return rc;
-  if ((rc = tmp.alloc(&dadj, 1))) return rc;
+  const AdjDev* dadj = nullptr;
+  int rc = adjoint_pack(pack, S, tan, A);
+  if (rc) return rc;
+  pack.add(&dadj, &A, 1);
+  pack.space(&dfr, fl * most);
+  pack.space(&dout, ol * most);
+  if ((rc = pack.alloc(tmp))) return rc;
+  A.frames = dfr;
+  A.nframes = most;
+  A.out = dout;
+  if ((rc = pack.copy())) return rc;
   for (int f0 = 0; f0 < nframes; f0 += chunk) {
     const int nf = std::min(chunk, nframes - f0);
-    A.frames = dfr;
-    A.nframes = nf;
-    A.out = dout;
     HIPCHK(hipMemcpyAsync(dfr, frames + fl * f0, sizeof(double) * fl * nf, hipMemcpyHostToDevice, h->stream));
-    HIPCHK(hipMemcpyAsync(dadj, &A, sizeof A, hipMemcpyHostToDevice, h->stream));
+    if (nf != A.nframes) {
+      A.nframes = nf;
+      HIPCHK(hipMemcpyAsync((void*)dadj, &A, sizeof A, hipMemcpyHostToDevice, h->stream));
+    }
     launch_adjoint(h->stream, S.prec, S.nstates, (long)nf * S.nqat, 1, h->dsys, dadj);
     HIPCHK(hipGetLastError());
     HIPCHK(hipMemcpyAsync(out + ol * f0, dout, sizeof(double) * ol * nf, hipMemcpyDeviceToHost, h->stream));

@@ -50,7 +50,7 @@ struct MdDev {
   double* xx;
   double* hist;   // [max_frames][QNB_FRAME_LEN]
   double* st;     // [8]: sfact of group 0, Tfree, Temp, Ekin, tfree of groups 0 and 1, sfact of group 1
-  int* ctr;       // [4]: frame, error flags
+  int* ctr;       // [4]: frames, error flags, snapshots, blocks that have integrated (qnb_batch::ctr)
   double* tfree;  // &tfree_all[k]
   int* istep;     // &istep_all[k]
   double* xs;     // [xs_max][natom*3] coordinate snapshots (counter ctr[2])
@@ -495,6 +495,7 @@ __global__ __launch_bounds__(256) void k_record(const DevSys* __restrict__ syste
 
 using namespace qnb;
 
+#define CTR_STRIDE 32  // ints: 128 bytes, one instance's counters to a cache line
 struct qnb_batch {
   int n = 0;
   std::vector<DevSys> hs;
@@ -513,6 +514,7 @@ struct qnb_batch {
   hipGraph_t cycle_graph = nullptr;
   int maxg = 0, maxat = 0, maxsw = 0, maxw = 0, maxs = 0, ns_max = 1, prec = 0;
   int nbblk = 1;  // k_bonded blocks per instance
+  int* ctr = nullptr;  // every instance's counters (MdDev::ctr), CTR_STRIDE apart: read in one copy
   bool anyq = false, anypol = false, static_q = true;
   int qchunks = 1, nq_max = 0, nqe_max = 0, nsol_max = 0;
   long sum_solute = 0, sum_solvent = 0;  // receiver groups of all instances
@@ -759,6 +761,13 @@ static void enqueue_min_step(qnb_batch* b, bool lists, double k0, double max_dis
   hipLaunchKernelGGL(k_shake, dim3((b->maxsw + 255) / 256, B), dim3(256), 0, b->stream, b->dsys, b->dmd);
 }
 
+// the counters of every instance, after the batch stream has been waited for
+static int counters(const qnb_batch* b, std::vector<int>& all) {
+  all.resize(CTR_STRIDE * (size_t)b->n);
+  HIPCHK(hipMemcpy(all.data(), b->ctr, sizeof(int) * all.size(), hipMemcpyDeviceToHost));
+  return 0;
+}
+
 // does MD step `step` sample energies in any instance
 static bool energy_step(const qnb_batch* b, long long step) {
   for (int e : b->ene_every)
@@ -839,6 +848,8 @@ extern "C" int32_t qnb_batch_create(int32_t n, const qnb_system* const* sys, con
   if ((rc = b->mem.alloc(&b->tfree, n)) || (rc = b->mem.alloc(&b->istep, n))) return rc;
   HIPCHK(hipMemset(b->istep, 0, sizeof(int) * n));
   // MD records
+  if ((rc = b->mem.alloc(&b->ctr, CTR_STRIDE * (size_t)n))) return rc;
+  HIPCHK(hipMemset(b->ctr, 0, sizeof(int) * CTR_STRIDE * n));
   for (int k = 0; k < n; k++) {
     const qnb_md_params* m = md[k];
     MdDev& M = b->hm[k];
@@ -882,7 +893,7 @@ extern "C" int32_t qnb_batch_create(int32_t n, const qnb_system* const* sys, con
     if ((rc = b->mem.upload(&M.winv, m->winv, S.natom)) ||
         (rc = b->mem.alloc(&M.v, 3 * (size_t)S.natom)) || (rc = b->mem.alloc(&M.xx, 3 * (size_t)S.natom)) ||
         (rc = b->mem.alloc(&M.hist, (size_t)std::max(m->max_frames, 1) * QNB_FRAME_LEN)) ||
-        (rc = b->mem.alloc(&M.st, 8)) || (rc = b->mem.alloc(&M.ctr, 4)))
+        (rc = b->mem.alloc(&M.st, 8)))
       return rc;
     // atom-centred incidence lists of the bonds and angles (k_bonded)
     if (m->nbonds < 0 || m->nangles < 0 || (m->nbonds > 0 && (!m->bond_ij || !m->bond_r0 || !m->bond_k)) ||
@@ -931,7 +942,7 @@ extern "C" int32_t qnb_batch_create(int32_t n, const qnb_system* const* sys, con
     }
     HIPCHK(hipMemcpy(M.v, v0[k], sizeof(double) * 3 * S.natom, hipMemcpyHostToDevice));
     HIPCHK(hipMemset(M.st, 0, 8 * sizeof(double)));
-    HIPCHK(hipMemset(M.ctr, 0, 4 * sizeof(int)));
+    M.ctr = b->ctr + CTR_STRIDE * k;
     M.tfree = b->tfree + k;
     M.istep = b->istep + k;
     // the nonbonded kernels accumulate energies on the sampled steps only
@@ -1105,9 +1116,10 @@ extern "C" int32_t qnb_batch_thermostat(qnb_batch* b, int32_t k, double* out) {
 extern "C" int32_t qnb_batch_sync(qnb_batch* b) {
   if (!b) return fail(QNB_EINVAL, "null batch");
   HIPCHK(hipStreamSynchronize(b->stream));
+  std::vector<int> all;
+  if (int rc = counters(b, all)) return rc;
   for (int k = 0; k < b->n; k++) {
-    int ctr[4];
-    HIPCHK(hipMemcpy(ctr, b->hm[k].ctr, sizeof ctr, hipMemcpyDeviceToHost));
+    const int* ctr = all.data() + CTR_STRIDE * k;
     if (ctr[1] & ERR_OVERFLOW) return fail(QNB_EOVERFLOW, "instance %d: neighbour list overflow", k);
     if (ctr[1] & ERR_NONFINITE) return fail(QNB_ENONFINITE, "instance %d: non-finite energy or gradient", k);
     if (ctr[1] & ERR_SHAKE) return fail(QNB_ENONFINITE, "instance %d: shake failure", k);
@@ -1292,18 +1304,16 @@ extern "C" int32_t qnb_batch_store_frames(qnb_batch* b, int32_t every, int32_t m
   return 0;
 }
 
-static int frames_stored(qnb_batch* b, int k, int* nf) {
-  int ctr[4];
-  HIPCHK(hipMemcpy(ctr, b->hm[k].ctr, sizeof ctr, hipMemcpyDeviceToHost));
-  *nf = b->hm[k].xs ? ctr[2] : 0;
-  return 0;
+static int frames_stored(const qnb_batch* b, int k, const std::vector<int>& all) {
+  return b->hm[k].xs ? all[CTR_STRIDE * k + 2] : 0;
 }
 
 extern "C" int32_t qnb_batch_frames(qnb_batch* b, int32_t k, double* out, int32_t cap, int32_t* nframes) {
   if (!b || k < 0 || k >= b->n || !nframes) return fail(QNB_EINVAL, "bad instance");
   HIPCHK(hipStreamSynchronize(b->stream));
-  int nf = 0, rc = frames_stored(b, k, &nf);
-  if (rc) return rc;
+  std::vector<int> all;
+  if (int rc = counters(b, all)) return rc;
+  const int nf = frames_stored(b, k, all);
   *nframes = nf;
   if (out && nf > 0 && nf <= cap)
     HIPCHK(hipMemcpy(out, b->hm[k].xs, sizeof(double) * 3 * b->hs[k].natom * nf, hipMemcpyDeviceToHost));
@@ -1314,40 +1324,47 @@ extern "C" int32_t qnb_batch_adjoint(qnb_batch* b, const qnb_qtangent* const* ta
                                      int64_t* n) {
   if (!b || !tan || !n) return fail(QNB_EINVAL, "null argument");
   HIPCHK(hipStreamSynchronize(b->stream));
-  std::vector<int> nf(b->n);
+  std::vector<int> nf(b->n), all;
+  if (int rc = counters(b, all)) return rc;
   std::vector<size_t> off(b->n + 1, 0);
-  long waves = 0;
+  long blocks = 0;
   for (int k = 0; k < b->n; k++) {
-    int rc = frames_stored(b, k, &nf[k]);
-    if (rc) return rc;
+    nf[k] = frames_stored(b, k, all);
     DevSys& S = b->hs[k];
     off[k + 1] = off[k] + (size_t)nf[k] * S.nstates * S.nqat * QNB_ADJ_NV;
-    waves = std::max(waves, (long)nf[k] * S.nqat);
+    blocks = std::max(blocks, (long)nf[k] * S.nqat);
   }
   *n = (int64_t)off[b->n];
   if (!out || *n == 0 || *n > cap) return 0;
   DevAlloc tmp;
+  DevPack pack;
   std::vector<AdjDev> A(b->n);
+  std::vector<int> of(b->n);  // the instance whose tables k uses
   double* dout = nullptr;
-  int rc = tmp.alloc(&dout, off[b->n]);
-  if (rc) return rc;
+  const AdjDev* dadj = nullptr;
+  int rc = 0;
   for (int k = 0; k < b->n; k++) {
     int same = -1;
     for (int m = 0; m < k && same < 0; m++)
       if (tan[m] == tan[k]) same = m;
     if (same >= 0) {
       if (b->topo_of[same] != b->topo_of[k]) return fail(QNB_EINVAL, "instances %d and %d share tangents but not a system", same, k);
-      A[k] = A[same];
-    } else if (b->hs[k].nqat > 0 && (rc = adjoint_upload(tmp, b->hs[k], tan[k], A[k]))) {
+    } else if (b->hs[k].nqat > 0 && (rc = adjoint_pack(pack, b->hs[k], tan[k], A[k]))) {
       return rc;
     }
+    of[k] = same >= 0 ? same : k;
+  }
+  pack.add(&dadj, (const AdjDev*)A.data(), A.size());
+  pack.space(&dout, off[b->n]);
+  if ((rc = pack.alloc(tmp))) return rc;
+  for (int k = 0; k < b->n; k++) {
+    if (of[k] != k) A[k] = A[of[k]];
     A[k].frames = b->hm[k].xs;
     A[k].nframes = nf[k];
     A[k].out = dout + off[k];
   }
-  AdjDev* dadj = nullptr;
-  if ((rc = tmp.upload((const AdjDev**)&dadj, A.data(), A.size()))) return rc;
-  launch_adjoint(b->stream, b->prec, b->ns_max, waves, b->n, b->dsys, dadj);
+  if ((rc = pack.copy())) return rc;
+  launch_adjoint(b->stream, b->prec, b->ns_max, blocks, b->n, b->dsys, dadj);
   HIPCHK(hipGetLastError());
   HIPCHK(hipMemcpyAsync(out, dout, sizeof(double) * off[b->n], hipMemcpyDeviceToHost, b->stream));
   HIPCHK(hipStreamSynchronize(b->stream));
@@ -1447,10 +1464,10 @@ extern "C" int32_t qnb_batch_free_energy(qnb_batch* b, const qnb_fep_params* p, 
   if (int rc = fep_params(p, ns, &P)) return rc;
   HIPCHK(hipStreamSynchronize(b->stream));
   std::vector<FepWin> hw(b->n);
+  std::vector<int> all;
+  if (int rc = counters(b, all)) return rc;
   for (int k = 0; k < b->n; k++) {
-    int nf = 0;
-    HIPCHK(hipMemcpy(&nf, b->hm[k].ctr, sizeof(int), hipMemcpyDeviceToHost));
-    nf = std::min(nf, b->hm[k].max_frames);
+    const int nf = std::min(all[CTR_STRIDE * k], b->hm[k].max_frames);
     if (nf <= P.nskip) return fail(QNB_EINVAL, "instance %d has %d frames, not more than the %d skipped", k, nf, P.nskip);
     FepWin& W = hw[k];
     W.hist = b->hm[k].hist;
@@ -1460,7 +1477,8 @@ extern "C" int32_t qnb_batch_free_energy(qnb_batch* b, const qnb_fep_params* p, 
     W.noffd = b->hm[k].noffd;
     for (int s = 0; s < QNB_MAX_STATES; s++) W.lam[s] = b->hs[k].lambda[s];
   }
-  return fep_run(b->stream, hw, P, out);
+  DevPack pack;
+  return fep_run(b->stream, hw, P, out, pack);
 }
 
 extern "C" int32_t qnb_batch_minimize(qnb_batch* b, int32_t nsteps, double max_disp) {

@@ -197,6 +197,7 @@ __global__ __launch_bounds__(FB_BINS) void k_fep_bins(const FepWin* __restrict__
   const int i = blockIdx.x, t = threadIdx.x, lane = t % QNB_WAVE;
   const FepWin& W = wins[i];
   const int ns = P.ns;
+  if (!(range[1] > range[0])) return;  // no bins to fill: the host refuses the result
   const double gapmin = range[0];
   const double xint = (range[1] - range[0]) / (double)P.nbins;
   __shared__ FepBinLds L;
@@ -272,8 +273,9 @@ __global__ __launch_bounds__(FB_BINS) void k_fep_bins(const FepWin* __restrict__
 
 // Part 3: per bin, the windows in order, FP3_U of them requested at a time
 #define FP3_U 8
-__global__ __launch_bounds__(256) void k_fep_part3(int n, FepPar P, const double* rec, const int* npts, double* bins,
-                                                   int* ptsum) {
+__global__ __launch_bounds__(256) void k_fep_part3(int n, FepPar P, const double* range, const double* rec,
+                                                   const int* npts, double* bins, int* ptsum) {
+  if (!(range[1] > range[0])) return;
   for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < P.nbins; k += gridDim.x * blockDim.x) {
     double b[4] = {0.0, 0.0, 0.0, 0.0};
     int pt = 0;
@@ -330,78 +332,67 @@ void launch_fep_part1(hipStream_t st, const FepWin* wins, int n, const FepPar& P
                      sd + off[2], sd + off[4]);
 }
 
-// Parts 2 and 3 (P.nbins > 0, a non-empty gap range)
+// Parts 2 and 3 (P.nbins > 0); nothing is written where the gap range is empty
 void launch_fep_bins(hipStream_t st, const FepWin* wins, int n, const FepPar& P, double* scratch) {
   size_t off[8];
   fep_layout(n, P.nbins, off);
   double* sd = scratch;
   int* npts = reinterpret_cast<int*>(sd + off[7]);
   hipLaunchKernelGGL(k_fep_bins, dim3(n), dim3(FB_BINS), 0, st, wins, P, sd + off[2], sd + off[4], sd + off[5], npts);
-  hipLaunchKernelGGL(k_fep_part3, dim3((P.nbins + 255) / 256), dim3(256), 0, st, n, P, sd + off[5], npts, sd + off[6],
-                     npts + (size_t)n * P.nbins);
+  hipLaunchKernelGGL(k_fep_part3, dim3((P.nbins + 255) / 256), dim3(256), 0, st, n, P, sd + off[4], sd + off[5], npts,
+                     sd + off[6], npts + (size_t)n * P.nbins);
 }
 
-// Runs the analysis for windows whose data already sit in device memory
-// (hw: host copies of the window records) and copies the results out.
-int fep_run(hipStream_t st, const std::vector<FepWin>& hw, const FepPar& P, qnb_fep_out* out) {
+// Runs the analysis and copies the results out.  hw: the window records, whose
+// data sit in device memory already or come with the tables of `pack`.
+int fep_run(hipStream_t st, std::vector<FepWin>& hw, const FepPar& P, qnb_fep_out* out, DevPack& pack) {
   const int n = (int)hw.size();
   DevAlloc mem;
   const FepWin* dw = nullptr;
   double* sd = nullptr;
-  if (int rc = mem.upload(&dw, hw.data(), hw.size())) return rc;
-  if (int rc = mem.alloc(&sd, fep_scratch_doubles(n, P.nbins))) return rc;
   size_t off[8];
   fep_layout(n, P.nbins, off);
+  const size_t nd = fep_scratch_doubles(n, P.nbins);
+  pack.add(&dw, (const FepWin*)hw.data(), hw.size());
+  pack.space(&sd, nd);
+  if (int rc = pack.alloc(mem)) return rc;
+  if (int rc = pack.copy()) return rc;
   launch_fep_part1(st, dw, n, P, sd);
+  if (P.nbins > 0) launch_fep_bins(st, dw, n, P, sd);
   HIPCHK(hipGetLastError());
-  double range[2];
-  HIPCHK(hipMemcpyAsync(range, sd + off[4], sizeof(range), hipMemcpyDeviceToHost, st));
+  std::unique_ptr<double[]> host(new (std::nothrow) double[nd]);
+  if (!host) return fail(QNB_ENOMEM, "no host memory for %zu results", nd);
+  const double* h = host.get();
+  HIPCHK(hipMemcpyAsync(host.get(), sd, nd * sizeof(double), hipMemcpyDeviceToHost, st));
   HIPCHK(hipStreamSynchronize(st));
-  if (P.nbins > 0) {
-    if (!(range[1] > range[0])) return fail(QNB_EINVAL, "energy gap range is empty: no bins to fill");
-    launch_fep_bins(st, dw, n, P, sd);
-    HIPCHK(hipGetLastError());
-  }
-  auto get = [&](void* dst, const void* src, size_t bytes) -> int {
-    if (dst && bytes) HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st));
-    return 0;
+  const double* range = h + off[4];
+  if (P.nbins > 0 && !(range[1] > range[0])) return fail(QNB_EINVAL, "energy gap range is empty: no bins to fill");
+  auto put = [](double* dst, const double* src, size_t k) {
+    if (dst) memcpy(dst, src, k * sizeof(double));
   };
-  int rc = 0;
-  rc = rc ? rc : get(out->dgf, sd + off[0], n * sizeof(double));
-  rc = rc ? rc : get(out->dgr, sd + off[1], n * sizeof(double));
-  rc = rc ? rc : get(out->dG, sd + off[2], n * sizeof(double));
-  rc = rc ? rc : get(out->gap_range, sd + off[4], 2 * sizeof(double));
-  std::vector<double> rec, bins;
-  std::vector<int32_t> ints;
+  put(out->dgf, h + off[0], n);
+  put(out->dgr, h + off[1], n);
+  put(out->dG, h + off[2], n);
+  put(out->gap_range, range, 2);
   const size_t nb = (size_t)n * P.nbins;
-  if (P.nbins > 0 && !rc) {
-    rec.resize(nb * FEP_REC);
-    bins.resize(4 * (size_t)P.nbins);
-    ints.resize(nb + P.nbins);
-    rc = rc ? rc : get(rec.data(), sd + off[5], rec.size() * sizeof(double));
-    rc = rc ? rc : get(bins.data(), sd + off[6], bins.size() * sizeof(double));
-    rc = rc ? rc : get(ints.data(), sd + off[7], ints.size() * sizeof(int32_t));
+  const double *rec = h + off[5], *bins = h + off[6];
+  const int32_t* ints = reinterpret_cast<const int32_t*>(h + off[7]);
+  for (size_t w = 0; w < nb; w++) {
+    const double* o = rec + w * FEP_REC;
+    if (out->dGg) out->dGg[w] = o[0];
+    if (out->c1) out->c1[w] = o[1];
+    if (out->c2) out->c2[w] = o[2];
+    if (out->r) out->r[w] = o[3];
+    if (out->dGv)
+      for (int s2 = 0; s2 < P.ns; s2++) out->dGv[w * P.ns + s2] = o[4 + s2];
+    if (out->npts) out->npts[w] = ints[w];
   }
-  if (rc) return rc;
-  HIPCHK(hipStreamSynchronize(st));
-  if (P.nbins > 0) {
-    for (size_t w = 0; w < nb; w++) {
-      const double* o = rec.data() + w * FEP_REC;
-      if (out->dGg) out->dGg[w] = o[0];
-      if (out->c1) out->c1[w] = o[1];
-      if (out->c2) out->c2[w] = o[2];
-      if (out->r) out->r[w] = o[3];
-      if (out->dGv)
-        for (int s2 = 0; s2 < P.ns; s2++) out->dGv[w * P.ns + s2] = o[4 + s2];
-      if (out->npts) out->npts[w] = ints[w];
-    }
-    for (int k = 0; k < P.nbins; k++) {
-      if (out->bin_dGg) out->bin_dGg[k] = bins[4 * k];
-      if (out->bin_c1) out->bin_c1[k] = bins[4 * k + 1];
-      if (out->bin_c2) out->bin_c2[k] = bins[4 * k + 2];
-      if (out->bin_r) out->bin_r[k] = bins[4 * k + 3];
-      if (out->ptsum) out->ptsum[k] = ints[nb + k];
-    }
+  for (int k = 0; k < P.nbins; k++) {
+    if (out->bin_dGg) out->bin_dGg[k] = bins[4 * k];
+    if (out->bin_c1) out->bin_c1[k] = bins[4 * k + 1];
+    if (out->bin_c2) out->bin_c2[k] = bins[4 * k + 2];
+    if (out->bin_r) out->bin_r[k] = bins[4 * k + 3];
+    if (out->ptsum) out->ptsum[k] = ints[nb + k];
   }
   return 0;
 }
@@ -439,7 +430,7 @@ extern "C" int32_t qnb_free_energy(int32_t nwin, int32_t nstates, const int32_t*
   if (nwin < 1 || !nframes || !V || !lambdas || !out) return fail(QNB_EINVAL, "bad arguments");
   FepPar P;
   if (int rc = fep_params(p, nstates, &P)) return rc;
-  DevAlloc mem;
+  DevPack pack;
   std::vector<FepWin> hw(nwin);
   for (int w = 0; w < nwin; w++) {
     if (!V[w] || nframes[w] <= P.nskip)
@@ -448,16 +439,10 @@ extern "C" int32_t qnb_free_energy(int32_t nwin, int32_t nstates, const int32_t*
     W.hist = nullptr;
     W.nf = nframes[w];
     W.noffd = (rkl && rkl[w]) ? 1 : 0;
-    const double* dv = nullptr;
-    if (int rc = mem.upload(&dv, V[w], (size_t)nframes[w] * nstates)) return rc;
-    W.V = dv;
     W.rkl = nullptr;
-    if (W.noffd) {
-      const double* dr = nullptr;
-      if (int rc = mem.upload(&dr, rkl[w], (size_t)nframes[w])) return rc;
-      W.rkl = dr;
-    }
+    pack.add(&W.V, V[w], (size_t)nframes[w] * nstates);
+    if (W.noffd) pack.add(&W.rkl, rkl[w], (size_t)nframes[w]);
     for (int s = 0; s < QNB_MAX_STATES; s++) W.lam[s] = s < nstates ? lambdas[(size_t)w * nstates + s] : 0.0;
   }
-  return fep_run(nullptr, hw, P, out);
+  return fep_run(nullptr, hw, P, out, pack);
 }

@@ -3,6 +3,9 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cstring>
+#include <memory>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -51,6 +54,48 @@ struct DevAlloc {
       (void)hipFree(p);
       ptrs.erase(it);
     }
+  }
+};
+
+// The tables of one call in one device allocation and one copy: a table of its
+// own costs an allocation, a copy and a free of about 20 us together, whatever
+// its size.  Tables are added first; alloc() sets their device pointers, and
+// copy() sends what they hold by then (so a table may hold such pointers).
+struct DevPack {
+  struct Item {
+    void** dst;
+    const void* src;  // null: space only
+    size_t off, bytes;
+  };
+  std::vector<Item> items;
+  size_t bytes = 0;
+  char* base = nullptr;
+  template <typename T>
+  void add(const T** dst, const T* src, size_t n) {
+    items.push_back({(void**)dst, src, bytes, src ? n * sizeof(T) : 0});
+    bytes += (std::max<size_t>(n, 1) * sizeof(T) + 255) & ~(size_t)255;
+  }
+  template <typename T>
+  void space(T** dst, size_t n) {
+    add((const T**)dst, (const T*)nullptr, n);
+  }
+  int alloc(DevAlloc& M) {
+    if (int rc = M.alloc(&base, bytes)) return rc;
+    for (const Item& i : items) *i.dst = base + i.off;
+    return 0;
+  }
+  int copy() const {
+    size_t end = 0;
+    for (const Item& i : items)
+      if (i.bytes) end = std::max(end, i.off + i.bytes);
+    if (end == 0) return 0;
+    std::unique_ptr<char[]> host(new (std::nothrow) char[end]);
+    if (!host) return fail(QNB_ENOMEM, "no host memory for %zu bytes of tables", end);
+    for (const Item& i : items)
+      if (i.bytes) memcpy(host.get() + i.off, i.src, i.bytes);
+    if (hipMemcpy(base, host.get(), end, hipMemcpyHostToDevice) != hipSuccess)
+      return fail(QNB_EDEVICE, "upload failed");
+    return 0;
   }
 };
 
@@ -124,10 +169,10 @@ struct FepPar {
 int fep_params(const qnb_fep_params* p, int ns, FepPar* P);
 // runs the analysis on stream st for windows whose data sit in device memory
 // (hw: host copies of the window records) and copies the results to out
-int fep_run(hipStream_t st, const std::vector<FepWin>& hw, const FepPar& P, qnb_fep_out* out);
+int fep_run(hipStream_t st, std::vector<FepWin>& hw, const FepPar& P, qnb_fep_out* out, DevPack& pack);
 
 // adjoint of the Q-atom energies: tangent upload and launch over frames
-int adjoint_upload(DevAlloc& M, const DevSys& S, const qnb_qtangent* t, AdjDev& A);
+int adjoint_pack(DevPack& M, const DevSys& S, const qnb_qtangent* t, AdjDev& A);
 void launch_adjoint(hipStream_t st, int prec, int ns_max, long blocks, int B, const DevSys* dsys, const AdjDev* dadj);
 // Q-atom bonded terms: validation and device copies (buffers recorded in
 // `owned` so a later set can release them), and the per-instance launch
