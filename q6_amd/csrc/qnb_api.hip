@@ -33,20 +33,28 @@ __global__ void k_pack_xq(const DevSys*);
 __global__ void k_pw_first(const DevSys*);
 __global__ void k_expand(const DevSys*);
 __global__ void k_watpol_theta(const DevSys*, const int*);
-template <bool BONDED>
 __global__ void k_pol_bonded(const DevSys*, int);
+__global__ void k_pol_forces(const DevSys*);
+__global__ void k_bonded_rows(const DevSys*);
 __global__ void k_watpol_finish(const DevSys*);
 
-void launch_watpol(hipStream_t st, int nwat, int B, const DevSys* dsys, const int* istep, bool theta, bool finish,
-                   int bonded_blocks) {
-  if (theta && nwat > 0)
+void launch_watpol(hipStream_t st, int nwat, int B, const DevSys* dsys, const int* istep, int with) {
+  if ((with & POL_THETA) && nwat > 0)
     hipLaunchKernelGGL(k_watpol_theta, dim3((nwat + WP_THREADS - 1) / WP_THREADS, B), dim3(WP_THREADS), 0, st, dsys,
                        istep);
-  const int pol = nwat > 0 ? nwat / WP_WATERS + QNB_MAXSH : 0;
-  const dim3 grid(pol + bonded_blocks, B);
-  if (bonded_blocks > 0) hipLaunchKernelGGL((k_pol_bonded<true>), grid, dim3(256), 0, st, dsys, pol);
-  else if (pol > 0) hipLaunchKernelGGL((k_pol_bonded<false>), grid, dim3(256), 0, st, dsys, pol);
-  if (finish && nwat > 0) hipLaunchKernelGGL(k_watpol_finish, dim3(B), dim3(64), 0, st, dsys);
+  if (nwat > 0) hipLaunchKernelGGL(k_pol_forces, dim3(nwat / WP_WATERS + QNB_MAXSH, B), dim3(256), 0, st, dsys);
+  if ((with & POL_FINISH) && nwat > 0) hipLaunchKernelGGL(k_watpol_finish, dim3(B), dim3(64), 0, st, dsys);
+}
+
+void launch_pol_bonded(hipStream_t st, int nwat, int bonded_atoms, int B, const DevSys* dsys) {
+  const int pol = nwat > 0 ? nwat / WP_WATERS + QNB_MAXSH : 0, bonded = (bonded_atoms + QNB_WAVE - 1) / QNB_WAVE;
+  if (pol + bonded > 0)
+    hipLaunchKernelGGL(k_pol_bonded, dim3(pol + bonded, B), dim3(QNB_WAVE * POL_SMALL_WAVES), 0, st, dsys, pol);
+}
+
+void launch_bonded_rows(hipStream_t st, int bonded_atoms, int B, const DevSys* dsys) {
+  if (bonded_atoms > 0)
+    hipLaunchKernelGGL(k_bonded_rows, dim3((bonded_atoms + 255) / 256, B), dim3(256), 0, st, dsys);
 }
 
 // Up to this many receiver waves (four per solute group, one per solvent
@@ -742,7 +750,7 @@ static void launch_eval(qnb_handle* h, uint32_t mask) {
     launch_forces_small(h->stream, S.prec, S.nstates, true, G, 1, h->dsys, mask, h->d_istep);
     hipLaunchKernelGGL(k_atom_terms, dim3((S.natom + 255) / 256, 1), dim3(256), 0, h->stream, h->dsys, mask,
                        (const double*)h->d_tfree, (G.qside ? QROWS_SIDE : 0) | (G.qq ? QROWS_QQ : 0));
-    if (with_pol) launch_watpol(h->stream, S.nwat, 1, h->dsys, h->d_istep, false, false, 0);
+    if (with_pol) launch_pol_bonded(h->stream, S.nwat, 0, 1, h->dsys);
     hipLaunchKernelGGL(k_reduce_part, dim3(QNB_RED_BLOCKS, 1), dim3(256), 0, h->stream, h->dsys);
     hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(256), 0, h->stream, h->dsys,
                        G.qq ? (int)QQ_RECORD_PER_BLOCK : 0, (int)with_pol);
@@ -771,7 +779,7 @@ static void launch_eval(qnb_handle* h, uint32_t mask) {
   }
   const int with_qq = S.nqat > 0 && (mask & (QNB_T_QQ | QNB_T_QQP)) ? QQ_ONE_RECORD : 0;
   if (with_qq) hipLaunchKernelGGL((k_qq<R, NS>), dim3(1), dim3(QQ_THREADS), 0, h->stream, h->dsys, mask);
-  if (with_pol) launch_watpol(h->stream, S.nwat, 1, h->dsys, (const int*)h->d_istep, true, false, 0);
+  if (with_pol) launch_watpol(h->stream, S.nwat, 1, h->dsys, (const int*)h->d_istep, POL_THETA);
   hipLaunchKernelGGL(k_reduce_part, dim3(QNB_RED_BLOCKS, 1), dim3(256), 0, h->stream, h->dsys);
   hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(256), 0, h->stream, h->dsys, with_qq, (int)with_pol);
 }

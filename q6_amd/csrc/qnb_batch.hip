@@ -162,17 +162,13 @@ __device__ void thermo_update(const MdDev& M, const double* ek, const double* ek
   }
 }
 
-// Closes an MD step, four waves of the last block of k_integrate.  Wave 0: the
-// kinetic energy from the block sums (lane l takes blocks l, l + 64, ..., then
-// a fixed tree), the temperature, Tfree and the Berendsen factor of the next
-// step (temperature, src/md.f90:1379-1447), the step counter and the errors;
-// the others close the polarisation restraint's step (watpol_finish).  A
-// launch of its own took 7 us for this.
-__device__ __forceinline__ void thermo(const DevSys& S, const MdDev& M, int nblk, int wid, int lane) {
-  if (wid != 0) {
-    watpol_finish(S, wid - 1, 3);
-    return;
-  }
+// Closes an MD step, one wave of the last block of k_integrate: the kinetic
+// energy from the block sums (lane l takes blocks l, l + 64, ..., then a fixed
+// tree), the temperature, Tfree and the Berendsen factor of the next step
+// (temperature, src/md.f90:1379-1447), the step counter and the errors.  A
+// launch of its own took 7 us for this and the polarisation restraint's sums
+// (watpol_finish), which a block of their own forms beside the integration.
+__device__ __forceinline__ void thermo(const DevSys& S, const MdDev& M, int nblk, int lane) {
   double s[4] = {0.0, 0.0, 0.0, 0.0};
   for (int k = lane; k < nblk; k += QNB_WAVE)
     for (int c = 0; c < 4; c++)
@@ -198,7 +194,11 @@ __device__ __forceinline__ void thermo(const DevSys& S, const MdDev& M, int nblk
 // of the step (LRF Taylor term, radial restraint, the rows of the bonded terms
 // and of the Q kernels: what k_atom_step adds) are formed here and not written,
 // on steps that neither record energies nor run the Q bonded terms in between:
-// a launch and a pass over the gradients less.
+// a launch and a pass over the gradients less.  Latency of dependent loads in a
+// small step, so an atom's data are all requested before any are used (one
+// window of 3,342 atoms 19.4 -> 15.0 us, with the restraint's sums moved out of
+// the last block); at 51 windows of 11,056 atoms memory: 766 -> 739 us per step
+// by the same.
 template <bool FUSED>
 __global__ __launch_bounds__(256) void k_integrate(const DevSys* __restrict__ systems, const MdDev* __restrict__ mds,
                                                    int rows) {
@@ -206,7 +206,11 @@ __global__ __launch_bounds__(256) void k_integrate(const DevSys* __restrict__ sy
   const MdDev& M = mds[blockIdx.y];
   const int nthr = S.nwat + S.nat_solute;
   const int nblk = (nthr + 255) / 256;
-  if ((int)blockIdx.x >= nblk) return;
+  const int lane = threadIdx.x % QNB_WAVE, wid = threadIdx.x / QNB_WAVE;
+  if ((int)blockIdx.x >= nblk) {
+    if ((int)blockIdx.x == nblk) watpol_finish(S, wid, 4);
+    return;
+  }
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   const double dt = M.dt;
   const auto xg = gpm(S.x);
@@ -218,28 +222,36 @@ __global__ __launch_bounds__(256) void k_integrate(const DevSys* __restrict__ sy
   const double s = (solvent && M.ngroup == 2) ? M.st[6] : M.st[0];
   double el = 0.0, er = 0.0;  // energies: not kept on these steps
   if (t < S.nwat) {
+    // everything the water needs is requested before any of it is used
     const int o = S.nat_solute + 3 * t;
-    double xo[3][3], xn[3][3], wi[3];
+    double xo[3][3], xn[3][3], v0[3][3], g[3][3], wi[3], q[3];
+    bool excl[3];
+    LrfGroup L;
     for (int k = 0; k < 3; k++) {
       wi[k] = ldg(M.winv + o + k);
-      double f[3] = {0.0, 0.0, 0.0};
+      excl[k] = ldg(S.excl + o + k);
+      q[k] = FUSED ? ldg(S.crg + o + k) : 0.0;
+      for (int c = 0; c < 3; c++) {
+        xo[k][c] = xg[3 * (o + k) + c];
+        v0[k][c] = vg[3 * (o + k) + c];
+        g[k][c] = dg[3 * (o + k) + c];
+      }
+    }
+    if constexpr (FUSED)
+      if (S.use_lrf) lrf_load(S, S.ncgp_solute + t, L);
+    for (int k = 0; k < 3; k++) {
       if constexpr (FUSED) {
-        if (S.use_lrf && !ldg(S.excl + o + k)) lrf_taylor_atom(S, o + k, S.ncgp_solute + t, f, el);
-        if (k == 0 && !ldg(S.excl + o)) {
+        double f[3] = {0.0, 0.0, 0.0};
+        if (S.use_lrf && !excl[k]) lrf_taylor(L, xo[k][0], xo[k][1], xo[k][2], q[k], f, el);
+        if (k == 0 && !excl[0]) {
           const double shift = S.fk_wsphere != 0.0 ? sqrt(S.Boltz * *M.tfree / S.fk_wsphere) : 0.0;
-          radial_restraint(S, o, shift, f, er);
+          radial_restraint(S, xo[0][0], xo[0][1], xo[0][2], shift, f, er);
         }
         if (o + k < S.nbat)
           for (int c = 0; c < 3; c++) f[c] += ldg(S.brow + 3 * (o + k) + c);
+        for (int c = 0; c < 3; c++) g[k][c] += f[c];
       }
-      for (int c = 0; c < 3; c++) {
-        const int q = 3 * (o + k) + c;
-        double g = dg[q];
-        if constexpr (FUSED) g += f[c];
-        const double v = (vg[q] - g * wi[k] * dt) * s;
-        xo[k][c] = xg[q];
-        xn[k][c] = xo[k][c] + v * dt;
-      }
+      for (int c = 0; c < 3; c++) xn[k][c] = xo[k][c] + (v0[k][c] - g[k][c] * wi[k] * dt) * s * dt;
     }
     const int ci[3] = {0, 0, 1}, cj[3] = {1, 2, 2};
     const double d2[3] = {M.roh2, M.roh2, M.rhh2};
@@ -276,33 +288,33 @@ __global__ __launch_bounds__(256) void k_integrate(const DevSys* __restrict__ sy
       }
       const double e = 0.5 * (1.0 / wi[k]) * v2;
       ek += e;
-      if (!ldg(S.excl + o + k)) ekf += e;
+      if (!excl[k]) ekf += e;
     }
   } else if (t < nthr) {
     const int i = t - S.nwat;
     const double wi = ldg(M.winv + i);
-    double f[3] = {0.0, 0.0, 0.0};
     const bool excl = ldg(S.excl + i);
-    // an excluded atom in no charge group has no pair gradient (store_atom_gradient)
-    bool grouped = true;
+    double xo[3], v0[3], g[3];
+    for (int c = 0; c < 3; c++) xo[c] = xg[3 * i + c], v0[c] = vg[3 * i + c], g[c] = dg[3 * i + c];
     if constexpr (FUSED) {
-      const int g = ldg(S.atom_group + i);
-      grouped = g >= 0;
-      if (S.use_lrf && !excl && ldg(S.iqatom + i) == 0) lrf_taylor_atom(S, i, g, f, el);
+      const int group = ldg(S.atom_group + i), iq = ldg(S.iqatom + i);
+      const double q = ldg(S.crg + i);
+      double f[3] = {0.0, 0.0, 0.0};
+      LrfGroup L;
+      if (S.use_lrf && group >= 0) lrf_load(S, group, L);
       if (i < S.nbat)
         for (int c = 0; c < 3; c++) f[c] += ldg(S.brow + 3 * i + c);
       add_qrows(S, i, rows, f);
+      if (S.use_lrf && group >= 0 && !excl && iq == 0) lrf_taylor(L, xo[0], xo[1], xo[2], q, f, el);
+      // an excluded atom in no charge group has no pair gradient (store_atom_gradient)
+      for (int c = 0; c < 3; c++) g[c] = group >= 0 ? g[c] + f[c] : f[c];
     }
     double v2 = 0.0;
     for (int c = 0; c < 3; c++) {
-      const int q = 3 * i + c;
-      double g = dg[q];
-      if constexpr (FUSED) g = grouped ? g + f[c] : f[c];
-      const double v0 = (vg[q] - g * wi * dt) * s;
-      const double xo = xg[q], xn = xo + v0 * dt;
-      const double v = (xn - xo) / dt;
-      xg[q] = xn;
-      vg[q] = v;
+      const double xn = xo[c] + (v0[c] - g[c] * wi * dt) * s * dt;
+      const double v = (xn - xo[c]) / dt;
+      xg[3 * i + c] = xn;
+      vg[3 * i + c] = v;
       v2 += v * v;
     }
     const double e = 0.5 * (1.0 / wi) * v2;
@@ -311,7 +323,6 @@ __global__ __launch_bounds__(256) void k_integrate(const DevSys* __restrict__ sy
   }
   // the four sums of the block, in wave order
   const bool g1 = solvent && M.ngroup == 2;
-  const int lane = threadIdx.x % QNB_WAVE, wid = threadIdx.x / QNB_WAVE;
   __shared__ double red[4][4];
   __shared__ bool last;
   const double sums[4] = {wave_sum_all(g1 ? 0.0 : ek), wave_sum_all(g1 ? 0.0 : ekf), wave_sum_all(g1 ? ek : 0.0),
@@ -336,7 +347,7 @@ __global__ __launch_bounds__(256) void k_integrate(const DevSys* __restrict__ sy
       last = __hip_atomic_fetch_add(&M.ctr[3], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nblk - 1;
   }
   __syncthreads();
-  if (last) thermo(S, M, nblk, wid, lane);
+  if (last && wid == 0) thermo(S, M, nblk, lane);
 }
 
 // shake (src/bondene.f90:1069-1151) on each rigid water (O-H1, O-H2, H1-H2),
@@ -514,6 +525,7 @@ struct qnb_batch {
   hipGraph_t cycle_graph = nullptr;
   int maxg = 0, maxat = 0, maxsw = 0, maxw = 0, maxs = 0, ns_max = 1, prec = 0;
   int nbblk = 1;  // k_bonded blocks per instance
+  int nbat_max = 0;
   int* ctr = nullptr;  // every instance's counters (MdDev::ctr), CTR_STRIDE apart: read in one copy
   bool anyq = false, anypol = false, static_q = true;
   int qchunks = 1, nq_max = 0, nqe_max = 0, nsol_max = 0;
@@ -661,12 +673,12 @@ static void enqueue_forces_forked(qnb_batch* b, bool energy, bool bonded) {
   const int wpb = 4, B = b->n;
   (void)hipEventRecord(b->ev_fork, b->stream);
   (void)hipStreamWaitEvent(b->side, b->ev_fork, 0);
-  if (bonded) launch_watpol(b->side, 0, B, b->dsys, (const int*)b->istep, false, false, b->nbblk);
+  if (bonded) launch_bonded_rows(b->side, b->nbat_max, B, b->dsys);
   if (b->anyq)
     hipLaunchKernelGGL((k_qforces<R, NS>), dim3(qforces_blocks(b->nq_max, b->qchunks, wpb), B), dim3(64 * wpb), 0,
                        b->side, b->dsys, kStepMask, b->qchunks, (int)QROWS_SIDE);
   if (b->maxw > 0) launch_forces_t<R, NS>(b, b->wpb_forces, energy, false, 1, b->side);
-  if (b->anypol) launch_watpol(b->side, b->maxw, B, b->dsys, (const int*)b->istep, true, false, 0);
+  if (b->anypol) launch_watpol(b->side, b->maxw, B, b->dsys, (const int*)b->istep, POL_THETA);
   launch_forces_t<R, NS>(b, b->wpb_forces, energy, false, 2);
   if (b->anyq) hipLaunchKernelGGL((k_qq<R, NS>), dim3(B), dim3(QQ_THREADS), 0, b->stream, b->dsys, kStepMask);
   (void)hipEventRecord(b->ev_join, b->side);
@@ -680,7 +692,7 @@ static bool small_step(const qnb_batch* b) { return small_launch(b->sum_solute, 
 static void enqueue_forces_small(qnb_batch* b, bool energy, bool bonded) {
   const SmallGrid G = small_grid(b->maxs, b->maxw, 3, b->nq_max, b->nsol_max, b->nqe_max, kStepMask, b->anypol);
   launch_forces_small(b->stream, b->prec, b->ns_max, energy, G, b->n, b->dsys, kStepMask, b->istep);
-  launch_watpol(b->stream, b->anypol ? b->maxw : 0, b->n, b->dsys, b->istep, false, false, bonded ? b->nbblk : 0);
+  launch_pol_bonded(b->stream, b->anypol ? b->maxw : 0, bonded ? b->nbat_max : 0, b->n, b->dsys);
 }
 
 template <typename R, int NS>
@@ -693,13 +705,13 @@ static void enqueue_forces(qnb_batch* b, bool energy = true, bool atom_terms = t
                        b->stream, b->dsys, mask, b->qchunks, 0);
     hipLaunchKernelGGL((k_qq<R, NS>), dim3(B), dim3(QQ_THREADS), 0, b->stream, b->dsys, mask);
   }
-  if (b->anypol) launch_watpol(b->stream, b->maxw, B, b->dsys, (const int*)b->istep, true, true, 0);
+  if (b->anypol) launch_watpol(b->stream, b->maxw, B, b->dsys, (const int*)b->istep, POL_THETA | POL_FINISH);
 }
 
 // leap-frog + SHAKE + new velocities, the temperatures and Berendsen factors
 // of the next step; fused: with the per-atom terms
 static void launch_integrate(qnb_batch* b, bool fused, int rows) {
-  const dim3 grid((b->maxsw + 255) / 256, b->n);
+  const dim3 grid((b->maxsw + 255) / 256 + 1, b->n);
   if (fused) hipLaunchKernelGGL((k_integrate<true>), grid, dim3(256), 0, b->stream, b->dsys, b->dmd, rows);
   else hipLaunchKernelGGL((k_integrate<false>), grid, dim3(256), 0, b->stream, b->dsys, b->dmd, rows);
 }
@@ -937,6 +949,7 @@ extern "C" int32_t qnb_batch_create(int32_t n, const qnb_system* const* sys, con
           (rc = b->mem.alloc(&S.brow, 3 * (size_t)std::max(nbat, 1))))
         return rc;
       b->nbblk = std::max(b->nbblk, (nbat + 255) / 256);
+      b->nbat_max = std::max(b->nbat_max, nbat);
       const int nib = (S.nwat + S.nat_solute + 255) / 256;
       if ((rc = b->mem.alloc(&M.tpart, 4 * (size_t)std::max(nib, 1)))) return rc;
     }

@@ -468,6 +468,8 @@ enum { QQ_ONE_RECORD = 1, QQ_RECORD_PER_BLOCK = 2 };
 
 // shell members per block of the polarisation-restraint force kernel
 #define WP_WATERS 64
+// waves per block of that kernel in a small step
+#define POL_SMALL_WAVES 16
 __host__ __device__ __forceinline__ bool has_pol(const DevSys& S) { return S.nwat > 0 && S.wpol && S.nshell > 0; }
 // restraint energy (c = 0) or theta (c = 1) of shell is, added over its n
 // members by one wave (every lane active): lane l takes ranks l, l + 64, ...,
@@ -749,39 +751,59 @@ __device__ __forceinline__ void bonded_atom(const DevSys& S, int i, double* f, d
   }
 }
 
-// LRF Taylor application for one atom (lrf_taylor, nonbondene.f90:507-571)
-__device__ __forceinline__ void lrf_taylor_atom(const DevSys& S, int i, int group, double* f, double& e) {
+// A charge group's LRF expansion, its symmetric tensors by their independent
+// components (xx xy xz yy yz zz; xxx xxy xxz xyy xyz xzz yyy yyz yzz zzz): 23
+// of the 43 stored numbers, all requested at once.
+struct LrfGroup {
+  double c[3], phi0, p1[3], p2[6], p3[10];
+};
+__device__ __forceinline__ void lrf_load(const DevSys& S, int group, LrfGroup& g) {
   const auto L = gp(S.lrf + (size_t)QNB_NLRF * group);
-  const auto x = gp(S.x);
-  const double drx = L[0] - x[3 * i], dry = L[1] - x[3 * i + 1], drz = L[2] - x[3 * i + 2];
-  const auto p1 = L + 4;
-  const auto p2 = L + 7;
-  const auto p3 = L + 16;
-  double t0 = drx * p2[0] + dry * p2[1] + drz * p2[2];
-  double t1 = drx * p2[3] + dry * p2[4] + drz * p2[5];
-  double t2 = drx * p2[6] + dry * p2[7] + drz * p2[8];
-  double V = L[3] + (drx * p1[0] + dry * p1[1] + drz * p1[2]) + 0.5 * (drx * t0 + dry * t1 + drz * t2);
-  const double q = ldg(S.crg + i);
+  for (int k = 0; k < 3; k++) g.c[k] = L[k], g.p1[k] = L[4 + k];
+  g.phi0 = L[3];
+  constexpr int i2[6] = {0, 1, 2, 4, 5, 8};
+  constexpr int i3[10] = {0, 1, 2, 4, 5, 8, 13, 14, 17, 26};
+#pragma unroll
+  for (int k = 0; k < 6; k++) g.p2[k] = L[7 + i2[k]];
+#pragma unroll
+  for (int k = 0; k < 10; k++) g.p3[k] = L[16 + i3[k]];
+}
+// LRF Taylor application for one atom at x (lrf_taylor, nonbondene.f90:507-571)
+__device__ __forceinline__ void lrf_taylor(const LrfGroup& g, double x, double y, double z, double q, double* f,
+                                           double& e) {
+  const double d[3] = {g.c[0] - x, g.c[1] - y, g.c[2] - z};
+  constexpr int s2[3][3] = {{0, 1, 2}, {1, 3, 4}, {2, 4, 5}};
+  constexpr int s3[3][3][3] = {{{0, 1, 2}, {1, 3, 4}, {2, 4, 5}},
+                               {{1, 3, 4}, {3, 6, 7}, {4, 7, 8}},
+                               {{2, 4, 5}, {4, 7, 8}, {5, 8, 9}}};
+  double t[3], df[3];
+#pragma unroll
+  for (int k = 0; k < 3; k++) t[k] = d[0] * g.p2[s2[k][0]] + d[1] * g.p2[s2[k][1]] + d[2] * g.p2[s2[k][2]];
+  const double V = g.phi0 + (d[0] * g.p1[0] + d[1] * g.p1[1] + d[2] * g.p1[2]) +
+                   0.5 * (d[0] * t[0] + d[1] * t[1] + d[2] * t[2]);
   e += 0.5 * q * V;
-  double df[3];
+#pragma unroll
   for (int k = 0; k < 3; k++) {
-    const auto P = p3 + 9 * k;
-    double u0 = drx * P[0] + dry * P[1] + drz * P[2];
-    double u1 = drx * P[3] + dry * P[4] + drz * P[5];
-    double u2 = drx * P[6] + dry * P[7] + drz * P[8];
-    df[k] = p1[k] + (drx * p2[3 * k] + dry * p2[3 * k + 1] + drz * p2[3 * k + 2]) +
-            0.5 * (drx * u0 + dry * u1 + drz * u2);
+    double u[3];
+#pragma unroll
+    for (int j = 0; j < 3; j++)
+      u[j] = d[0] * g.p3[s3[k][j][0]] + d[1] * g.p3[s3[k][j][1]] + d[2] * g.p3[s3[k][j][2]];
+    df[k] = g.p1[k] + t[k] + 0.5 * (d[0] * u[0] + d[1] * u[1] + d[2] * u[2]);
+    f[k] -= df[k] * q;
   }
-  f[0] -= df[0] * q;
-  f[1] -= df[1] * q;
-  f[2] -= df[2] * q;
+}
+__device__ __forceinline__ void lrf_taylor_atom(const DevSys& S, int i, int group, double* f, double& e) {
+  LrfGroup g;
+  lrf_load(S, group, g);
+  const auto x = gp(S.x);
+  lrf_taylor(g, x[3 * i], x[3 * i + 1], x[3 * i + 2], ldg(S.crg + i), f, e);
 }
 
 // SCAAS radial restraint on one water oxygen (restrain_solvent,
 // nonbondene.f90:6466-6544, 3-site branch)
-__device__ __forceinline__ void radial_restraint(const DevSys& S, int src, double shift, double* f, double& e) {
-  const auto x = gp(S.x);
-  double vx = x[3 * src] - S.xw[0], vy = x[3 * src + 1] - S.xw[1], vz = x[3 * src + 2] - S.xw[2];
+__device__ __forceinline__ void radial_restraint(const DevSys& S, double x, double y, double z, double shift, double* f,
+                                                 double& e) {
+  double vx = x - S.xw[0], vy = y - S.xw[1], vz = z - S.xw[2];
   double b = sqrt(vx * vx + vy * vy + vz * vz);
   double db = b - (S.rwat - shift);
   double erst, dv;
@@ -800,6 +822,11 @@ __device__ __forceinline__ void radial_restraint(const DevSys& S, int src, doubl
   f[1] += vy * dv;
   f[2] += vz * dv;
   e += erst;
+}
+
+__device__ __forceinline__ void radial_restraint(const DevSys& S, int src, double shift, double* f, double& e) {
+  const auto x = gp(S.x);
+  radial_restraint(S, x[3 * src], x[3 * src + 1], x[3 * src + 2], shift, f, e);
 }
 
 // The atom whose distance from xwcent drives atom i's SCAAS radial term

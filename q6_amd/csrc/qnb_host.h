@@ -126,11 +126,15 @@ void launch_forces_small(hipStream_t st, int prec, int ns_max, bool energy, cons
 // whether a force pass over so many receivers (of all instances) takes that
 // kernel
 bool small_launch(long solute_groups, long solvent);
-// polarisation restraint: angles and shells (theta), ranks and forces, and
-// the per-system sums (finish) where no later kernel of the caller runs them;
-// beside the forces, bonded_blocks blocks of bonded terms (DevSys::brow)
-void launch_watpol(hipStream_t st, int nwat, int B, const DevSys* dsys, const int* istep, bool theta, bool finish,
-                   int bonded_blocks);
+// polarisation restraint beside full force kernels: angles and shells (theta),
+// ranks and forces, and the per-system sums (finish) where no later kernel of
+// the caller runs them
+enum { POL_THETA = 1, POL_FINISH = 2 };
+void launch_watpol(hipStream_t st, int nwat, int B, const DevSys* dsys, const int* istep, int with);
+// the restraint's ranks and forces (nwat 0: none) and the bonded terms
+// (DevSys::brow) in a small step, which waits for them; the bonded terms alone
+void launch_pol_bonded(hipStream_t st, int nwat, int bonded_atoms, int B, const DevSys* dsys);
+void launch_bonded_rows(hipStream_t st, int bonded_atoms, int B, const DevSys* dsys);
 // per-instance device state (coordinates, gradient, lists, LRF, energies)
 int instance_alloc(DevSys& S, DevAlloc& M, const qnb_params* p, int nslots);
 // neighbour rows of `cap` groups; entries per partner-atom row that always

@@ -1887,41 +1887,27 @@ __global__ __launch_bounds__(256) void k_forces_small(const DevSys* __restrict__
   watpol_theta(S, b - G.qq, istep[blockIdx.y]);
 }
 
-// Phase 2, WP_WATERS members of one shell per block, four waves on the same
+// Phase 2, WP_WATERS members of one shell per block, WAVES waves on the same
 // members: each member's rank in its shell's stable ascending order of theta
 // (the reference's selection sort; ties by water index) is the number of
-// members before it, counted against the shell's list staged in LDS, a quarter
-// of it per wave; wave 0 then forms the target angle from the rank, the
-// restraint energy and the forces (adds to d), and writes energy and theta at
-// the member's rank (wp_rank), so the sums over a shell do not depend on the
-// order the angle kernel appended its members in.  Counting is n^2 compares,
-// but over all blocks it is a few microseconds of latency at n = 700, where
-// one block per shell running a bitonic network over its 55 steps took 14-23
-// us and was a launch of its own.  Blocks take the members of one shell, not
-// the waters in index order, so a wave counts one list: the index order, where
-// every block holds every shell, cost 51 windows of 2,352 waters 22 us per
-// step more.
-//
-// BONDED: blocks from pol on form the bonded terms of 256 atoms each into their
-// rows, for k_integrate.  In a small step they share the launch with the
-// polarisation blocks, whose latency is the longer one; where the restraint
-// runs beside full force kernels the two are launches of their own, because
-// the 106 registers of the bonded terms (32 without) keep those from the CUs:
-// 51 windows of 11,056 atoms, 847 us per step in one launch, 834 in two.
-template <bool BONDED>
-__global__ __launch_bounds__(256) void k_pol_bonded(const DevSys* __restrict__ systems, int pol) {
-  const DevSys& S = systems[blockIdx.y];
+// members before it, counted against the shell's list staged in LDS, an equal
+// part of it per wave (equal angles, which only coincidence brings, in a second
+// pass of the members concerned); wave 0 then forms the target angle from the
+// rank, the restraint energy and the forces (adds to d), and writes energy and
+// theta at the member's rank (wp_rank), so the sums over a shell do not depend
+// on the order the angle kernel appended its members in.  Counting is n^2
+// compares, but over all blocks it is a few microseconds of latency at n = 700,
+// where one block per shell running a bitonic network over its 55 steps took
+// 14-23 us and was a launch of its own.  Blocks take the members of one shell,
+// not the waters in index order, so a wave counts one list: the index order,
+// where every block holds every shell, cost 51 windows of 2,352 waters 22 us
+// per step more.
+// WAVES: a small step waits for this kernel, so 16 waves share a count (1,110
+// waters 10.5 -> 8.2 us, 2,352 waters 17 -> 8.5 us against 4); beside full
+// force kernels, whose blocks leave four wave slots sooner than 16, 4 do.
+template <int WAVES>
+__device__ __forceinline__ void pol_forces(const DevSys& S) {
   const int lane = threadIdx.x % QNB_WAVE, wid = threadIdx.x / QNB_WAVE;
-  if constexpr (BONDED) {
-    if ((int)blockIdx.x >= pol) {
-      const int i = ((int)blockIdx.x - pol) * blockDim.x + threadIdx.x;
-      if (i >= S.nbat) return;
-      double f[3] = {0.0, 0.0, 0.0}, eb = 0.0, ea = 0.0;
-      bonded_atom(S, i, f, eb, ea);
-      for (int c = 0; c < 3; c++) stg(S.brow + 3 * i + c, f[c]);
-      return;
-    }
-  }
   if (!has_pol(S)) return;
   const int nsh = S.nshell, nw = S.nwat;
   // block x of the system takes members 64 x' .. of shell sh, the blocks of
@@ -1940,34 +1926,38 @@ __global__ __launch_bounds__(256) void k_pol_bonded(const DevSys* __restrict__ s
   }
   if (sh < 0) return;
   __shared__ double c_th[WP_CHUNK];
-  __shared__ int c_w[WP_CHUNK];
-  __shared__ int s_cnt[4][QNB_WAVE];
+  __shared__ int s_cnt[WAVES][QNB_WAVE], s_eq[WAVES][QNB_WAVE];
   const int m = xb * WP_WATERS + lane;
   const double* L_th = S.sh_lth + (size_t)sh * nw;
   const int* L_w = S.sh_list + (size_t)sh * nw;
   const int w = m < n ? ldg(L_w + m) : 0;
   const double th = m < n ? ldg(L_th + m) : 0.0;
-  int before = 0;
+  int before = 0, equal = 0;
   for (int k0 = 0; k0 < n; k0 += WP_CHUNK) {
     const int nk = min(WP_CHUNK, n - k0);
     __syncthreads();
-    for (int k = threadIdx.x; k < nk; k += blockDim.x) {
-      c_th[k] = ldg(L_th + k0 + k);
-      c_w[k] = ldg(L_w + k0 + k);
-    }
+    for (int k = threadIdx.x; k < nk; k += blockDim.x) c_th[k] = ldg(L_th + k0 + k);
     __syncthreads();
-    const int q0 = nk * wid / 4, q1 = nk * (wid + 1) / 4;
-#pragma unroll 4
+    const int q0 = nk * wid / WAVES, q1 = nk * (wid + 1) / WAVES;
+#pragma unroll 8
     for (int k = q0; k < q1; k++) {
-      const double t2 = c_th[k];
-      before += (t2 < th) || (t2 == th && c_w[k] < w);
+      before += c_th[k] < th;
+      equal += c_th[k] == th;
     }
   }
   s_cnt[wid][lane] = before;
+  s_eq[wid][lane] = equal;
   __syncthreads();
   if (wid != 0 || m >= n) return;
+  int il = 1;
+  equal = 0;
+  for (int u = 0; u < WAVES; u++) {
+    il += s_cnt[u][lane];
+    equal += s_eq[u][lane];
+  }
+  if (equal > 1)  // members with the same angle: by water index
+    for (int k = 0; k < n; k++) il += ldg(L_th + k) == th && ldg(L_w + k) < w;
   const double pi = 3.141592653589793;
-  const int il = s_cnt[0][lane] + s_cnt[1][lane] + s_cnt[2][lane] + s_cnt[3][lane] + 1;
   const double tc = S.sh_state[sh];
   double arg = 1.0 + (1.0 - 2.0 * (double)il) / (double)n;
   double th0 = acos(arg);
@@ -1999,8 +1989,32 @@ __global__ __launch_bounds__(256) void k_pol_bonded(const DevSys* __restrict__ s
   stg(o + 1, th);
 }
 
-template __global__ void k_pol_bonded<false>(const DevSys*, int);
-template __global__ void k_pol_bonded<true>(const DevSys*, int);
+// the bonded terms of atom i into its rows, for k_integrate
+__device__ __forceinline__ void bonded_rows(const DevSys& S, int i) {
+  if (i >= S.nbat) return;
+  double f[3] = {0.0, 0.0, 0.0}, eb = 0.0, ea = 0.0;
+  bonded_atom(S, i, f, eb, ea);
+  for (int c = 0; c < 3; c++) stg(S.brow + 3 * i + c, f[c]);
+}
+
+// In a small step the bonded terms (blocks from pol on) share the launch of the
+// polarisation blocks, whose latency is the longer one; where the restraint
+// runs beside full force kernels the two are launches of their own, because the
+// 106 registers of the bonded terms (32 without) keep those from the CUs: 51
+// windows of 11,056 atoms, 847 us per step in one launch, 834 in two.  A block of
+// the small launch takes the atoms of one wave: 16 waves of FP64 angles on one
+// CU took 21 us for 4,000 atoms, spread 9 us.
+__global__ __launch_bounds__(64 * POL_SMALL_WAVES) void k_pol_bonded(const DevSys* __restrict__ systems, int pol) {
+  const DevSys& S = systems[blockIdx.y];
+  if ((int)blockIdx.x < pol) pol_forces<POL_SMALL_WAVES>(S);
+  else if (threadIdx.x < QNB_WAVE) bonded_rows(S, ((int)blockIdx.x - pol) * QNB_WAVE + threadIdx.x);
+}
+__global__ __launch_bounds__(256) void k_pol_forces(const DevSys* __restrict__ systems) {
+  pol_forces<4>(systems[blockIdx.y]);
+}
+__global__ __launch_bounds__(256) void k_bonded_rows(const DevSys* __restrict__ systems) {
+  bonded_rows(systems[blockIdx.y], blockIdx.x * blockDim.x + threadIdx.x);
+}
 
 // Phase 3 on its own, one wave per system (watpol_finish): the minimiser's
 // step; the MD step runs it in k_integrate, a single evaluation in
