@@ -59,11 +59,13 @@ void launch_bonded_rows(hipStream_t st, int bonded_atoms, int B, const DevSys* d
 
 // Up to this many receiver waves (four per solute group, one per solvent
 // molecule) a force pass is one launch of k_forces_small: 256 CUs hold 3,072
-// of its waves at a time.  Measured per MD step, that kernel against the
-// separate ones on two streams: 62 against 78 us at 1,160 waves, 92 / 97 at
-// 3,950 (FP64: 111 / 122), 87 / 99 at 9,300 of few solute groups, but 116 / 110
-// at 7,900 with 800 solute groups (FP64: 157 / 149).
-bool small_launch(long solute_groups, long solvent) { return 4 * solute_groups + solvent <= 6144; }
+// of its waves at a time.  Measured per MD step, the separate kernels on two
+// streams against that one: 74 and 55 us at 6,700 waves, 79 and 63 at 8,900, 87
+// and 81 at 7,900 with 800 solute groups (FP64: 104 and 92); at 11,900 with
+// 1,200 solute groups 103 and 106 (FP64: 125 and 122), where the four-way split
+// of a solute group costs what the launches save.  One evaluation at 6,500
+// waves: 260 and 202 us.
+bool small_launch(long solute_groups, long solvent) { return 4 * solute_groups + solvent <= 10240; }
 
 __global__ void k_reduce_part(const DevSys*);
 __global__ void k_reduce_final(const DevSys*, int, int);
