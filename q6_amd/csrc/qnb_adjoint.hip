@@ -26,24 +26,21 @@ struct AdjPar {
 template <typename R>
 __device__ __forceinline__ void adj_pair(double (&g)[QNB_ADJ_NV], R r2, R r, const AdjPar<R>& p, bool is14, bool lj,
                                          bool energy) {
-  double e_vdw = 0.0, gA = 0.0, gB = 0.0;
-  if (lj) {
-    R r6 = r2 * r2 * r2;
-    if (p.sc != R(0)) r6 = recip(recip(r6) + p.sc);
-    const R r12 = r6 * r6;
-    e_vdw = (double)(p.A * r12) - (double)(p.B * r6);
-    gA = (double)(p.tA * r12);
-    gB = -(double)(p.tB * r6);
-  }
   g[ADJ_DQ] += (double)(p.tq * r);
-  g[ADJ_DA] += is14 ? 0.0 : gA;
-  g[ADJ_DB] += is14 ? 0.0 : gB;
-  g[ADJ_DA14] += is14 ? gA : 0.0;
-  g[ADJ_DB14] += is14 ? gB : 0.0;
-  if (energy) {
-    g[ADJ_EEL] += (double)(p.el * r);
-    g[ADJ_EVDW] += e_vdw;
+  if (energy) g[ADJ_EEL] += (double)(p.el * r);
+  if (!lj) return;
+  R r6 = r2 * r2 * r2;
+  if (p.sc != R(0)) r6 = recip(recip(r6) + p.sc);
+  const R r12 = r6 * r6;
+  const double gA = (double)(p.tA * r12), gB = (double)(p.tB * r6);
+  if (is14) {
+    g[ADJ_DA14] += gA;
+    g[ADJ_DB14] -= gB;
+  } else {
+    g[ADJ_DA] += gA;
+    g[ADJ_DB] -= gB;
   }
+  if (energy) g[ADJ_EVDW] += (double)(p.A * r12) - (double)(p.B * r6);
 }
 
 // One block per (frame, Q-atom), its four waves taking every fourth 64 waters,
@@ -53,7 +50,8 @@ __device__ __forceinline__ void adj_pair(double (&g)[QNB_ADJ_NV], R r2, R r, con
 // tables of a site held over the waters, and each solute atom's list test from
 // its own word (qp_test) instead of through group, switch atom and exclusion
 // take 6 instances x 20 frames x 30 Q-atoms of 1,200 + 3,100 atoms from 175 to
-// 158 us (FP32 pairs), 24 frames x 18 Q-atoms from 50 to 20 us (FP64).
+// 158 us (FP32 pairs), and a water read once for its three sites to 100; 24
+// frames x 18 Q-atoms from 50 to 20 and 17 us (FP64).
 #define ADJ_WPB 4
 template <typename R, int NS>
 __global__ __launch_bounds__(QNB_WAVE* ADJ_WPB) void k_adjoint(const DevSys* __restrict__ systems,
@@ -89,28 +87,57 @@ __global__ __launch_bounds__(QNB_WAVE* ADJ_WPB) void k_adjoint(const DevSys* __r
   };
 
   // Q-water: every water whose oxygen lies within Rcq of the Q-list centre
-  for (int k = 0; k < sa; k++) {
-    AdjPar<R> p[NS];
-#pragma unroll
-    for (int s = 0; s < NS; s++) {
-      if (s >= ns || S.nwat <= 0) break;
-      const size_t t = (size_t)iq + (size_t)nq * ((size_t)k + (size_t)sa * s);
-      p[s] = AdjPar<R>{(R)S.qwA[t], (R)S.qwB[t], (R)S.qwEl[t], (R)S.qwSc[t],
-                       (R)A.qw_dq[t], (R)A.qw_dA[t], (R)A.qw_dB[t]};
-    }
-    const bool lj = k == 0 || !S.spc;
-#pragma unroll 2
+  const auto qw_par = [&](int k, int s) {
+    const size_t t = (size_t)iq + (size_t)nq * ((size_t)k + (size_t)sa * s);
+    return AdjPar<R>{(R)ldg(S.qwA + t), (R)ldg(S.qwB + t), (R)ldg(S.qwEl + t), (R)ldg(S.qwSc + t),
+                     (R)ldg(A.qw_dq + t), (R)ldg(A.qw_dA + t), (R)ldg(A.qw_dB + t)};
+  };
+  if (sa == 3) {
+    // a water's nine coordinates in one run, the parameters of its sites in LDS
+    // (the same for every lane): the loads' 72-byte strides, not the pairs, are
+    // what a pass per site waits for
+    __shared__ AdjPar<R> par[3][NS];
+    if (t0 < 3 * ns && S.nwat > 0) par[t0 / ns][t0 % ns] = qw_par(t0 / ns, t0 % ns);
+    __syncthreads();
     for (int w = t0; w < S.nwat; w += QNB_WAVE * ADJ_WPB) {
-      const int o = nsol + sa * w, j = o + k;
-      const double ox = x[3 * o], oy = x[3 * o + 1], oz = x[3 * o + 2];
-      const double jx = x[3 * j], jy = x[3 * j + 1], jz = x[3 * j + 2];
-      if (ldg(S.excl + o) || !inside(ox, oy, oz)) continue;
-      R r2, r;
-      inv(jx, jy, jz, xi0, xi1, xi2, r2, r);
+      const int o = nsol + 3 * w;
+      double xw[3][3];
+      for (int k = 0; k < 3; k++)
+        for (int c = 0; c < 3; c++) xw[k][c] = x[3 * (o + k) + c];
+      if (ldg(S.excl + o) || !inside(xw[0][0], xw[0][1], xw[0][2])) continue;
+      __asm__ volatile("" ::: "memory");  // the parameters stay in LDS, not in registers over the loop
+#pragma unroll
+      for (int k = 0; k < 3; k++) {
+        R r2, r;
+        inv(xw[k][0], xw[k][1], xw[k][2], xi0, xi1, xi2, r2, r);
+#pragma unroll
+        for (int s = 0; s < NS; s++) {
+          if (s >= ns) break;
+          adj_pair<R>(g[s], r2, r, par[k][s], false, k == 0 || !S.spc, true);
+        }
+      }
+    }
+  } else {
+    for (int k = 0; k < sa; k++) {
+      AdjPar<R> p[NS];
 #pragma unroll
       for (int s = 0; s < NS; s++) {
-        if (s >= ns) break;
-        adj_pair<R>(g[s], r2, r, p[s], false, lj, true);
+        if (s >= ns || S.nwat <= 0) break;
+        p[s] = qw_par(k, s);
+      }
+      const bool lj = k == 0 || !S.spc;
+      for (int w = t0; w < S.nwat; w += QNB_WAVE * ADJ_WPB) {
+        const int o = nsol + sa * w, j = o + k;
+        const double ox = x[3 * o], oy = x[3 * o + 1], oz = x[3 * o + 2];
+        const double jx = x[3 * j], jy = x[3 * j + 1], jz = x[3 * j + 2];
+        if (ldg(S.excl + o) || !inside(ox, oy, oz)) continue;
+        R r2, r;
+        inv(jx, jy, jz, xi0, xi1, xi2, r2, r);
+#pragma unroll
+        for (int s = 0; s < NS; s++) {
+          if (s >= ns) break;
+          adj_pair<R>(g[s], r2, r, p[s], false, lj, true);
+        }
       }
     }
   }
