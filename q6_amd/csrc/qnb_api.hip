@@ -31,7 +31,6 @@ template <typename R, int NS>
 __global__ void k_qq(const DevSys*, uint32_t);
 __global__ void k_pack_xq(const DevSys*);
 __global__ void k_pw_first(const DevSys*);
-__global__ void k_expand(const DevSys*);
 __global__ void k_watpol_theta(const DevSys*, const int*);
 __global__ void k_pol_bonded(const DevSys*, int);
 __global__ void k_pol_forces(const DevSys*);
@@ -708,7 +707,6 @@ static void launch_lists(qnb_handle* h) {
     hipLaunchKernelGGL(k_pw_first, dim3((h->hs.ncgp_solute + 3) / 4, 1), dim3(256), 0, h->stream, h->dsys);
   if (h->hs.any_atom) hipLaunchKernelGGL((k_lists_lrf<R, true>), grid, dim3(64 * wpb), 0, h->stream, h->dsys);
   else hipLaunchKernelGGL((k_lists_lrf<R, false>), grid, dim3(64 * wpb), 0, h->stream, h->dsys);
-  hipLaunchKernelGGL(k_expand, grid, dim3(64 * wpb), 0, h->stream, h->dsys);
 }
 
 extern "C" int32_t qnb_make_pair_lists(qnb_handle* h, const double* x) {
@@ -736,8 +734,8 @@ extern "C" int32_t qnb_make_pair_lists(qnb_handle* h, const double* x) {
     hipLaunchKernelGGL(k_qlists, dim3(1), dim3(1024), 0, h->stream, h->dsys);
     HIPCHK(hipGetLastError());
     h->qlists_built = true;
+    HIPCHK(hipStreamSynchronize(h->stream));
   }
-  HIPCHK(hipStreamSynchronize(h->stream));
   h->lists_built = true;
   return 0;
 }

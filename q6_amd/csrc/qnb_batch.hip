@@ -20,7 +20,6 @@ __global__ void k_lists_lrf(const DevSys*);
 __global__ void k_qlists(const DevSys*);
 __global__ void k_pack_xq(const DevSys*);
 __global__ void k_pw_first(const DevSys*);
-__global__ void k_expand(const DevSys*);
 template <typename R, int NS, bool E>
 __global__ void k_wforces(const DevSys*, uint32_t, int, int, int);
 template <typename R, int NS, bool E>
@@ -561,8 +560,7 @@ __global__ void k_exc_record(const DevSys* __restrict__ systems, const MdDev* __
                              const ExcDev* __restrict__ excs);
 
 // launchers shared by the step, the minimiser, the timer and the autotuner
-// `rows`: expand the neighbour rows into partner atoms too
-static void launch_lists(qnb_batch* b, int wpb, bool rows = true) {
+static void launch_lists(qnb_batch* b, int wpb) {
   dim3 g((b->maxg + wpb - 1) / wpb, b->n), t(64 * wpb);
   bool any = false, quirk = false;
   int maxsg = 0;
@@ -580,7 +578,6 @@ static void launch_lists(qnb_batch* b, int wpb, bool rows = true) {
     if (any) hipLaunchKernelGGL((k_lists_lrf<double, true>), g, t, 0, b->stream, b->dsys);
     else hipLaunchKernelGGL((k_lists_lrf<double, false>), g, t, 0, b->stream, b->dsys);
   }
-  if (rows) hipLaunchKernelGGL(k_expand, dim3((b->maxg + 3) / 4, b->n), dim3(256), 0, b->stream, b->dsys);
 }
 
 static const uint32_t kStepMask = QNB_T_NONBONDED | QNB_T_QQ | QNB_T_QQP | QNB_T_RAD | QNB_T_POL;
@@ -993,7 +990,7 @@ extern "C" int32_t qnb_batch_create(int32_t n, const qnb_system* const* sys, con
     HIPCHK(hipMemcpy(b->dsys, b->hs.data(), sizeof(DevSys) * n, hipMemcpyHostToDevice));
     for (int k = 0; k < n; k++) HIPCHK(hipMemset(b->hs[k].need, 0, sizeof(int)));
     const int wpb = 4;
-    launch_lists(b.get(), wpb, false);
+    launch_lists(b.get(), wpb);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(b->stream));
     bool again = false;

@@ -75,7 +75,7 @@ struct DevSys {
   // word of the list sweep's 64-group chunk
   const uint64_t* gbit;
   int ncgpat;
-  const int* cgentry;  // per group-ordered atom: its index, with AL_SKIP for a Q-atom (k_expand)
+  const int* cgentry;  // per group-ordered atom: its index, with AL_SKIP for a Q-atom (expand_row)
   const double* avdw;  // [t*3+k]
   const double* bvdw;
   const int* ljcod;    // [ti + tj*ntypes], 1-based code
@@ -170,7 +170,7 @@ struct DevSys {
   double* lrf;
   int* nbr;
   int* nnbr;
-  // partner atoms of each receiver (k_expand): rows of acap slots, the slots in
+  // partner atoms of each receiver (expand_row): rows of acap slots, the slots in
   // use [ncgp], slots per batch of groups
   int* alist;
   int* alist_n;

@@ -138,7 +138,7 @@ void launch_bonded_rows(hipStream_t st, int bonded_atoms, int B, const DevSys* d
 // per-instance device state (coordinates, gradient, lists, LRF, energies)
 int instance_alloc(DevSys& S, DevAlloc& M, const qnb_params* p, int nslots);
 // neighbour rows of `cap` groups; entries per partner-atom row that always
-// hold such a row's atoms (k_expand), and the rows themselves
+// hold such a row's atoms (expand_row), and the rows themselves
 int row_alloc(DevSys& S, DevAlloc& M, int cap);
 int atom_row_cap(const DevSys& S, const HostTopo& T);
 int atom_rows_alloc(DevSys& S, const HostTopo& T, DevAlloc& M);

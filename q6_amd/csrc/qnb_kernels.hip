@@ -253,6 +253,76 @@ __device__ __forceinline__ double dist4v(const d4v& a, const d4v& b) {
 }
 
 // ---------------------------------------------------------------------------
+// Partner atoms of receiver group a, written by its wave at the end of a list
+// update (nsr: the solute groups of its row) and read by the force kernels of
+// every step until the next one: the solute groups of the row's prefix as
+// atoms.  Lane = partner group; the groups are taken in batches of up to 64 whose atoms fit
+// in `batch` slots (al_batch) and every batch ends at a multiple of 64 slots,
+// so lane l of the force kernels, taking slots l, l + 64, ..., always adds the
+// same partners in the same order.  An entry is the atom's index with AL_OWN
+// (the receiver owns the energy of the two groups' pairs) and AL_FAR (a solute
+// receiver and a group that can hold no excluded or 1-4 pair with it: every
+// index more than 25 from the receiver's, no long-range partners in either);
+// AL_SKIP marks Q-atoms (their pairs belong to the Q kernels) and the padding.
+// The force kernels then read one coalesced list per receiver instead of
+// walking group -> atoms -> positions through LDS at every step.  A launch of
+// its own cost a list update 7 us.
+#define LS_WPB 8  // waves per block of the list sweep at most
+__device__ __forceinline__ void expand_row(const DevSys& S, int a, int nsr, int lane, int w) {
+  const int batch = S.al_batch;
+  const bool a_sol = a < S.ncgp_solute;
+  const int* row = S.nbr + (size_t)a * S.cap;
+  int* out = S.alist + (size_t)a * S.acap;
+  const bool along = a_sol && ldg(S.glong + a);
+  const int alo = a_sol ? ldg(S.gspan + 2 * a) : 0, ahi = a_sol ? ldg(S.gspan + 2 * a + 1) : 0;
+  __shared__ int s_incl[LS_WPB][QNB_WAVE], s_src[LS_WPB][QNB_WAVE], s_tag[LS_WPB][QNB_WAVE];
+  int n = 0;
+  for (int p0 = 0, ng = 0; p0 < nsr; p0 += ng) {
+    const int p = p0 + lane;
+    int f0 = 0, cnt = 0, tag = 0;
+    if (p < nsr) {
+      const int b = ldg(row + p);
+      f0 = ldg(S.gfirst + b);
+      cnt = ldg(S.glast + b) - f0 + 1;
+      const bool blong = ldg(S.glong + b);
+      const int blo = ldg(S.gspan + 2 * b), bhi = ldg(S.gspan + 2 * b + 1);
+      tag = owns(a, b) ? AL_OWN : 0;
+      if (a_sol && !along && !blong && (blo - ahi > 25 || alo - bhi > 25)) tag |= AL_FAR;
+    }
+    int incl = cnt;
+#pragma unroll
+    for (int o = 1; o < QNB_WAVE; o <<= 1) {
+      const int u = __shfl_up(incl, o, QNB_WAVE);
+      if (lane >= o) incl += u;
+    }
+    // inclusive sums never decrease, so the groups that fit are a prefix (a
+    // group always fits)
+    ng = min(__popcll(__ballot(incl <= batch)), nsr - p0);
+    const int total = __shfl(incl, ng - 1, QNB_WAVE);
+    // lane = slot: its group is the first whose inclusive count passes it
+    s_incl[w][lane] = incl;
+    s_src[w][lane] = f0 - (incl - cnt);
+    s_tag[w][lane] = tag;
+    __builtin_amdgcn_wave_barrier();
+    const int end = (total + QNB_WAVE - 1) / QNB_WAVE * QNB_WAVE;
+    for (int s = lane; s < end; s += QNB_WAVE) {
+      int e = AL_SKIP;
+      if (s < total) {
+        int g = 0;
+#pragma unroll
+        for (int h = 32; h > 0; h >>= 1)
+          if (s_incl[w][g + h - 1] <= s) g += h;
+        e = ldg(S.cgentry + s_src[w][g] + s) | s_tag[w][g];
+      }
+      stg(out + n + s, e);
+    }
+    __builtin_amdgcn_wave_barrier();
+    n += end;
+  }
+  if (lane == 0) S.alist_n[a] = n;
+}
+
+// ---------------------------------------------------------------------------
 // Pair-list update with LRF (make_pair_lists, nonbondene.f90:749-837, SPH):
 // one wavefront per receiver charge group a, sweeping the other groups in
 // chunks of 64 (lane = group b; reference atoms are L2-resident).  A pair
@@ -268,15 +338,15 @@ __device__ __forceinline__ double dist4v(const d4v& a, const d4v& b) {
 // for its 20 sums.  Around them: the run is read LRF_U records per lane at a
 // time (64 waters are three), the first before the group tests, from a base
 // that moves in scalar registers; FP32 has the next batch in flight while one
-// is summed, FP64 keeps the registers for a fourth wave.  A record's group is
+// is summed, FP64 the next chunk's groups.  A record's group is
 // one bit of a 64-bit word, so a test is two ANDs and reads past the run find
 // 0; FP64 takes the sums raw too, with rinv in place of a root and three
 // divisions.  Measured: 2,663 -> 2,270 us for 51 windows of 11,056 atoms
 // (FP32), 1,740 -> 870 us for 12 of them in FP64; a list update of 19,440 atoms
-// in FP64 775 -> 403 us.
+// in FP64 775 -> 380 us.
 #define LRF_U 3
 template <typename R, bool ANY>
-__global__ __launch_bounds__(512) void k_lists_lrf(const DevSys* __restrict__ systems) {
+__global__ __launch_bounds__(64 * LS_WPB) void k_lists_lrf(const DevSys* __restrict__ systems) {
   const DevSys& S = systems[blockIdx.y];
   const int a = uni(blockIdx.x * (blockDim.x / QNB_WAVE) + threadIdx.x / QNB_WAVE);
   if (a >= S.ncgp) return;
@@ -302,7 +372,7 @@ __global__ __launch_bounds__(512) void k_lists_lrf(const DevSys* __restrict__ sy
 #pragma unroll
   for (int k = 0; k < LRF_NF; k++) acc[k] = 0.0;
   int count = 0, count_sol = 0;
-  int* __restrict__ row = S.nbr + (size_t)a * S.cap;
+  int* row = S.nbr + (size_t)a * S.cap;
   // mixed path: the lane's FP32 sums since the last flush to FP64, flushed
   // after a chunk once a lane has been offered LRF_FLUSH atoms (at most
   // LRF_FLUSH - 1 plus one chunk's share)
@@ -324,13 +394,17 @@ __global__ __launch_bounds__(512) void k_lists_lrf(const DevSys* __restrict__ sy
     const bool quirk = pw_quirk(S), any_atom = ANY && S.any_atom;
     const double rclrf2 = S.use_lrf ? S.rclrf2 : -1.0;
     using Rec = decltype(lrf_rec<R>(grs, 0));
-    // the chunk's atoms: the run from b0's first to its last group's last
+    // the chunk's atoms: the run from b0's first to its last group's last; FP64
+    // requests the next chunk's groups while it sums this one (FP32 has no
+    // registers for that at four waves per SIMD)
     int k1 = ldc(S.gfirst);
+    d4v Gn = buf_d4(grs, (uint32_t)lane * 32);
     for (int b0 = 0; b0 < ncgp; b0 += QNB_WAVE) {
       const int b = b0 + lane;
-      const d4v G = buf_d4(grs, (uint32_t)b * 32);  // 0 past the last group
+      const d4v G = F32 ? buf_d4(grs, (uint32_t)b * 32) : Gn;  // 0 past the last group
       const int k0 = ldc(S.gfirst + b0);
       k1 = ldc(S.glast + min(b0 + QNB_WAVE, ncgp) - 1) + 1;
+      if constexpr (!F32) Gn = buf_d4(grs, (uint32_t)(b + QNB_WAVE) * 32);
       Rec r[LRF_U];
       u2v s[LRF_U];
       auto fetch = [&](int k, Rec* rr, u2v* ss) {
@@ -441,6 +515,10 @@ __global__ __launch_bounds__(512) void k_lists_lrf(const DevSys* __restrict__ sy
     for (int n = 0; n < 3; n++)
       for (int j = 0; j < 3; j++)
         for (int c = 0; c < 3; c++) L[16 + 3 * (j + 3 * n) + c] = t[t3index(n, j, c)];
+  }
+  if (S.alist) {  // null while the rows are being sized
+    __threadfence_block();  // the row's stores before its loads
+    expand_row(S, a, min(count_sol, S.cap), lane, threadIdx.x / QNB_WAVE);
   }
 }
 
@@ -659,86 +737,12 @@ __device__ __forceinline__ R qw_el(const DevSys& S, int iq, int k, int s) {
 }
 
 // ---------------------------------------------------------------------------
-// Partner atoms of every receiver group, written after each list update and
-// read by the force kernels of every step until the next one: the solute
-// groups of the row's prefix as atoms.  One wavefront per receiver, lane =
-// partner group; the groups are taken in batches of up to 64 whose atoms fit
-// in `batch` slots (al_batch) and every batch ends at a multiple of 64 slots,
-// so lane l of the force kernels, taking slots l, l + 64, ..., always adds the
-// same partners in the same order.  An entry is the atom's index with AL_OWN
-// (the receiver owns the energy of the two groups' pairs) and AL_FAR (a solute
-// receiver and a group that can hold no excluded or 1-4 pair with it: every
-// index more than 25 from the receiver's, no long-range partners in either);
-// AL_SKIP marks Q-atoms (their pairs belong to the Q kernels) and the padding.
-// The force kernels then read one coalesced list per receiver instead of
-// walking group -> atoms -> positions through LDS at every step.
-__global__ __launch_bounds__(256) void k_expand(const DevSys* __restrict__ systems) {
-  const DevSys& S = systems[blockIdx.y];
-  const int a = uni(blockIdx.x * (blockDim.x / QNB_WAVE) + threadIdx.x / QNB_WAVE);
-  if (a >= S.ncgp) return;
-  const int lane = threadIdx.x % QNB_WAVE, batch = S.al_batch;
-  const bool a_sol = a < S.ncgp_solute;
-  const int nsr = uni(min(ldg(S.nnsol + a), S.cap));
-  const int* __restrict__ row = S.nbr + (size_t)a * S.cap;
-  int* __restrict__ out = S.alist + (size_t)a * S.acap;
-  const bool along = a_sol && ldg(S.glong + a);
-  const int alo = a_sol ? ldg(S.gspan + 2 * a) : 0, ahi = a_sol ? ldg(S.gspan + 2 * a + 1) : 0;
-  __shared__ int s_incl[4][QNB_WAVE], s_src[4][QNB_WAVE], s_tag[4][QNB_WAVE];
-  const int w = threadIdx.x / QNB_WAVE;
-  int n = 0;
-  for (int p0 = 0, ng = 0; p0 < nsr; p0 += ng) {
-    const int p = p0 + lane;
-    int f0 = 0, cnt = 0, tag = 0;
-    if (p < nsr) {
-      const int b = ldg(row + p);
-      f0 = ldg(S.gfirst + b);
-      cnt = ldg(S.glast + b) - f0 + 1;
-      tag = owns(a, b) ? AL_OWN : 0;
-      if (a_sol && !along && !ldg(S.glong + b)) {
-        const int blo = ldg(S.gspan + 2 * b), bhi = ldg(S.gspan + 2 * b + 1);
-        if (blo - ahi > 25 || alo - bhi > 25) tag |= AL_FAR;
-      }
-    }
-    int incl = cnt;
-#pragma unroll
-    for (int o = 1; o < QNB_WAVE; o <<= 1) {
-      const int u = __shfl_up(incl, o, QNB_WAVE);
-      if (lane >= o) incl += u;
-    }
-    // inclusive sums never decrease, so the groups that fit are a prefix (a
-    // group always fits)
-    ng = min(__popcll(__ballot(incl <= batch)), nsr - p0);
-    const int total = __shfl(incl, ng - 1, QNB_WAVE);
-    // lane = slot: its group is the first whose inclusive count passes it
-    s_incl[w][lane] = incl;
-    s_src[w][lane] = f0 - (incl - cnt);
-    s_tag[w][lane] = tag;
-    __builtin_amdgcn_wave_barrier();
-    const int end = (total + QNB_WAVE - 1) / QNB_WAVE * QNB_WAVE;
-    for (int s = lane; s < end; s += QNB_WAVE) {
-      int e = AL_SKIP;
-      if (s < total) {
-        int g = 0;
-#pragma unroll
-        for (int h = 32; h > 0; h >>= 1)
-          if (s_incl[w][g + h - 1] <= s) g += h;
-        e = ldg(S.cgentry + s_src[w][g] + s) | s_tag[w][g];
-      }
-      stg(out + n + s, e);
-    }
-    __builtin_amdgcn_wave_barrier();
-    n += end;
-  }
-  if (lane == 0) S.alist_n[a] = n;
-}
-
-// ---------------------------------------------------------------------------
 // Solute receivers: one wavefront per solute charge group a, or, in a small
 // launch (SPLIT), the four waves of a block, each with a quarter of a's
 // partners.  a's atoms are taken in sweeps of up to SO_CH; they are the same
 // for every lane and live in scalar registers, and a lane takes one partner at
 // a time against them, the next partner's data in flight meanwhile:
-//  * solute partners from the receiver's atom list (k_expand; nonbond_pp,
+//  * solute partners from the receiver's atom list (expand_row; nonbond_pp,
 //    nonbondene.f90:4694-4760): those of a group without an excluded or 1-4
 //    pair (AL_FAR) take A, B and qq as products of per-atom factors when the
 //    system uses the geometric rule with LJ code 1 throughout (ppfast): the
@@ -1139,7 +1143,7 @@ __global__ __launch_bounds__(64 * FC_WPB) void k_sforces(const DevSys* __restric
 // Water receivers (rigid 3-site solvent): one wavefront per water a.  Its
 // neighbour row is sorted, so the solute groups (indices below ncgp_solute)
 // come first, then the waters.  Solute partners come from the receiver's atom
-// list (k_expand), one partner atom per lane against the three receiver atoms with
+// list (expand_row), one partner atom per lane against the three receiver atoms with
 // the pw parameters (nonbond_pw, nonbondene.f90:4856-4916; energy counted on
 // the solute side).  Partner waters need no staging: their atoms are
 // consecutive, so in each round lane l takes atom l % 3 of the row's water
