@@ -1896,7 +1896,9 @@ __global__ __launch_bounds__(256) void k_forces_small(const DevSys* __restrict__
 // (the reference's selection sort; ties by water index) is the number of
 // members before it, counted against the shell's list staged in LDS, an equal
 // part of it per wave (equal angles, which only coincidence brings, in a second
-// pass of the members concerned); wave 0 then forms the target angle from the
+// pass of the members concerned; an angle that is not a number, of a water
+// without a dipole direction, counts as the largest, so every member has a rank
+// of its own and its NaN reaches the sums); wave 0 then forms the target angle from the
 // rank, the restraint energy and the forces (adds to d), and writes energy and
 // theta at the member's rank (wp_rank), so the sums over a shell do not depend
 // on the order the angle kernel appended its members in.  Counting is n^2
@@ -1909,6 +1911,7 @@ __global__ __launch_bounds__(256) void k_forces_small(const DevSys* __restrict__
 // WAVES: a small step waits for this kernel, so 16 waves share a count (1,110
 // waters 10.5 -> 8.2 us, 2,352 waters 17 -> 8.5 us against 4); beside full
 // force kernels, whose blocks leave four wave slots sooner than 16, 4 do.
+__device__ __forceinline__ double pol_key(double theta) { return __builtin_fmin(theta, __builtin_inf()); }
 template <int WAVES>
 __device__ __forceinline__ void pol_forces(const DevSys& S) {
   const int lane = threadIdx.x % QNB_WAVE, wid = threadIdx.x / QNB_WAVE;
@@ -1935,18 +1938,18 @@ __device__ __forceinline__ void pol_forces(const DevSys& S) {
   const double* L_th = S.sh_lth + (size_t)sh * nw;
   const int* L_w = S.sh_list + (size_t)sh * nw;
   const int w = m < n ? ldg(L_w + m) : 0;
-  const double th = m < n ? ldg(L_th + m) : 0.0;
+  const double th = m < n ? ldg(L_th + m) : 0.0, key = pol_key(th);
   int before = 0, equal = 0;
   for (int k0 = 0; k0 < n; k0 += WP_CHUNK) {
     const int nk = min(WP_CHUNK, n - k0);
     __syncthreads();
-    for (int k = threadIdx.x; k < nk; k += blockDim.x) c_th[k] = ldg(L_th + k0 + k);
+    for (int k = threadIdx.x; k < nk; k += blockDim.x) c_th[k] = pol_key(ldg(L_th + k0 + k));
     __syncthreads();
     const int q0 = nk * wid / WAVES, q1 = nk * (wid + 1) / WAVES;
 #pragma unroll 8
     for (int k = q0; k < q1; k++) {
-      before += c_th[k] < th;
-      equal += c_th[k] == th;
+      before += c_th[k] < key;
+      equal += c_th[k] == key;
     }
   }
   s_cnt[wid][lane] = before;
@@ -1960,7 +1963,7 @@ __device__ __forceinline__ void pol_forces(const DevSys& S) {
     equal += s_eq[u][lane];
   }
   if (equal > 1)  // members with the same angle: by water index
-    for (int k = 0; k < n; k++) il += ldg(L_th + k) == th && ldg(L_w + k) < w;
+    for (int k = 0; k < n; k++) il += pol_key(ldg(L_th + k)) == key && ldg(L_w + k) < w;
   const double pi = 3.141592653589793;
   const double tc = S.sh_state[sh];
   double arg = 1.0 + (1.0 - 2.0 * (double)il) / (double)n;

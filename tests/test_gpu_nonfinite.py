@@ -1,0 +1,45 @@
+"""Coordinates without a finite answer: what such a call reports, and that it
+leaves the rest of its results and the next call alone.
+
+* A water of a polarisation shell whose dipole has no direction (its hydrogens
+  not a number): every call reports a non-finite energy, the other waters'
+  gradients stay finite, and the next call on finite coordinates equals the
+  oracle (1e-10, the bound of test_gpu_paths).
+"""
+import numpy as np
+import pytest
+
+from oracle.oracle import Oracle
+from q6_amd import abi, synth
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("lost", [1, 3])
+def test_polarisation_angle_not_a_number(lost):
+    from q6_amd.engine import NonbondedEngine
+    s = synth.build(9.0, 0, 1, 0, 1, seed=41, chain_region=4.5, lambdas=[1.0], cut=7.0, water_fill=9.0, name="shells")
+    mask = abi.T_RAD | abi.T_POL
+    x = s.x.copy()
+    out = np.argsort(np.linalg.norm(x[::3], axis=1))[-lost:]  # waters of the outermost shell
+    for w in out:
+        x[3 * w + 1:3 * w + 3] = np.nan
+    print(f"\n[gpu] {synth.describe(s)}: hydrogens of {lost} waters not a number", flush=True)
+    eng = NonbondedEngine(s, precision=abi.QNB_PREC_FP64)
+    eng.make_pair_lists(s.x)
+    state = eng.shell_state()
+    for _ in range(5):
+        d = np.zeros_like(x)
+        with pytest.raises(abi.QnbError, match="non-finite"):
+            eng.eval_terms(mask, x, Tfree=300.0, d=d)
+        lostatoms = np.isin(np.arange(len(x)) // 3, out)
+        assert np.all(np.isfinite(d[~lostatoms])) and np.all(np.isnan(d[lostatoms]).any(1))
+        eng.set_shell_state(state)
+    o = Oracle(s)
+    o.make_pair_lists(s.x)
+    do, Eo, _ = o.eval_terms(mask, s.x, Tfree=300.0)
+    d, E, _ = eng.eval_terms(mask, s.x, Tfree=300.0)
+    assert np.max(np.abs(d - do)) <= 1e-10 * np.max(np.abs(do))
+    assert abs(E["water_pol"] - Eo["water_pol"]) <= 1e-10 * abs(Eo["water_pol"])
+    assert np.allclose(eng.shell_state(), o.shell_state(), rtol=1e-10, atol=1e-12)
+    eng.close()
