@@ -77,16 +77,18 @@ __global__ __launch_bounds__(QNB_WAVE* ADJ_WPB) void k_adjoint(const DevSys* __r
     rinv(ux * ux + uy * uy + uz * uz, r2, r);
   };
   // dist4p's sum for the point (a, b, c) and the Q-list centre
-  auto inside = [&](double a, double b, double c) {
+  auto dist2 = [&](double a, double b, double c) {
 #pragma clang fp contract(off)
     const double dx = xp0 - a, dy = xp1 - b, dz = xp2 - c;
     double d = dx * dx;
     d = d + dy * dy;
     d = d + dz * dz;
-    return d <= rcq2;
+    return d;
   };
 
-  // Q-water: every water whose oxygen lies within Rcq of the Q-list centre
+  // Q-water: every water whose oxygen lies within Rcq of the Q-list centre; one
+  // whose position is not a number is not left out, so that its frame's results
+  // show it
   const auto qw_par = [&](int k, int s) {
     const size_t t = (size_t)iq + (size_t)nq * ((size_t)k + (size_t)sa * s);
     return AdjPar<R>{(R)ldg(S.qwA + t), (R)ldg(S.qwB + t), (R)ldg(S.qwEl + t), (R)ldg(S.qwSc + t),
@@ -104,7 +106,7 @@ __global__ __launch_bounds__(QNB_WAVE* ADJ_WPB) void k_adjoint(const DevSys* __r
       double xw[3][3];
       for (int k = 0; k < 3; k++)
         for (int c = 0; c < 3; c++) xw[k][c] = x[3 * (o + k) + c];
-      if (ldg(S.excl + o) || !inside(xw[0][0], xw[0][1], xw[0][2])) continue;
+      if (ldg(S.excl + o) || dist2(xw[0][0], xw[0][1], xw[0][2]) > rcq2) continue;
       __asm__ volatile("" ::: "memory");  // the parameters stay in LDS, not in registers over the loop
 #pragma unroll
       for (int k = 0; k < 3; k++) {
@@ -130,7 +132,7 @@ __global__ __launch_bounds__(QNB_WAVE* ADJ_WPB) void k_adjoint(const DevSys* __r
         const int o = nsol + sa * w, j = o + k;
         const double ox = x[3 * o], oy = x[3 * o + 1], oz = x[3 * o + 2];
         const double jx = x[3 * j], jy = x[3 * j + 1], jz = x[3 * j + 2];
-        if (ldg(S.excl + o) || !inside(ox, oy, oz)) continue;
+        if (ldg(S.excl + o) || dist2(ox, oy, oz) > rcq2) continue;
         R r2, r;
         inv(jx, jy, jz, xi0, xi1, xi2, r2, r);
 #pragma unroll
@@ -154,7 +156,7 @@ __global__ __launch_bounds__(QNB_WAVE* ADJ_WPB) void k_adjoint(const DevSys* __r
     if (sw < 0) continue;
     if (S.any_atom) {
       if (!qp_group_in(S, A.frames + (size_t)f * 3 * S.natom, ldg(S.atom_group + j))) continue;
-    } else if (!inside(x[3 * sw], x[3 * sw + 1], x[3 * sw + 2])) {
+    } else if (!(dist2(x[3 * sw], x[3 * sw + 1], x[3 * sw + 2]) <= rcq2)) {
       continue;
     }
     R r2, r;

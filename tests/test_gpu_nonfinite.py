@@ -5,6 +5,8 @@ leaves the rest of its results and the next call alone.
   not a number): every call reports a non-finite energy, the other waters'
   gradients stay finite, and the next call on finite coordinates equals the
   oracle (1e-10, the bound of test_gpu_paths).
+* A frame with a water that is not a number: the adjoint's sums over the waters
+  of that frame are not numbers, those of the other frames are unchanged.
 """
 import numpy as np
 import pytest
@@ -43,3 +45,27 @@ def test_polarisation_angle_not_a_number(lost):
     assert abs(E["water_pol"] - Eo["water_pol"]) <= 1e-10 * abs(Eo["water_pol"])
     assert np.allclose(eng.shell_state(), o.shell_state(), rtol=1e-10, atol=1e-12)
     eng.close()
+
+
+def nine_site():
+    s = synth.build(13.0, 3, 6, 1, 2, 41, chain_region=5.0, q_sigma=0.4, lambdas=[0.4, 0.6], water_fill=12.0)
+    return synth.replace_solvent(s, synth.ethanol(), 0.0085, 48)
+
+
+@pytest.mark.parametrize("precision", [abi.QNB_PREC_FP64, abi.QNB_PREC_MIXED])
+@pytest.mark.parametrize("build", [lambda: synth.build(11.0, 4, 8, 2, 2, seed=5, chain_region=5.0, q_sigma=0.4,
+                                                       lambdas=[0.3, 0.7], cut=7.0, q_per_chain=4), nine_site],
+                         ids=["water", "nine_site"])
+def test_adjoint_of_a_lost_water(build, precision):
+    from q6_amd import adjoint
+    from q6_amd.engine import NonbondedEngine
+    s = build()
+    frames = np.stack([s.x] * 3)
+    frames[1, s.n["nat_solute"]:s.n["nat_solute"] + s.n["solv_atom"]] = np.nan
+    print(f"\n[gpu] {synth.describe(s)} precision {precision}: first solvent molecule of frame 1 lost", flush=True)
+    tangent, _keep = adjoint.tangent_struct(s)
+    eng = NonbondedEngine(s, precision=precision)
+    out = eng.adjoint(tangent, frames)
+    eng.close()
+    assert np.all(np.isfinite(out[[0, 2]])) and np.array_equal(out[0], out[2])
+    assert np.all(np.isnan(out[1][..., [abi.ADJ_DQ, abi.ADJ_DA, abi.ADJ_DB, abi.ADJ_EEL, abi.ADJ_EVDW]]))
