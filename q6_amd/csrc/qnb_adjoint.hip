@@ -44,7 +44,7 @@ __device__ __forceinline__ void adj_pair(double (&g)[QNB_ADJ_NV], R r2, R r, con
 }
 
 // One block per (frame, Q-atom), its four waves taking every fourth 64 waters,
-// solute atoms and Q pairs; grid.y = instance.  A wave's pass is a few dozen
+// solute atoms and Q pairs; grid.y = instance, rows of blocks along z.  A wave's pass is a few dozen
 // iterations of dependent loads, so the kernel is bound by their latency until
 // the waves fill the chip: four waves per sum instead of one, the Q-water
 // tables of a site held over the waters, and each solute atom's list test from
@@ -61,7 +61,8 @@ __global__ __launch_bounds__(QNB_WAVE* ADJ_WPB) void k_adjoint(const DevSys* __r
   const int nq = S.nqat, ns = S.nstates, sa = S.sa, nsol = S.nat_solute;
   if (nq <= 0) return;
   const int t0 = threadIdx.x, lane = t0 % QNB_WAVE;
-  const int f = blockIdx.x / nq, iq = blockIdx.x % nq;
+  const uint32_t blk = blockIdx.z * gridDim.x + blockIdx.x;
+  const int f = (int)(blk / (uint32_t)nq), iq = (int)(blk % (uint32_t)nq);
   if (f >= A.nframes) return;
   const auto x = gp(A.frames + (size_t)f * 3 * S.natom);
   const int i = S.iqseq[iq];
@@ -259,9 +260,13 @@ int adjoint_pack(DevPack& M, const DevSys& S, const qnb_qtangent* t, AdjDev& A) 
   return 0;
 }
 
+// A launch holds fewer than 2^32 threads along x: 16.7 million blocks, which
+// 84,000 frames of 200 Q-atoms pass; more than 2^22 blocks are laid out in
+// several rows along z.
 template <typename R>
-static void launch_adj_r(hipStream_t st, int ns_max, int blocks, int B, const DevSys* dsys, const AdjDev* dadj) {
-  dim3 grid(blocks, B), block(QNB_WAVE * ADJ_WPB);
+static void launch_adj_r(hipStream_t st, int ns_max, long blocks, int B, const DevSys* dsys, const AdjDev* dadj) {
+  const long most = 1l << 22, rows = (blocks + most - 1) / most;
+  dim3 grid((unsigned)((blocks + rows - 1) / rows), B, (unsigned)rows), block(QNB_WAVE * ADJ_WPB);
   if (ns_max <= 1) hipLaunchKernelGGL((k_adjoint<R, 1>), grid, block, 0, st, dsys, dadj);
   else if (ns_max <= 2) hipLaunchKernelGGL((k_adjoint<R, 2>), grid, block, 0, st, dsys, dadj);
   else if (ns_max <= 4) hipLaunchKernelGGL((k_adjoint<R, 4>), grid, block, 0, st, dsys, dadj);
@@ -271,8 +276,8 @@ static void launch_adj_r(hipStream_t st, int ns_max, int blocks, int B, const De
 // blocks = max over instances of nframes * nqat
 void launch_adjoint(hipStream_t st, int prec, int ns_max, long blocks, int B, const DevSys* dsys, const AdjDev* dadj) {
   if (blocks <= 0 || B <= 0) return;
-  if (prec == QNB_PREC_MIXED) launch_adj_r<float>(st, ns_max, (int)blocks, B, dsys, dadj);
-  else launch_adj_r<double>(st, ns_max, (int)blocks, B, dsys, dadj);
+  if (prec == QNB_PREC_MIXED) launch_adj_r<float>(st, ns_max, blocks, B, dsys, dadj);
+  else launch_adj_r<double>(st, ns_max, blocks, B, dsys, dadj);
 }
 
 }  // namespace qnb
