@@ -895,18 +895,31 @@ __device__ __forceinline__ bool pp_param(const DevSys& S, int i, int j, double& 
   return set;
 }
 
-// 1/|u|^2 and 1/|u| from |u|^2: IEEE division and square root in FP64 (the
-// plain path evaluates them as q_dist does); in FP32 the hardware reciprocal
-// square root (v_rsq_f32, 1 ulp), the usual FP32 pair-kernel form
-// FP64: the hardware's reciprocal root (about 26 bits) with one third-order
-// step, y (1 + e/2 + 3 e^2/8) with e = 1 - d2 y^2, and 1/d2 from its square with
-// one Newton step: 15 slots and no branch, a division and a root took about 32
-__device__ __forceinline__ void rinv(double d2, double& r2, double& r) {
+// 1/|u|^2 and 1/|u| from |u|^2.  FP32: the hardware reciprocal square root
+// (v_rsq_f32, 1 ulp), the usual pair-kernel form.  FP64: the hardware's
+// reciprocal root (about 26 bits) with one third-order step,
+// y (1 + e/2 + 3 e^2/8) with e = 1 - d2 y^2, and 1/d2 from its square with one
+// Newton step: 15 slots and no branch, a division and a root took about 32.
+// The steps turn the limits (d2 = 0: infinite, d2 = inf: 0) into NaN, so rinv
+// takes the hardware's value there, 5 slots; the LRF sweep, whose q/r^3 r^2 is
+// NaN at both limits in any case, does without (rinv_inner).
+__device__ __forceinline__ void rinv_inner(double d2, double& r2, double& r) {
   const double y = __builtin_amdgcn_rsq(d2);
   const double e = __builtin_fma(-d2 * y, y, 1.0);
   r = __builtin_fma(y * e, __builtin_fma(0.375, e, 0.5), y);
   const double s = r * r;
   r2 = __builtin_fma(s, __builtin_fma(-d2, s, 1.0), s);
+}
+__device__ __forceinline__ void rinv(double d2, double& r2, double& r) {
+  rinv_inner(d2, r2, r);
+  const bool limit = __builtin_amdgcn_class(d2, 0x260);  // +0, -0, +inf
+  const double y = __builtin_amdgcn_rsq(d2);
+  r = limit ? y : r;
+  r2 = limit ? y : r2;
+}
+__device__ __forceinline__ void rinv_inner(float d2, float& r2, float& r) {
+  r = __builtin_amdgcn_rsqf(d2);
+  r2 = r * r;
 }
 __device__ __forceinline__ void rinv(float d2, float& r2, float& r) {
   r = __builtin_amdgcn_rsqf(d2);

@@ -102,7 +102,7 @@ typedef double d2v __attribute__((ext_vector_type(2)));
 template <typename R>
 __device__ __forceinline__ void lrf_accumulate(R* p, R dx, R dy, R dz, R q) {
   R ri2, ri;
-  rinv(norm2(dx, dy, dz), ri2, ri);
+  rinv_inner(norm2(dx, dy, dz), ri2, ri);
   const R qri = q * ri;
   p[0] += qri;
   const R f0 = qri * ri2;

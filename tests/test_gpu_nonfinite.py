@@ -7,10 +7,16 @@ leaves the rest of its results and the next call alone.
   oracle (1e-10, the bound of test_gpu_paths).
 * A frame with a water that is not a number: the adjoint's sums over the waters
   of that frame are not numbers, those of the other frames are unchanged.
+* Two atoms in one place and an atom 1e160 A away, whose squared distances are 0
+  and infinite: infinite sums where the enumeration in numpy has them, finite
+  ones beside them (1e-10; FP32 pairs 5e-6 of the largest of their kind, the
+  bound of test_gpu_shapes); the far atom adds nothing to an FP64 evaluation
+  (in FP32 its position itself is infinite).
 """
 import numpy as np
 import pytest
 
+from adjoint_ref import slot_sums
 from oracle.oracle import Oracle
 from q6_amd import abi, synth
 
@@ -69,3 +75,52 @@ def test_adjoint_of_a_lost_water(build, precision):
     eng.close()
     assert np.all(np.isfinite(out[[0, 2]])) and np.array_equal(out[0], out[2])
     assert np.all(np.isnan(out[1][..., [abi.ADJ_DQ, abi.ADJ_DA, abi.ADJ_DB, abi.ADJ_EEL, abi.ADJ_EVDW]]))
+
+
+def limits_case():
+    s = synth.build(11.0, 4, 8, 2, 2, seed=5, chain_region=5.0, q_sigma=0.4, lambdas=[0.3, 0.7], cut=7.0, q_per_chain=4)
+    a = s.a
+    away = [j for j in range(s.n["nat_solute"]) if not a["qconn3"][j] and j not in a["cgp_iswitch"]]
+    same, far = s.x.copy(), s.x.copy()
+    same[away[-1]] = s.x[a["iqseq"][0]]
+    far[away[-1], 0] = 1e160
+    return s, same, far
+
+
+@pytest.mark.parametrize("precision,tol", [(abi.QNB_PREC_FP64, 1e-10), (abi.QNB_PREC_MIXED, 5e-6)])
+def test_adjoint_at_the_limits_of_a_distance(precision, tol):
+    from q6_amd import adjoint
+    from q6_amd.engine import NonbondedEngine
+    s, same, far = limits_case()
+    print(f"\n[gpu] {synth.describe(s)} precision {precision}: an atom on a Q-atom; one far away", flush=True)
+    tangent, _keep = adjoint.tangent_struct(s)
+    eng = NonbondedEngine(s, precision=precision)
+    out = eng.adjoint(tangent, np.stack([same, far]))
+    eng.close()
+    tang = synth.q_tangents(s.md["qctx"], s.md["qcrg"], s.md["qA"], s.md["qB"])
+    with np.errstate(all="ignore"):
+        ref = np.stack([slot_sums(s, x, tang) for x in (same, far)])
+    assert np.isinf(ref[0]).any() and np.all(np.isfinite(ref[1]))
+    assert np.array_equal(np.isnan(out), np.isnan(ref))
+    assert np.array_equal(np.where(np.isinf(out), out, 0.0), np.where(np.isinf(ref), ref, 0.0))
+    m = np.isfinite(ref)
+    for c in range(abi.QNB_ADJ_NV):
+        o, r = out[..., c][m[..., c]], ref[..., c][m[..., c]]
+        assert np.max(np.abs(o - r)) <= tol * np.max(np.abs(r)), c
+
+
+def test_evaluation_with_a_far_atom():
+    from q6_amd.engine import NonbondedEngine
+    s, _, far = limits_case()
+    print(f"\n[gpu] {synth.describe(s)}: one atom far away", flush=True)
+    mask = abi.T_PP | abi.T_PW
+    o = Oracle(s)
+    o.make_pair_lists(s.x)
+    do, Eo, _ = o.eval_terms(mask, far, Tfree=300.0)
+    eng = NonbondedEngine(s, precision=abi.QNB_PREC_FP64)
+    eng.make_pair_lists(s.x)
+    d, E, _ = eng.eval_terms(mask, far, Tfree=300.0)
+    eng.close()
+    assert np.all(np.isfinite(do)) and np.max(np.abs(d - do)) <= 1e-10 * np.max(np.abs(do))
+    e, eo = (np.array([q[k] for k in ("pp_el", "pp_vdw", "pw_el", "pw_vdw")]) for q in (E, Eo))
+    assert np.max(np.abs(e - eo)) <= 1e-10 * np.max(np.abs(eo))
