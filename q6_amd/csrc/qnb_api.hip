@@ -484,20 +484,30 @@ int topo_build(DevSys& S, const qnb_system* s, HostTopo& T, DevAlloc& M) {
   return 0;
 }
 
-// A row of S.cap groups holds at most `atoms` atoms.  Of two batches in a row
-// the first ends because the next group would pass al_batch >= 128 slots, or
-// holds 64 groups, so batches hold 64 atoms on average and their padding (at
-// most 63 slots each, one batch more at the end) at most doubles the row.
-int atom_row_cap(const DevSys& S, const HostTopo& T) {
-  const long atoms = std::min((long)T.n_group_atoms, (long)S.cap * T.max_group);
-  return (int)((2 * atoms + 64 + 63) / 64 * 64);
+// Half as many again as the longest row seen and ten groups' worth (neighbour
+// rows get the same half and 64 groups), and no less than a cut-off sphere full
+// of solute: 0.1 atoms per A^3 out to 2 A beyond the cut-off, and a fifth of
+// them for the padding.  At most what any row of S.cap groups can hold: of two
+// batches in a row the first ends because the next group would pass
+// al_batch >= 128 slots, or holds 64 groups, so batches hold 64 atoms on average
+// and their padding (at most 63 slots each, one batch more at the end) at most
+// doubles the row.  For 4,000 solute atoms and 2,687 groups with rows of up to
+// 576 slots: 1,504 slots, 16 MB; rows that hold any S.cap groups took 8,064, 87 MB.
+int atom_row_slots(const DevSys& S, const HostTopo& T, int longest) {
+  const long atoms = std::min((long)T.n_group_atoms, (long)S.cap * T.max_group), most = 2 * atoms + 64;
+  const double r = std::sqrt(std::max(S.rcpp2, S.rcpw2)) + 2.0;
+  const double sphere = std::min(0.5 * r * r * r + 64.0, (double)most);
+  const long seen = longest > 0 ? longest + longest / 2 + 640l : 0l;
+  return (int)((std::min(most, std::max(seen, (long)sphere)) + 63) / 64 * 64);
 }
 
-int atom_rows_alloc(DevSys& S, const HostTopo& T, DevAlloc& M) {
+int atom_rows_alloc(DevSys& S, DevAlloc& M, int slots) {
   M.release(S.alist);
   S.alist = nullptr;
-  S.acap = atom_row_cap(S, T);
-  return M.alloc(&S.alist, (size_t)S.acap * S.ncgp);
+  S.acap = 0;
+  if (int rc = M.alloc(&S.alist, (size_t)slots * S.atom_rows)) return rc;
+  S.acap = slots;
+  return 0;
 }
 
 int row_alloc(DevSys& S, DevAlloc& M, int cap) {
@@ -532,7 +542,7 @@ int instance_alloc(DevSys& S, DevAlloc& M, const qnb_params* p, int nslots) {
   AL(nnbr, S.ncgp);
   AL(nnsol, S.ncgp);
   AL(pw_first, S.ncgp_solute);
-  AL(need, 1);
+  AL(need, 2);
   AL(qw_in, nw1);
   AL(qp_in, S.ncgp_solute);
   AL(qw_list, nw1);
@@ -560,6 +570,8 @@ int instance_alloc(DevSys& S, DevAlloc& M, const qnb_params* p, int nslots) {
   for (int k = 0; k < S.nshell; k++) sh0[k] = p->wshell_theta_corr[k];
   HIPCHK(hipMemcpy(S.sh_state, sh0, sizeof sh0, hipMemcpyHostToDevice));
   S.nbr = S.alist = nullptr;
+  S.acap = 0;
+  S.atom_rows = S.sa == 3 ? S.ncgp : S.ncgp_solute;
   return row_alloc(S, M, S.cap > 0 ? S.cap : 256);
 }
 
@@ -679,7 +691,7 @@ extern "C" int32_t qnb_create(const qnb_system* s, const qnb_params* p, qnb_hand
   memset(&S, 0, sizeof S);
   fill_params(S, s, p);
   if ((rc = topo_build(S, s, h->T, h->mem)) || (rc = instance_alloc(S, h->mem, p, s->ncgp + qq_slots(S))) ||
-      (rc = atom_rows_alloc(S, h->T, h->mem)) ||
+      (rc = atom_rows_alloc(S, h->mem, atom_row_slots(S, h->T, 0))) ||
       (rc = h->mem.alloc(&h->d_tfree, 1)) || (rc = h->mem.alloc(&h->d_istep, 1)) || (rc = h->mem.alloc(&h->dsys, 1))) {
     delete h;
     return rc;
@@ -713,20 +725,23 @@ extern "C" int32_t qnb_make_pair_lists(qnb_handle* h, const double* x) {
   if (!h) return fail(QNB_EINVAL, "null handle");
   int rc = upload_x(h, x);
   if (rc) return rc;
-  for (int attempt = 0; attempt < 4; attempt++) {
-    HIPCHK(hipMemsetAsync(h->hs.need, 0, sizeof(int), h->stream));
+  for (int attempt = 0;; attempt++) {
+    HIPCHK(hipMemsetAsync(h->hs.need, 0, 2 * sizeof(int), h->stream));
     if (h->hs.prec == QNB_PREC_MIXED) launch_lists<float>(h);
     else launch_lists<double>(h);
     HIPCHK(hipGetLastError());
-    int need = 0;
-    HIPCHK(hipMemcpyAsync(&need, h->hs.need, sizeof(int), hipMemcpyDeviceToHost, h->stream));
+    int need[2] = {0, 0};
+    HIPCHK(hipMemcpyAsync(need, h->hs.need, sizeof need, hipMemcpyDeviceToHost, h->stream));
     HIPCHK(hipStreamSynchronize(h->stream));
-    if (need <= h->hs.cap) break;
-    // reallocate_nonbondlist_* (qalloc.f90:370-605): grow and rebuild
-    int ncap = ((need * 5 / 4) + 63) / 64 * 64;
-    if ((rc = row_alloc(h->hs, h->mem, ncap)) || (rc = atom_rows_alloc(h->hs, h->T, h->mem))) return rc;
+    const bool groups = need[0] > h->hs.cap, atoms = need[1] > h->hs.acap;
+    if (!groups && !atoms) break;
+    // reallocate_nonbondlist_* (qalloc.f90:370-605): grow and rebuild; no
+    // evaluation until that is done
+    h->lists_built = false;
+    if (attempt == 4) return fail(QNB_EOVERFLOW, "neighbour list capacity");
+    if (groups && (rc = row_alloc(h->hs, h->mem, ((need[0] * 5 / 4) + 63) / 64 * 64))) return rc;
+    if (atoms && (rc = atom_rows_alloc(h->hs, h->mem, atom_row_slots(h->hs, h->T, need[1])))) return rc;
     HIPCHK(hipMemcpy(h->dsys, &h->hs, sizeof(DevSys), hipMemcpyHostToDevice));
-    if (attempt == 3) return fail(QNB_EOVERFLOW, "neighbour list capacity");
   }
   // Q lists: rebuilt every update unless Rcq exceeds the exclusion radius,
   // then built once (the `save`d list_done of nbqplist/nbqwlist)

@@ -179,7 +179,7 @@ __device__ __forceinline__ void thermo(const DevSys& S, const MdDev& M, int nblk
   thermo_update(M, ek, ekf);
   const double T = M.st[2];
   if (!isfinite(T) || !isfinite(S.ered[E_PP_EL] + S.ered[E_WW_EL])) atomicOr(&M.ctr[1], ERR_NONFINITE);
-  if (*S.need > S.cap) atomicOr(&M.ctr[1], ERR_OVERFLOW);
+  if (S.need[0] > S.cap || S.need[1] > S.acap) atomicOr(&M.ctr[1], ERR_OVERFLOW);
   M.ctr[3] = 0;
   *M.istep = *M.istep + 1;
 }
@@ -442,7 +442,7 @@ __global__ __launch_bounds__(256) void k_temperature(const DevSys* __restrict__ 
     thermo_update(M, ek, ekf);
     const double T = M.st[2];
     if (!isfinite(T) || !isfinite(S.ered[E_PP_EL] + S.ered[E_WW_EL])) atomicOr(&M.ctr[1], ERR_NONFINITE);
-    if (*S.need > S.cap) atomicOr(&M.ctr[1], ERR_OVERFLOW);
+    if (S.need[0] > S.cap || S.need[1] > S.acap) atomicOr(&M.ctr[1], ERR_OVERFLOW);
   }
 }
 
@@ -986,9 +986,10 @@ extern "C" int32_t qnb_batch_create(int32_t n, const qnb_system* const* sys, con
     DevSys& S = b->hs[k];
     if ((rc = row_alloc(S, b->mem, std::min(((S.ncgp + 63) / 64) * 64, 1024)))) return rc;
   }
+  std::vector<int> slots(n, 0);  // of each instance's longest partner-atom row
   for (int attempt = 0;; attempt++) {
     HIPCHK(hipMemcpy(b->dsys, b->hs.data(), sizeof(DevSys) * n, hipMemcpyHostToDevice));
-    for (int k = 0; k < n; k++) HIPCHK(hipMemset(b->hs[k].need, 0, sizeof(int)));
+    for (int k = 0; k < n; k++) HIPCHK(hipMemset(b->hs[k].need, 0, 2 * sizeof(int)));
     const int wpb = 4;
     launch_lists(b.get(), wpb);
     HIPCHK(hipGetLastError());
@@ -996,10 +997,11 @@ extern "C" int32_t qnb_batch_create(int32_t n, const qnb_system* const* sys, con
     bool again = false;
     for (int k = 0; k < n; k++) {
       DevSys& S = b->hs[k];
-      int need = 0;
-      HIPCHK(hipMemcpy(&need, S.need, sizeof(int), hipMemcpyDeviceToHost));
-      if (need > S.cap) {
-        if ((rc = row_alloc(S, b->mem, ((need + 63) / 64) * 64))) return rc;
+      int need[2] = {0, 0};
+      HIPCHK(hipMemcpy(need, S.need, sizeof need, hipMemcpyDeviceToHost));
+      slots[k] = need[1];
+      if (need[0] > S.cap) {
+        if ((rc = row_alloc(S, b->mem, ((need[0] + 63) / 64) * 64))) return rc;
         again = true;
       }
     }
@@ -1017,21 +1019,21 @@ extern "C" int32_t qnb_batch_create(int32_t n, const qnb_system* const* sys, con
       // shrink: rebuild happens at the first step of the run
       if ((rc = row_alloc(S, b->mem, cap))) return rc;
     }
-    HIPCHK(hipMemset(S.need, 0, sizeof(int)));
+    HIPCHK(hipMemset(S.need, 0, 2 * sizeof(int)));
   }
   // the partner-atom rows of all instances in one allocation
   {
     size_t total = 0;
     for (int k = 0; k < n; k++) {
       DevSys& S = b->hs[k];
-      S.acap = atom_row_cap(S, *b->topos[b->topo_of[k]]);
-      total += (size_t)S.acap * S.ncgp;
+      S.acap = atom_row_slots(S, *b->topos[b->topo_of[k]], slots[k]);
+      total += (size_t)S.acap * S.atom_rows;
     }
     int* rows = nullptr;
     if ((rc = b->mem.alloc(&rows, total))) return rc;
     for (int k = 0; k < n; k++) {
       b->hs[k].alist = rows;
-      rows += (size_t)b->hs[k].acap * b->hs[k].ncgp;
+      rows += (size_t)b->hs[k].acap * b->hs[k].atom_rows;
     }
   }
   HIPCHK(hipMemcpy(b->dsys, b->hs.data(), sizeof(DevSys) * n, hipMemcpyHostToDevice));

@@ -170,11 +170,12 @@ struct DevSys {
   double* lrf;
   int* nbr;
   int* nnbr;
-  // partner atoms of each receiver (expand_row): rows of acap slots, the slots in
-  // use [ncgp], slots per batch of groups
+  // partner atoms of receivers 0 .. atom_rows - 1 (expand_row; a solvent other
+  // than 3-site water has none, solvent_receiver walks its groups): rows of acap
+  // slots, the slots in use [ncgp], slots per batch of groups
   int* alist;
   int* alist_n;
-  int acap, al_batch;
+  int acap, al_batch, atom_rows;
   int* nnsol;  // [ncgp] length of the row's solute prefix (rows are sorted)
   // reference test-point reuse of the LRF-off switch-atom solute-water list
   // (quirk bit 0 with use_lrf = 0): per solute group, the first water within
@@ -182,7 +183,7 @@ struct DevSys {
   // against atom glast + 1
   int* pw_first;
   int cap;
-  int* need;        // [1] max neighbours seen (overflow detection)
+  int* need;        // [2] most groups of a row seen, and most slots of an atom row that did not fit
   uint8_t* qw_in;   // [nwat] water on the Q-water list
   uint8_t* qp_in;   // [ncgp_solute] group on the Q-solute list
   int* qw_list;     // compacted waters on the Q list

@@ -137,11 +137,12 @@ void launch_pol_bonded(hipStream_t st, int nwat, int bonded_atoms, int B, const 
 void launch_bonded_rows(hipStream_t st, int bonded_atoms, int B, const DevSys* dsys);
 // per-instance device state (coordinates, gradient, lists, LRF, energies)
 int instance_alloc(DevSys& S, DevAlloc& M, const qnb_params* p, int nslots);
-// neighbour rows of `cap` groups; entries per partner-atom row that always
-// hold such a row's atoms (expand_row), and the rows themselves
+// neighbour rows of `cap` groups
 int row_alloc(DevSys& S, DevAlloc& M, int cap);
-int atom_row_cap(const DevSys& S, const HostTopo& T);
-int atom_rows_alloc(DevSys& S, const HostTopo& T, DevAlloc& M);
+// slots of the partner-atom rows (expand_row) where the longest row seen has
+// `longest` (0: none seen yet), and rows of so many slots
+int atom_row_slots(const DevSys& S, const HostTopo& T, int longest);
+int atom_rows_alloc(DevSys& S, DevAlloc& M, int slots);
 // group contributions (qnb_exc.hip): the pair lists of each energy array
 // and state, built on the host from the system's Q tables
 struct ExcHost {

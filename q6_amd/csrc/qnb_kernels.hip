@@ -266,17 +266,20 @@ __device__ __forceinline__ double dist4v(const d4v& a, const d4v& b) {
 // AL_SKIP marks Q-atoms (their pairs belong to the Q kernels) and the padding.
 // The force kernels then read one coalesced list per receiver instead of
 // walking group -> atoms -> positions through LDS at every step.  A launch of
-// its own cost a list update 7 us.
+// its own cost a list update 7 us.  A row longer than acap slots ends before
+// the batch that does not fit and its length goes to need[1] (as a neighbour
+// row's does to need[0]); with acap 0 the call only counts.
 #define LS_WPB 8  // waves per block of the list sweep at most
 __device__ __forceinline__ void expand_row(const DevSys& S, int a, int nsr, int lane, int w) {
   const int batch = S.al_batch;
   const bool a_sol = a < S.ncgp_solute;
   const int* row = S.nbr + (size_t)a * S.cap;
-  int* out = S.alist + (size_t)a * S.acap;
+  const int acap = S.acap;
+  int* out = S.alist + (size_t)a * acap;
   const bool along = a_sol && ldg(S.glong + a);
   const int alo = a_sol ? ldg(S.gspan + 2 * a) : 0, ahi = a_sol ? ldg(S.gspan + 2 * a + 1) : 0;
   __shared__ int s_incl[LS_WPB][QNB_WAVE], s_src[LS_WPB][QNB_WAVE], s_tag[LS_WPB][QNB_WAVE];
-  int n = 0;
+  int n = 0, stored = 0;
   for (int p0 = 0, ng = 0; p0 < nsr; p0 += ng) {
     const int p = p0 + lane;
     int f0 = 0, cnt = 0, tag = 0;
@@ -299,12 +302,14 @@ __device__ __forceinline__ void expand_row(const DevSys& S, int a, int nsr, int 
     // group always fits)
     ng = min(__popcll(__ballot(incl <= batch)), nsr - p0);
     const int total = __shfl(incl, ng - 1, QNB_WAVE);
+    const int end = uni((total + QNB_WAVE - 1) / QNB_WAVE * QNB_WAVE);
+    n += end;
+    if (n > acap) continue;
     // lane = slot: its group is the first whose inclusive count passes it
     s_incl[w][lane] = incl;
     s_src[w][lane] = f0 - (incl - cnt);
     s_tag[w][lane] = tag;
     __builtin_amdgcn_wave_barrier();
-    const int end = (total + QNB_WAVE - 1) / QNB_WAVE * QNB_WAVE;
     for (int s = lane; s < end; s += QNB_WAVE) {
       int e = AL_SKIP;
       if (s < total) {
@@ -314,12 +319,15 @@ __device__ __forceinline__ void expand_row(const DevSys& S, int a, int nsr, int 
           if (s_incl[w][g + h - 1] <= s) g += h;
         e = ldg(S.cgentry + s_src[w][g] + s) | s_tag[w][g];
       }
-      stg(out + n + s, e);
+      stg(out + stored + s, e);
     }
     __builtin_amdgcn_wave_barrier();
-    n += end;
+    stored = n;
   }
-  if (lane == 0) S.alist_n[a] = n;
+  if (lane == 0) {
+    S.alist_n[a] = stored;
+    if (n > acap) atomicMax(S.need + 1, n);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -516,7 +524,7 @@ __global__ __launch_bounds__(64 * LS_WPB) void k_lists_lrf(const DevSys* __restr
       for (int j = 0; j < 3; j++)
         for (int c = 0; c < 3; c++) L[16 + 3 * (j + 3 * n) + c] = t[t3index(n, j, c)];
   }
-  if (S.alist) {  // null while the rows are being sized
+  if (a < S.atom_rows) {
     __threadfence_block();  // the row's stores before its loads
     expand_row(S, a, min(count_sol, S.cap), lane, threadIdx.x / QNB_WAVE);
   }
