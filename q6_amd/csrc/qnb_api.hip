@@ -16,8 +16,6 @@
 #include "qnb_host.h"
 
 namespace qnb {
-template <typename R, bool ANY>
-__global__ void k_lists_lrf(const DevSys*);
 __global__ void k_qlists(const DevSys*);
 template <typename R, int NS, bool E>
 __global__ void k_wforces(const DevSys*, uint32_t, int, int, int);
@@ -710,15 +708,12 @@ static int upload_x(qnb_handle* h, const double* x) {
   return 0;
 }
 
-template <typename R>
 static void launch_lists(qnb_handle* h) {
-  const int wpb = 4;
-  dim3 grid((h->hs.ncgp + wpb - 1) / wpb, 1);
-  hipLaunchKernelGGL(k_pack_xq, dim3((h->hs.ncgpat + 255) / 256, 1), dim3(256), 0, h->stream, h->dsys);
-  if (pw_quirk(h->hs))
-    hipLaunchKernelGGL(k_pw_first, dim3((h->hs.ncgp_solute + 3) / 4, 1), dim3(256), 0, h->stream, h->dsys);
-  if (h->hs.any_atom) hipLaunchKernelGGL((k_lists_lrf<R, true>), grid, dim3(64 * wpb), 0, h->stream, h->dsys);
-  else hipLaunchKernelGGL((k_lists_lrf<R, false>), grid, dim3(64 * wpb), 0, h->stream, h->dsys);
+  const DevSys& S = h->hs;
+  hipLaunchKernelGGL(k_pack_xq, dim3((S.ncgpat + 255) / 256, 1), dim3(256), 0, h->stream, h->dsys);
+  if (pw_quirk(S))
+    hipLaunchKernelGGL(k_pw_first, dim3((S.ncgp_solute + 3) / 4, 1), dim3(256), 0, h->stream, h->dsys);
+  launch_sweep(h->stream, S.prec, S.any_atom, S.use_lrf, S.ncgp, 4, 1, h->dsys);
 }
 
 extern "C" int32_t qnb_make_pair_lists(qnb_handle* h, const double* x) {
@@ -727,8 +722,7 @@ extern "C" int32_t qnb_make_pair_lists(qnb_handle* h, const double* x) {
   if (rc) return rc;
   for (int attempt = 0;; attempt++) {
     HIPCHK(hipMemsetAsync(h->hs.need, 0, 2 * sizeof(int), h->stream));
-    if (h->hs.prec == QNB_PREC_MIXED) launch_lists<float>(h);
-    else launch_lists<double>(h);
+    launch_lists(h);
     HIPCHK(hipGetLastError());
     int need[2] = {0, 0};
     HIPCHK(hipMemcpyAsync(need, h->hs.need, sizeof need, hipMemcpyDeviceToHost, h->stream));

@@ -15,8 +15,6 @@
 #include "qnb_host.h"
 
 namespace qnb {
-template <typename R, bool ANY>
-__global__ void k_lists_lrf(const DevSys*);
 __global__ void k_qlists(const DevSys*);
 __global__ void k_pack_xq(const DevSys*);
 __global__ void k_pw_first(const DevSys*);
@@ -561,23 +559,17 @@ __global__ void k_exc_record(const DevSys* __restrict__ systems, const MdDev* __
 
 // launchers shared by the step, the minimiser, the timer and the autotuner
 static void launch_lists(qnb_batch* b, int wpb) {
-  dim3 g((b->maxg + wpb - 1) / wpb, b->n), t(64 * wpb);
-  bool any = false, quirk = false;
+  bool any = false, quirk = false, lrf = false;
   int maxsg = 0;
   for (const DevSys& S : b->hs) {
     any = any || S.any_atom;
     quirk = quirk || pw_quirk(S);
+    lrf = lrf || S.use_lrf;
     maxsg = std::max(maxsg, S.ncgp_solute);
   }
   if (quirk) hipLaunchKernelGGL(k_pw_first, dim3((maxsg + 3) / 4, b->n), dim3(256), 0, b->stream, b->dsys);
   hipLaunchKernelGGL(k_pack_xq, dim3((b->maxat + 255) / 256, b->n), dim3(256), 0, b->stream, b->dsys);
-  if (b->prec == QNB_PREC_MIXED) {
-    if (any) hipLaunchKernelGGL((k_lists_lrf<float, true>), g, t, 0, b->stream, b->dsys);
-    else hipLaunchKernelGGL((k_lists_lrf<float, false>), g, t, 0, b->stream, b->dsys);
-  } else {
-    if (any) hipLaunchKernelGGL((k_lists_lrf<double, true>), g, t, 0, b->stream, b->dsys);
-    else hipLaunchKernelGGL((k_lists_lrf<double, false>), g, t, 0, b->stream, b->dsys);
-  }
+  launch_sweep(b->stream, b->prec, any, lrf, b->maxg, wpb, b->n, b->dsys);
 }
 
 static const uint32_t kStepMask = QNB_T_NONBONDED | QNB_T_QQ | QNB_T_QQP | QNB_T_RAD | QNB_T_POL;

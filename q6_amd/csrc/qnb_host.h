@@ -117,6 +117,10 @@ void fill_params(DevSys& S, const qnb_system* s, const qnb_params* p);
 int topo_build(DevSys& S, const qnb_system* s, HostTopo& T, DevAlloc& M);
 // host twin of the device solute-solute filter (pp_param), for list export
 bool host_pp_param(const HostTopo& T, int i, int j);
+// the list sweep over `groups` receivers of B systems, wpb of them per block; any:
+// some system takes any atom pair for its group tests, lrf: some system wants
+// the expansion
+void launch_sweep(hipStream_t st, int prec, bool any, bool lrf, int groups, int wpb, int B, const DevSys* dsys);
 // the force pass of a small launch as one kernel (k_forces_small): the grid
 // for systems of at most these sizes (pol: the polarisation angles too), and
 // the launch

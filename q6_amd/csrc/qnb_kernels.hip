@@ -352,8 +352,10 @@ __device__ __forceinline__ void expand_row(const DevSys& S, int a, int nsr, int 
 // divisions.  Measured: 2,663 -> 2,270 us for 51 windows of 11,056 atoms
 // (FP32), 1,740 -> 870 us for 12 of them in FP64; a list update of 19,440 atoms
 // in FP64 775 -> 380 us.
+// LRF: the expansion is wanted by some system of the launch; without it the
+// sweep reads no records and has the next chunk's groups in flight.
 #define LRF_U 3
-template <typename R, bool ANY>
+template <typename R, bool ANY, bool LRF>
 __global__ __launch_bounds__(64 * LS_WPB) void k_lists_lrf(const DevSys* __restrict__ systems) {
   const DevSys& S = systems[blockIdx.y];
   const int a = uni(blockIdx.x * (blockDim.x / QNB_WAVE) + threadIdx.x / QNB_WAVE);
@@ -400,19 +402,21 @@ __global__ __launch_bounds__(64 * LS_WPB) void k_lists_lrf(const DevSys* __restr
     // the cut-off of a pair with a solute group and with a water, given a
     const double cut_sol = a_sol ? S.rcpp2 : S.rcpw2, cut_wat = a_sol ? S.rcpw2 : S.rcww2;
     const bool quirk = pw_quirk(S), any_atom = ANY && S.any_atom;
-    const double rclrf2 = S.use_lrf ? S.rclrf2 : -1.0;
+    const bool lrf = LRF && S.use_lrf;
+    const double rclrf2 = lrf ? S.rclrf2 : -1.0;
+    constexpr bool AHEAD = !F32 || !LRF;  // next chunk's groups in flight
     using Rec = decltype(lrf_rec<R>(grs, 0));
     // the chunk's atoms: the run from b0's first to its last group's last; FP64
     // requests the next chunk's groups while it sums this one (FP32 has no
-    // registers for that at four waves per SIMD)
+    // registers for that beside the sums at four waves per SIMD)
     int k1 = ldc(S.gfirst);
     d4v Gn = buf_d4(grs, (uint32_t)lane * 32);
     for (int b0 = 0; b0 < ncgp; b0 += QNB_WAVE) {
       const int b = b0 + lane;
-      const d4v G = F32 ? buf_d4(grs, (uint32_t)b * 32) : Gn;  // 0 past the last group
+      const d4v G = AHEAD ? Gn : buf_d4(grs, (uint32_t)b * 32);  // 0 past the last group
       const int k0 = ldc(S.gfirst + b0);
       k1 = ldc(S.glast + min(b0 + QNB_WAVE, ncgp) - 1) + 1;
-      if constexpr (!F32) Gn = buf_d4(grs, (uint32_t)(b + QNB_WAVE) * 32);
+      if constexpr (AHEAD) Gn = buf_d4(grs, (uint32_t)(b + QNB_WAVE) * 32);
       Rec r[LRF_U];
       u2v s[LRF_U];
       auto fetch = [&](int k, Rec* rr, u2v* ss) {
@@ -425,7 +429,7 @@ __global__ __launch_bounds__(64 * LS_WPB) void k_lists_lrf(const DevSys* __restr
           ss[u] = buf_u2(bs, (uint32_t)(lane + u * QNB_WAVE) * 8);
         }
       };
-      fetch(k0, r, s);
+      if (lrf) fetch(k0, r, s);
       bool in = false, far = false;
       if (G.w != 0.0 && b != a) {
         const bool b_sol = b < nsol;
@@ -456,6 +460,7 @@ __global__ __launch_bounds__(64 * LS_WPB) void k_lists_lrf(const DevSys* __restr
         count += __popcll(m);
         if (b0 < nsol) count_sol += __popcll(__ballot(in && b < nsol));
       }
+      if (!lrf) continue;
       const uint64_t fw = __ballot(far);
       if (fw == 0) continue;
       const uint32_t f0 = (uint32_t)fw, f1 = (uint32_t)(fw >> 32);
@@ -497,12 +502,14 @@ __global__ __launch_bounds__(64 * LS_WPB) void k_lists_lrf(const DevSys* __restr
       }
     }
   }
-  if constexpr (F32)
+  if constexpr (LRF) {
+    if constexpr (F32)
 #pragma unroll
-    for (int c = 0; c < LRF_NF; c++) acc[c] += (double)pf[c];
-  const double tr = wave_sum_tr<double, LRF_NF>(acc, lane);
+      for (int c = 0; c < LRF_NF; c++) acc[c] += (double)pf[c];
+    const double tr = wave_sum_tr<double, LRF_NF>(acc, lane);
 #pragma unroll
-  for (int k = 0; k < LRF_NF; k++) acc[k] = lane_value(tr, wave_sum_tr_lane<LRF_NF>(k));
+    for (int k = 0; k < LRF_NF; k++) acc[k] = lane_value(tr, wave_sum_tr_lane<LRF_NF>(k));
+  }
   if (lane == 0) {
     double t[LRF_NF];
     lrf_tensors(t, acc);
@@ -2088,6 +2095,20 @@ __global__ __launch_bounds__(256) void k_reduce_final(const DevSys* __restrict__
   if (with_pol) watpol_finish(S, threadIdx.x / QNB_WAVE, 4);
 }
 
+void launch_sweep(hipStream_t st, int prec, bool any, bool lrf, int groups, int wpb, int B, const DevSys* dsys) {
+  const dim3 g((groups + wpb - 1) / wpb, B), t(QNB_WAVE * wpb);
+  if (!lrf) {
+    if (any) hipLaunchKernelGGL((k_lists_lrf<double, true, false>), g, t, 0, st, dsys);
+    else hipLaunchKernelGGL((k_lists_lrf<double, false, false>), g, t, 0, st, dsys);
+  } else if (prec == QNB_PREC_MIXED) {
+    if (any) hipLaunchKernelGGL((k_lists_lrf<float, true, true>), g, t, 0, st, dsys);
+    else hipLaunchKernelGGL((k_lists_lrf<float, false, true>), g, t, 0, st, dsys);
+  } else {
+    if (any) hipLaunchKernelGGL((k_lists_lrf<double, true, true>), g, t, 0, st, dsys);
+    else hipLaunchKernelGGL((k_lists_lrf<double, false, true>), g, t, 0, st, dsys);
+  }
+}
+
 SmallGrid small_grid(int solute_groups, int nwat, int sa, int nqat, int nat_solute, int nqe, uint32_t mask, bool pol) {
   SmallGrid G{};
   G.solute = solute_groups;
@@ -2131,10 +2152,6 @@ void launch_forces_small(hipStream_t st, int prec, int ns_max, bool energy, cons
 }
 
 // explicit instantiations used by the host code
-template __global__ void k_lists_lrf<double, false>(const DevSys*);
-template __global__ void k_lists_lrf<float, false>(const DevSys*);
-template __global__ void k_lists_lrf<double, true>(const DevSys*);
-template __global__ void k_lists_lrf<float, true>(const DevSys*);
 #define QNB_INST(R, NS)                                                            \
   template __global__ void k_qforces<R, NS>(const DevSys*, uint32_t, int, int);                       \
   template __global__ void k_sforces<R, NS, true>(const DevSys*, uint32_t, int, int, int); \
