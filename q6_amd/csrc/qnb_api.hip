@@ -713,7 +713,7 @@ static void launch_lists(qnb_handle* h) {
   hipLaunchKernelGGL(k_pack_xq, dim3((S.ncgpat + 255) / 256, 1), dim3(256), 0, h->stream, h->dsys);
   if (pw_quirk(S))
     hipLaunchKernelGGL(k_pw_first, dim3((S.ncgp_solute + 3) / 4, 1), dim3(256), 0, h->stream, h->dsys);
-  launch_sweep(h->stream, S.prec, S.any_atom, S.use_lrf, S.ncgp, 4, 1, h->dsys);
+  launch_sweep(h->stream, S.prec, S.any_atom, S.use_lrf ? SWEEP_LRF : SWEEP_PLAIN, S.ncgp, 4, 1, h->dsys);
 }
 
 extern "C" int32_t qnb_make_pair_lists(qnb_handle* h, const double* x) {

@@ -559,12 +559,12 @@ __global__ void k_exc_record(const DevSys* __restrict__ systems, const MdDev* __
 
 // launchers shared by the step, the minimiser, the timer and the autotuner
 static void launch_lists(qnb_batch* b, int wpb) {
-  bool any = false, quirk = false, lrf = false;
-  int maxsg = 0;
+  bool any = false, quirk = false;
+  int maxsg = 0, lrf = 0;
   for (const DevSys& S : b->hs) {
     any = any || S.any_atom;
     quirk = quirk || pw_quirk(S);
-    lrf = lrf || S.use_lrf;
+    lrf |= S.use_lrf ? SWEEP_LRF : SWEEP_PLAIN;
     maxsg = std::max(maxsg, S.ncgp_solute);
   }
   if (quirk) hipLaunchKernelGGL(k_pw_first, dim3((maxsg + 3) / 4, b->n), dim3(256), 0, b->stream, b->dsys);

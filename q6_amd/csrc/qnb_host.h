@@ -119,8 +119,9 @@ int topo_build(DevSys& S, const qnb_system* s, HostTopo& T, DevAlloc& M);
 bool host_pp_param(const HostTopo& T, int i, int j);
 // the list sweep over `groups` receivers of B systems, wpb of them per block; any:
 // some system takes any atom pair for its group tests, lrf: some system wants
-// the expansion
-void launch_sweep(hipStream_t st, int prec, bool any, bool lrf, int groups, int wpb, int B, const DevSys* dsys);
+// the expansion, some does not
+enum { SWEEP_LRF = 1, SWEEP_PLAIN = 2 };
+void launch_sweep(hipStream_t st, int prec, bool any, int lrf, int groups, int wpb, int B, const DevSys* dsys);
 // the force pass of a small launch as one kernel (k_forces_small): the grid
 // for systems of at most these sizes (pol: the polarisation angles too), and
 // the launch

@@ -348,18 +348,21 @@ __device__ __forceinline__ void expand_row(const DevSys& S, int a, int nsr, int 
 // that moves in scalar registers; FP32 has the next batch in flight while one
 // is summed, FP64 the next chunk's groups.  A record's group is
 // one bit of a 64-bit word, so a test is two ANDs and reads past the run find
-// 0; FP64 takes the sums raw too, with rinv in place of a root and three
+// 0; FP64 takes the sums raw too, with rinv_inner in place of a root and three
 // divisions.  Measured: 2,663 -> 2,270 us for 51 windows of 11,056 atoms
 // (FP32), 1,740 -> 870 us for 12 of them in FP64; a list update of 19,440 atoms
 // in FP64 775 -> 380 us.
-// LRF: the expansion is wanted by some system of the launch; without it the
-// sweep reads no records and has the next chunk's groups in flight.
+// LRF: for the systems that want the expansion, the others leave at once (and
+// the other way round): without it the sweep reads no records and has the next
+// chunk's groups in flight.  ANY reads a batch of records when it sums it: held
+// over the group tests, which loop over atom pairs, they leave three waves per
+// SIMD (51 windows of 11,056 atoms in FP32 6.6 ms, 6.15 so).
 #define LRF_U 3
 template <typename R, bool ANY, bool LRF>
 __global__ __launch_bounds__(64 * LS_WPB) void k_lists_lrf(const DevSys* __restrict__ systems) {
   const DevSys& S = systems[blockIdx.y];
   const int a = uni(blockIdx.x * (blockDim.x / QNB_WAVE) + threadIdx.x / QNB_WAVE);
-  if (a >= S.ncgp) return;
+  if (a >= S.ncgp || (S.use_lrf != 0) != LRF) return;
   const int lane = threadIdx.x % QNB_WAVE;
   const double* __restrict__ x = S.x;
   const int ra = group_ref_atom(S, a);
@@ -402,8 +405,7 @@ __global__ __launch_bounds__(64 * LS_WPB) void k_lists_lrf(const DevSys* __restr
     // the cut-off of a pair with a solute group and with a water, given a
     const double cut_sol = a_sol ? S.rcpp2 : S.rcpw2, cut_wat = a_sol ? S.rcpw2 : S.rcww2;
     const bool quirk = pw_quirk(S), any_atom = ANY && S.any_atom;
-    const bool lrf = LRF && S.use_lrf;
-    const double rclrf2 = lrf ? S.rclrf2 : -1.0;
+    const double rclrf2 = LRF ? S.rclrf2 : -1.0;
     constexpr bool AHEAD = !F32 || !LRF;  // next chunk's groups in flight
     using Rec = decltype(lrf_rec<R>(grs, 0));
     // the chunk's atoms: the run from b0's first to its last group's last; FP64
@@ -429,7 +431,7 @@ __global__ __launch_bounds__(64 * LS_WPB) void k_lists_lrf(const DevSys* __restr
           ss[u] = buf_u2(bs, (uint32_t)(lane + u * QNB_WAVE) * 8);
         }
       };
-      if (lrf) fetch(k0, r, s);
+      if constexpr (LRF && !ANY) fetch(k0, r, s);
       bool in = false, far = false;
       if (G.w != 0.0 && b != a) {
         const bool b_sol = b < nsol;
@@ -460,9 +462,10 @@ __global__ __launch_bounds__(64 * LS_WPB) void k_lists_lrf(const DevSys* __restr
         count += __popcll(m);
         if (b0 < nsol) count_sol += __popcll(__ballot(in && b < nsol));
       }
-      if (!lrf) continue;
+      if constexpr (!LRF) continue;
       const uint64_t fw = __ballot(far);
       if (fw == 0) continue;
+      if constexpr (ANY) fetch(k0, r, s);
       const uint32_t f0 = (uint32_t)fw, f1 = (uint32_t)(fw >> 32);
       auto sum = [&](const Rec* rr, const u2v* ss) {
 #pragma unroll
@@ -472,7 +475,7 @@ __global__ __launch_bounds__(64 * LS_WPB) void k_lists_lrf(const DevSys* __restr
             else lrf_accumulate<double>(acc, rr[u].x - cxr, rr[u].y - cyr, rr[u].z - czr, rr[u].w);
           }
       };
-      if constexpr (F32) {
+      if constexpr (F32 && !ANY) {
         for (int k = k0 + LRF_U * QNB_WAVE; k < k1; k += LRF_U * QNB_WAVE) {
           Rec rn[LRF_U];
           u2v sn[LRF_U];
@@ -2095,12 +2098,14 @@ __global__ __launch_bounds__(256) void k_reduce_final(const DevSys* __restrict__
   if (with_pol) watpol_finish(S, threadIdx.x / QNB_WAVE, 4);
 }
 
-void launch_sweep(hipStream_t st, int prec, bool any, bool lrf, int groups, int wpb, int B, const DevSys* dsys) {
+void launch_sweep(hipStream_t st, int prec, bool any, int lrf, int groups, int wpb, int B, const DevSys* dsys) {
   const dim3 g((groups + wpb - 1) / wpb, B), t(QNB_WAVE * wpb);
-  if (!lrf) {
+  if (lrf & SWEEP_PLAIN) {
     if (any) hipLaunchKernelGGL((k_lists_lrf<double, true, false>), g, t, 0, st, dsys);
     else hipLaunchKernelGGL((k_lists_lrf<double, false, false>), g, t, 0, st, dsys);
-  } else if (prec == QNB_PREC_MIXED) {
+  }
+  if (!(lrf & SWEEP_LRF)) return;
+  if (prec == QNB_PREC_MIXED) {
     if (any) hipLaunchKernelGGL((k_lists_lrf<float, true, true>), g, t, 0, st, dsys);
     else hipLaunchKernelGGL((k_lists_lrf<float, false, true>), g, t, 0, st, dsys);
   } else {
