@@ -203,6 +203,11 @@ int topo_build(DevSys& S, const qnb_system* s, HostTopo& T, DevAlloc& M) {
       return fail(QNB_EINVAL, "atom %d is in no charge group", i);
   // charge groups are consecutive runs of cgpatom, as the topology reader
   // lays them out
+  // per-atom tables of the force and list kernels that go up together
+  DevPack pack;
+  std::vector<int> entry(T.cgpatom), qp_test, qe_of;
+  std::vector<double> qw_d;
+  std::vector<float> qw_f;
   std::vector<uint64_t> gbit(ncgpat);
   for (int g = 0; g < s->ncgp; g++) {
     if (s->cgp_first[g] != (g == 0 ? 0 : s->cgp_last[g - 1] + 1) || s->cgp_last[g] < s->cgp_first[g])
@@ -292,13 +297,10 @@ int topo_build(DevSys& S, const qnb_system* s, HostTopo& T, DevAlloc& M) {
   UP(gswitch, s->cgp_iswitch, s->ncgp);
   UP(cgpatom, s->cgpatom, ncgpat);
   UP(atom_group, atom_group.data(), nat);
-  UP(gbit, gbit.data(), ncgpat);
-  {
-    std::vector<int> entry(T.cgpatom);
-    for (int& e : entry)
-      if (s->iqatom[e] != 0) e |= AL_SKIP;
-    UP(cgentry, entry.data(), entry.size());
-  }
+  pack.add(&S.gbit, gbit.data(), ncgpat);
+  for (int& e : entry)
+    if (s->iqatom[e] != 0) e |= AL_SKIP;
+  pack.add(&S.cgentry, entry.data(), entry.size());
   T.n_group_atoms = s->ncgp_solute > 0 ? s->cgp_last[s->ncgp_solute - 1] + 1 : 0;
   for (int g = 0; g < s->ncgp_solute; g++)
     T.max_group = std::max(T.max_group, s->cgp_last[g] - s->cgp_first[g] + 1);
@@ -374,12 +376,12 @@ int topo_build(DevSys& S, const qnb_system* s, HostTopo& T, DevAlloc& M) {
     }
   }
   UP(qconn3, T.qconn3.data(), T.qconn3.size());
-  std::vector<int> qp_test(nsol1, -1);
+  qp_test.assign(nsol1, -1);
   for (int i = 0; i < nsol; i++) {
     const int g = atom_group[i];
     if (!T.qconn3[i] && g >= 0 && !s->excl[s->cgp_iswitch[g]]) qp_test[i] = s->cgp_iswitch[g];
   }
-  UP(qp_test, qp_test.data(), qp_test.size());
+  pack.add(&S.qp_test, qp_test.data(), qp_test.size());
   if (nq > 0) {
     UP(iqseq, s->iqseq, nq);
     if (nsol > 0) {
@@ -404,21 +406,21 @@ int topo_build(DevSys& S, const qnb_system* s, HostTopo& T, DevAlloc& M) {
       UP(qwB, s->qw_B, n);
       UP(qwEl, s->qw_el, n);
       UP(qwSc, s->qw_sc, n);
-      std::vector<double> pd(4 * n);
+      qw_d.resize(4 * n);
       for (int iq = 0; iq < nq; iq++)
         for (int k = 0; k < sa; k++)
           for (int st = 0; st < ns; st++) {
             const size_t a = (size_t)iq + nq * ((size_t)k + (size_t)sa * st), b = 4 * ((size_t)(iq * sa + k) * ns + st);
-            pd[b] = s->qw_A[a];
-            pd[b + 1] = s->qw_B[a];
-            pd[b + 2] = s->qw_el[a];
-            pd[b + 3] = s->qw_sc[a];
+            qw_d[b] = s->qw_A[a];
+            qw_d[b + 1] = s->qw_B[a];
+            qw_d[b + 2] = s->qw_el[a];
+            qw_d[b + 3] = s->qw_sc[a];
           }
       if (S.prec == QNB_PREC_MIXED) {
-        const std::vector<float> pf(pd.begin(), pd.end());
-        UP(qw_f, pf.data(), pf.size());
+        qw_f.assign(qw_d.begin(), qw_d.end());
+        pack.add(&S.qw_f, qw_f.data(), qw_f.size());
       } else {
-        UP(qw_d, pd.data(), pd.size());
+        pack.add(&S.qw_d, qw_d.data(), qw_d.size());
       }
     }
     S.nqq = (int)qq_iq.size();
@@ -474,28 +476,28 @@ int topo_build(DevSys& S, const qnb_system* s, HostTopo& T, DevAlloc& M) {
     UP(qe_atom, ent_atom.data(), ent_atom.size());
     UP(qe_off, off.data(), off.size());
     UP(qe_item, item.data(), item.size());
-    std::vector<int> qe_of(nsol1, -1);
+    qe_of.assign(nsol1, -1);
     for (int e = 0; e < nent; e++) qe_of[ent_atom[e]] = e;
-    UP(qe_of, qe_of.data(), qe_of.size());
+    pack.add(&S.qe_of, qe_of.data(), qe_of.size());
   }
 #undef UP
-  return 0;
+  if (int rc2 = pack.alloc(M)) return rc2;
+  return pack.copy();
 }
 
-// Half as many again as the longest row seen and ten groups' worth (neighbour
-// rows get the same half and 64 groups), and no less than a cut-off sphere full
-// of solute: 0.1 atoms per A^3 out to 2 A beyond the cut-off, and a fifth of
-// them for the padding.  At most what any row of S.cap groups can hold: of two
+// Half as many again as the longest row seen and 64, and no less than a cut-off
+// sphere full of solute: 0.1 atoms per A^3 out to 2 A beyond the cut-off, and a
+// fifth of them for the padding.  At most what any row of S.cap groups can hold: of two
 // batches in a row the first ends because the next group would pass
 // al_batch >= 128 slots, or holds 64 groups, so batches hold 64 atoms on average
 // and their padding (at most 63 slots each, one batch more at the end) at most
 // doubles the row.  For 4,000 solute atoms and 2,687 groups with rows of up to
-// 576 slots: 1,504 slots, 16 MB; rows that hold any S.cap groups took 8,064, 87 MB.
+// 576 slots: 960 slots, 10 MB; rows that hold any S.cap groups took 8,064, 87 MB.
 int atom_row_slots(const DevSys& S, const HostTopo& T, int longest) {
   const long atoms = std::min((long)T.n_group_atoms, (long)S.cap * T.max_group), most = 2 * atoms + 64;
   const double r = std::sqrt(std::max(S.rcpp2, S.rcpw2)) + 2.0;
   const double sphere = std::min(0.5 * r * r * r + 64.0, (double)most);
-  const long seen = longest > 0 ? longest + longest / 2 + 640l : 0l;
+  const long seen = longest > 0 ? longest + longest / 2 + 64l : 0l;
   return (int)((std::min(most, std::max(seen, (long)sphere)) + 63) / 64 * 64);
 }
 
@@ -516,54 +518,52 @@ int row_alloc(DevSys& S, DevAlloc& M, int cap) {
 }
 
 int instance_alloc(DevSys& S, DevAlloc& M, const qnb_params* p, int nslots) {
-  // one allocation for all of the instance's buffers but the rows, which are
-  // sized and resized on their own
-  std::vector<std::pair<void**, size_t>> want;
-  size_t total = 0;
-  auto add = [&](auto** field, size_t n) {
-    want.push_back({(void**)field, total});
-    total += (std::max(n, (size_t)1) * sizeof(**field) + 255) & ~(size_t)255;
-  };
-#define AL(field, n) add(&S.field, (size_t)(n))
+  int rc = 0;
   const int nat = S.natom, nsol1 = std::max(S.nat_solute, 1), nw1 = std::max(S.nwat, 1);
-  AL(x, 3 * nat);
+  S.nslots = nslots;
   S.xqg = nullptr;
   S.xqgd = nullptr;
+#define AL(field, n)                                      \
+  do {                                                    \
+    if ((rc = M.alloc(&S.field, (size_t)(n)))) return rc; \
+  } while (0)
+  AL(x, 3 * nat);
   if (p->precision == QNB_PREC_MIXED) AL(xqg, 4 * (size_t)S.ncgpat);
   else AL(xqgd, 4 * (size_t)S.ncgpat);
   AL(gref, 4 * (size_t)S.ncgp);
   AL(d, 3 * nat);
-  AL(dq, 3 * (size_t)S.nqat);
   AL(dqq, 3 * (size_t)S.nqe);
   AL(lrf, (size_t)QNB_NLRF * S.ncgp);
-  AL(alist_n, S.ncgp);
-  AL(nnbr, S.ncgp);
-  AL(nnsol, S.ncgp);
   AL(pw_first, S.ncgp_solute);
-  AL(need, 2);
-  AL(qw_in, nw1);
-  AL(qp_in, S.ncgp_solute);
   AL(qw_list, nw1);
   AL(qp_list, nsol1);
-  AL(nq_lists, 2);
-  S.nslots = nslots;
   AL(epart, (size_t)QNB_NE * nslots);
   AL(ered_part, (size_t)QNB_NE * QNB_RED_BLOCKS);
-  AL(ered, QNB_NE);
   AL(eatom, 2 * (size_t)nat);
-  AL(sh_state, 3 * QNB_MAXSH);
   AL(w_theta, nw1);
   AL(w_shell, nw1);
   AL(sh_list, (size_t)QNB_MAXSH * nw1);
   AL(sh_lth, (size_t)QNB_MAXSH * nw1);
-  AL(sh_n, QNB_MAXSH);
   AL(wp_rank, 2 * (size_t)QNB_MAXSH * nw1);
 #undef AL
-  unsigned char* base = nullptr;
-  if (int rc = M.alloc(&base, total)) return rc;
-  for (auto& w : want) *w.first = base + w.second;
-  // counts, flags, energies and the Q-atom rows start at zero
-  HIPCHK(hipMemset(base, 0, total));
+  // what starts at zero (counts, flags, energies, the Q-atom rows), small all of
+  // it, is one allocation and one fill; one allocation for everything would be
+  // megabytes, which the driver maps anew each time (22 us a call on average over
+  // a batch's creation, 2.5 us below that)
+  DevPack zero;
+  zero.space(&S.dq, 3 * (size_t)S.nqat);
+  zero.space(&S.alist_n, S.ncgp);
+  zero.space(&S.nnbr, S.ncgp);
+  zero.space(&S.nnsol, S.ncgp);
+  zero.space(&S.need, 2);
+  zero.space(&S.qw_in, nw1);
+  zero.space(&S.qp_in, S.ncgp_solute);
+  zero.space(&S.nq_lists, 2);
+  zero.space(&S.ered, QNB_NE);
+  zero.space(&S.sh_state, 3 * QNB_MAXSH);
+  zero.space(&S.sh_n, QNB_MAXSH);
+  if ((rc = zero.alloc(M))) return rc;
+  HIPCHK(hipMemset(zero.base, 0, zero.bytes));
   double sh0[3 * QNB_MAXSH] = {0};
   for (int k = 0; k < S.nshell; k++) sh0[k] = p->wshell_theta_corr[k];
   HIPCHK(hipMemcpy(S.sh_state, sh0, sizeof sh0, hipMemcpyHostToDevice));

@@ -891,12 +891,7 @@ extern "C" int32_t qnb_batch_create(int32_t n, const qnb_system* const* sys, con
       M.ndegf = 3.0 * S.natom - 3.0 * S.nwat;
       M.ndegfree = (double)(long long)(M.ndegf - 3.0 * (nex[0] + nex[1]) + (exsh[0] + exsh[1]));
     }
-    if ((rc = b->mem.upload(&M.winv, m->winv, S.natom)) ||
-        (rc = b->mem.alloc(&M.v, 3 * (size_t)S.natom)) || (rc = b->mem.alloc(&M.xx, 3 * (size_t)S.natom)) ||
-        (rc = b->mem.alloc(&M.hist, (size_t)std::max(m->max_frames, 1) * QNB_FRAME_LEN)) ||
-        (rc = b->mem.alloc(&M.st, 8)))
-      return rc;
-    // atom-centred incidence lists of the bonds and angles (k_bonded)
+    // atom-centred records of the bonds and angles (bonded_atom)
     if (m->nbonds < 0 || m->nangles < 0 || (m->nbonds > 0 && (!m->bond_ij || !m->bond_r0 || !m->bond_k)) ||
         (m->nangles > 0 && (!m->angle_ijk || !m->angle_t0 || !m->angle_k)))
       return fail(QNB_EINVAL, "instance %d: bad bond/angle arrays", k);
@@ -931,19 +926,25 @@ extern "C" int32_t qnb_batch_create(int32_t n, const qnb_system* const* sys, con
           arec[apos[p[role]]++] = AngleRec{role, p[role == 0 ? 1 : 0], p[role == 2 ? 1 : 2], 0, m->angle_t0[q], m->angle_k[q]};
       }
       S.nbat = nbat;
-      if ((rc = b->mem.upload(&S.boff, boff.data(), boff.size())) ||
-          (rc = b->mem.upload(&S.brec, brec.data(), brec.size())) ||
-          (rc = b->mem.upload(&S.aoff, aoff.data(), aoff.size())) ||
-          (rc = b->mem.upload(&S.arec, arec.data(), arec.size())) ||
-          (rc = b->mem.alloc(&S.brow, 3 * (size_t)std::max(nbat, 1))))
-        return rc;
       b->nbblk = std::max(b->nbblk, (nbat + 255) / 256);
       b->nbat_max = std::max(b->nbat_max, nbat);
       const int nib = (S.nwat + S.nat_solute + 255) / 256;
-      if ((rc = b->mem.alloc(&M.tpart, 4 * (size_t)std::max(nib, 1)))) return rc;
+      const double st0[8] = {0};
+      DevPack pack;
+      pack.add(&S.boff, boff.data(), boff.size());
+      pack.add(&S.brec, brec.data(), brec.size());
+      pack.add(&S.aoff, aoff.data(), aoff.size());
+      pack.add(&S.arec, arec.data(), arec.size());
+      pack.add(&M.winv, (const double*)m->winv, S.natom);
+      pack.add((const double**)&M.st, st0, 8);
+      if ((rc = pack.alloc(b->mem)) || (rc = pack.copy()) || (rc = b->mem.alloc(&M.v, 3 * (size_t)S.natom)) ||
+          (rc = b->mem.alloc(&M.xx, 3 * (size_t)S.natom)) ||
+          (rc = b->mem.alloc(&M.hist, (size_t)std::max(m->max_frames, 1) * QNB_FRAME_LEN)) ||
+          (rc = b->mem.alloc(&M.tpart, 4 * (size_t)std::max(nib, 1))) ||
+          (rc = b->mem.alloc(&S.brow, 3 * (size_t)std::max(nbat, 1))))
+        return rc;
     }
     HIPCHK(hipMemcpy(M.v, v0[k], sizeof(double) * 3 * S.natom, hipMemcpyHostToDevice));
-    HIPCHK(hipMemset(M.st, 0, 8 * sizeof(double)));
     M.ctr = b->ctr + CTR_STRIDE * k;
     M.tfree = b->tfree + k;
     M.istep = b->istep + k;
@@ -1000,33 +1001,27 @@ extern "C" int32_t qnb_batch_create(int32_t n, const qnb_system* const* sys, con
     if (!again) break;
     if (attempt > 3) return fail(QNB_EOVERFLOW, "neighbour list capacity");
   }
+  // neighbour rows of the size needed and partner-atom rows, both in the space of
+  // the first build's rows where it holds them (mapping 16 MB anew took half a
+  // millisecond per 30 A window); rebuilt below
   for (int k = 0; k < n; k++) {
     DevSys& S = b->hs[k];
     std::vector<int> nn(S.ncgp);
     HIPCHK(hipMemcpy(nn.data(), S.nnbr, sizeof(int) * S.ncgp, hipMemcpyDeviceToHost));
     int mx = 0;
     for (int v : nn) mx = std::max(mx, v);
-    const int cap = ((mx * 3 / 2 + 64) + 63) / 64 * 64;
-    if (cap < S.cap) {
-      // shrink: rebuild happens at the first step of the run
-      if ((rc = row_alloc(S, b->mem, cap))) return rc;
+    const int first = S.cap, cap = std::min(first, ((mx * 3 / 2 + 64) + 63) / 64 * 64);
+    S.cap = cap;
+    const int slot = atom_row_slots(S, *b->topos[b->topo_of[k]], slots[k]);
+    if (cap + slot <= first) {
+      S.alist = S.nbr;
+      S.acap = first - cap;
+      S.nbr += (size_t)S.acap * S.ncgp;
+    } else {
+      if (cap < first && (rc = row_alloc(S, b->mem, cap))) return rc;
+      if ((rc = atom_rows_alloc(S, b->mem, slot))) return rc;
     }
     HIPCHK(hipMemset(S.need, 0, 2 * sizeof(int)));
-  }
-  // the partner-atom rows of all instances in one allocation
-  {
-    size_t total = 0;
-    for (int k = 0; k < n; k++) {
-      DevSys& S = b->hs[k];
-      S.acap = atom_row_slots(S, *b->topos[b->topo_of[k]], slots[k]);
-      total += (size_t)S.acap * S.atom_rows;
-    }
-    int* rows = nullptr;
-    if ((rc = b->mem.alloc(&rows, total))) return rc;
-    for (int k = 0; k < n; k++) {
-      b->hs[k].alist = rows;
-      rows += (size_t)b->hs[k].acap * b->hs[k].atom_rows;
-    }
   }
   HIPCHK(hipMemcpy(b->dsys, b->hs.data(), sizeof(DevSys) * n, hipMemcpyHostToDevice));
   {

@@ -1,12 +1,13 @@
 """Partner-atom rows of the receivers: their memory and their growth.
 
 * Memory: a batch's rows follow the longest row of its systems (half as many
-  slots again and 640 more), not the solute's size times the number of groups.
-  1,500 solute atoms in 150 ten-atom groups at a cut-off of 7 A: the longest row
-  holds 110 atoms, 192 slots with its padding, so 928 slots of 4 bytes for each
-  of the 2,166 groups, 8 MB, and at most 7 MB for everything else of an instance
-  (44 numbers per group and 65 per atom, of 8 bytes, and neighbour rows of 320
-  groups); rows for all solute atoms would take 26.5 MB.
+  slots again, or a cut-off sphere of solute), not the solute's size times the
+  number of groups.  1,500 solute atoms in 150 ten-atom groups at a cut-off of
+  7 A: the longest row holds 110 atoms, so its rows and the neighbour rows fit
+  the 1,024 numbers of 4 bytes that the first list build has for each of the
+  2,166 groups, 9 MB, and at most 7 MB are left for everything else of an
+  instance (44 numbers per group and 65 per atom, of 8 bytes); rows for all
+  solute atoms alone would take 26.5 MB.
 * Growth: rows longer than the slots an engine starts with (a cut-off sphere of
   solute, 256 slots at 5.2 A; two groups of 140 atoms take 320; seed 1 has such
   rows, seed 2 none), against the oracle with the bounds of test_gpu_shapes,
