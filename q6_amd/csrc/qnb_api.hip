@@ -540,8 +540,6 @@ int instance_alloc(DevSys& S, DevAlloc& M, const qnb_params* p, int nslots) {
   AL(epart, (size_t)QNB_NE * nslots);
   AL(ered_part, (size_t)QNB_NE * QNB_RED_BLOCKS);
   AL(eatom, 2 * (size_t)nat);
-  AL(w_theta, nw1);
-  AL(w_shell, nw1);
   AL(sh_list, (size_t)QNB_MAXSH * nw1);
   AL(sh_lth, (size_t)QNB_MAXSH * nw1);
   AL(wp_rank, 2 * (size_t)QNB_MAXSH * nw1);
@@ -622,7 +620,7 @@ struct qnb_handle {
   std::unique_ptr<DevAlloc> exc_mem;    // their lists, freed when the arrays are replaced
 };
 
-// host twin of the device pp_param filter, for list export
+// host twin of the device solute-solute filter (pp_pair), for list export
 bool qnb::host_pp_param(const HostTopo& T, int i, int j) {
   int lo = std::min(i, j), hi = std::max(i, j), dk = hi - lo;
   bool is14 = false;

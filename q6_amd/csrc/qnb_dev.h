@@ -196,8 +196,6 @@ struct DevSys {
   double* eatom;    // [natom][2]: per-atom LRF and radial-restraint energies
   // polarisation restraint state
   double* sh_state;  // [3*QNB_MAXSH]: theta_corr, avtheta, avn_insh
-  double* w_theta;   // [nwat]
-  int* w_shell;      // [nwat]
   int* sh_list;      // [QNB_MAXSH][nwat] members of each shell
   double* sh_lth;    // [QNB_MAXSH][nwat] their theta
   int* sh_n;         // [QNB_MAXSH] members per shell
@@ -857,45 +855,6 @@ __device__ __forceinline__ bool qp_group_in(const DevSys& S, const double* __res
   return false;
 }
 
-// Solute-solute pair parameters computed from atom data exactly as
-// pp_int_comp / precompute_set_values_pp (simprep.f90:2952-3065, 3321-3350)
-// would tabulate them.  Returns false when the pair does not interact.
-__device__ __forceinline__ bool pp_param(const DevSys& S, int i, int j, double& A, double& B, double& el) {
-  int lo = i < j ? i : j, hi = i < j ? j : i, dk = hi - lo;
-  bool is14 = false;
-  if (dk <= 25) {
-    uint32_t bit = 1u << (dk - 1);
-    if (ldg(S.exmask + lo) & bit) return false;
-    is14 = (ldg(S.m14mask + lo) & bit) != 0;
-  } else {
-    bool ex = false;
-    for (int m = ldg(S.lx_off + lo); m < ldg(S.lx_off + (lo + 1)); m++)
-      if (ldg(S.lx_j + m) == hi) {
-        if (ldg(S.lx_kind + m) == 0) ex = true;
-        else is14 = true;
-      }
-    if (ex) return false;
-  }
-  int ti = ldg(S.iac + i), tj = ldg(S.iac + j);
-  int vdw = is14 ? 3 : ldg(S.ljcod + (ti + tj * S.ntypes));
-  int k = vdw - 1;
-  if (S.ivdw_rule == 1) {
-    A = ldg(S.avdw + (ti * 3 + k)) * ldg(S.avdw + (tj * 3 + k));
-    B = ldg(S.bvdw + (ti * 3 + k)) * ldg(S.bvdw + (tj * 3 + k));
-  } else {
-    double tA = ldg(S.avdw + (ti * 3 + k)) + ldg(S.avdw + (tj * 3 + k));
-    tA = tA * tA;
-    tA = tA * tA * tA;
-    double tB = ldg(S.bvdw + (ti * 3 + k)) * ldg(S.bvdw + (tj * 3 + k));
-    A = (tA * tA) * tB;
-    B = 2.0 * tA * tB;
-  }
-  el = ldg(S.crg + i) * ldg(S.crg + j);
-  bool set = fabs(A) > 1.0e-10 || fabs(B) > 1.0e-10 || fabs(el) > 1.0e-10;
-  if (vdw == 3) el = el * S.el14;
-  return set;
-}
-
 // 1/|u|^2 and 1/|u| from |u|^2.  FP32: the hardware reciprocal square root
 // (v_rsq_f32, 1 ulp), the usual pair-kernel form.  FP64: the hardware's
 // reciprocal root (about 26 bits) with one third-order step,
@@ -1057,13 +1016,6 @@ __device__ __forceinline__ bool map_block(int imap, int nb, int ninst, int& inst
   inst = (int)(g / nb);
   blk = (int)(g % nb);
   return true;
-}
-
-// largest solute charge group of a system (gfirst/glast span)
-inline int max_solute_group(const int* gfirst, const int* glast, int ncgp_solute) {
-  int m = 0;
-  for (int g = 0; g < ncgp_solute; g++) m = glast[g] - gfirst[g] + 1 > m ? glast[g] - gfirst[g] + 1 : m;
-  return m;
 }
 
 // Adjoint of the per-state Q-atom energies over a set of frames: tangent

@@ -115,7 +115,7 @@ int validate_system(const qnb_system* s, const qnb_params* p);
 void fill_params(DevSys& S, const qnb_system* s, const qnb_params* p);
 // derived tables and device copies of the topology (shareable by instances)
 int topo_build(DevSys& S, const qnb_system* s, HostTopo& T, DevAlloc& M);
-// host twin of the device solute-solute filter (pp_param), for list export
+// host twin of the device solute-solute filter (pp_pair), for list export
 bool host_pp_param(const HostTopo& T, int i, int j);
 // the list sweep over `groups` receivers of B systems, wpb of them per block; any:
 // some system takes any atom pair for its group tests, lrf: some system wants

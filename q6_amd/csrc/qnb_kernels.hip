@@ -619,12 +619,9 @@ enum : uint32_t { T_WW = QNB_T_WW, T_QW = QNB_T_QW, T_PW = QNB_T_PW, T_PP = QNB_
 // Pair forms: water-water as nonbond_ww_spc / nonbond_ww
 // (nonbondene.f90:5886-5975, 5509-5573: O-O LJ + Coulomb, the other 8
 // Coulomb only for SPC), pw from the pw table (nonbond_pw 4856-4916), pp from
-// pp_param (nonbond_pp 4694-4760).  Writes (not adds) d for every atom of a,
+// pp_pair (nonbond_pp 4694-4760).  Writes (not adds) d for every atom of a,
 // and the wave's energy partials into epart[a] on the sampled steps.
 
-// pp_param from data at hand: the two atoms' types, charges and exclusion
-// masks (bit 31: partners beyond the 25-atom window, looked up in the long
-// list).  Same result as pp_param.
 // the pair (lo, hi) in lo's long exclusion / 1-4 list: 1 excluded, 2 1-4,
 // 0 neither (kept out of line: rare, and its loop would stop the callers'
 // receiver-atom loops from unrolling)
@@ -652,6 +649,10 @@ __device__ __forceinline__ int pair_kind(const DevSys& S, int i, uint32_t xi, ui
   return (xm >> 31) ? long_pair_kind(S, il ? i : j, il ? j : i) : 0;
 }
 
+// Solute-solute pair parameters from the two atoms' types, charges and exclusion
+// masks (bit 31: partners beyond the 25-atom window, looked up in the long
+// list), as pp_int_comp / precompute_set_values_pp (simprep.f90:2952-3065,
+// 3321-3350) would tabulate them; false: the pair does not interact.
 struct PPAtom {
   int i, t;
   uint32_t xm, m14;
@@ -764,8 +765,8 @@ __device__ __forceinline__ R qw_el(const DevSys& S, int iq, int k, int s) {
 //    nonbondene.f90:4694-4760): those of a group without an excluded or 1-4
 //    pair (AL_FAR) take A, B and qq as products of per-atom factors when the
 //    system uses the geometric rule with LJ code 1 throughout (ppfast): the
-//    products pp_param forms for such a pair, same operands; every other pair
-//    goes through the exclusion masks and pp_param's rules;
+//    products pp_pair forms for such a pair, same operands; every other pair
+//    goes through the exclusion masks and pp_pair's rules;
 //  * partner waters with the fixed mapping of k_wforces (lane l takes site
 //    l % 3 of water l / 3 of the round; nonbond_pw 4856-4916);
 //  * the pairs inside the group (ig == jgr, i < j, nonbondene.f90:1610) and
@@ -896,7 +897,7 @@ __device__ __forceinline__ void solute_receiver(const DevSys& S, uint32_t mask, 
       rQ[k] = lane_get(fc, k);
       f[k][0] = f[k][1] = f[k][2] = R(0);
     }
-    // A, B and qq of sweep atom k with atom j (pp_param); false: no pair
+    // A, B and qq of sweep atom k with atom j (pp_pair); false: no pair
     auto general = [&](int k, int i, int j, const double* qf, double qc, uint32_t qx, uint32_t qm, R& A, R& B,
                        R& el) {
       double Ad, Bd, eld;
@@ -967,7 +968,7 @@ __device__ __forceinline__ void solute_receiver(const DevSys& S, uint32_t mask, 
           if (ri[k] < 0) continue;
           R A = rA[k] * qA, B = rB[k] * qB, el = rQ[k] * qQ;
           if (far) {
-            // pp_param's `set` test (QREAL_EPS, src/sizes.f90:50); in FP32
+            // pp_pair's `set` test (QREAL_EPS, src/sizes.f90:50); in FP32
             // a pair of zero parameters adds exactly zero, so it is skipped
             // only on the FP64 path
             if constexpr (sizeof(R) == 8)
@@ -1830,8 +1831,6 @@ __device__ __forceinline__ void watpol_theta(const DevSys& S, int blk, int step)
       sh = is;
     }
   }
-  stg(S.w_theta + w, th);
-  stg(S.w_shell + w, sh);
   // append to the shell lists with one atomic per (wave, shell): the lanes of
   // a shell take consecutive places (ranks are counted by (theta, water index),
   // so the order of appending does not matter)
