@@ -60,8 +60,8 @@ void launch_bonded_rows(hipStream_t st, int bonded_atoms, int B, const DevSys* d
 // streams against that one: 74 and 55 us at 6,700 waves, 79 and 63 at 8,900, 87
 // and 81 at 7,900 with 800 solute groups (FP64: 104 and 92); at 11,900 with
 // 1,200 solute groups 103 and 106 (FP64: 125 and 122), where the four-way split
-// of a solute group costs what the launches save.  One evaluation at 6,500
-// waves: 260 and 202 us.
+// of a solute group costs what the launches save in FP32 and almost that in
+// FP64; one bound serves both.  One evaluation at 6,500 waves: 260 and 202 us.
 bool small_launch(long solute_groups, long solvent) { return 4 * solute_groups + solvent <= 10240; }
 
 __global__ void k_reduce_part(const DevSys*);

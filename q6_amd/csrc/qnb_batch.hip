@@ -648,8 +648,6 @@ static void launch_qforces(qnb_batch* b) {
 #undef QNB_LQ
 }
 
-// atom_terms = false: the caller runs the per-atom terms itself (the MD step
-// fuses them with the bonded terms in k_atom_step)
 // The MD step's force pass on two streams: the Q-atom side (first: its few
 // blocks start beside the solute receivers), the water receivers and the
 // polarisation restraint on the side stream, the solute receivers and the
@@ -1497,7 +1495,8 @@ extern "C" int32_t qnb_batch_minimize(qnb_batch* b, int32_t nsteps, double max_d
 
 // Autotuner: times the list/LRF sweep and the force kernel on the live batch
 // for 1, 2, 4 and 8 receiver groups (wavefronts) per block and keeps the
-// fastest shape of each.  Both kernels recompute their outputs from the
+// fastest shape of each (a step small enough for one force launch has a fixed
+// shape; its minimiser takes the one picked here).  Both kernels recompute their outputs from the
 // current coordinates, so the trials leave the state unchanged.
 extern "C" int32_t qnb_batch_autotune(qnb_batch* b, int32_t reps, int32_t* wpb_out) {
   if (!b || reps <= 0) return fail(QNB_EINVAL, "bad arguments");

@@ -158,8 +158,8 @@ struct DevSys {
   float* xqg;
   double* xqgd;
   // [ncgp][4] per group, packed with them: its reference atom's position
-  // (switch atom of a solute group, oxygen of a water) and 1 if that atom is
-  // excluded, else 0
+  // (switch atom of a solute group, oxygen of a water) and 0 if that atom is
+  // excluded, else 1
   double* gref;
   double* d;
   // gradient rows of the Q-atom side [nqat][3] and of the Q-Q entities
@@ -988,8 +988,8 @@ struct SmallGrid {
 // of groups where every solute group fits in them, else FC_CAP
 enum : int { AL_ATOM = (1 << 28) - 1, AL_OWN = 1 << 28, AL_FAR = 1 << 29, AL_SKIP = 1 << 30 };
 #define AL_BATCH 128
-// Solute-receiver force kernel (k_sforces): receiver atoms per sweep, at most
-// as many as the scalar registers hold (6 values of R each), and per-wave LDS
+// Solute receivers (solute_receiver): atoms per sweep, whose values (an index and
+// 6 of R each) are the same in every lane, and per-wave LDS
 template <typename R>
 __host__ __device__ constexpr int so_ch() { return sizeof(R) == 4 ? 10 : 5; }
 template <typename R>

@@ -608,15 +608,14 @@ enum : uint32_t { T_WW = QNB_T_WW, T_QW = QNB_T_QW, T_PW = QNB_T_PW, T_PP = QNB_
                   T_SINT = QNB_T_SINT };
 
 // ---------------------------------------------------------------------------
-// Receiver-side forces: one wavefront per charge group a.  The wave expands
-// its neighbour row into partner atoms 64 groups at a time (a wave prefix sum
-// over the groups' atom counts, staged in LDS) and gives every lane one
-// partner atom at a time, so lanes stay balanced however the row mixes 3-atom
-// waters and larger solute groups.  A lane forms the partner's position
-// relative to the receiver's reference atom once in FP64, rounds it to R and
-// evaluates it against the receiver atoms (offsets from the same reference
-// point), accumulating per-lane forces in R; the wave reduces them in FP64.
-// Pair forms: water-water as nonbond_ww_spc / nonbond_ww
+// Receiver-side forces: one wavefront per charge group a (or four, see
+// solute_receiver) walks its partners, every lane one partner atom at a time:
+// solute partners from the receiver's atom list (expand_row), so lanes stay
+// balanced however large the groups are, waters from the neighbour row.  A lane
+// forms the partner's position relative to the receiver's reference atom once in
+// FP64, rounds it to R and evaluates it against the receiver atoms (offsets from
+// the same reference point), accumulating per-lane forces in R; the wave reduces
+// them in FP64.  Pair forms: water-water as nonbond_ww_spc / nonbond_ww
 // (nonbondene.f90:5886-5975, 5509-5573: O-O LJ + Coulomb, the other 8
 // Coulomb only for SPC), pw from the pw table (nonbond_pw 4856-4916), pp from
 // pp_pair (nonbond_pp 4694-4760).  Writes (not adds) d for every atom of a,
@@ -758,9 +757,11 @@ __device__ __forceinline__ R qw_el(const DevSys& S, int iq, int k, int s) {
 // ---------------------------------------------------------------------------
 // Solute receivers: one wavefront per solute charge group a, or, in a small
 // launch (SPLIT), the four waves of a block, each with a quarter of a's
-// partners.  a's atoms are taken in sweeps of up to SO_CH; they are the same
-// for every lane and live in scalar registers, and a lane takes one partner at
-// a time against them, the next partner's data in flight meanwhile:
+// partners.  a's atoms are taken in sweeps of up to so_ch; they are the same
+// for every lane and are read into scalar registers (70 values in FP32 beside the
+// pointers: about 116 words of them the compiler keeps in lanes of vector
+// registers and reads back), and a lane takes one partner at a time against
+// them, the next partner's data in flight meanwhile:
 //  * solute partners from the receiver's atom list (expand_row; nonbond_pp,
 //    nonbondene.f90:4694-4760): those of a group without an excluded or 1-4
 //    pair (AL_FAR) take A, B and qq as products of per-atom factors when the
@@ -1756,9 +1757,12 @@ __global__ __launch_bounds__(QQ_THREADS) void k_qq(const DevSys* __restrict__ sy
 
 // ---------------------------------------------------------------------------
 // SCAAS polarisation restraint (watpol, nonbondene.f90:6548-6746,
-// md = .true.): one block per system.  The reference's per-shell
-// selection sort by theta is a stable ascending sort; here each member's rank
-// is counted directly (ties broken by water index, as the selection sort does).
+// md = .true.): the angles and shells (watpol_theta), the ranks and forces
+// (pol_forces, blocks of 64 members of one shell), the per-shell sums
+// (watpol_finish).  The reference's per-shell selection sort by theta is a
+// stable ascending sort; here each member's rank is counted directly (ties
+// broken by water index, as the selection sort does).
+//
 // Dipole and radial directions of the molecule whose first atom is i
 // (nonbondene.f90:6572-6604): a 3-site solvent takes H1 + H2 - 2 O and the
 // radial vector of O; any other the charge-weighted sum of its positions
