@@ -205,7 +205,7 @@ int topo_build(DevSys& S, const qnb_system* s, HostTopo& T, DevAlloc& M) {
   // lays them out
   // per-atom tables of the force and list kernels that go up together
   DevPack pack;
-  std::vector<int> entry(T.cgpatom), qp_test, qe_of;
+  std::vector<int> entry(T.cgpatom), qp_test, qe_of, iq_of;
   std::vector<double> qw_d;
   std::vector<float> qw_f;
   std::vector<uint64_t> gbit(ncgpat);
@@ -384,6 +384,9 @@ int topo_build(DevSys& S, const qnb_system* s, HostTopo& T, DevAlloc& M) {
   pack.add(&S.qp_test, qp_test.data(), qp_test.size());
   if (nq > 0) {
     UP(iqseq, s->iqseq, nq);
+    iq_of.assign(nsol1, -1);
+    for (int iq = 0; iq < nq; iq++) iq_of[s->iqseq[iq]] = iq;
+    pack.add(&S.iq_of, iq_of.data(), iq_of.size());
     if (nsol > 0) {
       size_t n = (size_t)nsol * nq * ns;
       UP(qpA, s->qp_A, n);

@@ -108,6 +108,7 @@ struct DevSys {
   const int* sint_ij;
   const double* sint_par;
   const int* iqseq;
+  const int* iq_of;  // [nat_solute] the atom's place in iqseq, -1 where it has none
   const uint8_t* qconn3;
   // per solute atom: the switch atom that decides whether its group is on the
   // Q-solute list, or -1 where no group test can put it there (within two
@@ -644,9 +645,9 @@ enum { QROWS_SIDE = 1, QROWS_QQ = 2 };
 // adds atom i's rows to f; the Q-atom side's row is cleared for the next step
 __device__ __forceinline__ void add_qrows(const DevSys& S, int i, int rows, double* f) {
   if (rows == 0 || i >= S.nat_solute || S.nqat <= 0) return;
-  const int iq = (rows & QROWS_SIDE) ? ldg(S.iqatom + i) : 0;
-  if (iq > 0) {
-    const auto q = gpm(S.dq) + 3 * (iq - 1);
+  const int iq = (rows & QROWS_SIDE) ? ldg(S.iq_of + i) : -1;
+  if (iq >= 0) {
+    const auto q = gpm(S.dq) + 3 * iq;
     for (int c = 0; c < 3; c++) {
       f[c] += q[c];
       q[c] = 0.0;

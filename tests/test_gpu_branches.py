@@ -123,3 +123,22 @@ def test_unlike_systems_in_one_batch(every):
             xr, vr = alone[k % 5]
             assert np.max(np.abs(x - xr)) <= 1e-9, (copies, k)
             assert np.max(np.abs(v - vr)) <= 1e-7 * np.max(np.abs(vr)), (copies, k)
+
+
+def test_q_atoms_are_taken_from_iqseq():
+    """An evaluation takes the Q-atoms' places from iqseq; iqatom only says
+    which atoms they are (a caller may hold plain flags there)."""
+    from q6_amd.engine import NonbondedEngine
+    s = synth.build(14.0, 60, 5, 3, 4, seed=23, chain_region=7.0, q_sigma=0.4, lambdas=[0.1, 0.2, 0.3, 0.4], cut=7.0)
+    print(f"\n[gpu] {synth.describe(s)}: flags for Q-atom numbers", flush=True)
+    o = Oracle(s)
+    o.make_pair_lists(s.x)
+    do, Eo, EQo = o.eval_terms(abi.T_ALL, s.x, Tfree=300.0)
+    s.a["iqatom"] = (s.a["iqatom"] > 0).astype(np.int32)
+    eng = NonbondedEngine(s, precision=abi.QNB_PREC_FP64)
+    eng.make_pair_lists(s.x)
+    d, E, EQ = eng.eval_terms(abi.T_ALL, s.x, Tfree=300.0)
+    eng.close()
+    assert np.max(np.abs(d - do)) <= 1e-10 * np.max(np.abs(do))
+    e, eo = (np.array(list(a.values()) + [v for q in b for v in q.values()]) for a, b in ((E, EQ), (Eo, EQo)))
+    assert np.max(np.abs(e - eo)) <= 1e-10 * np.max(np.abs(eo))
