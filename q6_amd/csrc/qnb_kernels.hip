@@ -349,9 +349,9 @@ __device__ __forceinline__ void expand_row(const DevSys& S, int a, int nsr, int 
 // is summed, FP64 the next chunk's groups.  A record's group is
 // one bit of a 64-bit word, so a test is two ANDs and reads past the run find
 // 0; FP64 takes the sums raw too, with rinv_inner in place of a root and three
-// divisions.  Measured: 2,663 -> 2,270 us for 51 windows of 11,056 atoms
-// (FP32), 1,740 -> 870 us for 12 of them in FP64; a list update of 19,440 atoms
-// in FP64 775 -> 380 us.
+// divisions.  Measured, the partner-atom rows included: 2,620 -> 2,330 us for 51
+// windows of 11,056 atoms in FP32, 6,970 -> 3,420 us in FP64; 19,440 atoms in
+// FP64 710 -> 331 us.
 // LRF: for the systems that want the expansion, the others leave at once (and
 // the other way round): without it the sweep reads no records and has the next
 // chunk's groups in flight.  ANY reads a batch of records when it sums it: held
