@@ -305,6 +305,7 @@ int topo_build(DevSys& S, const qnb_system* s, HostTopo& T, DevAlloc& M) {
   for (int g = 0; g < s->ncgp_solute; g++)
     T.max_group = std::max(T.max_group, s->cgp_last[g] - s->cgp_first[g] + 1);
   S.al_batch = T.max_group <= AL_BATCH ? AL_BATCH : FC_CAP;
+  S.al_group = std::max((T.max_group + QNB_WAVE - 1) / QNB_WAVE, 1) * QNB_WAVE;
 
   UP(avdw, s->avdw, 3 * s->ntypes);
   UP(bvdw, s->bvdw, 3 * s->ntypes);
@@ -488,7 +489,8 @@ int topo_build(DevSys& S, const qnb_system* s, HostTopo& T, DevAlloc& M) {
   return pack.copy();
 }
 
-// Half as many again as the longest row seen and 64, and no less than a cut-off
+// Slots of the atom rows (a row may outgrow them, partner_row): half as many
+// again as the longest row seen and 64, and no less than a cut-off
 // sphere full of solute: 0.1 atoms per A^3 out to 2 A beyond the cut-off, and a
 // fifth of them for the padding.  At most what any row of S.cap groups can hold: of two
 // batches in a row the first ends because the next group would pass
@@ -553,7 +555,7 @@ int instance_alloc(DevSys& S, DevAlloc& M, const qnb_params* p, int nslots) {
   // a batch's creation, 2.5 us below that)
   DevPack zero;
   zero.space(&S.dq, 3 * (size_t)S.nqat);
-  zero.space(&S.alist_n, S.ncgp);
+  zero.space(&S.alist_end, 2 * (size_t)S.ncgp);
   zero.space(&S.nnbr, S.ncgp);
   zero.space(&S.nnsol, S.ncgp);
   zero.space(&S.need, 2);

@@ -177,7 +177,7 @@ __device__ __forceinline__ void thermo(const DevSys& S, const MdDev& M, int nblk
   thermo_update(M, ek, ekf);
   const double T = M.st[2];
   if (!isfinite(T) || !isfinite(S.ered[E_PP_EL] + S.ered[E_WW_EL])) atomicOr(&M.ctr[1], ERR_NONFINITE);
-  if (S.need[0] > S.cap || S.need[1] > S.acap) atomicOr(&M.ctr[1], ERR_OVERFLOW);
+  if (S.need[0] > S.cap) atomicOr(&M.ctr[1], ERR_OVERFLOW);
   M.ctr[3] = 0;
   *M.istep = *M.istep + 1;
 }
@@ -440,7 +440,7 @@ __global__ __launch_bounds__(256) void k_temperature(const DevSys* __restrict__ 
     thermo_update(M, ek, ekf);
     const double T = M.st[2];
     if (!isfinite(T) || !isfinite(S.ered[E_PP_EL] + S.ered[E_WW_EL])) atomicOr(&M.ctr[1], ERR_NONFINITE);
-    if (S.need[0] > S.cap || S.need[1] > S.acap) atomicOr(&M.ctr[1], ERR_OVERFLOW);
+    if (S.need[0] > S.cap) atomicOr(&M.ctr[1], ERR_OVERFLOW);
   }
 }
 

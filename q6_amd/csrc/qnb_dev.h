@@ -173,10 +173,11 @@ struct DevSys {
   int* nnbr;
   // partner atoms of receivers 0 .. atom_rows - 1 (expand_row; a solvent other
   // than 3-site water has none, solvent_receiver walks its groups): rows of acap
-  // slots, the slots in use [ncgp], slots per batch of groups
+  // slots; [ncgp][2] the slots in use and the groups they hold; slots per batch of
+  // groups; slots a group takes where a row was too short (partner_row)
   int* alist;
-  int* alist_n;
-  int acap, al_batch, atom_rows;
+  int* alist_end;
+  int acap, al_batch, al_group, atom_rows;
   int* nnsol;  // [ncgp] length of the row's solute prefix (rows are sorted)
   // reference test-point reuse of the LRF-off switch-atom solute-water list
   // (quirk bit 0 with use_lrf = 0): per solute group, the first water within

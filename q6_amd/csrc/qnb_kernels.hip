@@ -267,8 +267,10 @@ __device__ __forceinline__ double dist4v(const d4v& a, const d4v& b) {
 // The force kernels then read one coalesced list per receiver instead of
 // walking group -> atoms -> positions through LDS at every step.  A launch of
 // its own cost a list update 7 us.  A row longer than acap slots ends before
-// the batch that does not fit and its length goes to need[1] (as a neighbour
-// row's does to need[0]); with acap 0 the call only counts.
+// the batch that does not fit (alist_end: slots and groups stored) and its length
+// goes to need[1], as a neighbour row's does to need[0]; the force kernels take
+// the groups after it from the neighbour row (row_tail).  With acap 0 the call
+// only counts.
 #define LS_WPB 8  // waves per block of the list sweep at most
 __device__ __forceinline__ void expand_row(const DevSys& S, int a, int nsr, int lane, int w) {
   const int batch = S.al_batch;
@@ -279,7 +281,7 @@ __device__ __forceinline__ void expand_row(const DevSys& S, int a, int nsr, int 
   const bool along = a_sol && ldg(S.glong + a);
   const int alo = a_sol ? ldg(S.gspan + 2 * a) : 0, ahi = a_sol ? ldg(S.gspan + 2 * a + 1) : 0;
   __shared__ int s_incl[LS_WPB][QNB_WAVE], s_src[LS_WPB][QNB_WAVE], s_tag[LS_WPB][QNB_WAVE];
-  int n = 0, stored = 0;
+  int n = 0, stored = 0, groups = 0;
   for (int p0 = 0, ng = 0; p0 < nsr; p0 += ng) {
     const int p = p0 + lane;
     int f0 = 0, cnt = 0, tag = 0;
@@ -323,9 +325,11 @@ __device__ __forceinline__ void expand_row(const DevSys& S, int a, int nsr, int 
     }
     __builtin_amdgcn_wave_barrier();
     stored = n;
+    groups = p0 + ng;
   }
   if (lane == 0) {
-    S.alist_n[a] = stored;
+    S.alist_end[2 * a] = stored;
+    S.alist_end[2 * a + 1] = groups;
     if (n > acap) atomicMax(S.need + 1, n);
   }
 }
@@ -754,6 +758,34 @@ __device__ __forceinline__ R qw_el(const DevSys& S, int iq, int k, int s) {
   return ldg(qp_tab<R>(S.qw_d, S.qw_f) + 4 * ((size_t)(iq * S.sa + k) * S.nstates + s) + 2);
 }
 
+// A receiver's partner atoms as its force kernel reads them: `stored` slots of its
+// atom row, then, where the row was too short, al_group slots for each further
+// group, its atoms from the neighbour row.  `n` slots in all.
+struct PartnerRow {
+  const int* al;
+  int stored, groups, n;
+};
+__device__ __forceinline__ PartnerRow partner_row(const DevSys& S, int a, int nsr) {
+  PartnerRow r;
+  r.al = S.alist + (size_t)a * S.acap;
+  r.stored = uni(ldg(S.alist_end + 2 * a));
+  r.groups = uni(ldg(S.alist_end + 2 * a + 1));
+  r.n = r.stored + (nsr - r.groups) * S.al_group;
+  return r;
+}
+// slot q past the stored ones
+__device__ __forceinline__ int row_tail(const DevSys& S, int a, int groups, int q) {
+  const int p = groups + q / S.al_group, m = q % S.al_group;
+  const int b = ldg(S.nbr + (size_t)a * S.cap + p);
+  const int f0 = ldg(S.gfirst + b), cnt = ldg(S.glast + b) - f0 + 1;
+  return m < cnt ? ldg(S.cgentry + f0 + m) | (owns(a, b) ? AL_OWN : 0) : (int)AL_SKIP;
+}
+// out of line for the solute receivers: rare, and their loops call in any case
+// (long_pair_kind); a call would cost the water receivers two waves per SIMD
+__device__ __noinline__ int row_tail_call(const DevSys& S, int a, int groups, int q) {
+  return row_tail(S, a, groups, q);
+}
+
 // ---------------------------------------------------------------------------
 // Solute receivers: one wavefront per solute charge group a, or, in a small
 // launch (SPLIT), the four waves of a block, each with a quarter of a's
@@ -820,7 +852,6 @@ __device__ __forceinline__ void solute_receiver(const DevSys& S, uint32_t mask, 
   const auto d = gpm(S.d);
   const int nn = uni(min(ldg(S.nnbr + a), S.cap)), nsr = uni(min(ldg(S.nnsol + a), nn));
   const int* __restrict__ row = S.nbr + (size_t)a * S.cap;
-  const int* __restrict__ al = S.alist + (size_t)a * S.acap;
   const bool want_e = E && want_energies(S);
   const int nsol = S.nat_solute, sa = S.sa, ncs = S.ncgp_solute;
   const int ra = uni(ldg(S.gswitch + a));
@@ -835,7 +866,9 @@ __device__ __forceinline__ void solute_receiver(const DevSys& S, uint32_t mask, 
   const int nq = S.nqat, ns = S.nstates;
   const bool qin = (mask & T_QP) && nq > 0 && uni(ldg(S.qp_in + a));
   const bool pp = (mask & T_PP) && !aexcl;
-  const int nsl = pp ? uni(ldg(S.alist_n + a)) : 0;
+  PartnerRow partners = partner_row(S, a, nsr);
+  if (!pp) partners.stored = partners.n = 0;
+  const int nsl = partners.n;
   const bool pw = (mask & T_PW) && !aexcl && nsr < nn;
   // SPLIT: sets of waves with receiver atoms of their own (nset), the waves of
   // a set sharing the partners
@@ -844,7 +877,10 @@ __device__ __forceinline__ void solute_receiver(const DevSys& S, uint32_t mask, 
   // the first two rounds' entries are requested before the receiver's own
   // chain of loads
   const int t0 = lane + QNB_WAVE * part, ts = QNB_WAVE * parts;
-  auto entry = [&](int t) { return t < nsl ? ldg(al + t) : (int)AL_SKIP; };
+  auto entry = [&](int t) {
+    if (t < partners.stored) return ldg(partners.al + t);
+    return t < nsl ? row_tail_call(S, a, partners.groups, t - partners.stored) : (int)AL_SKIP;
+  };
   const int e0 = entry(t0), e1 = entry(t0 + ts);
   for (int cb = 0; cb < na; cb += nset * CH) {
     const int c0 = cb + set * CH, nk = max(0, min(CH, na - c0));
@@ -1203,8 +1239,9 @@ __device__ __forceinline__ void water_receiver(const DevSys& S, uint32_t mask, i
     // solute partners from the receiver's atom list, one per lane, the next
     // one's data in flight
     if (mask & T_PW) {
-      const int* __restrict__ al = S.alist + (size_t)a * S.acap;
-      const int n = uni(ldg(S.alist_n + a));
+      const PartnerRow partners = partner_row(S, a, nsr);
+      const int n = partners.stored;
+      const int* __restrict__ al = partners.al;
       int e = lane < n ? ldg(al + lane) : 0;
       int en = lane + QNB_WAVE < n ? ldg(al + lane + QNB_WAVE) : 0;
       double px = 0.0, py = 0.0, pz = 0.0;
@@ -1227,17 +1264,7 @@ __device__ __forceinline__ void water_receiver(const DevSys& S, uint32_t mask, i
           }
         }
       };
-      if (n > 0) fetch(e & AL_ATOM);
-      for (int t = lane; t < n; t += QNB_WAVE) {
-        const R dx = (R)(px - xr0), dy = (R)(py - xr1), dz = (R)(pz - xr2);
-        R pw[9];
-#pragma unroll
-        for (int k = 0; k < 9; k++) pw[k] = pl[k];
-        const int ec = e;
-        e = en;
-        fetch(e & AL_ATOM);
-        en = t + 2 * QNB_WAVE < n ? ldg(al + t + 2 * QNB_WAVE) : 0;
-        if (ec & AL_SKIP) continue;
+      auto pairs = [&](R dx, R dy, R dz, const R* pw) {
 #pragma unroll
         for (int k = 0; k < 3; k++) {
           const R ux = dx - o[k][0], uy = dy - o[k][1], uz = dz - o[k][2];
@@ -1250,6 +1277,25 @@ __device__ __forceinline__ void water_receiver(const DevSys& S, uint32_t mask, i
           f[k][1] += uy * dv;
           f[k][2] += uz * dv;
         }
+      };
+      if (n > 0) fetch(e & AL_ATOM);
+      for (int t = lane; t < n; t += QNB_WAVE) {
+        const R dx = (R)(px - xr0), dy = (R)(py - xr1), dz = (R)(pz - xr2);
+        R pw[9];
+#pragma unroll
+        for (int k = 0; k < 9; k++) pw[k] = pl[k];
+        const int ec = e;
+        e = en;
+        fetch(e & AL_ATOM);
+        en = t + 2 * QNB_WAVE < n ? ldg(al + t + 2 * QNB_WAVE) : 0;
+        if (!(ec & AL_SKIP)) pairs(dx, dy, dz, pw);
+      }
+      // groups that the row had no room for
+      for (int q = lane; q < partners.n - n; q += QNB_WAVE) {
+        const int ec = row_tail(S, a, partners.groups, q);
+        if (ec & AL_SKIP) continue;
+        fetch(ec & AL_ATOM);
+        pairs((R)(px - xr0), (R)(py - xr1), (R)(pz - xr2), pl);
       }
     }
     // partner waters: lane l takes atom kb = l % 3 of water (l / 3) of the round
