@@ -862,23 +862,24 @@ __device__ __forceinline__ bool qp_group_in(const DevSys& S, const double* __res
 // reciprocal root (about 26 bits) with one third-order step,
 // y (1 + e/2 + 3 e^2/8) with e = 1 - d2 y^2, and 1/d2 from its square with one
 // Newton step: 15 slots and no branch, a division and a root took about 32.
-// The steps turn the limits (d2 = 0: infinite, d2 = inf: 0) into NaN, so rinv
-// takes the hardware's value there, 5 slots; the LRF sweep, whose q/r^3 r^2 is
-// NaN at both limits in any case, does without (rinv_inner).
-__device__ __forceinline__ void rinv_inner(double d2, double& r2, double& r) {
+// At the limits (d2 = 0: y infinite; d2 = inf: y = 0) both steps' residuals are
+// 0 inf = NaN, and v_min_f64 takes its other operand then: 1, with which each
+// step leaves its limit as it is (a residual proper is about 0, and a NaN d2
+// still gives NaN through y).  That is 2 slots; the LRF sweep, whose
+// q/r^3 r^2 is NaN at both limits in any case, does without (rinv_inner).
+template <bool LIMITS>
+__device__ __forceinline__ void rinv_steps(double d2, double& r2, double& r) {
   const double y = __builtin_amdgcn_rsq(d2);
-  const double e = __builtin_fma(-d2 * y, y, 1.0);
+  double e = __builtin_fma(-d2 * y, y, 1.0);
+  if (LIMITS) e = __builtin_fmin(e, 1.0);
   r = __builtin_fma(y * e, __builtin_fma(0.375, e, 0.5), y);
   const double s = r * r;
-  r2 = __builtin_fma(s, __builtin_fma(-d2, s, 1.0), s);
+  double f = __builtin_fma(-d2, s, 1.0);
+  if (LIMITS) f = __builtin_fmin(f, 1.0);
+  r2 = __builtin_fma(s, f, s);
 }
-__device__ __forceinline__ void rinv(double d2, double& r2, double& r) {
-  rinv_inner(d2, r2, r);
-  const bool limit = __builtin_amdgcn_class(d2, 0x260);  // +0, -0, +inf
-  const double y = __builtin_amdgcn_rsq(d2);
-  r = limit ? y : r;
-  r2 = limit ? y : r2;
-}
+__device__ __forceinline__ void rinv_inner(double d2, double& r2, double& r) { rinv_steps<false>(d2, r2, r); }
+__device__ __forceinline__ void rinv(double d2, double& r2, double& r) { rinv_steps<true>(d2, r2, r); }
 __device__ __forceinline__ void rinv_inner(float d2, float& r2, float& r) {
   r = __builtin_amdgcn_rsqf(d2);
   r2 = r * r;
