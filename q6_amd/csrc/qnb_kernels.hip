@@ -791,7 +791,7 @@ __device__ __noinline__ int row_tail_call(const DevSys& S, int a, int groups, in
 // launch (SPLIT), the four waves of a block, each with a quarter of a's
 // partners.  a's atoms are taken in sweeps of up to so_ch; they are the same
 // for every lane and are read into scalar registers (70 values in FP32 beside the
-// pointers: about 116 words of them the compiler keeps in lanes of vector
+// pointers: about 118 words of them the compiler keeps in lanes of vector
 // registers and reads back), and a lane takes one partner at a time against
 // them, the next partner's data in flight meanwhile:
 //  * solute partners from the receiver's atom list (expand_row; nonbond_pp,
@@ -876,10 +876,11 @@ __device__ __forceinline__ void solute_receiver(const DevSys& S, uint32_t mask, 
   const int set = SPLIT ? wave / parts : 0, part = SPLIT ? wave % parts : 0;
   // the first two rounds' entries are requested before the receiver's own
   // chain of loads
-  const int t0 = lane + QNB_WAVE * part, ts = QNB_WAVE * parts;
+  // (every count of slots is a multiple of 64, so a round's place is the wave's)
+  const int t0 = QNB_WAVE * part, ts = QNB_WAVE * parts;
   auto entry = [&](int t) {
-    if (t < partners.stored) return ldg(partners.al + t);
-    return t < nsl ? row_tail_call(S, a, partners.groups, t - partners.stored) : (int)AL_SKIP;
+    if (t < partners.stored) return ldg(partners.al + t + lane);
+    return t < nsl ? row_tail_call(S, a, partners.groups, t + lane - partners.stored) : (int)AL_SKIP;
   };
   const int e0 = entry(t0), e1 = entry(t0 + ts);
   for (int cb = 0; cb < na; cb += nset * CH) {
