@@ -812,7 +812,7 @@ __device__ __noinline__ int row_tail_call(const DevSys& S, int a, int groups, in
 // in vector registers (167 of them, three waves per SIMD), took 213 us at 51
 // windows of 400 ten-atom groups and 52 us for one FP64 window; staging by
 // blocks of four waves 310 us at 51 windows (its barriers wait on four chains
-// of loads); from the atom lists it takes 151 us, and about 20
+// of loads); from the atom lists it takes 145 us, and about 20
 // us split four ways.
 
 __device__ __forceinline__ float lane_get(float v, int lane) {
